@@ -49,7 +49,24 @@ LinearProblem problem(const void* x, const void* w, const void* bias, void* y, l
     return p;
 }
 
-int attend(const mi_attn_block_args* a, const BlockDims& d, const void* q, const void* k, const void* v, void* o, int kv_len) {
+// What the attention launch of a block of these sizes may use to cut the key axis into pieces, whichever head count its
+// channels turn out to have.
+size_t split_bytes(int batch, int q_len, int kv_len, int inner) {
+    size_t most = 0;
+    if (q_len == 0 || kv_len == 0) return 0;
+    for (int hd = 8; hd <= inner; hd += 8) {
+        if (inner % hd || !sdpa_supported(MI_DTYPE_F16, hd)) continue;
+        SdpaDev p;
+        std::memset(&p, 0, sizeof(p));
+        p.B = batch; p.H = inner / hd; p.Lq = q_len; p.Lk = kv_len;
+        const size_t n = sdpa_split_scratch_bytes(p, MI_DTYPE_F16, hd);
+        most = n > most ? n : most;
+    }
+    return most;
+}
+
+// [scratch_used, scratch_bytes) of the caller's scratch is lent to the attention launch.
+int attend(const mi_attn_block_args* a, const BlockDims& d, const void* q, const void* k, const void* v, void* o, int kv_len, size_t scratch_used) {
     mi_sdpa_args s;
     std::memset(&s, 0, sizeof(s));
     s.struct_size = sizeof(s);
@@ -59,6 +76,8 @@ int attend(const mi_attn_block_args* a, const BlockDims& d, const void* q, const
     s.q_len = a->q_len; s.kv_len = kv_len;
     s.key_mask = a->key_mask; s.key_mask_batch_stride = a->key_mask_batch_stride;
     if (a->causal) { s.mask_mode = MI_MASK_CAUSAL; s.q_offset = kv_len - a->q_len; }
+    s.split_scratch = static_cast<char*>(a->scratch) + scratch_used;
+    s.split_scratch_bytes = a->scratch_bytes - scratch_used;
     s.stream = a->stream;
     return mi_sdpa_forward(&s);
 }
@@ -106,7 +125,7 @@ size_t mi_flash_attention_scratch_bytes(int32_t batch, int32_t q_len, int32_t kv
     if (batch <= 0 || q_len < 0 || kv_len < 0 || inner <= 0) return 0;
     const size_t q = mi::round_up(static_cast<size_t>(batch) * q_len * inner * 2);
     const size_t kv = mi::round_up(static_cast<size_t>(batch) * kv_len * inner * 2);
-    return 2 * q + (with_kv ? 2 * kv : 0);
+    return 2 * q + (with_kv ? 2 * kv : 0) + mi::round_up(mi::split_bytes(batch, q_len, kv_len, inner));
 }
 
 int mi_flash_attention_project_kv(const mi_attn_block_args* a) {
@@ -153,7 +172,7 @@ int mi_flash_attention_qkvo_forward(const mi_attn_block_args* a) {
         n = 3;
     }
     if (mi::launch_linear(b, n, a->dtype, st) != 0) return -1;
-    if (mi::attend(a, d, sq, sk, sv, sa, kv_len) != 0) return -1;
+    if (mi::attend(a, d, sq, sk, sv, sa, kv_len, need) != 0) return -1;
     std::memset(&b, 0, sizeof(b));
     b.p[0] = mi::problem(sa, a->wo, a->bo, a->out, d.q_rows, a->out_channels, a->inner, a->wo_scales);
     return mi::launch_linear(b, 1, a->dtype, st);
@@ -178,7 +197,7 @@ int mi_flash_attention_q_with_kv_cached_forward(const mi_attn_block_args* a) {
     std::memset(&b, 0, sizeof(b));
     b.p[0] = mi::problem(a->x, a->wq, a->bq, sq, d.q_rows, a->inner, a->channels, a->wq_scales);
     if (mi::launch_linear(b, 1, a->dtype, st) != 0) return -1;
-    if (mi::attend(a, d, sq, a->k, a->v, sa, a->kv_len) != 0) return -1;
+    if (mi::attend(a, d, sq, a->k, a->v, sa, a->kv_len, need) != 0) return -1;
     std::memset(&b, 0, sizeof(b));
     b.p[0] = mi::problem(sa, a->wo, a->bo, a->out, d.q_rows, a->out_channels, a->inner, a->wo_scales);
     return mi::launch_linear(b, 1, a->dtype, st);

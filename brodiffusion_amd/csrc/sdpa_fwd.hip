@@ -1305,6 +1305,7 @@ bool sdpa_supported(int dtype, int head_dim) {
 
 size_t sdpa_split_scratch_bytes(const SdpaDev& p, int dtype, int head_dim) {
     if (dtype != MI_DTYPE_BF16 && dtype != MI_DTYPE_F16) return 0;
+    if (sdpa_wide_head(head_dim)) return sdpa_wide_split_scratch_bytes(p, head_dim);
     const int n_cu = device_cu_count();
     if (head_dim == 72) return split_scratch_bytes_d<72>(p, n_cu);
     if (head_dim == 128) return split_scratch_bytes_d<128>(p, n_cu);

@@ -2,17 +2,28 @@
 // (src/vae.cpp:259-277: one head over all 512 channels of a 64 x 64 latent; src/vae_qwenimage.cpp:322-340: 384 channels),
 // through the same entry point as every other head dimension.
 //
-// At these widths the output accumulator of a query row (head_dim floats per lane pair) no longer fits the registers of one
-// wavefront, so the head dimension is dealt out to the four wavefronts of a work group instead of the query rows: all four
-// work on the SAME 32 query rows, wavefront w owns elements [w D/4, (w+1) D/4) of the head dimension. Per 64-key tile
-//   1. every wavefront multiplies its quarter of the contraction: a partial score tile (K Q^T over D/4 elements);
-//   2. the four partial tiles meet in LDS and every wavefront adds them in the same fixed order, so all four hold
-//      bit-identical scores and run the same online softmax (same reference, same denominator, same P);
-//   3. every wavefront multiplies P with its quarter of V's columns into its quarter of the output.
-// K and V tiles go through registers into padded LDS, single buffered: the operator runs once per image on a few thousand
-// tokens, so the kernel is written for clarity, not for the last microsecond. Masks work as everywhere (per-row visible
-// key interval, kv_valid_len, key mask); cached prefixes, logit bias, lse output, packed sequences and K rotated tile by
-// tile are not offered at these widths (K rotated into a scratch and Q rotated on load are).
+// Bound: MFMA (4 L^2 d FLOPs against 8 L d bytes). A work group is 4 wavefronts, one per SIMD, each with 32 query rows of its
+// own and all of the head dimension: at 512 the output accumulator of 32 rows is 256 registers per lane, the Q fragments
+// are 128, and one wavefront per SIMD may use 512. So no partial score ever leaves a wavefront (the earlier form dealt the
+// head dimension out to the wavefronts and summed four FP32 score tiles through LDS at every step: 240 TFLOP/s at 16384
+// tokens, 2.37 ms). The key axis goes in steps of 32: with rows of up to 1 KB two stages of K and two of V are 128 KB of LDS.
+//
+// With one wavefront per SIMD nothing but the wavefront itself can cover its softmax, so the step is one instruction
+// stream in which the two overlap: the MFMAs of S_{t+1} = K_{t+1} Q^T carry the exponentials of tile t between them
+// (elementwise: the softmax is taken relative to a reference that is raised only when a tile grows past it, see
+// softmax_tile_rel), then O^T += V_t^T P_t. The DMA of tiles K_{t+2} and V_{t+1} is dealt out under the first half, so it
+// has the rest of the step to land; one barrier per step.
+//   LDS: rows back to back as the DMA deposits them, 16-byte chunk c of row r at position c ^ f(r) within its group of 16
+//   chunks, f(r) = 4 (r % 4) + (r / 4) % 4: the K fragment reads (16 rows, one chunk column) and the V transpose reads
+//   (4 rows, one 64-byte window) are both free of bank conflicts.
+//
+// A query tile is 128 rows, so a VAE mid-block has 32 (64 x 64 latent) to 128 tiles for 256 compute units: the key axis is
+// cut into as many pieces as shorten the launch (wide_split), each leaving a normalised partial output and its softmax
+// statistics in the caller's scratch, merged in a fixed order by wide_combine_kernel.
+//
+// Masks work as everywhere (per-row visible key interval, kv_valid_len, key mask); cached prefixes, logit bias, lse output,
+// packed sequences and K rotated tile by tile are not offered at these widths (K rotated into a scratch and Q rotated on
+// load are).
 #include "sdpa_tiles.h"
 
 namespace mi {
@@ -21,178 +32,437 @@ namespace {
 using namespace sdpa;
 
 constexpr int kWideThreads = 256;
-constexpr int kWideRows = 32;     // query rows per work group
+constexpr int kWideRows = 128;    // query rows per work group, 32 per wavefront
+constexpr int kWideKeys = 32;     // key rows per step
 
 template <int D> struct WideGeo {
     using G = HeadGeo<D>;
-    static constexpr int DW = D / 4;                 // head-dim elements per wavefront
-    static constexpr int KCW = DW / 16;              // its 16-element contraction chunks
-    static constexpr int VBW = DW / 32;              // its 32-row blocks of O^T
-    static constexpr int EX_BYTES = 4 * 2 * 16 * 64 * 4;   // four partial score tiles (2 blocks x 16 registers x 64 lanes, FP32)
-    static constexpr int Q_BYTES = kWideRows * G::O_STRIDE;
-    // the K tile's space also takes the staged Q rows (before the key loop), the partial score tiles (after K has been
-    // read) and the staged output (after the loop)
-    static constexpr int A_BYTES = G::K_BYTES > EX_BYTES ? (G::K_BYTES > Q_BYTES ? G::K_BYTES : Q_BYTES) : (EX_BYTES > Q_BYTES ? EX_BYTES : Q_BYTES);
-    static constexpr int LDS_BYTES = A_BYTES + G::V_BYTES + kBN * 4;
-    static_assert(D % 128 == 0, "four wavefronts with whole 32-row blocks each");
+    static constexpr int ROWB = D * 2;                  // bytes per row in LDS
+    static constexpr int TILE = kWideKeys * ROWB;       // one operand stage
+    static constexpr int VOFF = 2 * TILE;               // the V stages follow the K stages
+    static constexpr int NDMA = TILE / 1024 / 4;        // DMA instructions per wavefront and operand tile
+    static constexpr int KC = D / 16;                   // 16-element contraction chunks of K Q^T
+    static constexpr int VB = D / 32;                   // 32-row blocks of O^T
+    static constexpr int STAGED = kWideRows * G::O_STRIDE;   // the staged Q tile, later the staged output, over the rings
+    static constexpr int LDS_BYTES = 4 * TILE > STAGED ? 4 * TILE : STAGED;
+    static_assert(D % 128 == 0 && TILE % 4096 == 0, "whole swizzle groups per row, whole DMA instructions per wavefront");
     static_assert(LDS_BYTES <= 160 * 1024, "one work group must fit the LDS of a compute unit");
+    // a partial result: 128 rows of D 16-bit values, then 128 references and 128 denominators
+    static constexpr long SLOT = static_cast<long>(kWideRows) * (D * 2 + 8);
 };
 
+// The MFMAs of this kernel are inline assembly. At head_dim 512 the output accumulator of a wavefront is exactly the 256
+// accumulation registers; left to the compiler, which also puts every other MFMA result there, the scores spill (640 to
+// 1840 bytes of scratch per lane). Here O lives in a[0 : 16 VB) by name (block vb in a[16 vb : 16 vb + 16)), every statement
+// that touches it declares all of a0..a255 clobbered, so that the compiler keeps nothing of its own there, and the scores are
+// in ordinary registers. The compiler does not see the wait that VALU code needs before it touches the result of an
+// MFMA of 8 passes (11 wait states); it is kept by construction: the last MFMA of a score tile and the two that follow it
+// are one statement (wide_tail), so the scores are complete before anything can read them, and wide_settle stands in front
+// of the code that works on O.
+#define MI_A10(t) "a" #t "0", "a" #t "1", "a" #t "2", "a" #t "3", "a" #t "4", "a" #t "5", "a" #t "6", "a" #t "7", "a" #t "8", "a" #t "9"
+#define MI_AGPRS                                                                                                              \
+    "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", MI_A10(1), MI_A10(2), MI_A10(3), MI_A10(4), MI_A10(5),       \
+        MI_A10(6), MI_A10(7), MI_A10(8), MI_A10(9), MI_A10(10), MI_A10(11), MI_A10(12), MI_A10(13), MI_A10(14), MI_A10(15),  \
+        MI_A10(16), MI_A10(17), MI_A10(18), MI_A10(19), MI_A10(20), MI_A10(21), MI_A10(22), MI_A10(23), MI_A10(24), "a250",  \
+        "a251", "a252", "a253", "a254", "a255"
+template <typename T> struct WideMma;
+#define MI_WIDE_MMA(TYPE, NAME)                                                                                               \
+    template <> struct WideMma<TYPE> {                                                                                        \
+        using V8 = typename Mma<TYPE>::v8;                                                                                    \
+        static __device__ __forceinline__ void first(f32x16& s, V8 a, V8 b) {                                                 \
+            asm volatile(NAME " %0, %1, %2, 0" : "=&v"(s) : "v"(a), "v"(b));                                                  \
+        }                                                                                                                     \
+        static __device__ __forceinline__ void score(f32x16& s, V8 a, V8 b) {                                                 \
+            asm volatile(NAME " %0, %1, %2, %0" : "+v"(s) : "v"(a), "v"(b));                                                  \
+        }                                                                                                                     \
+        /* O block VB += a b */                                                                                               \
+        template <int VB> static __device__ __forceinline__ void out(V8 a, V8 b) {                                            \
+            asm volatile(NAME " a[%2:%3], %0, %1, a[%2:%3]" : : "v"(a), "v"(b), "n"(16 * VB), "n"(16 * VB + 15) : MI_AGPRS);  \
+        }                                                                                                                     \
+        /* the last MFMA of a score tile together with the first two of the PV product (O blocks 0 and 1) */                  \
+        static __device__ __forceinline__ void tail(f32x16& s, V8 ak, V8 q, V8 a0, V8 a1, V8 p) {                             \
+            asm volatile(NAME " %0, %1, %2, %0\n\t" NAME " a[0:15], %3, %5, a[0:15]\n\t" NAME " a[16:31], %4, %5, a[16:31]"   \
+                         : "+v"(s) : "v"(ak), "v"(q), "v"(a0), "v"(a1), "v"(p) : MI_AGPRS);                                   \
+        }                                                                                                                     \
+    };
+MI_WIDE_MMA(__bf16, "v_mfma_f32_32x32x16_bf16")
+MI_WIDE_MMA(_Float16, "v_mfma_f32_32x32x16_f16")
+#undef MI_WIDE_MMA
+// every MFMA in flight has written its result when this returns
+__device__ __forceinline__ void wide_settle(f32x16& s) { asm volatile("s_nop 15\n\ts_nop 15" : "+v"(s) : : MI_AGPRS); }
+template <int R> __device__ __forceinline__ float o_get() {
+    float f;
+    asm volatile("v_accvgpr_read_b32 %0, a[%1]" : "=v"(f) : "n"(R) : MI_AGPRS);
+    return f;
+}
+template <int R> __device__ __forceinline__ void o_set(float f) { asm volatile("v_accvgpr_write_b32 a[%1], %0" : : "v"(f), "n"(R) : MI_AGPRS); }
+// O = 0; O *= f (the reads of a block go out before its writes: a value just read is not touched in the next instruction)
+template <int N> __device__ __forceinline__ void o_clear() {
+    [&]<int... I>(std::integer_sequence<int, I...>) { (o_set<I>(0.f), ...); }(std::make_integer_sequence<int, N>{});
+}
+template <int B> __device__ __forceinline__ void o_scale_block(float f) {
+    [&]<int... I>(std::integer_sequence<int, I...>) {
+        const float v[16] = {o_get<16 * B + I>()...};
+        (o_set<16 * B + I>(v[I] * f), ...);
+    }(std::make_integer_sequence<int, 16>{});
+}
+template <int N> __device__ __forceinline__ void o_scale(float f) {
+    [&]<int... B>(std::integer_sequence<int, B...>) { (o_scale_block<B>(f), ...); }(std::make_integer_sequence<int, N / 16>{});
+    asm volatile("s_nop 7" : : : MI_AGPRS);   // accumulation registers written by the VALU and read by the next MFMA
+}
+
+// position of 16-byte chunk `c` of row `row` (XOR within groups of 16 chunks)
+__device__ __forceinline__ int wide_swz(int row) { return 4 * (row & 3) + ((row >> 2) & 3); }
+
 template <typename T, int D>
-__global__ void __launch_bounds__(kWideThreads) sdpa_wide_kernel(const SdpaDev p, int n_q_tiles) {
+__global__ void __launch_bounds__(kWideThreads, 1) sdpa_wide_kernel(const SdpaDev p, int n_q_tiles, int n_split, int n_blocks) {
     using G = HeadGeo<D>;
     using W = WideGeo<D>;
-    using GW = HeadGeo<W::DW>;            // softmax_tile rescales an accumulator of this many blocks
     using V8 = typename Mma<T>::v8;
-    static_assert(GW::VB == W::VBW, "accumulator blocks per wavefront");
+    constexpr int KC = W::KC, VB = W::VB;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    unsigned char* const Ks = smem;
-    unsigned char* const Vs = smem + W::A_BYTES;
-    float* const Ms = reinterpret_cast<float*>(Vs + G::V_BYTES);
-    float* const Ex = reinterpret_cast<float*>(smem);
 
-    const int bh = static_cast<int>(blockIdx.x) / n_q_tiles;
-    const int qt = static_cast<int>(blockIdx.x) - bh * n_q_tiles;
+    // pieces of the key axis outermost: the work groups of one XCD walk the same keys
+    const int logical = logical_block(n_blocks);
+    if (logical < 0) return;
+    const int tiles = n_blocks / n_split;
+    const int piece = logical / tiles, tile = logical - piece * tiles;
+    const int bh = tile / n_q_tiles, qt = tile - bh * n_q_tiles;
     const int h = bh % p.H, b = bh / p.H;
     const int hk = h / p.kv_group;
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
     const int q0 = qt * kWideRows;
-    const int qrow = q0 + lq;                         // every wavefront holds the same 32 rows
+    const int qrow = q0 + wave * 32 + lq;
     const bool qvalid = qrow < p.Lq;
-    const int d_w = wave * W::DW;                     // first head-dim element of this wavefront
     const T* const q_base = static_cast<const T*>(p.q) + b * p.q_bs + h * D;
     T* const o_base = static_cast<T*>(p.o) + b * p.o_bs + h * D;
-    const unsigned char* const k_base = reinterpret_cast<const unsigned char*>(static_cast<const T*>(p.k) + b * p.k_bs + hk * D);
-    const unsigned char* const v_base = reinterpret_cast<const unsigned char*>(static_cast<const T*>(p.v) + b * p.v_bs + hk * D);
     const float* const key_mask = p.key_mask ? p.key_mask + b * p.key_mask_bs : nullptr;
 
     int lo, hi;
     row_interval(p, b, qrow, qvalid, lo, hi);
-    const WaveExtent we = wave_extent(lo, hi);        // the same in all four wavefronts
+    if (n_split > 1) {   // this work group's piece of the key axis, in whole steps
+        const int steps = (p.Lk + kWideKeys - 1) / kWideKeys;
+        lo = max(lo, static_cast<int>(static_cast<long>(piece) * steps / n_split) * kWideKeys);
+        hi = min(hi, static_cast<int>(static_cast<long>(piece + 1) * steps / n_split) * kWideKeys);
+        if (hi <= lo) { lo = 0; hi = 0; }
+    }
+    const bool dead_row = hi <= lo;
+    const WaveExtent we = wave_extent(lo, hi);
 
-    // this wavefront's share of the Q fragments (RoPE, if any, applied while the rows are staged)
-    stage_q_tile<T, D, kWideThreads, kWideRows>(smem, p, q_base, q0, tid);
+    // ── Q rows through LDS (RoPE, if any, applied on the way), 32 rows at a time; every lane picks its row's fragments ──
+    V8 qf[KC];
+#pragma unroll 1
+    for (int r = 0; r < 4; ++r) stage_q_tile<T, D, kWideThreads, 32>(smem + r * 32 * G::O_STRIDE, p, q_base, q0 + 32 * r, tid);
     __syncthreads();
-    V8 qf[W::KCW];
+    read_q_frags<T, D>(qf, smem, wave * 32 + lq, lh);
+    __syncthreads();
+    // the extents of the four wavefronts
+    if (lane == 0) { reinterpret_cast<int*>(smem)[wave] = we.lo_min; reinterpret_cast<int*>(smem)[4 + wave] = we.hi_max; }
+    __syncthreads();
+    int g_lo = 0x7fffffff, g_hi = 0;
 #pragma unroll
-    for (int c = 0; c < W::KCW; ++c)
-        qf[c] = __builtin_bit_cast(V8, *reinterpret_cast<const u32x4*>(smem + lq * G::O_STRIDE + (d_w + 16 * c + 8 * lh) * 2));
+    for (int w = 0; w < 4; ++w) { g_lo = min(g_lo, reinterpret_cast<int*>(smem)[w]); g_hi = max(g_hi, reinterpret_cast<int*>(smem)[4 + w]); }
+    g_lo = __builtin_amdgcn_readfirstlane(g_lo);
+    g_hi = __builtin_amdgcn_readfirstlane(g_hi);
     __syncthreads();
+    const int k_first = g_lo == 0x7fffffff ? 0 : g_lo / kWideKeys * kWideKeys;
+    const int n_steps = g_lo == 0x7fffffff ? 0 : (g_hi - k_first + kWideKeys - 1) / kWideKeys;
 
-    f32x16 oacc[W::VBW];
-#pragma unroll
-    for (int vb = 0; vb < W::VBW; ++vb)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) oacc[vb][e] = 0.f;
-    SoftmaxState st;
+    o_clear<16 * VB>();
+    float l_sum = 0.f, neg_ref = 0.f;     // as RelSoftmaxState
+    bool started = false;
     const float cl2 = p.scale_log2;
-    const float lazy_raw = kLazyLog2 / cl2;
 
-    const int t_begin = we.lo_min == 0x7fffffff ? 0 : we.lo_min / kBN;
-    const int t_end = we.lo_min == 0x7fffffff ? 0 : (we.hi_max + kBN - 1) / kBN;
+    // ── DMA duty: instructions wave, wave + 4, ... of a tile; instruction j fills LDS bytes [1024 j, 1024 j + 1024) ──
     const unsigned k_rsb = static_cast<unsigned>(p.k_rs) * 2u, v_rsb = static_cast<unsigned>(p.v_rs) * 2u;
-    const int trow = (lane & 15) >> 2;
-    const int tcol = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+    const unsigned char* kptr = reinterpret_cast<const unsigned char*>(static_cast<const T*>(p.k) + b * p.k_bs + hk * D) + static_cast<unsigned long>(k_first) * k_rsb;
+    const unsigned char* vptr = reinterpret_cast<const unsigned char*>(static_cast<const T*>(p.v) + b * p.v_bs + hk * D) + static_cast<unsigned long>(k_first) * v_rsb;
+    int k_left = g_hi - k_first, v_left = k_left;     // rows from the tile under the cursor on
+    // this lane's tile row in its m-th instruction, and the byte offset of its chunk in that row (at 512 a row is one instruction,
+    // and the chunk depends on m % 4 only: a scalar row and four registers)
+    auto drow = [&](int m) -> int { return D == 512 ? wave + 4 * m : (64 * (wave + 4 * m) + lane) / G::CPR; };
+    constexpr int NCOL = D == 512 ? 4 : W::NDMA;
+    unsigned dcol[NCOL];
+#pragma unroll
+    for (int m = 0; m < NCOL; ++m) dcol[m] = static_cast<unsigned>((64 * (wave + 4 * m) + lane - drow(m) * G::CPR) ^ wide_swz(drow(m))) * 16u;
+    const unsigned lds_base = static_cast<unsigned>(reinterpret_cast<size_t>((__attribute__((address_space(3))) unsigned char*)smem));
+    // (inline assembly: for the compiler's builtin every later LDS read may alias the DMA's LDS write, so it would wait for the
+    //  load to land before the next LDS read. The s_nop is the wait state an LDS-DMA instruction needs behind a write of m0.
+    //  Rows past the last visible key repeat it: their scores are blanked.)
+    auto dma = [&](const unsigned char* base, unsigned rsb, int left, int m, unsigned dst) {
+        const unsigned voff = dcol[m % NCOL] + static_cast<unsigned>(min(drow(m), left - 1)) * rsb;
+        asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(base), "{m0}"(lds_base + dst + (wave + 4 * m) * 1024) : "memory");
+    };
+    auto dma_tile = [&](bool is_k, unsigned dst) {
+#pragma unroll
+        for (int m = 0; m < W::NDMA; ++m) dma(is_k ? kptr : vptr, is_k ? k_rsb : v_rsb, is_k ? k_left : v_left, m, dst);
+    };
 
-    for (int t = t_begin; t < t_end; ++t) {
-        const int j0 = t * kBN;
-        // ── K and V rows [j0, j0 + 64) into LDS; rows past the last key repeat it and are stored as zeros ──
-        {
-            const int last = min(p.Lk - j0, kBN) - 1;
-            constexpr int NLD = G::NCH / kWideThreads;     // 16-byte pieces per thread and operand (D / 8 pieces per row)
-            static_assert(G::NCH % kWideThreads == 0, "whole pieces per thread");
-#pragma unroll 4
-            for (int i = 0; i < NLD; ++i) {
-                const int idx = tid + kWideThreads * i;
-                const int row = idx / G::CPR, cc = idx - row * G::CPR;
-                const unsigned long src_row = static_cast<unsigned long>(j0 + min(row, last));
-                u32x4 kv = *reinterpret_cast<const u32x4*>(k_base + src_row * k_rsb + cc * 16u);
-                u32x4 vv = *reinterpret_cast<const u32x4*>(v_base + src_row * v_rsb + cc * 16u);
-                if (row > last) { kv = u32x4{0, 0, 0, 0}; vv = u32x4{0, 0, 0, 0}; }
-                *reinterpret_cast<u32x4*>(Ks + row * G::K_STRIDE + cc * 16) = kv;
-                *reinterpret_cast<u32x4*>(Vs + row * G::V_STRIDE + cc * 16) = vv;
-            }
-            if (key_mask && tid < kBN) Ms[tid] = j0 + tid < p.Lk ? key_mask[j0 + tid] : 0.f;
+    // ── LDS read addresses (stage, 32-row and 256-byte group offsets are immediates) ──
+    const int fk = wide_swz(lq);
+    unsigned kaddr[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) kaddr[c] = lq * W::ROWB + (((2 * c + lh) ^ fk) << 4);
+    const int trow = (lane & 15) >> 2, j4 = lane & 3, g1 = (lane >> 4) & 1;
+    unsigned vaddr[4][2];
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh) {
+            const int row = 4 * lh + 8 * hh + trow;
+            vaddr[v][hh] = W::VOFF + row * W::ROWB + (((4 * v + 2 * g1 + (j4 >> 1)) ^ wide_swz(row)) << 4) + 8 * (j4 & 1);
         }
-        __syncthreads();
 
-        // ── 1. partial scores over this wavefront's quarter of the head dimension ──
-        f32x16 sacc[2];
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-#pragma unroll
-            for (int e = 0; e < 16; ++e) sacc[kb][e] = 0.f;
-#pragma unroll
-            for (int c = 0; c < W::KCW; ++c) {
-                const u32x4 a = *reinterpret_cast<const u32x4*>(Ks + (32 * kb + lq) * G::K_STRIDE + (d_w + 16 * c + 8 * lh) * 2);
-                sacc[kb] = Mma<T>::run(__builtin_bit_cast(V8, a), qf[c], sacc[kb]);
-            }
-        }
-        __syncthreads();                               // every wavefront has read the K tile: its space takes the partial tiles
-        // ── 2. the four partial tiles, added in wavefront order by everybody ──
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) Ex[((wave * 2 + kb) * 16 + e) * 64 + lane] = sacc[kb][e];
+    f32x16 x;           // scores of the tile whose softmax is due
+    V8 pf[2];
+    constexpr int kFetch = 6;    // LDS reads run this many operands ahead of their MFMA
+    auto fetch_k = [&](int stage, int c) -> V8 {
+        return __builtin_bit_cast(V8, *reinterpret_cast<const u32x4*>(smem + stage * W::TILE + (c >> 3) * 256 + kaddr[c & 7]));
+    };
+    auto fetch_v = [&](int stage, int j) -> V8 {
+        const int c2 = j / VB, vb = j % VB;
+        const unsigned off = stage * W::TILE + c2 * 16 * W::ROWB + (vb >> 2) * 256;
+        const s16x4 v_lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(smem + off + vaddr[vb & 3][0]));
+        const s16x4 v_hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(smem + off + vaddr[vb & 3][1]));
+        return __builtin_bit_cast(V8, __builtin_shufflevector(v_lo, v_hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    };
+    auto step_end = [&]() {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
+    };
+
+    if (n_steps > 0) {
+        // prologue: K_0, K_1 and V_0 in LDS, x = raw scores of tile 0
+        dma_tile(true, 0);
+        dma_tile(false, W::VOFF);
+        if (n_steps > 1) {
+            kptr += kWideKeys * k_rsb; k_left -= kWideKeys;
+            dma_tile(true, W::TILE);
+        }
+        step_end();
+        WideMma<T>::first(x, fetch_k(0, 0), qf[0]);
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
+        for (int c = 1; c < KC; ++c) WideMma<T>::score(x, fetch_k(0, c), qf[c]);
+        wide_settle(x);
+    }
+    // K_0 has been read by everybody before its stage is overwritten
+    __syncthreads();
+
+    // Step t (PAR = t % 2): reads K_{t+1} (stage 1 - PAR) and V_t (stage PAR), loads K_{t+2} into stage PAR and V_{t+1} into
+    // stage 1 - PAR (their former tiles were used up in step t - 1).
+    auto step = [&](auto par_tag, int t) {
+        constexpr int PAR = decltype(par_tag)::value;
+        if (t + 2 < n_steps) { kptr += kWideKeys * k_rsb; k_left -= kWideKeys; }
+        if (t + 1 < n_steps) { vptr += kWideKeys * v_rsb; v_left -= kWideKeys; }
+        const int j0 = k_first + t * kWideKeys;
+        if (j0 < we.lo_max || j0 + kWideKeys > we.hi_min || key_mask != nullptr) {   // wave-uniform
+            const int d0 = j0 + 4 * lh - lo, top = hi - 1 - lo;
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
-                float s = Ex[((0 * 2 + kb) * 16 + e) * 64 + lane];
-#pragma unroll
-                for (int w = 1; w < 4; ++w) s += Ex[((w * 2 + kb) * 16 + e) * 64 + lane];
-                sacc[kb][e] = s;
+                const int c = 8 * (e >> 2) + (e & 3);
+                int hidden = 0;
+                // a key-mask value of +-0 hides the key: (bits of |m|) - 1 is negative exactly then
+                if (key_mask) hidden = static_cast<int>(__builtin_bit_cast(unsigned, key_mask[min(j0 + 4 * lh + c, p.Lk - 1)]) & 0x7fffffffu) - 1;
+                const float score = x[e];
+                x[e] = blank_outside(score, d0 + c, top, hidden);
             }
-        // ── softmax (identical in the four wavefronts), then 3. this wavefront's quarter of O^T += V^T P^T ──
-        V8 pf[4];
-        const bool interior = (j0 >= we.lo_max) && (j0 + kBN <= min(we.hi_min, p.Lk)) && (key_mask == nullptr);
-        softmax_tile<T, W::DW>(sacc, pf, oacc, st, cl2, lazy_raw, !interior, j0, lo, min(hi, p.Lk), lh, key_mask ? Ms : nullptr);
+        }
+        f32x16 s;
+        float s0 = 0.f, s1 = 0.f;
+        const float nr = neg_ref;
+        V8 ring[kFetch];
+        constexpr int NPV = 2 * VB, N = KC + NPV;
+        auto fetch = [&](auto i_tag) {
+            constexpr int i = decltype(i_tag)::value;
+            if constexpr (i < KC) ring[i % kFetch] = fetch_k(1 - PAR, i);
+            else if constexpr (i < N) ring[i % kFetch] = fetch_v(PAR, i - KC);
+        };
+        auto exponentials = [&](int e0, int e1) {
 #pragma unroll
-        for (int c4 = 0; c4 < 4; ++c4)
-#pragma unroll
-            for (int vb = 0; vb < W::VBW; ++vb) {
-                const unsigned char* vptr = Vs + (16 * c4 + 4 * lh + trow) * G::V_STRIDE + (d_w + 32 * vb + tcol) * 2;
-                const s16x4 v_lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(vptr));
-                const s16x4 v_hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(vptr + 8 * G::V_STRIDE));
-                const s16x8 a = __builtin_shufflevector(v_lo, v_hi, 0, 1, 2, 3, 4, 5, 6, 7);
-                oacc[vb] = Mma<T>::run(__builtin_bit_cast(V8, a), pf[c4], oacc[vb]);
+            for (int e = e0; e < e1; ++e) {
+                const float pr = __builtin_amdgcn_exp2f(x[e]);
+                pf[e >> 3][e & 7] = static_cast<T>(pr);
+                if (e & 1) s1 += pr; else s0 += pr;
             }
-        __syncthreads();                               // tiles and partial scores are used up
+        };
+        [&]<int... I>(std::integer_sequence<int, I...>) { (fetch(std::integral_constant<int, I>{}), ...); }(std::make_integer_sequence<int, kFetch>{});
+        // ── S_{t+1} = K_{t+1} Q^T (after the last tile: of a stage that holds none, never read) over the exponentials of tile t;
+        //    the last of these MFMAs goes out with the first of the PV product ──
+        [&]<int... I>(std::integer_sequence<int, I...>) {
+            ([&] {
+                constexpr int i = I;
+                if constexpr (i == 0) WideMma<T>::first(s, ring[0], qf[0]);
+                else WideMma<T>::score(s, ring[i % kFetch], qf[i]);
+                fetch(std::integral_constant<int, i + kFetch>{});
+                constexpr int e0 = 16 * i / (KC - 1), e1 = 16 * (i + 1) / (KC - 1);
+#pragma unroll
+                for (int e = e0; e < e1; ++e) x[e] = __builtin_fmaf(x[e], cl2, nr);
+                exponentials(e0, e1);
+                // (past the last tile the cursors stand still and that tile is loaded again, into a stage nobody reads)
+                constexpr int m0 = W::NDMA * i / (KC - 1), m1 = W::NDMA * (i + 1) / (KC - 1);
+#pragma unroll
+                for (int m = m0; m < m1; ++m) {
+                    dma(kptr, k_rsb, k_left, m, PAR * W::TILE);
+                    dma(vptr, v_rsb, v_left, m, W::VOFF + (1 - PAR) * W::TILE);
+                }
+                MI_SCHED_BARRIER
+            }(), ...);
+        }(std::make_integer_sequence<int, KC - 1>{});
+        const bool fine = (started || dead_row) && s0 + s1 < kRelSumMax;   // false also for inf / nan sums
+        if (__any(!fine)) {   // first visible tile of a row, or its terms grew: move the reference (see softmax_tile_rel)
+            wide_settle(s);
+            float mloc = x[0];
+#pragma unroll
+            for (int e = 1; e < 16; ++e) mloc = fmaxf(mloc, x[e]);
+            mloc = exchange_max(mloc);
+            const bool visible = mloc > kNegInf;
+            const float shift = !visible ? 0.f : (started ? fmaxf(mloc, 0.f) : mloc);
+            const float alpha = started ? __builtin_amdgcn_exp2f(-shift) : 1.f;
+            started = started || visible;
+            l_sum *= alpha;
+            o_scale<16 * VB>(alpha);
+#pragma unroll
+            for (int e = 0; e < 16; ++e) x[e] -= shift;
+            neg_ref -= shift;
+            s0 = s1 = 0.f;
+            exponentials(0, 16);
+        }
+        l_sum += s0 + s1;
+        MI_SCHED_BARRIER
+        // ── O^T += V_t^T P_t ──
+        WideMma<T>::tail(s, ring[(KC - 1) % kFetch], qf[KC - 1], ring[KC % kFetch], ring[(KC + 1) % kFetch], pf[0]);
+        fetch(std::integral_constant<int, KC - 1 + kFetch>{});
+        fetch(std::integral_constant<int, KC + kFetch>{});
+        fetch(std::integral_constant<int, KC + 1 + kFetch>{});
+        MI_SCHED_BARRIER
+        [&]<int... I>(std::integer_sequence<int, I...>) {
+            ([&] {
+                constexpr int i = KC + 2 + I, c2 = (I + 2) / VB, vb = (I + 2) % VB;
+                WideMma<T>::template out<vb>(ring[i % kFetch], pf[c2]);
+                fetch(std::integral_constant<int, i + kFetch>{});
+                MI_SCHED_BARRIER
+            }(), ...);
+        }(std::make_integer_sequence<int, NPV - 2>{});
+        x = s;
+        step_end();
+    };
+    for (int t = 0; t < n_steps; t += 2) {
+        step(std::integral_constant<int, 0>{}, t);
+        if (t + 1 >= n_steps) break;
+        step(std::integral_constant<int, 1>{}, t + 1);
     }
 
-    const float l_tot = exchange_sum(st.l);
+    wide_settle(x);
+    const float l_tot = exchange_sum(l_sum);
     const float inv = row_inverse(l_tot);
-    {
-        typedef T t4 __attribute__((ext_vector_type(4)));
-#pragma unroll
-        for (int vb = 0; vb < W::VBW; ++vb)
-#pragma unroll
-            for (int bb = 0; bb < 4; ++bb) {
-                t4 ov;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) ov[i] = static_cast<T>(oacc[vb][4 * bb + i] * inv);
-                *reinterpret_cast<t4*>(smem + lq * G::O_STRIDE + (d_w + 32 * vb + 8 * bb + 4 * lh) * 2) = ov;
-            }
-    }
+    [&]<int... B>(std::integer_sequence<int, B...>) {   // accumulation registers 4 B .. 4 B + 3: head-dim elements 8 B + 4 lh ..
+        ([&] {
+            typedef T t4 __attribute__((ext_vector_type(4)));
+            const float o0 = o_get<4 * B>(), o1 = o_get<4 * B + 1>(), o2 = o_get<4 * B + 2>(), o3 = o_get<4 * B + 3>();
+            const t4 ov = {static_cast<T>(o0 * inv), static_cast<T>(o1 * inv), static_cast<T>(o2 * inv), static_cast<T>(o3 * inv)};
+            *reinterpret_cast<t4*>(smem + (wave * 32 + lq) * G::O_STRIDE + (8 * B + 4 * lh) * 2) = ov;
+        }(), ...);
+    }(std::make_integer_sequence<int, 4 * VB>{});
     __syncthreads();
-    write_output<T, D, kWideThreads>(smem, o_base, p.o_rs, q0, p.Lq, kWideRows, tid);
+    if (n_split == 1) {
+        write_output<T, D, kWideThreads>(smem, o_base, p.o_rs, q0, p.Lq, kWideRows, tid);
+    } else {
+        unsigned char* const slot = p.split_scratch + (static_cast<long>(tile) * n_split + piece) * W::SLOT;
+        write_output<T, D, kWideThreads>(smem, reinterpret_cast<T*>(slot), D, 0, min(kWideRows, p.Lq - q0), kWideRows, tid);
+        if (lh == 0) {   // the weight of the part in the merge is l * 2^ref
+            float* const stat = reinterpret_cast<float*>(slot + static_cast<long>(kWideRows) * D * 2);
+            stat[wave * 32 + lq] = -neg_ref;
+            stat[kWideRows + wave * 32 + lq] = l_tot;
+        }
+    }
+}
+
+// out = sum_k w_k O_k / sum_k w_k with w_k = l_k 2^(ref_k - max ref) over the pieces of a query tile, in a fixed order; one
+// 16-byte piece of a row per thread, blockIdx.x = query tile.
+template <typename T, int D>
+__global__ void __launch_bounds__(256) wide_combine_kernel(const SdpaDev p, int n_q_tiles, int n_split) {
+    using W = WideGeo<D>;
+    typedef T t8 __attribute__((ext_vector_type(8)));
+    constexpr int CPR = D / 8;
+    const int tile = blockIdx.x;
+    const int bh = tile / n_q_tiles, q0 = (tile - bh * n_q_tiles) * kWideRows;
+    const int h = bh % p.H, b = bh / p.H;
+    const int idx = static_cast<int>(blockIdx.y) * 256 + static_cast<int>(threadIdx.x);
+    const int row = idx / CPR, cc = idx - row * CPR;
+    if (row >= kWideRows || q0 + row >= p.Lq) return;
+    const unsigned char* const slots = p.split_scratch + static_cast<long>(tile) * n_split * W::SLOT;
+    // (a part without visible keys has denominator 0 and is skipped; one whose denominator is NaN is not. The bits pass
+    //  through an empty asm statement because -fno-honor-nans entitles the optimiser to a comparison that is false for NaN.)
+    auto empty = [](float l) {
+        unsigned bits = __builtin_bit_cast(unsigned, l);
+        asm volatile("" : "+v"(bits));
+        return (bits & 0x7fffffffu) == 0u;
+    };
+    float ref = kNegInf;
+    for (int k = 0; k < n_split; ++k) {
+        const float* stat = reinterpret_cast<const float*>(slots + k * W::SLOT + static_cast<long>(kWideRows) * D * 2);
+        if (!empty(stat[kWideRows + row])) ref = fmaxf(ref, stat[row]);
+    }
+    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float wsum = 0.f;
+    for (int k = 0; k < n_split; ++k) {
+        const unsigned char* slot = slots + k * W::SLOT;
+        const float* stat = reinterpret_cast<const float*>(slot + static_cast<long>(kWideRows) * D * 2);
+        const float l = stat[kWideRows + row];
+        if (empty(l)) continue;
+        const float w = l * __builtin_amdgcn_exp2f(stat[row] - ref);
+        wsum += w;
+        const t8 o = *reinterpret_cast<const t8*>(slot + (static_cast<long>(row) * D + cc * 8) * 2);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] = __builtin_fmaf(w, static_cast<float>(o[e]), acc[e]);
+    }
+    const float inv = row_inverse(wsum);
+    t8 out;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) out[e] = static_cast<T>(acc[e] * inv);
+    *reinterpret_cast<t8*>(static_cast<T*>(p.o) + b * p.o_bs + static_cast<long>(q0 + row) * p.o_rs + h * D + cc * 8) = out;
+}
+
+// Pieces of the key axis: as many as minimise rounds x (steps of a piece + what a work group costs beyond its steps, about
+// kOverhead of them: Q staging, first tiles, write-out), plus the merge pass when there is one. Only unmasked calls (a valid
+// length or key mask may be on): with causal masks the tiles are unequal and fill the GPU in their own way.
+int wide_split(const SdpaDev& p, int n_cu) {
+    if (p.mask_mode != MI_MASK_NONE) return 1;
+    const long tiles = static_cast<long>(p.B) * p.H * ((p.Lq + kWideRows - 1) / kWideRows);
+    const int steps = (p.Lk + kWideKeys - 1) / kWideKeys;
+    constexpr int kOverhead = 6, kMerge = 4, kMaxSplit = 16, kMinSteps = 6;
+    int best = 1;
+    long best_cost = 0;
+    for (int s = 1; s <= kMaxSplit && (s == 1 || steps / s >= kMinSteps); ++s) {
+        const long rounds = (tiles * s + n_cu - 1) / n_cu;
+        const long cost = rounds * ((steps + s - 1) / s + kOverhead) + (s > 1 ? kMerge : 0);
+        if (s == 1 || cost < best_cost) { best = s; best_cost = cost; }
+    }
+    return best;
 }
 
 template <typename T, int D>
 int launch_wide_d(const SdpaDev& p, hipStream_t stream) {
+    using W = WideGeo<D>;
     const int n_q_tiles = (p.Lq + kWideRows - 1) / kWideRows;
-    const long blocks = static_cast<long>(p.B) * p.H * n_q_tiles;
-    if (blocks > 0x7fffffffL) return fail("mi_sdpa_forward: problem too large for one launch");
+    const long tiles = static_cast<long>(p.B) * p.H * n_q_tiles;
+    int n_split = wide_split(p, device_cu_count());
+    if (p.split_scratch == nullptr || p.split_scratch_bytes < static_cast<size_t>(tiles) * n_split * W::SLOT) n_split = 1;
+    const long blocks = tiles * n_split;
+    if (blocks > 0x7fffff00L) return fail("mi_sdpa_forward: problem too large for one launch");
     static thread_local bool raised = false;
     if (!raised) {
         MI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&sdpa_wide_kernel<T, D>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         WideGeo<D>::LDS_BYTES));
+                                         W::LDS_BYTES));
         raised = true;
     }
-    hipLaunchKernelGGL((sdpa_wide_kernel<T, D>), dim3(static_cast<unsigned>(blocks)), dim3(kWideThreads), WideGeo<D>::LDS_BYTES, stream, p, n_q_tiles);
+    hipLaunchKernelGGL((sdpa_wide_kernel<T, D>), dim3(static_cast<unsigned>((blocks + 7) / 8 * 8)), dim3(kWideThreads), W::LDS_BYTES, stream, p,
+                       n_q_tiles, n_split, static_cast<int>(blocks));
+    if (n_split > 1)
+        hipLaunchKernelGGL((wide_combine_kernel<T, D>), dim3(static_cast<unsigned>(tiles), kWideRows * (D / 8) / 256), dim3(256), 0, stream, p,
+                           n_q_tiles, n_split);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail("sdpa_wide launch: %s", hipGetErrorString(e));
     return 0;
@@ -201,6 +471,13 @@ int launch_wide_d(const SdpaDev& p, hipStream_t stream) {
 }  // namespace
 
 bool sdpa_wide_head(int head_dim) { return head_dim == 256 || head_dim == 384 || head_dim == 512; }
+
+size_t sdpa_wide_split_scratch_bytes(const SdpaDev& p, int head_dim) {
+    const int n_split = wide_split(p, device_cu_count());
+    if (n_split == 1) return 0;
+    const size_t slot = static_cast<size_t>(kWideRows) * (static_cast<size_t>(head_dim) * 2 + 8);
+    return static_cast<size_t>(p.B) * p.H * ((p.Lq + kWideRows - 1) / kWideRows) * n_split * slot;
+}
 
 int launch_sdpa_wide(const SdpaDev& p, int dtype, int head_dim, hipStream_t stream) {
     const char* what = nullptr;

@@ -443,7 +443,8 @@ MI_API int mi_rms_norm_forward(const void* x, const void* gain, void* out, int32
  *
  * Weights are (out_features, in_features) row-major, biases may be NULL. Q, K, V and the attention
  * output are rounded to `dtype` between the stages (they are tensors of that dtype in the reference too) and
- * live in `scratch`, which the caller lends: mi_flash_attention_scratch_bytes() bytes, 16-byte aligned.
+ * live in `scratch`, which the caller lends: mi_flash_attention_scratch_bytes() bytes, 16-byte aligned (of
+ * these only the projections are required; the rest, if lent, lets the attention launch cut its key axis into pieces).
  * The three projections of the qkvo form run as ONE launch, attention as one, the output projection as
  * one. Rows are batch-major: item b of x is rows [b*q_len, (b+1)*q_len); with ctx == NULL kv_len is
  * taken as q_len. head_dim = inner / num_heads must be one mi_sdpa_supported() accepts. */

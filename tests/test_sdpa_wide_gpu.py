@@ -130,3 +130,25 @@ def test_wide_head_rope(oracle, dtype, d, split_half):
     # before anything is enqueued
     with pytest.raises(RuntimeError, match="does not offer K rotated tile by tile|needs rope_k_scratch"):
         bd.joint_attention(dq, dk, dv, dcos, dsin, d, H, split_half=split_half)
+
+
+@pytest.mark.parametrize("dtype,B,H,d,Lq,Lk,valid", [
+    ("fp16", 1, 1, 512, 129, 512, None),          # two query tiles, the second of one row; pieces of whole steps
+    ("bf16", 1, 1, 512, 128, 1025, None),         # the last piece ends in a step of one key
+    ("bf16", 2, 1, 384, 100, 800, [800, 33]),     # one batch item's keys lie in the first piece only
+    ("fp16", 1, 2, 256, 260, 450, None),
+])
+def test_wide_head_key_axis_in_pieces(oracle, dtype, B, H, d, Lq, Lk, valid):
+    """With a scratch lent the key axis is cut into pieces whose partial results are merged: as the checker, and as the
+    launch in one piece to two units in the last place (each part is rounded once more before the merge)."""
+    q, k, v = (randn(8541 + i, (B, n, H * d), dtype) for i, n in enumerate((Lq, Lk, Lk)))
+    dq, dk, dv = (to_dev(x, dtype) for x in (q, k, v))
+    kw = {} if valid is None else {"kv_valid_len": torch.tensor(valid, dtype=torch.int32, device="cuda")}
+    whole = bd.sdpa_forward(dq, dk, dv, H, split_scratch=False, **kw)
+    pieces = bd.sdpa_forward(dq, dk, dv, H, split_scratch=torch.full((1 << 23,), 0xFF, dtype=torch.uint8, device="cuda"), **kw)
+    assert not torch.equal(whole, pieces), "this shape is expected to be cut"
+    unit = 2.0 ** (-8 if dtype == "bf16" else -11)
+    assert (whole.float() - pieces.float()).abs().max().item() <= 2 * unit * max(1.0, whole.float().abs().max().item())
+    for b in range(B):
+        n = Lk if valid is None else valid[b]
+        assert_close(oracle.sdpa(q[b], k[b, :n], v[b, :n], H), to_np(pieces[b]), dtype, f"pieces d={d} batch {b}")
