@@ -131,8 +131,10 @@ struct LinearBatch { LinearProblem p[kMaxLinearProblems]; };
 // Validates and launches up to kMaxLinearProblems problems as one grid.
 // geglu: problem 0 has W (2 N, K) and bias (2 N), value half first; Y (M, N) = value * gelu_exact(gate).
 int launch_linear(const LinearBatch& batch, int n_problems, int dtype, hipStream_t stream, bool geglu = false);
-// The 256 x 256-tile form with LDS-DMA operand rings (linear_dma.hip): whether it takes a validated launch, and the launch.
-bool linear_dma_takes(const LinearBatch& batch, int n_problems, int n_cu);
+// The forms with LDS-DMA operand rings: whether they take a validated launch, and the launch (linear_pipe.hip); the one with
+// 256 x 256 tiles (linear_dma.hip).
+bool linear_pipe_takes(const LinearBatch& batch, int n_problems, bool geglu);
+int launch_linear_pipe(const LinearBatch& batch, int n_problems, int dtype, bool geglu, hipStream_t stream);
 int launch_linear_dma(const LinearBatch& batch, int n_problems, int dtype, hipStream_t stream);
 
 }  // namespace mi

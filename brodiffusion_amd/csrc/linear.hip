@@ -6,50 +6,25 @@
 // output features of one token per accumulator group; bias is added in FP32 before the single rounding and the tile
 // leaves through LDS as whole 16-byte pieces of rows of Y.
 //
-// Streaming form (linear_kernel): 256 threads = 4 wavefronts in a 2 x 2 arrangement over a BM x BN output tile,
+// launch_linear validates a launch and hands it to the LDS-DMA kernels of linear_pipe.hip. What those do not take (contractions
+// that are no multiple of 64, operands beyond 32-bit tile offsets) runs here:
+//
+// linear_kernel: 256 threads = 4 wavefronts in a 2 x 2 arrangement over a BM x BN output tile,
 // contraction step 64. Operand tiles go global -> registers -> LDS with 16-byte accesses, double buffered so that the
 // loads of step t+1 are in flight while step t multiplies; one barrier per step. LDS rows are 144 bytes (128 + 16): 16
 // consecutive rows start on distinct 16-byte bank groups, so the ds_read_b128 fragment reads are conflict free.
 // Up to three problems share one launch (blockIdx.y): the Q, K and V projections of an attention block.
-// Ring form (linear_ring_kernel): work groups that stay and walk tiles with five contraction steps in flight, for the
-// GEGLU FF1 of the U-Net (launch_t decides).
-// Large problems with 16-bit weights go to the 256 x 256-tile kernel of linear_dma.hip instead (launch_linear decides).
 #include <type_traits>
 #include <utility>
 
-#include "internal.h"
+#include "linear_math.h"
 
 namespace mi {
 namespace gemm {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-
-template <typename T> struct Mma;
-template <> struct Mma<__bf16> {
-    using v8 = bf16x8;
-    using v4 = bf16x4;
-    static __device__ __forceinline__ f32x16 run(v8 a, v8 b, f32x16 c) {
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-    }
-};
-template <> struct Mma<_Float16> {
-    using v8 = f16x8;
-    using v4 = f16x4;
-    static __device__ __forceinline__ f32x16 run(v8 a, v8 b, f32x16 c) {
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-    }
-};
-
 constexpr int kBK = 64;                // contraction elements per step
 constexpr int kRowBytes = kBK * 2 + 16;  // LDS row stride
 constexpr int kThreads = 256;
-constexpr int kRing = 5;               // contraction steps in flight in the ring form (K a multiple of 320)
 
 // One 16-byte chunk column (tid % 8) and 32 rows per pass: ROWS / 32 loads per thread and tile.
 // GATED (the W tile of the GEGLU form): the tile's 32-row groups alternate between the value half and the gate half
@@ -109,43 +84,7 @@ __device__ __forceinline__ void store_tile_int8(const u32x2 (&raw)[ROWS / 32], c
     }
 }
 
-// x * Phi(x), the erf form of GELU (gelu_exact_scalar, src/fused_transformer.cu:89-92), branch free. With z = |x| / sqrt 2,
-// erfc(z) = t exp(-z^2 + P(t)), t = 1 / (1 + z / 2) (the Chebyshev fit of Numerical Recipes' erfcc, fractional error below
-// 1.2e-7 for all z >= 0), and Phi(x) = erfc(z) / 2 for x < 0, 1 - erfc(z) / 2 otherwise - so the left tail keeps its
-// relative accuracy, which the sum 1 + erf loses to cancellation. Here in base 2 with the constants folded: the
-// coefficients of P are multiplied by log2 e, its constant term also takes the factor 1/2 (-1 in the exponent), and
-// z^2 log2 e = (|x| sqrt(log2 e / 2))^2. 19 FP32 instructions and 2 transcendentals; against x Phi(x) in double the
-// relative error stays below 4e-6 for |x| < 6 and 1.5e-5 down to x = -12.
-__device__ __forceinline__ float gelu_erf(float x) {
-    const float ax = fabsf(x);
-    const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(ax, 0.35355339059327373f, 1.f));
-    const float zs = ax * 0.849321800288f;
-    float q = 0.246517298f;
-    q = __builtin_fmaf(q, t, -1.18611495f);
-    q = __builtin_fmaf(q, t, 2.14747446f);
-    q = __builtin_fmaf(q, t, -1.63775315f);
-    q = __builtin_fmaf(q, t, 0.402321582f);
-    q = __builtin_fmaf(q, t, -0.26875686f);
-    q = __builtin_fmaf(q, t, 0.139630057f);
-    q = __builtin_fmaf(q, t, 0.539700616f);
-    q = __builtin_fmaf(q, t, 1.4427292f);
-    q = __builtin_fmaf(q, t, -2.82574822f);
-    const float half_erfc = t * __builtin_amdgcn_exp2f(__builtin_fmaf(-zs, zs, q));
-    return x * (x < 0.f ? half_erfc : 1.f - half_erfc);
-}
-
-// acc * scale + bias of the INT8-weight forms as an FP32 value of its own. Left to itself the compiler merges the
-// multiply-add with the rounding to T that follows (v_fma_mixlo_f16: one rounding of the exact result) in some places and
-// not in others, and the plain and the GEGLU form of the same layer then disagree by a unit in the last place in about 3
-// outputs of 100 000; as a separate FP32 operation it is the FP32 multiply-add and conversion of the reference's kernel
-// everywhere.
-__device__ __forceinline__ float scaled_acc(float acc, float scale, float bias) {
-    float r = __builtin_fmaf(acc, scale, bias);
-    asm volatile("" : "+v"(r));
-    return r;
-}
-
-// What the two kernels below share: the MFMA step and the epilogue of a BM x BN tile held by WM x WN wavefronts. GEGLU: W is (2 N, K) and bias (2 N): value half on top, gate half below; the output (M, N) is
+// The MFMA step and the epilogue of a BM x BN tile held by WM x WN wavefronts. GEGLU: W is (2 N, K) and bias (2 N): value half on top, gate half below; the output (M, N) is
 // value * gelu_exact(gate) (diffusers' GEGLU with the erf form of GELU). A work group's 128 W-tile rows are 64 output
 // features times {value, gate}; each wavefront holds both accumulators of its 32 features, so the product of the two
 // halves never leaves registers and the (M, 2 N) intermediate does not exist.
@@ -294,7 +233,7 @@ struct TileMath {
     }
 };
 
-// The streaming form: one work group per output tile, one contraction step prefetched while the previous one is multiplied.
+// One work group per output tile, one contraction step prefetched while the previous one is multiplied.
 template <typename T, int BM, int BN, bool GEGLU = false, bool W8 = false>
 __global__ __launch_bounds__(kThreads) void linear_kernel(const LinearBatch batch) {
     using TM_ = TileMath<T, BM, BN, GEGLU, W8>;
@@ -353,120 +292,6 @@ __global__ __launch_bounds__(kThreads) void linear_kernel(const LinearBatch batc
     tm.write_tile(acc, braw, p, lds, m0, n0);
 }
 
-// The ring form, for contractions that are a multiple of kRing steps (the channel counts of the U-Net: 320, 640, 1280 and
-// their FF multiples). A work group of the streaming form lives a few microseconds, most of them waiting: every step for
-// the one tile it prefetched, at the start for its first, and the tile's few hundred cycles of MFMAs hide none of it.
-// Here a work group stays and walks output tiles (a contiguous run per XCD, so that the tiles sharing X rows meet in one
-// L2), and the operand tiles of kRing consecutive steps are in flight at any time, across tile boundaries: the registers
-// of step t + 1 go to LDS during step t and are at once requested again for step t + 1 + kRing (of this output tile or of
-// the next). All loads are unconditional, straight-line code (past the last tile they re-read the first rows of the
-// operands), so the waits the compiler places count exactly, and nothing ever waits for a store.
-template <typename T, int BM, int BN, bool GEGLU = false, int WM = 2, int WN = 2>
-__global__ __launch_bounds__(64 * WM * WN) void linear_ring_kernel(const LinearBatch batch) {
-    using TM_ = TileMath<T, BM, BN, GEGLU, false, WM, WN>;
-    constexpr int RP = TM_::NT / 8;             // tile rows per pass of the work group (8 threads per 128-byte row piece)
-    constexpr int XL = BM / RP, WL = BN / RP;   // loads per thread, operand and step
-    static_assert(BM % RP == 0 && BN % RP == 0 && RP % 32 == 0, "whole passes; a pass covers whole 32-row groups");
-    constexpr int TM = TM_::TM, TN = TM_::TN, BN_OUT = TM_::BN_OUT, X_BYTES = TM_::X_BYTES, W_BYTES = TM_::W_BYTES;
-    constexpr int R = kRing;
-    extern __shared__ __attribute__((aligned(16))) char lds[];  // [2][X tile ; W tile], then the staged output
-    char* const stage = lds + 2 * (X_BYTES + W_BYTES);
-
-    const LinearProblem& p = batch.p[blockIdx.y];
-    const int tiles_n = (p.N + BN_OUT - 1) / BN_OUT;
-    const int tiles_m = (p.M + BM - 1) / BM;
-    const int n_tiles = tiles_m * tiles_n;
-    // consecutive work-group ids go to the 8 XCDs in turn: every XCD takes a contiguous run of tiles
-    const int run = (n_tiles + 7) >> 3;
-    const int stride = static_cast<int>(gridDim.x) >> 3;
-    const int run_end = min(((static_cast<int>(blockIdx.x) & 7) + 1) * run, n_tiles);
-    int tile = (static_cast<int>(blockIdx.x) & 7) * run + (static_cast<int>(blockIdx.x) >> 3);
-    if (tile >= run_end) return;   // uniform
-
-    const int tid = threadIdx.x;
-    const TM_ tm(tid);
-    const char* xg = static_cast<const char*>(p.x);
-    const char* wg = static_cast<const char*>(p.w);
-    const unsigned x_pitch = static_cast<unsigned>(p.ldx) * 2u, w_pitch = static_cast<unsigned>(p.ldw) * 2u;
-    const unsigned k_bytes = static_cast<unsigned>(p.K) * 2u;
-
-    // ── the load cursor: kRing steps ahead of the multiplication; 32-bit byte offsets from the operand bases ──
-    int c_tile = tile;
-    unsigned c_k = 0;                       // byte offset of the cursor's step in a row (uniform)
-    const unsigned kcol = (tid & 7) * 16u;  // this thread's 16 bytes of a step
-    unsigned xrow[XL], wrow[WL];
-    auto cursor_rows = [&]() {
-        if (c_tile < run_end) {
-            const int m0 = (c_tile / tiles_n) * BM, n0 = (c_tile % tiles_n) * BN_OUT;
-#pragma unroll
-            for (int i = 0; i < XL; ++i) xrow[i] = static_cast<unsigned>(min(m0 + (tid >> 3) + RP * i, p.M - 1)) * x_pitch + kcol;
-#pragma unroll
-            for (int i = 0; i < WL; ++i) {
-                // (GEGLU: the tile's 32-row groups alternate between the value and the gate half of W, see load_tile)
-                const int r = (tid >> 3) + RP * i, grp = r >> 5;
-                const int row = GEGLU ? min(n0 + 32 * (grp >> 1) + (r & 31), p.N - 1) + (grp & 1) * p.N : min(n0 + r, p.N - 1);
-                wrow[i] = static_cast<unsigned>(row) * w_pitch + kcol;
-            }
-        } else {   // past the last tile: the first row of either operand
-#pragma unroll
-            for (int i = 0; i < XL; ++i) xrow[i] = kcol;
-#pragma unroll
-            for (int i = 0; i < WL; ++i) wrow[i] = kcol;
-        }
-    };
-    u32x4 xs_[R][XL], ws_[R][WL];
-    auto request = [&](auto s_tag) {
-        constexpr int s = decltype(s_tag)::value;
-#pragma unroll
-        for (int i = 0; i < XL; ++i) xs_[s][i] = *reinterpret_cast<const u32x4*>(xg + (xrow[i] + c_k));
-#pragma unroll
-        for (int i = 0; i < WL; ++i) ws_[s][i] = *reinterpret_cast<const u32x4*>(wg + (wrow[i] + c_k));
-        c_k += kBK * 2;
-        if (c_k == k_bytes) {   // uniform: on to the next output tile of this work group
-            c_k = 0;
-            c_tile += stride;
-            cursor_rows();
-        }
-    };
-    auto to_lds = [&](auto s_tag, char* dst) {
-        constexpr int s = decltype(s_tag)::value;
-#pragma unroll
-        for (int i = 0; i < XL; ++i) *reinterpret_cast<u32x4*>(dst + ((tid >> 3) + RP * i) * kRowBytes + (tid & 7) * 16) = xs_[s][i];
-#pragma unroll
-        for (int i = 0; i < WL; ++i) *reinterpret_cast<u32x4*>(dst + X_BYTES + ((tid >> 3) + RP * i) * kRowBytes + (tid & 7) * 16) = ws_[s][i];
-    };
-    cursor_rows();
-    [&]<int... S>(std::integer_sequence<int, S...>) { (request(std::integral_constant<int, S>{}), ...); }(std::make_integer_sequence<int, R>{});
-    to_lds(std::integral_constant<int, 0>{}, lds);
-    request(std::integral_constant<int, 0>{});
-    __syncthreads();
-
-    const int groups = p.K / (R * kBK);
-    int par = 0;   // LDS buffer of the step about to be multiplied
-    f32x16 acc[TN][TM];
-    for (; tile < run_end; tile += stride) {
-        const int m0 = (tile / tiles_n) * BM, n0 = (tile % tiles_n) * BN_OUT;
-        typename TM_::V4 braw[TN][4];
-        tm.request_bias(braw, p, n0);
-        TM_::clear(acc);
-        int g = 0;
-        do {   // (at least one group: a loop that may not run would make the wait for the bias a wait for every load)
-            [&]<int... S>(std::integer_sequence<int, S...>) {
-                ([&] {
-                    // step S of the group: the registers of the following step go to the other buffer and are requested anew
-                    constexpr int nxt = (S + 1) % R;
-                    to_lds(std::integral_constant<int, nxt>{}, lds + (par ^ 1) * (X_BYTES + W_BYTES));
-                    request(std::integral_constant<int, nxt>{});
-                    tm.multiply(acc, lds + par * (X_BYTES + W_BYTES));
-                    __syncthreads();
-                    par ^= 1;
-                }(), ...);
-            }(std::make_integer_sequence<int, R>{});
-        } while (++g < groups);
-        tm.write_tile(acc, braw, p, stage, m0, n0);
-    }
-}
-
 template <typename T, int BM, int BN, bool GEGLU = false, bool W8 = false>
 int launch_tiles(const LinearBatch& batch, int n_problems, hipStream_t st) {
     constexpr int BN_OUT = GEGLU ? BN / 2 : BN;
@@ -492,78 +317,10 @@ int launch_tiles(const LinearBatch& batch, int n_problems, hipStream_t st) {
     return 0;
 }
 
-// The ring form: 16-bit weights, contractions that are a multiple of kRing steps, operands addressable with 32-bit byte
-// offsets from their bases.
-inline bool ring_form_takes(const LinearBatch& batch, int n_problems, bool geglu) {
-    for (int i = 0; i < n_problems; ++i) {
-        const LinearProblem& p = batch.p[i];
-        if (p.w_scale != nullptr || p.K % (kRing * kBK) != 0) return false;
-        if (static_cast<long>(p.M) * p.ldx * 2 >= (1L << 32) || static_cast<long>(p.N) * (geglu ? 2 : 1) * p.ldw * 2 >= (1L << 32)) return false;
-    }
-    return true;
-}
-
-template <typename T, int BM, int BN, bool GEGLU = false, int WM = 2, int WN = 2>
-int launch_ring(const LinearBatch& batch, int n_problems, hipStream_t st) {
-    using TM_ = TileMath<T, BM, BN, GEGLU, false, WM, WN>;
-    int max_tiles = 0;
-    for (int i = 0; i < n_problems; ++i) {
-        const LinearProblem& p = batch.p[i];
-        max_tiles = max(max_tiles, ((p.M + BM - 1) / BM) * ((p.N + TM_::BN_OUT - 1) / TM_::BN_OUT));
-    }
-    constexpr size_t lds = 2 * static_cast<size_t>(BM + BN) * kRowBytes + TM_::kOutBytes;
-    static_assert(lds <= 160 * 1024, "operand buffers and staged output exceed the LDS of a compute unit");
-    const void* const kern = reinterpret_cast<const void*>(&linear_ring_kernel<T, BM, BN, GEGLU, WM, WN>);
-    static thread_local int per_cu = 0;   // work groups a compute unit holds at once
-    if (per_cu == 0) {
-        if (lds > 64 * 1024)
-            MI_HIP_CHECK(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-        int n = 0;
-        MI_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kern, TM_::NT, lds));
-        per_cu = max(n, 1);
-    }
-    // as many work groups as the GPU holds at once, split over the problems; a multiple of 8 (one run of tiles per XCD)
-    const int grid_x = min((max_tiles + 7) / 8 * 8, max(8, per_cu * device_cu_count() / n_problems / 8 * 8));
-    hipLaunchKernelGGL((linear_ring_kernel<T, BM, BN, GEGLU, WM, WN>), dim3(grid_x, n_problems), dim3(TM_::NT), lds, st, batch);
-    MI_HIP_CHECK(hipGetLastError());
-    return 0;
-}
-
 template <typename T>
 int launch_t(const LinearBatch& batch, int n_problems, hipStream_t st, bool geglu) {
-    if (geglu) {
-        // the ring form when its 128-token tiles give every compute unit two: FF1 of the U-Net's widest levels
-        // (8192 x 320 -> 2 x 1280: 31 us against 40 for the streaming form, 33 with 256-token tiles, whose 640 tiles are
-        // 2.5 per compute unit; 2048 x 640 -> 2 x 2560: 28 against 33)
-        if (ring_form_takes(batch, 1, true) && static_cast<long>((batch.p[0].M + 127) / 128) * ((batch.p[0].N + 63) / 64) >= 2L * device_cu_count())
-            return launch_ring<T, 128, 128, true, 4, 2>(batch, 1, st);
-        // 64-token tiles unless 128-token tiles alone fill the GPU twice over
-        const long big = static_cast<long>((batch.p[0].M + 127) / 128) * ((batch.p[0].N + 63) / 64);
-        const bool w8g = batch.p[0].w_scale != nullptr;
-        if (big >= 2L * device_cu_count() && batch.p[0].K >= 1024)
-            return w8g ? launch_tiles<T, 128, 128, true, true>(batch, 1, st) : launch_tiles<T, 128, 128, true>(batch, 1, st);
-        return w8g ? launch_tiles<T, 64, 128, true, true>(batch, 1, st) : launch_tiles<T, 64, 128, true>(batch, 1, st);
-    }
-    // 128 x 128 tiles when they alone fill the GPU twice over and the contraction is long enough to pay for their
-    // longer prologue, else 64 x 64 (more, smaller work groups: the projections of one attention block are small
-    // problems)
-    long big = 0;
-    int min_k = 0x7fffffff;
-    for (int i = 0; i < n_problems; ++i) {
-        big += static_cast<long>((batch.p[i].M + 127) / 128) * ((batch.p[i].N + 127) / 128);
-        min_k = min(min_k, batch.p[i].K);
-    }
     const bool w8 = batch.p[0].w_scale != nullptr;
-    if (big >= 2L * device_cu_count() && min_k >= 1024)
-        return w8 ? launch_tiles<T, 128, 128, false, true>(batch, n_problems, st) : launch_tiles<T, 128, 128>(batch, n_problems, st);
-    // long contractions over few tiles (FF2 of the U-Net: 2048 x 2560 -> 640, 30 -> 21 us; 8192 x 1280 -> 320, 22 -> 17 us): the
-    // ring form, whose five steps in flight shorten the per-step chain of memory latencies; at 320 it measures the same
-    // (with many tiles per compute unit the streaming form's work groups cover for each other: 2048 x 640 -> 5120, 2560
-    // tiles, 28 us against 34)
-    long tiles64 = 0;
-    for (int i = 0; i < n_problems; ++i) tiles64 += static_cast<long>((batch.p[i].M + 63) / 64) * ((batch.p[i].N + 63) / 64);
-    if (min_k >= 2 * kRing * kBK && tiles64 <= 4L * device_cu_count() && ring_form_takes(batch, n_problems, false))
-        return launch_ring<T, 64, 64>(batch, n_problems, st);
+    if (geglu) return w8 ? launch_tiles<T, 64, 128, true, true>(batch, 1, st) : launch_tiles<T, 64, 128, true>(batch, 1, st);
     return w8 ? launch_tiles<T, 64, 64, false, true>(batch, n_problems, st) : launch_tiles<T, 64, 64>(batch, n_problems, st);
 }
 
@@ -587,7 +344,7 @@ int launch_linear(const LinearBatch& batch, int n_problems, int dtype, hipStream
         if (static_cast<long>((p.M + 63) / 64) * ((p.N + 63) / 64) > 0x7fffffffL) return fail("linear: problem too large for one launch");
     }
     if (dtype != MI_DTYPE_BF16 && dtype != MI_DTYPE_F16) return fail("linear: dtype %d is neither MI_DTYPE_F16 nor MI_DTYPE_BF16", dtype);
-    if (!geglu && linear_dma_takes(batch, n_problems, device_cu_count())) return launch_linear_dma(batch, n_problems, dtype, st);
+    if (linear_pipe_takes(batch, n_problems, geglu)) return launch_linear_pipe(batch, n_problems, dtype, geglu, st);
     if (dtype == MI_DTYPE_BF16) return gemm::launch_t<__bf16>(batch, n_problems, st, geglu);
     if (dtype == MI_DTYPE_F16) return gemm::launch_t<_Float16>(batch, n_problems, st, geglu);
     return fail("linear: dtype %d is neither MI_DTYPE_F16 nor MI_DTYPE_BF16", dtype);

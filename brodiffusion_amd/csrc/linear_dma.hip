@@ -1,4 +1,4 @@
-// Y = X W^T + b for large problems on gfx950: 256 x 256 output tiles, 8 wavefronts, operand blocks moved global -> LDS
+// Y = X W^T + b for large problems on gfx950 (linear_pipe.hip says which): 256 x 256 output tiles, 8 wavefronts, operand blocks moved global -> LDS
 // by DMA into rings.
 //
 // The work group's 512 threads are 8 wavefronts in a 2 (feature halves) x 4 (token quarters) arrangement; a wavefront owns
@@ -258,18 +258,6 @@ int launch_t(const LinearBatch& batch, int n_problems, hipStream_t st) {
 }
 
 }  // namespace gemm_dma
-
-// Large plain problems (16-bit weights, no GEGLU) whose 256 x 256 tiles give most compute units one work group.
-bool linear_dma_takes(const LinearBatch& batch, int n_problems, int n_cu) {
-    long tiles = 0;
-    for (int i = 0; i < n_problems; ++i) {
-        const LinearProblem& p = batch.p[i];
-        if (p.w_scale != nullptr || p.K % gemm_dma::kBK != 0 || p.K < 512) return false;
-        if (static_cast<long>(p.ldx) * 2 * gemm_dma::kTile >= (1L << 31) || static_cast<long>(p.ldw) * 2 * gemm_dma::kTile >= (1L << 31)) return false;
-        tiles += static_cast<long>((p.M + gemm_dma::kTile - 1) / gemm_dma::kTile) * ((p.N + gemm_dma::kTile - 1) / gemm_dma::kTile);
-    }
-    return 4 * tiles >= 3L * n_cu;
-}
 
 int launch_linear_dma(const LinearBatch& batch, int n_problems, int dtype, hipStream_t st) {
     if (dtype == MI_DTYPE_BF16) return gemm_dma::launch_t<__bf16>(batch, n_problems, st);

@@ -1,0 +1,480 @@
+// Y = X W^T + b for problems between the smallest and the 256 x 256-tile kernel's on gfx950 (contractions that are a
+// multiple of 64; 16-bit or INT8 weights; plain or GEGLU).
+//
+// Operands go global -> LDS by DMA into a ring of S stages of 64 contraction elements each: no staging registers, no LDS
+// store instructions, and as many steps in flight as the LDS holds (a problem of this size is a chain of memory latencies
+// before it is anything else: with one step in flight, 2048 x 640 x 640 took 10 to 12 us of which 1 us is arithmetic). A
+// stage holds BM rows of X and BN rows of W, 128 bytes each (INT8: 64), back to back as the DMA deposits them; bank
+// conflicts of the fragment reads (one row per lane, 16 consecutive rows per phase) are avoided by an XOR swizzle applied on
+// the global side: the 16-byte piece in position c of row r is piece c ^ ((r >> 1) & 7) (INT8 rows: c ^ ((r >> 2) & 3)).
+//
+// A work group is WM x WN wavefronts over tokens x features; a wavefront owns TM x TN blocks of 32 x 32 (as in linear.hip the
+// product is computed transposed: MFMA rows are features). A stage is read in two halves into two register sets. Step t:
+//   read half 1 of stage t; multiply half 0
+//   wait until stage t + 1 has landed and this wavefront's reads of stage t have returned; barrier (for everybody)
+//   read half 0 of stage t + 1; multiply half 1 of stage t
+// and the DMA of stage t + S, which goes into the ring slot of stage t, is dealt out between the MFMAs of the second half of
+// step t and the first half of step t + 1: issued in one burst behind the barrier it made a step of 128 x 128 take 0.57 us
+// on an otherwise empty compute unit, 0.4 dealt out. The accumulation order is the same in every form (and in linear_dma.hip):
+// a problem gives the same bits whichever one takes it, alone or in a launch with others.
+//
+// Measured (fp16 / bf16, one launch; before: 64 x 64 tiles through registers, one step ahead): 4096 x 1152 x 1152 30 -> 19 us,
+// three of them 90 -> 45; 1024 x 2240 x 2240 30 -> 18, three 90 -> 38; 2048 x 640 x 640 8.4 -> 6.7 (INT8 weights 11.5 -> 7.5);
+// 128 x 1280 x 1280 8.2 -> 6.0; GEGLU 3072 x 640 -> 2 x 2560 39 -> 33, INT8 54 -> 37.
+#include <cmath>
+#include <type_traits>
+#include <utility>
+
+#include "linear_math.h"
+
+namespace mi {
+namespace gemm {
+namespace {
+
+constexpr int kBK = 64;   // contraction elements per stage
+struct PanelWidths { int w[kMaxLinearProblems]; };   // per problem: columns of tiles walked together
+
+template <typename T, bool W8, bool GEGLU, int WM, int WN, int TM, int TN, int S>
+struct PipeGeo {
+    static constexpr int NW = WM * WN, NT = 64 * NW;
+    static constexpr int BM = WM * TM * 32, BN = WN * TN * 32;
+    static constexpr int BN_OUT = GEGLU ? BN / 2 : BN;
+    static constexpr int WROW = W8 ? 64 : 128;                    // bytes of a W row in a stage
+    static constexpr int X_BYTES = BM * 128, W_BYTES = BN * WROW, STAGE = X_BYTES + W_BYTES;
+    static constexpr int MX = X_BYTES / 1024 / NW, MW = W_BYTES / 1024 / NW;   // DMA instructions per wavefront and stage
+    static constexpr int MI = MX + MW;
+    static constexpr int OUT_ROW = BN_OUT * 2 + 16;
+    static constexpr int LDS = S * STAGE > BM * OUT_ROW ? S * STAGE : BM * OUT_ROW;
+    static_assert(MX * NW * 1024 == X_BYTES && MW * NW * 1024 == W_BYTES, "the same DMA duty for every wavefront");
+    static_assert(!GEGLU || TN == 2, "the GEGLU form pairs the two feature blocks of a wavefront");
+    static_assert(LDS <= 160 * 1024, "LDS of a compute unit");
+    static_assert((S - 1) * MI < 64, "outstanding loads fit the counter");
+};
+
+// 8 INT8 weights -> 8 values of T, exactly
+template <typename T> __device__ __forceinline__ typename Mma<T>::v8 widen(u32x2 raw);
+template <> __device__ __forceinline__ f16x8 widen<_Float16>(u32x2 raw) {
+    // u = w + 128 as the low byte of 1024 + u (0x6400 | u), minus 1152
+    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+    const f16x2 off = {static_cast<_Float16>(1152.f), static_cast<_Float16>(1152.f)};
+    u32x4 r;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const unsigned u = raw[i] ^ 0x80808080u;
+        const unsigned lo = __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u), hi = __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u);
+        r[2 * i] = __builtin_bit_cast(unsigned, __builtin_bit_cast(f16x2, lo) - off);
+        r[2 * i + 1] = __builtin_bit_cast(unsigned, __builtin_bit_cast(f16x2, hi) - off);
+    }
+    return __builtin_bit_cast(f16x8, r);
+}
+template <> __device__ __forceinline__ bf16x8 widen<__bf16>(u32x2 raw) {
+    // |w| <= 128 has at most 8 significant bits: the upper half of the FP32 value is the bf16 value
+    u32x4 r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const unsigned pair = i & 1 ? raw[i >> 1] >> 16 : raw[i >> 1];
+        const float a = static_cast<float>(static_cast<signed char>(pair & 0xffu)), b = static_cast<float>(static_cast<signed char>((pair >> 8) & 0xffu));
+        r[i] = __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, b), __builtin_bit_cast(unsigned, a), 0x07060302u);
+    }
+    return __builtin_bit_cast(bf16x8, r);
+}
+
+template <typename T, bool W8, bool GEGLU, int WM, int WN, int TM, int TN, int S>
+__global__ void __launch_bounds__(64 * WM * WN, 2) linear_pipe_kernel(const LinearBatch batch, int n_problems, const PanelWidths panels) {
+    using G = PipeGeo<T, W8, GEGLU, WM, WN, TM, TN, S>;
+    using M = Mma<T>;
+    using V8 = typename M::v8;
+    using V4 = typename M::v4;
+    constexpr int BM = G::BM, BN = G::BN, BN_OUT = G::BN_OUT, MI = G::MI;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+
+    // Tiles of all problems in one row; consecutive work-group ids go to the 8 XCDs in turn, and every XCD (one L2) takes a
+    // contiguous run of it. A problem's tiles are numbered panel by panel (panels.w columns of tiles, row by row), so that a
+    // run is about as many rows of X as rows of W: what a run touches comes from the last-level cache, which serves a
+    // compute unit 28 bytes per ns when all of them ask, once, and from then on from the L2 at 95.
+    auto tiles_of = [&](int i) { return ((batch.p[i].M + BM - 1) / BM) * ((batch.p[i].N + BN_OUT - 1) / BN_OUT); };
+    const int n0_tiles = tiles_of(0), n1_tiles = n_problems > 1 ? tiles_of(1) : 0, n2_tiles = n_problems > 2 ? tiles_of(2) : 0;
+    const int n_tiles = n0_tiles + n1_tiles + n2_tiles;
+    const int chunk = (n_tiles + 7) >> 3;
+    int tile = (static_cast<int>(blockIdx.x) & 7) * chunk + (static_cast<int>(blockIdx.x) >> 3);
+    if (tile >= n_tiles) return;
+    int pi = 0;
+    if (tile >= n0_tiles) { tile -= n0_tiles; pi = 1; if (tile >= n1_tiles) { tile -= n1_tiles; pi = 2; } }
+    const LinearProblem& p = batch.p[__builtin_amdgcn_readfirstlane(pi)];
+    const int tiles_n = (p.N + BN_OUT - 1) / BN_OUT, tiles_m = (p.M + BM - 1) / BM;
+    const int pw = panels.w[__builtin_amdgcn_readfirstlane(pi)];
+    const int panel = tile / (tiles_m * pw), in_panel = tile - panel * tiles_m * pw;
+    const int w_here = min(pw, tiles_n - panel * pw);
+    const int m0 = (in_panel / w_here) * BM, n0 = (panel * pw + in_panel % w_here) * BN_OUT;
+
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
+    const int wm = wave % WM, wn = wave / WM;
+
+    // a pointer that is the same for the whole wavefront, in scalar registers
+    auto uniform = [](const unsigned char* q) {
+        const unsigned long u = reinterpret_cast<unsigned long>(q);
+        const unsigned lo = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(u)), hi = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(u >> 32));
+        return reinterpret_cast<const unsigned char*>(static_cast<unsigned long>(hi) << 32 | lo);
+    };
+    // ── DMA duty: X instructions wave + NW m (8 rows of 128 bytes each), W instructions likewise (INT8: 16 rows of 64) ──
+    const unsigned char* xg = uniform(static_cast<const unsigned char*>(p.x) + static_cast<long>(m0) * p.ldx * 2);
+    const unsigned char* wg = uniform(static_cast<const unsigned char*>(p.w) + (GEGLU ? 0L : static_cast<long>(n0) * p.ldw * (W8 ? 1 : 2)));
+    unsigned xoff[G::MX], woff[G::MW];
+#pragma unroll
+    for (int u = 0; u < G::MX; ++u) {
+        const int r = 8 * (wave + G::NW * u) + (lane >> 3);
+        xoff[u] = static_cast<unsigned>(min(r, p.M - 1 - m0)) * (static_cast<unsigned>(p.ldx) * 2u) + ((lane & 7) ^ ((r >> 1) & 7)) * 16u;
+    }
+#pragma unroll
+    for (int u = 0; u < G::MW; ++u) {
+        const int r = W8 ? 16 * (wave + G::NW * u) + (lane >> 2) : 8 * (wave + G::NW * u) + (lane >> 3);
+        const unsigned piece = W8 ? (lane & 3) ^ ((r >> 2) & 3) : (lane & 7) ^ ((r >> 1) & 7);
+        // GEGLU: 32-row groups of the tile alternate between the value and the gate rows of the same features
+        const int row = GEGLU ? min(n0 + 32 * (r >> 6) + (r & 31), p.N - 1) + ((r >> 5) & 1) * p.N : min(r, p.N - 1 - n0);
+        woff[u] = static_cast<unsigned>(row) * (static_cast<unsigned>(p.ldw) * (W8 ? 1u : 2u)) + piece * 16u;
+    }
+    const unsigned lds_base = static_cast<unsigned>(reinterpret_cast<size_t>((__attribute__((address_space(3))) unsigned char*)lds));
+    // (the LDS destination travels in m0; the s_nop is the wait state an LDS-DMA instruction needs behind a write of m0)
+    auto dma = [&](unsigned voff, const unsigned char* base, unsigned dst) {
+        asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(base), "{m0}"(dst) : "memory");
+    };
+    // pieces [J0, J1) of this wavefront's share of a stage; xg / wg stand on that stage
+    auto dma_piece = [&](int j, unsigned slot) {
+        if (j < G::MX) dma(xoff[j < G::MX ? j : 0], xg, lds_base + slot + (wave + G::NW * j) * 1024);
+        else dma(woff[j < G::MX ? 0 : j - G::MX], wg, lds_base + slot + G::X_BYTES + (wave + G::NW * (j - G::MX)) * 1024);
+    };
+    auto next_stage = [&]() {
+        xg += kBK * 2;
+        wg += W8 ? kBK : kBK * 2;
+    };
+    // Waits until at most `stages` of this wavefront's stages are in flight and its LDS reads have returned, then meets the others.
+    auto wait_barrier = [&](int stages) {
+        if (stages == S - 2) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"((S - 2) * MI) : "memory");
+        else {
+            [&]<int... I>(std::integer_sequence<int, I...>) {
+                ([&] { if (stages == I) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(I * MI) : "memory"); }(), ...);
+            }(std::make_integer_sequence<int, S>{});
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        }
+    };
+
+    // ── fragment reads: a stage is four chunks of 16 contraction elements, read two at a time ──
+    unsigned xaddr[4], waddr[4];
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+        xaddr[kk] = wm * TM * 4096 + lq * 128 + (((2 * kk + lh) ^ ((lq >> 1) & 7)) << 4);
+        waddr[kk] = G::X_BYTES + wn * TN * 32 * G::WROW + (W8 ? lq * 64 + ((kk ^ ((lq >> 2) & 3)) << 4) + 8 * lh : lq * 128 + (((2 * kk + lh) ^ ((lq >> 1) & 7)) << 4));
+    }
+    using WRaw = std::conditional_t<W8, u32x2, V8>;
+    V8 xf[2][2][TM];
+    WRaw wf[2][2][TN];
+    auto read_half = [&](auto half_tag, unsigned slot) {
+        constexpr int H = decltype(half_tag)::value;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+#pragma unroll
+            for (int b = 0; b < TM; ++b) xf[H][i][b] = *reinterpret_cast<const V8*>(lds + slot + xaddr[2 * H + i] + b * 4096);
+#pragma unroll
+            for (int a = 0; a < TN; ++a) wf[H][i][a] = *reinterpret_cast<const WRaw*>(lds + slot + waddr[2 * H + i] + a * 32 * G::WROW);
+        }
+    };
+    f32x16 acc[TN][TM];
+#pragma unroll
+    for (int a = 0; a < TN; ++a)
+#pragma unroll
+        for (int b = 0; b < TM; ++b)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[a][b][e] = 0.f;
+    // the MFMAs of a half stage, with DMA pieces [J0, J1) of the stage that goes to `slot` between them: issued in one burst they
+    // would keep the wavefront from its MFMAs for as long as the burst takes (16 clocks per instruction and compute unit)
+    auto multiply_half = [&](auto half_tag, auto j0_tag, auto j1_tag, unsigned slot) {
+        constexpr int H = decltype(half_tag)::value, J0 = decltype(j0_tag)::value, J1 = decltype(j1_tag)::value, NM = 2 * TM * TN;
+        V8 w[2][TN];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int a = 0; a < TN; ++a) {
+                if constexpr (W8) w[i][a] = widen<T>(wf[H][i][a]);
+                else w[i][a] = wf[H][i][a];
+            }
+        [&]<int... Q>(std::integer_sequence<int, Q...>) {
+            ([&] {
+                constexpr int i = Q / (TM * TN), a = Q / TM % TN, b = Q % TM;
+                acc[a][b] = M::run(w[i][a], xf[H][i][b], acc[a][b]);
+                constexpr int j0 = J0 + (J1 - J0) * Q / NM, j1 = J0 + (J1 - J0) * (Q + 1) / NM;
+                if constexpr (j1 > j0) {
+#pragma unroll
+                    for (int j = j0; j < j1; ++j) dma_piece(j, slot);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }(), ...);
+        }(std::make_integer_sequence<int, NM>{});
+    };
+
+    using Half0 = std::integral_constant<int, 0>;
+    using Half1 = std::integral_constant<int, 1>;
+    using Mid = std::integral_constant<int, MI / 2>;
+    using All = std::integral_constant<int, MI>;
+    const int n = p.K / kBK;
+    unsigned cur = 0, prev = (S - 1) * G::STAGE;      // ring slots of stages t and t - 1
+    // Step t. D0: the second part of stage t + S - 1 is loaded, into the slot of stage t - 1; D1: the first part of stage t + S,
+    // into the slot of stage t.
+    auto step = [&](auto d0_tag, auto d1_tag, int t) {
+        constexpr bool D0 = decltype(d0_tag)::value, D1 = decltype(d1_tag)::value;
+        const unsigned nxt = cur + G::STAGE == S * G::STAGE ? 0u : cur + G::STAGE;
+        read_half(Half1{}, cur);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (D0) {
+            multiply_half(Half0{}, Mid{}, All{}, prev);
+            next_stage();
+        } else {
+            multiply_half(Half0{}, Half0{}, Half0{}, 0u);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (D1 || t + 1 < n) {
+            wait_barrier(D1 ? S - 2 : (t + S - 1 < n - 1 ? t + S - 1 : n - 1) - (t + 1));
+            read_half(Half0{}, nxt);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (D1) multiply_half(Half1{}, Half0{}, Mid{}, cur);
+        else multiply_half(Half1{}, Half0{}, Half0{}, 0u);
+        __builtin_amdgcn_sched_barrier(0);
+        prev = cur;
+        cur = nxt;
+    };
+    if (n < S) {   // everything fits the ring
+        for (int s = 0; s < n; ++s) {
+#pragma unroll
+            for (int j = 0; j < MI; ++j) dma_piece(j, s * G::STAGE);
+            next_stage();
+        }
+        wait_barrier(n - 1);
+        read_half(Half0{}, 0);
+        for (int t = 0; t < n; ++t) step(std::false_type{}, std::false_type{}, t);
+    } else {
+        for (int s = 0; s < S - 1; ++s) {
+#pragma unroll
+            for (int j = 0; j < MI; ++j) dma_piece(j, s * G::STAGE);
+            next_stage();
+        }
+#pragma unroll
+        for (int j = 0; j < MI / 2; ++j) dma_piece(j, prev);
+        // stage 0 has landed: behind it are S - 2 stages and the first part of another
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"((S - 2) * MI + MI / 2) : "memory");
+        read_half(Half0{}, 0);
+        int t = 0;
+        for (; t < n - S; ++t) step(std::true_type{}, std::true_type{}, t);
+        step(std::true_type{}, std::false_type{}, t);
+        for (++t; t < n; ++t) step(std::false_type{}, std::false_type{}, t);
+    }
+
+    // the bias of this lane's features, requested ahead of the barrier
+    const T* const bias = static_cast<const T*>(p.bias);
+    V4 braw[TN][4];
+#pragma unroll
+    for (int a = 0; a < TN; ++a)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int feat = GEGLU ? n0 + wn * 32 + 8 * g + 4 * lh : n0 + (wn * TN + a) * 32 + 8 * g + 4 * lh;
+            const bool there = bias != nullptr && feat < p.N;
+            const V4 raw = *reinterpret_cast<const V4*>(there ? bias + feat + (GEGLU ? a * p.N : 0) : static_cast<const T*>(p.w));
+            const V4 zero = {static_cast<T>(0.f), static_cast<T>(0.f), static_cast<T>(0.f), static_cast<T>(0.f)};
+            braw[a][g] = there ? raw : zero;
+        }
+
+    __syncthreads();   // the ring is used up
+    // ── epilogue: acc[a][b][4g + i] is feature n0 + (wn TN + a) 32 + 8g + 4 lh + i of token m0 + (wm TM + b) 32 + lq; the tile
+    //    leaves through LDS as 16-byte pieces of rows of Y ──
+    if constexpr (GEGLU) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int feat = wn * 32 + 8 * g + 4 * lh;
+            float sv[4] = {1.f, 1.f, 1.f, 1.f}, sg[4] = {1.f, 1.f, 1.f, 1.f};
+            if constexpr (W8) {
+                if (n0 + feat < p.N) {   // N is a multiple of 8, so the 4 features are in or out together
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) { sv[i] = p.w_scale[n0 + feat + i]; sg[i] = p.w_scale[p.N + n0 + feat + i]; }
+                }
+            }
+#pragma unroll
+            for (int b = 0; b < TM; ++b) {
+                    V4 o;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float bv = static_cast<float>(braw[0][g][i]), bg = static_cast<float>(braw[1][g][i]);
+                        float val, gate;
+                        if constexpr (W8) {   // the two halves are rounded where the reference's 16-bit intermediate would
+                            val = static_cast<float>(static_cast<T>(scaled_acc(acc[0][b][4 * g + i], sv[i], bv)));
+                            gate = static_cast<float>(static_cast<T>(scaled_acc(acc[1][b][4 * g + i], sg[i], bg)));
+                        } else {
+                            val = acc[0][b][4 * g + i] + bv;
+                            gate = acc[1][b][4 * g + i] + bg;
+                        }
+                        o[i] = static_cast<T>(val * gelu_erf(gate));
+                    }
+                    *reinterpret_cast<V4*>(lds + ((wm * TM + b) * 32 + lq) * G::OUT_ROW + feat * 2) = o;
+                }
+        }
+    } else {
+#pragma unroll
+        for (int a = 0; a < TN; ++a)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int feat = (wn * TN + a) * 32 + 8 * g + 4 * lh;
+                float sc[4] = {1.f, 1.f, 1.f, 1.f};
+                if constexpr (W8) {
+                    if (n0 + feat < p.N) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) sc[i] = p.w_scale[n0 + feat + i];
+                    }
+                }
+#pragma unroll
+                for (int b = 0; b < TM; ++b) {
+                        V4 o;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const float bv = static_cast<float>(braw[a][g][i]);
+                            if constexpr (W8) o[i] = static_cast<T>(scaled_acc(acc[a][b][4 * g + i], sc[i], bv));
+                            else o[i] = static_cast<T>(acc[a][b][4 * g + i] + bv);
+                        }
+                        *reinterpret_cast<V4*>(lds + ((wm * TM + b) * 32 + lq) * G::OUT_ROW + feat * 2) = o;
+                    }
+            }
+    }
+    __syncthreads();
+    unsigned char* const yg = static_cast<unsigned char*>(p.y);
+    constexpr int PPR = BN_OUT / 8;   // 16-byte pieces per staged row
+#pragma unroll
+    for (int idx = tid; idx < BM * PPR; idx += G::NT) {
+        const int row = idx / PPR, piece = idx % PPR;
+        if (m0 + row < p.M && n0 + piece * 8 < p.N)
+            *reinterpret_cast<u32x4*>(yg + (static_cast<long>(m0 + row) * p.ldy + n0 + piece * 8) * 2) =
+                *reinterpret_cast<const u32x4*>(lds + row * G::OUT_ROW + piece * 16);
+    }
+}
+
+template <typename T, bool W8, bool GEGLU, int WM, int WN, int TM, int TN, int S>
+int launch_pipe(const LinearBatch& batch, int n_problems, hipStream_t st) {
+    using G = PipeGeo<T, W8, GEGLU, WM, WN, TM, TN, S>;
+    long tiles = 0;
+    for (int i = 0; i < n_problems; ++i)
+        tiles += static_cast<long>((batch.p[i].M + G::BM - 1) / G::BM) * ((batch.p[i].N + G::BN_OUT - 1) / G::BN_OUT);
+    PanelWidths panels{};
+    for (int i = 0; i < n_problems; ++i) {
+        const int tiles_n = (batch.p[i].N + G::BN_OUT - 1) / G::BN_OUT;
+        panels.w[i] = min(tiles_n, max(1, static_cast<int>(std::sqrt(static_cast<double>(tiles) / 8 * G::BM / G::BN) + 0.5)));
+    }
+    if (tiles > 0x7ffffff0L) return fail("linear: problem too large for one launch");
+    if (G::LDS > 64 * 1024) {
+        static thread_local bool raised = false;
+        if (!raised) {
+            MI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&linear_pipe_kernel<T, W8, GEGLU, WM, WN, TM, TN, S>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS));
+            raised = true;
+        }
+    }
+    hipLaunchKernelGGL((linear_pipe_kernel<T, W8, GEGLU, WM, WN, TM, TN, S>), dim3(static_cast<unsigned>((tiles + 7) / 8 * 8)), dim3(G::NT), G::LDS, st,
+                       batch, n_problems, panels);
+    MI_HIP_CHECK(hipGetLastError());
+    return 0;
+}
+
+// ── which form a launch takes ──
+// A launch of n tiles on a GPU of C compute units costs about
+//     phi + steps lam + (m - 1) (steps tau + eps),   m = ceil(n / C) tiles on the busiest compute unit,
+// with steps = K / 64: phi what a launch of one tile per compute unit costs beyond its steps (start, first loads, write-out), lam
+// a step when the compute unit has one tile, tau and eps a step and the rest of every further tile. The constants (us) are fitted
+// to 90 problems between 32 x 1280 x 1280 and 4096 x 6720 x 2240 on MI355X, rms error 6 to 13 %; the form with the
+// smallest estimate is within 1 % of the fastest one on average, 14 % at worst. Large tiles need fewer bytes per FLOP
+// (a step of 128 x 128 moves 32 KB for 0.5 us of a saturated compute unit), small ones fill the GPU: 128 x 1280 x 1280
+// takes 6 us with 80 tiles of 64 x 32, 8 with 20 of 128 x 64, 16 with 10 of 256 x 128; 1024 x 2240 x 2240 takes 18 us
+// with 144 tiles of 128 x 128, 24 with 288 of 128 x 64, 50 with 36 of 256 x 256.
+struct Form {
+    int bm, bn_out;
+    float phi, lam, tau, eps;
+};
+enum { k64x32, k64x64, k128x64, k128x128, k128x128_2, k256x128, k256x256, kPlainForms };
+constexpr Form kPlain[kPlainForms] = {
+    {64, 32, 2.8f, 0.164f, 0.129f, 0.5f},   {64, 64, 2.8f, 0.199f, 0.197f, 0.9f},   {128, 64, 3.5f, 0.289f, 0.319f, 1.2f}, {128, 128, 4.6f, 0.350f, 0.556f, 3.8f},
+    {128, 128, 3.9f, 0.617f, 0.380f, 3.5f}, {256, 128, 5.7f, 0.613f, 0.920f, 7.0f}, {256, 256, 8.3f, 1.216f, 1.888f, 8.6f}};
+// INT8 weights: the widening makes small steps dearer and the large tiles no better (the 256-row forms are not built)
+constexpr Form kPlainW8[] = {
+    {64, 32, 1e9f, 0.f, 0.f, 0.f},          {64, 64, 3.1f, 0.257f, 0.149f, 1.1f},   {128, 64, 4.2f, 0.315f, 0.237f, 1.7f}, {128, 128, 5.3f, 0.370f, 0.609f, 3.6f},
+    {128, 128, 4.9f, 0.644f, 0.390f, 2.3f}, {256, 128, 1e9f, 0.f, 0.f, 0.f},        {256, 256, 1e9f, 0.f, 0.f, 0.f}};
+enum { kG64x64, kG128x64, kG256x64, kGegluForms };   // output features; the W tile holds twice as many rows
+constexpr Form kGeglu[kGegluForms] = {{64, 64, 3.2f, 0.378f, 0.282f, 1.8f}, {128, 64, 5.9f, 0.628f, 0.217f, 4.5f}, {256, 64, 7.5f, 0.674f, 0.957f, 7.7f}};
+constexpr Form kGegluW8[kGegluForms] = {{64, 64, 4.2f, 0.427f, 0.298f, 2.0f}, {128, 64, 6.5f, 0.682f, 0.384f, 3.3f}, {256, 64, 8.2f, 0.866f, 1.007f, 8.2f}};
+
+// 256 x 256 tiles take contractions from 512 on (below, their prologue is most of the launch).
+int pick_form(const Form* forms, int n_forms, const LinearBatch& batch, int n_problems) {
+    const int n_cu = device_cu_count();
+    int best = 0;
+    double best_cost = 1e30;
+    for (int f = 0; f < n_forms; ++f) {
+        long tiles = 0;
+        int k = 0;
+        for (int i = 0; i < n_problems; ++i) {
+            const LinearProblem& p = batch.p[i];
+            tiles += static_cast<long>((p.M + forms[f].bm - 1) / forms[f].bm) * ((p.N + forms[f].bn_out - 1) / forms[f].bn_out);
+            k = max(k, p.K);
+        }
+        if (forms[f].bn_out == 256 && k < 512) continue;
+        const double steps = k / kBK, m = static_cast<double>((tiles + n_cu - 1) / n_cu);
+        const double cost = forms[f].phi + steps * forms[f].lam + (m - 1) * (steps * forms[f].tau + forms[f].eps);
+        if (cost < best_cost) { best_cost = cost; best = f; }
+    }
+    return best;
+}
+
+template <typename T>
+int launch_form(const LinearBatch& b, int n, bool geglu, int dtype, hipStream_t st) {
+    const bool w8 = b.p[0].w_scale != nullptr;
+    if (geglu) {
+        switch (pick_form(w8 ? kGegluW8 : kGeglu, kGegluForms, b, n)) {
+            case kG64x64: return w8 ? launch_pipe<T, true, true, 2, 2, 1, 2, 3>(b, n, st) : launch_pipe<T, false, true, 2, 2, 1, 2, 3>(b, n, st);
+            case kG128x64: return w8 ? launch_pipe<T, true, true, 2, 2, 2, 2, 2>(b, n, st) : launch_pipe<T, false, true, 2, 2, 2, 2, 2>(b, n, st);
+            default: return w8 ? launch_pipe<T, true, true, 4, 2, 2, 2, 3>(b, n, st) : launch_pipe<T, false, true, 4, 2, 2, 2, 3>(b, n, st);
+        }
+    }
+    if (w8) {
+        switch (pick_form(kPlainW8, kPlainForms, b, n)) {
+            case k64x64: return launch_pipe<T, true, false, 2, 2, 1, 1, 4>(b, n, st);
+            case k128x64: return launch_pipe<T, true, false, 2, 2, 2, 1, 3>(b, n, st);
+            case k128x128: return launch_pipe<T, true, false, 2, 4, 2, 1, 4>(b, n, st);
+            default: return launch_pipe<T, true, false, 2, 2, 2, 2, 2>(b, n, st);
+        }
+    }
+    switch (pick_form(kPlain, kPlainForms, b, n)) {
+        case k64x32: return launch_pipe<T, false, false, 2, 1, 1, 1, 4>(b, n, st);
+        case k64x64: return launch_pipe<T, false, false, 2, 2, 1, 1, 4>(b, n, st);
+        case k128x64: return launch_pipe<T, false, false, 2, 2, 2, 1, 3>(b, n, st);
+        case k128x128: return launch_pipe<T, false, false, 2, 4, 2, 1, 4>(b, n, st);
+        case k128x128_2: return launch_pipe<T, false, false, 2, 2, 2, 2, 2>(b, n, st);
+        case k256x128: return launch_pipe<T, false, false, 4, 2, 2, 2, 3>(b, n, st);
+        default: return launch_linear_dma(b, n, dtype, st);
+    }
+}
+
+}  // namespace
+}  // namespace gemm
+
+// Contractions of whole stages; operands whose tiles (GEGLU: whose whole W) are addressable with 32-bit byte offsets.
+bool linear_pipe_takes(const LinearBatch& batch, int n_problems, bool geglu) {
+    for (int i = 0; i < n_problems; ++i) {
+        const LinearProblem& p = batch.p[i];
+        if (p.K % gemm::kBK != 0) return false;
+        if (p.w_scale != nullptr && (p.ldw % 16 != 0)) return false;   // (rows of 16-byte pieces)
+        if (static_cast<long>(p.ldx) * 2 * 256 >= (1L << 31) || static_cast<long>(p.ldw) * 2 * 256 >= (1L << 31)) return false;
+        if (geglu && static_cast<long>(p.N) * 2 * p.ldw * 2 >= (1L << 32)) return false;
+    }
+    return true;
+}
+
+int launch_linear_pipe(const LinearBatch& batch, int n_problems, int dtype, bool geglu, hipStream_t st) {
+    if (dtype == MI_DTYPE_BF16) return gemm::launch_form<__bf16>(batch, n_problems, geglu, dtype, st);
+    return gemm::launch_form<_Float16>(batch, n_problems, geglu, dtype, st);
+}
+
+}  // namespace mi

@@ -1,0 +1,92 @@
+"""The projection GEMM's forms with LDS-DMA operand rings at the sizes where they can go wrong: contractions of fewer stages
+than the ring has, exactly as many and one more; one row, one 8-feature piece past a tile; every tile size the dispatch
+knows, 16-bit and INT8 weights, plain and GEGLU; three problems of different sizes in one launch. Against the CPU checker, one
+unit in the last place of the result's magnitude (FP32 accumulation and one rounding, as in tests/test_attn_block_gpu.py)."""
+import numpy as np
+import pytest
+import torch
+
+import brodiffusion_amd as bd
+from helpers import randn, to_dev, to_np
+
+pytestmark = pytest.mark.gpu
+
+
+def _weight(oracle, seed, n_out, n_in, dtype):
+    return oracle.round_to(randn(seed, (n_out, n_in), "fp32") / np.sqrt(n_in), dtype)
+
+
+def _int8(seed, n_out, n_in):
+    rng = np.random.default_rng(seed)
+    return rng.integers(-128, 128, (n_out, n_in)).astype(np.int8), (rng.uniform(0.5, 1.5, (n_out, 1)) / (74.0 * np.sqrt(n_in))).astype(np.float32)
+
+
+def _one_ulp(ref, got, dtype, what):
+    unit = 2.0 ** -8 if dtype == "bf16" else 2.0 ** -11
+    assert np.isfinite(got).all(), what
+    assert np.all(np.abs(got - ref) <= unit * np.maximum(np.abs(ref), 2.0 ** -6) * 1.05 + 2e-6), what
+
+
+def _rows(M):
+    return np.unique(np.concatenate([[0, M - 1], np.arange(31, M, 97), [r for t in (64, 128, 256) for r in (t - 1, t, M // t * t - 1, M // t * t) if 0 <= r < M]]))
+
+
+SHAPES = [(65, 40, 64), (65, 40, 128), (63, 32, 192), (1, 8, 256), (130, 96, 320),          # 64 x 32 tiles; 1 to 5 stages, ring of 4
+          (513, 1288, 1280), (2049, 648, 640),                                              # 64 x 64, 128 x 64
+          (1030, 2248, 2240), (8200, 1032, 128), (4099, 1160, 1152)]                        # 128 x 128 twice, 256 x 128
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_pipe_linear_matches_checker(oracle, dtype, M, N, K):
+    x, w, b = randn(81 + M, (M, K), dtype), _weight(oracle, 82 + N, N, K, dtype), randn(83 + K, (N,), dtype)
+    y = to_np(bd.linear_batched(to_dev(w, dtype), to_dev(b, dtype), to_dev(x, dtype)))
+    r = _rows(M)
+    _one_ulp(oracle.linear(x[r], w, b), y[r], dtype, f"linear {M}x{N}x{K}")
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("M,N,K", SHAPES[:8])
+def test_pipe_linear_int8_matches_checker(oracle, dtype, M, N, K):
+    x, b = randn(91 + M, (M, K), dtype), randn(93 + K, (N,), dtype)
+    w, s = _int8(92 + N, N, K)
+    y = to_np(bd.linear_forward_batched_int8w_fp16(torch.from_numpy(w).cuda(), torch.from_numpy(s).cuda(), to_dev(b, dtype), to_dev(x, dtype)))
+    r = _rows(M)
+    _one_ulp(oracle.linear(x[r], w.astype(np.float32)) * s.reshape(1, -1) + b, y[r], dtype, f"linear int8 {M}x{N}x{K}")
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("int8", [False, True], ids=["w16", "w8"])
+@pytest.mark.parametrize("M,N,K", [(65, 72, 64), (127, 8, 128), (129, 200, 320), (1030, 2568, 640), (770, 5128, 1280)])
+def test_pipe_geglu_is_the_linear_layer_and_the_gate(oracle, dtype, int8, M, N, K):
+    """Against the checker's linear layer in FP32 followed by y = v gelu(g). Bound: one unit u of the output's magnitude; with
+    INT8 weights v and g are rounded to the dtype on both sides, and a sum at a rounding boundary may go either way: another
+    u |y| from v and u |g| |v gelu'(g)| <= 1.13 u |v g| from g."""
+    import math
+    x, b = randn(101 + M, (M, K), dtype), randn(103 + K, (2 * N,), dtype)
+    r = _rows(M)
+    if int8:
+        w, s = _int8(102 + N, 2 * N, K)
+        y = bd.fused_linear_geglu_int8w(to_dev(x, dtype), torch.from_numpy(w).cuda(), torch.from_numpy(s).cuda(), to_dev(b, dtype))
+        lin = oracle.round_to((oracle.linear(x[r], w.astype(np.float32)) * s.reshape(1, -1) + b).astype(np.float32), dtype)
+    else:
+        w = _weight(oracle, 102 + N, 2 * N, K, dtype)
+        y = bd.fused_linear_geglu(to_dev(x, dtype), to_dev(w, dtype), to_dev(b, dtype))
+        lin = oracle.linear(x[r], w, b)
+    gate = lin[:, N:].astype(np.float64)
+    ref = (lin[:, :N] * gate * 0.5 * (1.0 + np.vectorize(math.erf)(gate / math.sqrt(2.0)))).astype(np.float32)
+    unit = 2.0 ** -8 if dtype == "bf16" else 2.0 ** -11
+    bound = unit * (np.abs(ref) + (np.abs(ref) + 1.13 * np.abs(lin[:, :N] * gate) if int8 else 0.0)) * 1.05 + 2e-6
+    assert np.all(np.abs(to_np(y)[r] - ref) <= bound), f"geglu {M}x{N}x{K} int8={int8}"
+
+
+def test_pipe_three_unequal_problems_in_one_launch(oracle):
+    """Q from 300 rows of 320 channels, K and V from 77 rows of 768: tiles of all three problems in one row, different
+    contractions. The block equals its parts bit for bit (every form accumulates in the same order)."""
+    dtype, L, Lc, C, Cc, H = "fp16", 300, 77, 320, 768, 8
+    x, ctx = to_dev(randn(111, (L, C), dtype), dtype), to_dev(randn(112, (Lc, Cc), dtype), dtype)
+    wq, wo = (to_dev(_weight(oracle, 113 + i, C, C, dtype), dtype) for i in range(2))
+    wk, wv = (to_dev(_weight(oracle, 115 + i, C, Cc, dtype), dtype) for i in range(2))
+    out = bd.flash_attention_qkvo_forward(x, ctx, wq, None, wk, None, wv, None, wo, None, None, H, False)
+    q, k, v = bd.linear_batched(wq, None, x), bd.linear_batched(wk, None, ctx), bd.linear_batched(wv, None, ctx)
+    assert torch.equal(bd.linear_batched(wo, None, bd.flash_attention_forward(q, k, v, None, H, False)), out)
