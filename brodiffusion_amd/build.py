@@ -96,6 +96,30 @@ def build_host(with_test: bool = True, verbose: bool = False) -> str:
     return HOST_LIB
 
 
+NATIVE = os.path.join(HERE, "_native.so")
+
+
+def build_native(verbose: bool = False) -> str:
+    """The extension module behind ops.py (CPython C API and torch's C++ headers; no HIP code in it; g++)."""
+    import sysconfig
+
+    from torch.utils import cpp_extension
+    import torch
+    cmd = [CXX, "-std=c++20", "-O2", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I" + os.path.join(ROOT, "include"),
+           "-I" + sysconfig.get_paths()["include"], *("-isystem" + p for p in cpp_extension.include_paths("cuda")),
+           os.path.join(HOST_DIR, "py_ops.cpp"), "-o", NATIVE, *("-L" + p for p in cpp_extension.library_paths("cuda")),
+           "-ltorch_python", "-ltorch_cpu", "-ltorch", "-lc10", "-lc10_hip", "-ldl"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        sys.stderr.write(r.stdout + r.stderr)
+        raise RuntimeError("native host module build failed")
+    if verbose:
+        print("built", NATIVE)
+    return NATIVE
+
+
 if __name__ == "__main__":
     build(save_temps="--save-temps" in sys.argv, verbose=True)
     build_host(verbose=True)
+    build_native(verbose=True)

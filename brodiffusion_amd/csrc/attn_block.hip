@@ -82,6 +82,29 @@ int attend(const mi_attn_block_args* a, const BlockDims& d, const void* q, const
     return mi_sdpa_forward(&s);
 }
 
+LinearProblem problem_of(const mi_linear_args& a) {
+    LinearProblem p = problem(a.x, a.w, a.bias, a.y, a.rows, a.out_features, a.in_features, a.w_scales);
+    if (a.x_row_stride) p.ldx = a.x_row_stride;
+    if (a.w_row_stride) p.ldw = a.w_row_stride;
+    if (a.y_row_stride) p.ldy = a.y_row_stride;
+    return p;
+}
+
+int linear_n(const mi_linear_args* a, int n, const char* op) {
+    clear_error();
+    if (!a) return fail("%s: null args", op);
+    LinearBatch b;
+    std::memset(&b, 0, sizeof(b));
+    int used = 0;
+    for (int i = 0; i < n; ++i) {
+        if (a[i].struct_size != sizeof(mi_linear_args)) return fail("%s: struct_size %u != %zu (header mismatch)", op, a[i].struct_size, sizeof(mi_linear_args));
+        if (a[i].rows < 0) return fail("%s: negative rows", op);
+        if (a[i].dtype != a[0].dtype) return fail("%s: one dtype per launch", op);
+        if (a[i].rows > 0) b.p[used++] = problem_of(a[i]);
+    }
+    return used == 0 ? 0 : launch_linear(b, used, a[0].dtype, resolve_stream(a[0].stream));
+}
+
 }  // namespace
 }  // namespace mi
 
@@ -89,20 +112,12 @@ using mi::fail;
 
 extern "C" {
 
-int mi_linear_forward(const mi_linear_args* a) {
+int mi_linear_forward(const mi_linear_args* a) { return mi::linear_n(a, 1, "mi_linear_forward"); }
+
+int mi_linear_forward_n(const mi_linear_args* a, int32_t n) {
     mi::clear_error();
-    if (!a) return fail("mi_linear_forward: null args");
-    if (a->struct_size != sizeof(mi_linear_args))
-        return fail("mi_linear_forward: struct_size %u != %zu (header mismatch)", a->struct_size, sizeof(mi_linear_args));
-    if (a->rows < 0) return fail("mi_linear_forward: negative rows");
-    if (a->rows == 0) return 0;
-    mi::LinearBatch b;
-    std::memset(&b, 0, sizeof(b));
-    b.p[0] = mi::problem(a->x, a->w, a->bias, a->y, a->rows, a->out_features, a->in_features, a->w_scales);
-    if (a->x_row_stride) b.p[0].ldx = a->x_row_stride;
-    if (a->w_row_stride) b.p[0].ldw = a->w_row_stride;
-    if (a->y_row_stride) b.p[0].ldy = a->y_row_stride;
-    return mi::launch_linear(b, 1, a->dtype, mi::resolve_stream(a->stream));
+    if (n < 1 || n > mi::kMaxLinearProblems) return fail("mi_linear_forward_n: %d layers in one launch (1..%d)", n, mi::kMaxLinearProblems);
+    return mi::linear_n(a, n, "mi_linear_forward_n");
 }
 
 int mi_linear_geglu_forward(const mi_linear_args* a) {
@@ -114,10 +129,7 @@ int mi_linear_geglu_forward(const mi_linear_args* a) {
     if (a->rows == 0) return 0;
     mi::LinearBatch b;
     std::memset(&b, 0, sizeof(b));
-    b.p[0] = mi::problem(a->x, a->w, a->bias, a->y, a->rows, a->out_features, a->in_features, a->w_scales);
-    if (a->x_row_stride) b.p[0].ldx = a->x_row_stride;
-    if (a->w_row_stride) b.p[0].ldw = a->w_row_stride;
-    if (a->y_row_stride) b.p[0].ldy = a->y_row_stride;
+    b.p[0] = mi::problem_of(*a);
     return mi::launch_linear(b, 1, a->dtype, mi::resolve_stream(a->stream), true);
 }
 

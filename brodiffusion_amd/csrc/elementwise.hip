@@ -52,10 +52,14 @@ __global__ void __launch_bounds__(256) add_row_bias_kernel(T* y, const T* bias, 
 
 // RMS normalisation of whole rows: one work group per row (grid-stride over rows), the row held in registers between
 // the sum of squares and the scaling (up to kRmsChunks 16-byte chunks per thread), FP32 arithmetic, one rounding.
+// blockIdx.y: which of up to two tensors (q and k of one call site share a launch: 1024 x 2240 twice, 7 -> 4 us).
+template <typename T> struct RmsOperands { const T* x; const T* gain; T* out; };
 constexpr int kRmsChunks = 8;   // 256 threads x 8 chunks x 8 elements = rows of up to 16384 columns
 template <typename T>
-__global__ void __launch_bounds__(256) rms_norm_rows_kernel(const T* x, const T* __restrict__ gain, T* out, int rows, int cols,
-                                                            long x_rs, long o_rs, float eps) {
+__global__ void __launch_bounds__(256) rms_norm_rows_kernel(RmsOperands<T> a, RmsOperands<T> b, int rows, int cols, long x_rs, long o_rs, float eps) {
+    const T* const x = blockIdx.y == 0 ? a.x : b.x;
+    const T* const gain = blockIdx.y == 0 ? a.gain : b.gain;
+    T* const out = blockIdx.y == 0 ? a.out : b.out;
     typedef T t8 __attribute__((ext_vector_type(8)));
     __shared__ float red[4];
     const int cpr = cols / 8;
@@ -95,6 +99,34 @@ __global__ void __launch_bounds__(256) rms_norm_rows_kernel(const T* x, const T*
 long grid_for(long work) {
     long blocks = (work + 255) / 256;
     return blocks < 1 ? 1 : (blocks > 256 * 32 ? 256 * 32 : blocks);
+}
+
+int rms_norm_n(const char* op, int n, const void* x0, const void* gain0, void* out0, const void* x1, const void* gain1, void* out1, int rows, int cols,
+               int64_t x_row_stride, int64_t out_row_stride, float eps, int dtype, void* stream) {
+    clear_error();
+    if (rows < 0 || cols <= 0 || cols % 8 != 0) return fail("%s: cols must be a positive multiple of 8, rows >= 0", op);
+    if (cols > 256 * 8 * kRmsChunks) return fail("%s: rows of more than %d columns are not supported", op, 256 * 8 * kRmsChunks);
+    if (rows == 0) return 0;
+    if (!x0 || !gain0 || !out0 || !x1 || !gain1 || !out1) return fail("%s: null tensor", op);
+    if (!(eps >= 0.f)) return fail("%s: eps must be >= 0", op);
+    const long x_rs = x_row_stride ? x_row_stride : cols, o_rs = out_row_stride ? out_row_stride : cols;
+    if (x_rs < cols || o_rs < cols || x_rs % 8 != 0 || o_rs % 8 != 0) return fail("%s: row strides must be multiples of 8 elements and at least cols", op);
+    uintptr_t al = 0;
+    for (const void* p : {x0, gain0, static_cast<const void*>(out0), x1, gain1, static_cast<const void*>(out1)}) al |= reinterpret_cast<uintptr_t>(p);
+    if (al & 15u) return fail("%s: pointers must be 16-byte aligned", op);
+    const dim3 grid(static_cast<unsigned>(rows < 256 * 16 ? rows : 256 * 16), n);
+    auto launch = [&](auto tag) {
+        using T = decltype(tag);
+        const RmsOperands<T> a{static_cast<const T*>(x0), static_cast<const T*>(gain0), static_cast<T*>(out0)};
+        const RmsOperands<T> b{static_cast<const T*>(x1), static_cast<const T*>(gain1), static_cast<T*>(out1)};
+        hipLaunchKernelGGL(rms_norm_rows_kernel<T>, grid, dim3(256), 0, resolve_stream(stream), a, b, rows, cols, x_rs, o_rs, eps);
+    };
+    if (dtype == MI_DTYPE_BF16) launch(__bf16{});
+    else if (dtype == MI_DTYPE_F16) launch(_Float16{});
+    else return fail("%s: dtype %d not supported", op, dtype);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail("%s launch: %s", op, hipGetErrorString(e));
+    return 0;
 }
 
 }  // namespace
@@ -147,30 +179,12 @@ int mi_add_row_bias(void* y, const void* bias, int32_t rows, int32_t cols, int64
 
 int mi_rms_norm_forward(const void* x, const void* gain, void* out, int32_t rows, int32_t cols, int64_t x_row_stride,
                         int64_t out_row_stride, float eps, int32_t dtype, void* stream) {
-    mi::clear_error();
-    if (rows < 0 || cols <= 0 || cols % 8 != 0) return fail("mi_rms_norm_forward: cols must be a positive multiple of 8, rows >= 0");
-    if (cols > 256 * 8 * mi::kRmsChunks) return fail("mi_rms_norm_forward: rows of more than %d columns are not supported", 256 * 8 * mi::kRmsChunks);
-    if (rows == 0) return 0;
-    if (!x || !gain || !out) return fail("mi_rms_norm_forward: null tensor");
-    if (!(eps >= 0.f)) return fail("mi_rms_norm_forward: eps must be >= 0");
-    const long x_rs = x_row_stride ? x_row_stride : cols, o_rs = out_row_stride ? out_row_stride : cols;
-    if (x_rs < cols || o_rs < cols || x_rs % 8 != 0 || o_rs % 8 != 0)
-        return fail("mi_rms_norm_forward: row strides must be multiples of 8 elements and at least cols");
-    if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(gain) | reinterpret_cast<uintptr_t>(out)) & 15u)
-        return fail("mi_rms_norm_forward: pointers must be 16-byte aligned");
-    hipStream_t st = mi::resolve_stream(stream);
-    const dim3 grid(static_cast<unsigned>(rows < 256 * 16 ? rows : 256 * 16));
-    if (dtype == MI_DTYPE_BF16)
-        hipLaunchKernelGGL(mi::rms_norm_rows_kernel<__bf16>, grid, dim3(256), 0, st, static_cast<const __bf16*>(x), static_cast<const __bf16*>(gain),
-                           static_cast<__bf16*>(out), rows, cols, x_rs, o_rs, eps);
-    else if (dtype == MI_DTYPE_F16)
-        hipLaunchKernelGGL(mi::rms_norm_rows_kernel<_Float16>, grid, dim3(256), 0, st, static_cast<const _Float16*>(x), static_cast<const _Float16*>(gain),
-                           static_cast<_Float16*>(out), rows, cols, x_rs, o_rs, eps);
-    else
-        return fail("mi_rms_norm_forward: dtype %d not supported", dtype);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return fail("mi_rms_norm_forward launch: %s", hipGetErrorString(e));
-    return 0;
+    return mi::rms_norm_n("mi_rms_norm_forward", 1, x, gain, out, x, gain, out, rows, cols, x_row_stride, out_row_stride, eps, dtype, stream);
+}
+
+int mi_rms_norm_pair_forward(const void* x0, const void* gain0, void* out0, const void* x1, const void* gain1, void* out1, int32_t rows, int32_t cols,
+                             int64_t x_row_stride, int64_t out_row_stride, float eps, int32_t dtype, void* stream) {
+    return mi::rms_norm_n("mi_rms_norm_pair_forward", 2, x0, gain0, out0, x1, gain1, out1, rows, cols, x_row_stride, out_row_stride, eps, dtype, stream);
 }
 
 }  // extern "C"

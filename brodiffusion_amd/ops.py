@@ -40,6 +40,26 @@ import torch
 from . import _capi as capi
 
 
+class _Unbuilt:
+    """Stands for the native module until it is bound: the first call binds it, and fails loudly where it is not built."""
+
+    def __getattr__(self, name):
+        global _native
+        capi.lib()
+        try:
+            from . import _native as module
+        except ImportError as e:
+            raise RuntimeError(f"brodiffusion_amd._native cannot be loaded ({e}): build it first (python -m brodiffusion_amd.build)") from e
+        module.bind(capi.LIB_PATH, lambda index, nbytes: _own_split_scratch(torch.device("cuda", index), nbytes))
+        _native = module
+        return getattr(module, name)
+
+
+# The calls below try the native form first (host/py_ops.cpp). It returns None, having done nothing, unless the call is plainly
+# valid; the Python code behind it then finds what is wrong, and words it.
+_native = _Unbuilt()
+
+
 @dataclass
 class SdpaMask:
     """Visibility rule of one attention call (see mi_sdpa_args in include/mi_attention.h)."""
@@ -162,6 +182,12 @@ def sdpa_forward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, num_heads: i
     """General entry: everything mi_sdpa_forward offers. Returns `out` (allocated like q if None).
     split_scratch: None = lend the module's own scratch (grown on demand, one per device, shared by all calls of the
     process: use one stream at a time) when the launch can use one, False = never split, a uint8 tensor = lend that."""
+    if logit_bias is None and lse_out is None and prefix_k_row_scale is None and prefix_v_row_scale is None and prefix_k_scale == 1.0 \
+            and prefix_v_scale == 1.0:
+        r = _native.sdpa(q, k, v, num_heads, out, num_kv_heads, k_prefix, v_prefix, scale, mask, kv_valid_len, key_mask, rope_q, rope_k,
+                         rope_k_scratch, rope_split_half, split_scratch, op)
+        if r is not None:
+            return r
     _dev(op, q, k, v, out, k_prefix, v_prefix, kv_valid_len, key_mask, rope_k_scratch)
     dt = _dtype_code(op, q)
     if k.dtype != q.dtype or v.dtype != q.dtype:
@@ -392,6 +418,9 @@ def linear_batched(W, bias, X, Y: Optional[torch.Tensor] = None, W_scales: Optio
                    op: str = "linear_batched"):
     """Y = X W^T + bias; W (out_features, in_features), X (..., in_features). With W_scales, W is INT8 and
     Y = (X W^T) * scales + bias (see linear_forward_batched_int8w_fp16)."""
+    r = _native.linear(W, bias, X, Y, W_scales, op)
+    if r is not None:
+        return r
     _dev(op, W, X)
     if W.dim() != 2 or X.shape[-1] != W.shape[1]:
         _fail(op, f"X has {X.shape[-1]} columns, W is {tuple(W.shape)}")
@@ -426,6 +455,9 @@ def fused_linear_geglu(X, W, b, Y: Optional[torch.Tensor] = None, W_scales: Opti
     """Y = a * gelu_exact(g), [a | g] = X W^T + b with W (2*D_out, D_in), b (2*D_out): the fused FF1 + GEGLU of the
     U-Net transformer block (brodiffusion::fused_linear_geglu, include/brodiffusion/fused_transformer.h:20-35). With
     W_scales, W is INT8 with one FP32 scale per row (see fused_linear_geglu_int8w)."""
+    r = _native.geglu(X, W, b, Y, W_scales, op)
+    if r is not None:
+        return r
     _dev(op, X, W, b, Y, W_scales)
     if W.dim() != 2 or W.shape[0] % 2 != 0 or X.shape[-1] != W.shape[1]:
         _fail(op, f"W must be (2*D_out, D_in) with D_in = {X.shape[-1]}, got {tuple(W.shape)}")
@@ -460,6 +492,9 @@ def fused_linear_geglu_int8w(X, W_int8, W_scales, b, Y: Optional[torch.Tensor] =
 
 def add_inplace_vec(Y, X):
     """Y += X, same shape and dtype (brodiffusion::add_inplace_vec, include/brodiffusion/fused_transformer.h:50-53)."""
+    r = _native.add_inplace(Y, X)
+    if r is not None:
+        return r
     op = "add_inplace_vec"
     _dev(op, Y, X)
     if tuple(Y.shape) != tuple(X.shape) or Y.dtype != X.dtype or not Y.is_contiguous() or not X.is_contiguous():
@@ -487,6 +522,9 @@ def flash_attention_scratch_bytes(batch: int, q_len: int, kv_len: int, inner: in
 
 def _attn_block(op: str, fn_name: str, X, Ctx, K, V, Wq, bq, Wk, bk, Wv, bv, Wo, bo, d_mask, num_heads, causal, out, scratch,
                 scales=(None, None, None, None)):
+    r = _native.attn_block(X, Ctx, K, V, Wq, bq, Wk, bk, Wv, bv, Wo, bo, d_mask, num_heads, causal, out, scratch, *scales, op)
+    if r is not None:
+        return r
     _dev(op, X, Ctx, K, V, Wq, Wk, Wv, Wo, d_mask, out, scratch)
     dt = X.dtype
     B, Lq, Cx, _, _ = _as3(op, X, "X")
@@ -623,6 +661,9 @@ def flash_attention_project_kv(ctx, Wk, bk, Wv, bv, K_out: Optional[torch.Tensor
 
 
 def _rope(op: str, X, cos, sin, head_dim, num_heads, out, per_head: bool, split_half: bool):
+    r = _native.rope(X, cos, sin, head_dim, num_heads, out, per_head, split_half, op)
+    if r is not None:
+        return r
     _dev(op, X, cos, sin, out)
     dt = _dtype_code(op, X)
     if X.dim() != 2 or X.stride(1) != 1:
@@ -691,6 +732,9 @@ def headnorm_rope(X, gain, eps: float, cos, sin, head_dim: int, num_heads: int, 
     one pass: per (row, head) RMS normalisation with `gain` (head_dim), then the rotation (cos = sin = None: the
     normalisation alone). cache_out (rows <= X's rows): its rows also receive the result — the prefix rows of K going
     into the prefix cache (qwenimage21_forward.cpp:587-597)."""
+    r = _native.headnorm_rope(X, gain, eps, cos, sin, head_dim, num_heads, out, cache_out, split_half)
+    if r is not None:
+        return r
     op = "headnorm_rope"
     _dev(op, X, gain, cos, sin, out, cache_out)
     if X.dim() != 2 or X.stride(1) != 1 or X.shape[1] != head_dim * num_heads:
@@ -733,6 +777,9 @@ def joint_attention(Q, K, V, cos, sin, head_dim: int, num_heads: int, out: Optio
     pass and, as in the reference, Kr holds RoPE(K) afterwards; without one K is rotated tile by tile
     inside the attention kernel (slower; adjacent pairs only). Qr is accepted and left untouched. split_half selects the
     pair convention of the rotation as in rope_apply."""
+    r = _native.joint(Q, K, V, cos, sin, head_dim, num_heads, out, Kr, split_half)
+    if r is not None:
+        return r
     op = "joint_attention"
     if Q.dim() != 2 or Q.shape[1] != head_dim * num_heads:
         _fail(op, "D must equal head_dim * num_heads")
@@ -847,9 +894,13 @@ def mha_forward(X, Wq, Wk, Wv, Wo, bq, bk, bv, bo, d_mask, num_heads: int, qh: O
                 yc: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None):
     """bt::mha_forward as PixArt's self attention calls it on the reference's FP32 path (src/dit/pixart.cpp:325-328):
     qh = X Wq^T + bq, kh, vh likewise, yc = attention(qh, kh, vh) with the optional key mask (float32 (L,), 1 = valid),
-    out = yc Wo^T + bo; biases may be None. For float16 / bfloat16 device tensors: four GEMMs and one attention launch,
+    out = yc Wo^T + bo; biases may be None. For float16 / bfloat16 device tensors: the three projections in one launch, attention, output
+    projection,
     intermediates in the caller's tensors when given. The scores are never materialised, so `attn` is ignored.
     Returns (out, qh, kh, vh, yc)."""
+    r = _native.mha(X, Wq, Wk, Wv, Wo, bq, bk, bv, bo, d_mask, num_heads, qh, kh, vh, yc, out)
+    if r is not None:
+        return r
     op = "mha_forward"
     _dev(op, X, Wq, Wk, Wv, Wo, bq, bk, bv, bo, d_mask, qh, kh, vh, yc, out)
     if X.dim() != 2:
@@ -926,6 +977,9 @@ def linear_attention_relu_forward(Q, K, V, num_heads: int, out: Optional[torch.T
     partial states of token chunks; None allocates one, False runs without (one work group per batch item and head).
     `form`: 0 = the library picks, 1 = three launches (state per token chunk, reduction, apply), 2 = one launch with the
     state split along its value channels (mi_linear_attn_args.form)."""
+    r = _native.linear_attn(Q, K, V, num_heads, out, eps, workspace, accumulate_state, scratch, form)
+    if r is not None:
+        return r
     op = "linear_attention_relu_forward"
     _dev(op, Q, K, V, out, workspace, scratch if scratch is not False else None)
     if out is None:
@@ -1011,6 +1065,9 @@ def linear_attention_relu_forward_static_scratch(Q, K, V, num_heads: int, out: t
 def rms_norm_rows(X, gain, eps: float, out: Optional[torch.Tensor] = None):
     """RMS normalisation of whole rows with a per-column gain: bt::rms_norm_forward(X, gain, eps, out) as Sana-Sprint's
     qk_norm uses it (src/dit/sana.cpp:449-461). X (rows, cols), gain (cols) of X's dtype; in place is allowed."""
+    r = _native.rms_norm(X, gain, eps, out)
+    if r is not None:
+        return r
     op = "rms_norm_rows"
     _dev(op, X, gain, out)
     dt = _dtype_code(op, X)
@@ -1036,6 +1093,10 @@ def sana_self_attention(x_mod, Wq, Wk, Wv, Wo, bo, num_heads: int, *, nq=None, n
     not exist here. ref_mode "capture" writes this call's (S, z) into ref_state (float32, heads x (head_dim + 1) x head_dim:
     S rows then z, the reference's FP32 cache layout, :489-497); "inject" adds ref_weight * ref_state to this call's state
     before the queries read it (:498-505) and leaves ref_state untouched."""
+    if ref_mode == "off" or (ref_mode == "capture" and ref_state is not None):
+        r = _native.sana(x_mod, Wq, Wk, Wv, Wo, bo, num_heads, nq, nk, rms_eps, attn_eps, None if ref_mode == "off" else ref_state, out)
+        if r is not None:
+            return r
     op = "sana_self_attention"
     _dev(op, x_mod, Wq, Wk, Wv, Wo, bo, nq, nk, ref_state, out)
     if x_mod.dim() != 2:

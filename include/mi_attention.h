@@ -407,6 +407,9 @@ typedef struct mi_linear_args {
     void* stream;
 } mi_linear_args;
 MI_API int mi_linear_forward(const mi_linear_args* args);
+/* 1 to 3 independent linear layers of one dtype and weight type in ONE launch on args[0]'s stream (the projections of an attention
+ * block: three times the work groups of one of them). Each result is bit for bit that of mi_linear_forward. */
+MI_API int mi_linear_forward_n(const mi_linear_args* args, int32_t n);
 /* Y (rows, out_features) = a * gelu_exact(g) with [a | g] = X W^T + bias, W (2*out_features, in_features) and bias
  * (2*out_features): value half first, gate half second; gelu_exact(g) = 0.5 g (1 + erf(g / sqrt 2)). The fused FF1 +
  * GEGLU of the U-Net transformer block, brodiffusion::fused_linear_geglu (include/brodiffusion/fused_transformer.h:20-35,
@@ -427,6 +430,9 @@ MI_API int mi_add_row_bias(void* y, const void* bias, int32_t rows, int32_t cols
  * (0 = dense), multiples of 8; gain (cols) of `dtype`; in place (out == x) is allowed. */
 MI_API int mi_rms_norm_forward(const void* x, const void* gain, void* out, int32_t rows, int32_t cols, int64_t x_row_stride,
                                int64_t out_row_stride, float eps, int32_t dtype, void* stream);
+/* Two tensors of one shape, each with its own gain, in one launch (the q and k of that call site). */
+MI_API int mi_rms_norm_pair_forward(const void* x0, const void* gain0, void* out0, const void* x1, const void* gain1, void* out1, int32_t rows,
+                                    int32_t cols, int64_t x_row_stride, int64_t out_row_stride, float eps, int32_t dtype, void* stream);
 
 /* ── attention with its projections ────────────────────────────────────────
  * The three operators the U-Net spatial transformer calls (src/unet_blocks.cpp:255-327,
