@@ -2,7 +2,7 @@
 // sdpa_common.h; launch_d picks one per call:
 //
 //   sdpa_fwd_kernel         4 wavefronts = 128 query rows per work group, K/V tiles through registers into padded LDS,
-//                           double buffered. Small problems, head_dim 160, calls with a key mask, a logit bias, a
+//                           double buffered. Few keys or few work groups (rows256_pay), head_dim 160, calls with a key mask, a logit bias, a
 //                           request for the softmax denominators, or packed variable-length sequences.
 //   sdpa_fwd_pp_kernel      8 wavefronts = 256 query rows, 2 wavefronts per SIMD, one work-group barrier per key tile:
 //                           between two barriers every wavefront runs the MFMA stream (O += V^T P of tile t, then
@@ -374,11 +374,13 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_shortkv_kernel(const SdpaDe
 // In the shadow of the stream the wavefront stores its share of tiles K_{t+2}, V_{t+1} into the LDS buffers
 // of K_t, V_{t-1} (last read in step t-1) and issues the global loads of K_{t+3}, V_{t+2}; two buffers per
 // operand suffice.
-// DENSE: as in the DMA form below (no mask, no prefix, whole key tiles only); instantiated for head_dim up to 64, where
-// it measures 2-3 % faster (at 80 the compiler's allocation of that instance goes wrong: twice as slow).
+// FORM: as in the DMA form below, without prefix; kDense and kRagged are instantiated for head_dim up to 64, where kDense
+// measures 2-3 % faster (at 80 the compiler's allocation of that instance goes wrong: twice as slow) and kRagged 17 %
+// (head_dim 40, 8 heads, 3600 tokens: 73.5 -> 61.1 us).
 // XTRA: key mask, logit bias and softmax denominators (see sdpa_fwd_pp_dma_kernel).
-template <typename T, int D, bool ROPE_K, bool DENSE = false, bool XTRA = false>
+template <typename T, int D, bool ROPE_K, int FORM = kGeneral, bool XTRA = false>
 __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_kernel(const SdpaDev p) {
+    constexpr bool DENSE = FORM != kGeneral, RAGGED = FORM == kRagged;
     static_assert(!XTRA || (!DENSE && !ROPE_K), "key mask, bias and denominators belong to the general form");
     using G = HeadGeo<D>;
     using V8 = typename Mma<T>::v8;
@@ -406,9 +408,10 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_kernel(const SdpaDev
     const T* const q_base = static_cast<const T*>(p.q) + b * p.q_bs + h * D;
     T* const o_base = static_cast<T*>(p.o) + b * p.o_bs + h * D;
 
-    int lo = 0, hi = p.Lk;   // DENSE: rows past the end of Q repeat its last row and are never stored
+    const int n_keys = RAGGED ? visible_keys(p, b) : p.Lk;
+    int lo = 0, hi = n_keys;   // DENSE: rows past the end of Q repeat its last row and are never stored
     if constexpr (!DENSE) row_interval(p, b, qrow, qvalid, lo, hi);
-    WaveExtent we{0, 0, p.Lk, p.Lk};
+    WaveExtent we{0, 0, n_keys, n_keys};
     if constexpr (!DENSE) {
         we = wave_extent(lo, hi);
         if (lane == 0) { red[wave] = we.lo_min; red[8 + wave] = we.hi_max; }
@@ -423,7 +426,7 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_kernel(const SdpaDev
     zero_pads<D, kThreads8>(Kbuf, Vbuf, G::K_BYTES, G::V_BYTES, 2, tid);
     for (int i = tid; i < 2 * G::V_BYTES / 16; i += kThreads8) *reinterpret_cast<u32x4*>(Vbuf + i * 16) = u32x4{0, 0, 0, 0};
     __syncthreads();
-    int g_lo = 0, kv_stop = p.Lk;
+    int g_lo = 0, kv_stop = n_keys;
     if constexpr (!DENSE) {
         g_lo = red[0]; kv_stop = red[8];
 #pragma unroll
@@ -452,7 +455,7 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_kernel(const SdpaDev
     const unsigned char* const v_head = reinterpret_cast<const unsigned char*>(static_cast<const T*>(p.v) + b * p.v_bs + hk * D);
     // (the dense launch is whole tiles of one segment: its mover does no arithmetic per tile)
     auto make_mover = [&]() {
-        if constexpr (DENSE) return DenseMover<T, D, kThreads8>(k_head, p.k_rs, v_head, p.v_rs, tid, wave);
+        if constexpr (DENSE) return DenseMover<T, D, kThreads8, RAGGED>(k_head, p.k_rs, v_head, p.v_rs, tid, wave, n_keys);
         else return TileMover<T, D, kThreads8, ROPE_K>{p, plan, k_head, v_head,
                                                        reinterpret_cast<const unsigned char*>(static_cast<const T*>(p.kp) + b * p.kp_bs + hk * D),
                                                        reinterpret_cast<const unsigned char*>(static_cast<const T*>(p.vp) + b * p.vp_bs + hk * D),
@@ -505,7 +508,8 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_kernel(const SdpaDev
         auto softmax_of = [&](int tt) {
             if constexpr (DENSE) {
                 if (tt >= 0 && tt < n_tiles) {
-                    softmax_tile_rel<T, D>(sacc, pf, oacc, st, false, false, 0, 0, p.Lk, lh);
+                    const int rows = RAGGED ? min(n_keys - tt * kBN, kBN) : kBN;
+                    softmax_tile_rel<T, D>(sacc, pf, oacc, st, RAGGED && rows < kBN, false, 0, 0, rows, lh);
                     return;
                 }
             }
@@ -619,15 +623,21 @@ __device__ __forceinline__ int swz(int row) { return 4 * (row & 3) + ((row >> 2)
 // SPLIT: the launch follows p.split — a work group either processes one whole query tile or one piece of the last
 // round, i.e. one or more (tile, key range) parts in sequence, each leaving a partial result in its scratch slot
 // (merged by sdpa_combine_kernel). Only for unmasked calls without prefix.
-// DENSE: no mask of any kind and key counts (cached prefix, if any, and fresh) that are multiples of 64: every tile is whole and visible to
-// every row, so the masked form of the softmax and the per-step bookkeeping (which tile, its limit, whether this
-// wavefront sees it whole) drop out of the kernel, and with them their registers: measured 6 % faster at head_dim 128
-// and 8 % at 72 than the general form on the same dense call.
+// FORM kDense: no mask of any kind and key counts (cached prefix, if any, and fresh) that are multiples of 64: every tile is
+// whole and visible to every row, so the masked form of the softmax and the per-step bookkeeping (which tile, its limit,
+// whether this wavefront sees it whole) drop out of the kernel, and with them their registers: measured 6 % faster at
+// head_dim 128 and 8 % at 72 than the general form on the same dense call.
+// FORM kRagged: every row sees the same keys, their number is free. All tiles but the last of a segment are as in kDense; that
+// one is met by scalar branches (DMA rows clamped to the last that exists, scores past it blanked). The general form clamps and
+// compares in every step, on the path that bounds this kernel (a wavefront's own chain of issue, MFMAs and softmax):
+// 24 heads of 128, 1997 tokens 65.3 -> 54.0 us, 2280 tokens + 669 cached 97.0 -> 81.6, 16 heads of 72, 3000 tokens 80.3 -> 64.6,
+// all within 4 % of the next multiple of 64 on kDense.
 // PSCALE: the general form with the prefix-KV dial (factors on the rows of the cached prefix) in its softmax.
 // XTRA: the general form with a key mask (one visibility bit per key, 64-bit words per key tile built once per work group
 // in LDS behind the rings), an additive logit bias and the softmax denominators as an output (traced attention).
-template <typename T, int D, bool SPLIT, bool DENSE = false, bool PSCALE = false, bool XTRA = false>
+template <typename T, int D, bool SPLIT, int FORM = kGeneral, bool PSCALE = false, bool XTRA = false>
 __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const SdpaDev p) {
+    constexpr bool DENSE = FORM != kGeneral, RAGGED = FORM == kRagged;
     static_assert(!(SPLIT && DENSE), "the split launch clips key ranges per part");
     static_assert(!PSCALE || (!SPLIT && !DENSE), "the dial belongs to the general form");
     static_assert(!XTRA || (!SPLIT && !DENSE && !PSCALE), "key mask, bias and denominators belong to the general form");
@@ -703,7 +713,7 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
     const T* const q_base = static_cast<const T*>(p.q) + b * p.q_bs + h * D;
     T* const o_base = static_cast<T*>(p.o) + b * p.o_bs + h * D;
 
-    const int n_keys = p.Lk;   // counts the cached prefix rows, which come first
+    const int n_keys = RAGGED ? visible_keys(p, b) : p.Lk;   // counts the cached prefix rows, which come first
     int lo = 0, hi = n_keys;   // DENSE: rows past the end of Q repeat its last row and are never stored
     if constexpr (!DENSE) row_interval(p, b, qrow, qvalid, lo, hi);
     if constexpr (SPLIT) {
@@ -773,7 +783,7 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
         drow[m] = row;
         dcol[m] = static_cast<unsigned>(cc) * 16u;
         if constexpr (DENSE) {
-            // whole tiles of one segment only: the lane's byte offset inside a tile never changes
+            // the lane's byte offset inside a (whole) tile never changes
             const bool is_k = DG::NDMA % 8 == 0 ? m < DG::MAXI / 2 : i < DG::NDMA;
             dcol[m] += static_cast<unsigned>(row) * (static_cast<unsigned>(is_k ? p.k_rs : p.v_rs) * 2u);
         }
@@ -785,6 +795,8 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
     auto dma = [&](const TileCursor& c, int m, int j, int lds_off) {
         unsigned voff = dcol[m];
         if constexpr (!DENSE) voff += static_cast<unsigned>(min(drow[m], min(c.rows_left, kBN) - 1)) * c.rsb;
+        // the last tile of a segment: rows past its end repeat the last one (a scalar branch, untaken for every other tile)
+        if (RAGGED && c.rows_left < kBN) voff -= static_cast<unsigned>(max(drow[m] - (c.rows_left - 1), 0)) * c.rsb;
         const unsigned dst = lds_base + lds_off + j * 1024;
         // (the LDS base travels in m0 as a declared input: the compiler writes the register itself and knows it is taken;
         //  the s_nop is the wait state an LDS-DMA instruction needs behind a write of m0)
@@ -873,7 +885,8 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
         auto softmax_of = [&](int tt) {
             if constexpr (DENSE) {
                 if (tt >= 0 && tt < n_tiles) {
-                    softmax_tile_rel<T, D>(sacc, pf, oacc, st, false, false, 0, 0, n_keys, lh);
+                    const int rows = RAGGED ? plan.limit(tt) - plan.j0(tt) : kBN;
+                    softmax_tile_rel<T, D>(sacc, pf, oacc, st, RAGGED && rows < kBN, false, 0, 0, rows, lh);
                     return;
                 }
             }
@@ -900,7 +913,7 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
         // LDS access ahead of it for a long time: right before its softmax.
         auto issue_dma = [&]() {
             issued = dma_tiles(load_k, KD, load_v, VD);
-            if (DENSE && p.Lp == 0) {
+            if (DENSE && !RAGGED && p.Lp == 0) {
                 if (load_k) kc.ptr += kBN * kc.rsb;
                 if (load_v) vc.ptr += kBN * vc.rsb;
             } else {
@@ -1170,6 +1183,40 @@ size_t split_scratch_bytes_d(SdpaDev p, int n_cu) {
     return static_cast<size_t>(8) * p.split.max_tail * p.split.max_parts * SplitGeo::slot_bytes(D);
 }
 
+// Every query row sees the same keys of its batch item: the kRagged form (and, with whole tiles, kDense) can take the call.
+bool same_keys_for_all_rows(const SdpaDev& p) {
+    return p.mask_mode == MI_MASK_NONE && !p.prefix_scaled && (p.Lp == 0 || (p.kp_rs == p.k_rs && p.vp_rs == p.v_rs));
+}
+
+// Whether a launch runs on 256-row tiles (8 wavefronts, two per SIMD, softmax of one under the MFMAs of the other) or on
+// 128-row tiles. With a 256-row tile or more per CU the former always. Below that the 128-row kernel keeps more CUs busy, but
+// each of them runs one wavefront per SIMD whose softmax nothing hides, and from the 257th work group on two share a CU
+// anyway ("crowded"); a CU with eight wavefronts needs 2/3 of the time per row and key, and costs about 1.5 us more to start
+// (rings, two-part Q staging). The lines are where the two sides met (us, 128-row / 256-row, one head count each):
+//   128, no mask:      T = 4 11.7 / 12.5, 6 14.9 / 15.0, 8 18.5 / 17.6, 16 31.3 / 27.2, 32 (192 tiles) 74 / 52; cross, 3 key
+//                      tiles, 216 query tiles 15.2 / 14.5, 96 query tiles 11.2 / 12.6
+//   72, no mask:       T = 4 11.5 / 11.3, cross with 4: 12.2 / 12.5, 9 19.5 / 17.7, 36 (144 tiles) 72 / 50
+//   40 and 64:         faster from one key tile on (6.1 / 5.7; 1024 tokens 24.4 / 18.1)
+//   128, 72 masked:    T = 8 18.8 / 19.6 and 18.0 / 17.7, 16 31.4 / 29.8 and 30.3 / 27.3, 32 (192 tiles, block-causal) 79 / 54
+//   80, 96, 112:       crowded only: 144 tiles of 80 72 / 64, 192 of 96 98 / 92, 128 of 80 102 / 114; masked never (96: 70 / 79)
+//   K rotated by tile: crowded only: 144 tiles 72 / 57, 120 tiles 40 / 41
+template <int D>
+bool rows256_pay(const SdpaDev& p, int n_cu, bool xtra) {
+    const long heads = static_cast<long>(p.B) * p.H;
+    const int T = (p.Lk + kBN - 1) / kBN;
+    if (heads * ((p.Lq + 255) / 256) >= n_cu) return true;
+    if (p.prefix_scaled) return false;
+    const bool crowded = heads * ((p.Lq + 127) / 128) > n_cu;
+    if (p.cos_k != nullptr) return crowded && T >= 16;
+    const bool plain = !xtra && same_keys_for_all_rows(p);
+    if constexpr (dma_kernel_available<D>()) {
+        if (!plain) return T >= (crowded ? 12 : 16);
+        return crowded ? T >= 3 : T >= (D == 72 ? 5 : 8);
+    }
+    if (D <= 64) return plain && p.Lp == 0;
+    return plain && crowded && T >= 16;
+}
+
 template <typename T, int D>
 int launch_d(SdpaDev p, int n_cu, hipStream_t stream) {
     const bool rope_k = p.cos_k != nullptr;
@@ -1197,8 +1244,7 @@ int launch_d(SdpaDev p, int n_cu, hipStream_t stream) {
         }
         p.split = SplitGeo{};
     }
-    // 256-row tiles when they give every CU at least one work group; head_dim above 128 does not fit
-    // two wavefronts per SIMD and stays on the 128-row kernel.
+    // head_dim above 128 does not fit two wavefronts per SIMD and stays on the 128-row kernel
     const long tiles256 = static_cast<long>(p.B) * p.H * ((p.Lq + 255) / 256);
     const int choice = sdpa_kernel_choice();
     // calls with a key mask, a logit bias or a request for the softmax denominators take the XTRA instances of the 256-row
@@ -1209,7 +1255,7 @@ int launch_d(SdpaDev p, int n_cu, hipStream_t stream) {
     const bool xtra_ok = !xtra || (!rope_k && !p.prefix_scaled && kbits_bytes <= 24 * 1024);   // (the words share the LDS with rings and Q staging)
     // calls with the prefix-KV dial stay on the 128-row kernel unless the DMA kernel (which has an instance for it) takes them
     const bool dial_ok = !p.prefix_scaled || (dma_kernel_available<D>() && !rope_k && choice != 3);
-    const bool pingpong = D <= 128 && xtra_ok && dial_ok && (choice >= 2 || (choice == 0 && tiles256 >= n_cu));
+    const bool pingpong = D <= 128 && xtra_ok && dial_ok && (choice >= 2 || (choice == 0 && rows256_pay<D>(p, n_cu, xtra)));
     // short key sequences whose K and V fit in LDS next to a query tile: one work group walks several query tiles
     const int n_kt = (p.Lk + kBN - 1) / kBN;
     if (D <= 128 && choice == 0 && p.mask_mode == MI_MASK_NONE && p.bias == nullptr && p.lse == nullptr &&
@@ -1237,13 +1283,13 @@ int launch_d(SdpaDev p, int n_cu, hipStream_t stream) {
                 if constexpr (dma_kernel_available<D>()) {
                     if (dma) {
                         p.kbits_off = DmaGeo<D>::lds_bytes();
-                        hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, false, false, false, true>), grid, block,
+                        hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, false, kGeneral, false, true>), grid, block,
                                            DmaGeo<D>::lds_bytes() + kbits_bytes, stream, p);
                     }
                 }
                 if (!dma) {
                     p.kbits_off = lds_bytes_8<D>();
-                    hipLaunchKernelGGL((sdpa_fwd_pp_kernel<T, D, false, false, true>), grid, block, lds_bytes_8<D>() + kbits_bytes, stream, p);
+                    hipLaunchKernelGGL((sdpa_fwd_pp_kernel<T, D, false, kGeneral, true>), grid, block, lds_bytes_8<D>() + kbits_bytes, stream, p);
                 }
             }
             else if (rope_k) hipLaunchKernelGGL((sdpa_fwd_pp_kernel<T, D, true>), grid, block, lds_bytes_8<D>(), stream, p);
@@ -1252,13 +1298,18 @@ int launch_d(SdpaDev p, int n_cu, hipStream_t stream) {
                     // whole key tiles only; a cached prefix may come first if it is whole tiles too and laid out like K / V
                     const bool dense = p.mask_mode == MI_MASK_NONE && p.kv_valid_len == nullptr && p.Lk % kBN == 0 && !p.prefix_scaled &&
                                        (p.Lp == 0 || (p.Lp % kBN == 0 && p.kp_rs == p.k_rs && p.vp_rs == p.v_rs));
-                    if (dense) hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, false, true>), grid, block, DmaGeo<D>::lds_bytes(), stream, p);
-                    else if (p.prefix_scaled) hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, false, false, true>), grid, block, DmaGeo<D>::lds_bytes(), stream, p);
+                    const bool ragged = same_keys_for_all_rows(p);
+                    if (dense) hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, false, kDense>), grid, block, DmaGeo<D>::lds_bytes(), stream, p);
+                    else if (ragged) hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, false, kRagged>), grid, block, DmaGeo<D>::lds_bytes(), stream, p);
+                    else if (p.prefix_scaled) hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, false, kGeneral, true>), grid, block, DmaGeo<D>::lds_bytes(), stream, p);
                     else hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, false>), grid, block, DmaGeo<D>::lds_bytes(), stream, p);
                 }
             }
-            else if (D <= 64 && p.mask_mode == MI_MASK_NONE && p.kv_valid_len == nullptr && p.Lp == 0 && p.Lk % kBN == 0) {
-                if constexpr (D <= 64) hipLaunchKernelGGL((sdpa_fwd_pp_kernel<T, D, false, true>), grid, block, lds_bytes_8<D>(), stream, p);
+            else if (D <= 64 && p.mask_mode == MI_MASK_NONE && p.Lp == 0) {
+                if constexpr (D <= 64) {
+                    if (p.kv_valid_len == nullptr && p.Lk % kBN == 0) hipLaunchKernelGGL((sdpa_fwd_pp_kernel<T, D, false, kDense>), grid, block, lds_bytes_8<D>(), stream, p);
+                    else hipLaunchKernelGGL((sdpa_fwd_pp_kernel<T, D, false, kRagged>), grid, block, lds_bytes_8<D>(), stream, p);
+                }
             }
             else hipLaunchKernelGGL((sdpa_fwd_pp_kernel<T, D, false>), grid, block, lds_bytes_8<D>(), stream, p);
         }

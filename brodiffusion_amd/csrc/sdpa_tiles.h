@@ -108,6 +108,17 @@ struct TileCursor {
     }
 };
 
+// Forms of the 256-row kernels by what the launch can look like:
+//   kGeneral  any mask: a visible-key interval per query row, K and V of prefix and fresh rows with their own strides
+//   kDense    no mask of any kind and whole key tiles only
+//   kRagged   every query row sees the same keys [0, n) of its batch item, n any number (kv_valid_len included), prefix of any length
+enum { kGeneral = 0, kDense = 1, kRagged = 2 };
+
+// keys that every query row of batch item b sees, where no mask but kv_valid_len applies (uniform)
+__device__ __forceinline__ int visible_keys(const SdpaDev& p, int b) {
+    return __builtin_amdgcn_readfirstlane(p.kv_valid_len ? max(min(p.Lk, p.kv_valid_len[b]), 0) : p.Lk);
+}
+
 // Cooperative K/V tile movement for a work group of NT threads: global -> registers -> LDS.
 // kreg / vreg hold this thread's 16-byte chunks of one K tile and one V tile (possibly different tiles).
 template <typename T, int D, int NT, bool ROPE_K>
@@ -259,7 +270,8 @@ struct TileMover {
 // base address of the next tile advances in scalar registers and this thread's byte offsets inside a tile (global and
 // LDS) are computed once, so a load is one instruction with a scalar base and a fixed vector offset, a store has no
 // select, and whether a thread takes part in round i is the same for its whole wavefront (a scalar branch).
-template <typename T, int D, int NT>
+// RAGGED: the last tile may be partial; its missing rows are read from the last row that exists and stored as zeros.
+template <typename T, int D, int NT, bool RAGGED = false>
 struct DenseMover {
     using G = HeadGeo<D>;
     static constexpr int NLD = (G::NCH + NT - 1) / NT;
@@ -270,8 +282,11 @@ struct DenseMover {
     unsigned kgo[NLD], vgo[NLD];    // byte offsets of this thread's chunks inside a tile in memory
     unsigned klo[NLD], vlo[NLD];    // ... and inside the LDS tile
     u32x4 kreg[NLD], vreg[NLD];
-    __device__ __forceinline__ DenseMover(const unsigned char* k_base, long k_rs, const unsigned char* v_base, long v_rs, int tid, int wave_)
-        : kptr(k_base), vptr(v_base), k_tile_bytes(static_cast<unsigned>(k_rs) * 2u * kBN), v_tile_bytes(static_cast<unsigned>(v_rs) * 2u * kBN), wave(wave_) {
+    // RAGGED: rows from the next tile to fetch on, and rows of the tile held in kreg / vreg
+    int k_left, v_left, k_rows = kBN, v_rows = kBN, tid0;
+    __device__ __forceinline__ DenseMover(const unsigned char* k_base, long k_rs, const unsigned char* v_base, long v_rs, int tid, int wave_, int n_keys)
+        : kptr(k_base), vptr(v_base), k_tile_bytes(static_cast<unsigned>(k_rs) * 2u * kBN), v_tile_bytes(static_cast<unsigned>(v_rs) * 2u * kBN), wave(wave_),
+          k_left(n_keys), v_left(n_keys), tid0(tid) {
 #pragma unroll
         for (int i = 0; i < NLD; ++i) {
             const int idx = min(tid + NT * i, G::NCH - 1);
@@ -289,17 +304,33 @@ struct DenseMover {
 #pragma unroll
         for (int i = 0; i < NLD; ++i)
             if (mine(i)) {
-                if constexpr (WHICH == 0) kreg[i] = *reinterpret_cast<const u32x4*>(kptr + kgo[i]);
-                else vreg[i] = *reinterpret_cast<const u32x4*>(vptr + vgo[i]);
+                unsigned off = WHICH == 0 ? kgo[i] : vgo[i];
+                if constexpr (RAGGED) {
+                    const int left = WHICH == 0 ? k_left : v_left;
+                    if (left < kBN) off -= static_cast<unsigned>(max(row_of(i) - (left - 1), 0)) * ((WHICH == 0 ? k_tile_bytes : v_tile_bytes) / kBN);
+                }
+                if constexpr (WHICH == 0) kreg[i] = *reinterpret_cast<const u32x4*>(kptr + off);
+                else vreg[i] = *reinterpret_cast<const u32x4*>(vptr + off);
             }
+        if constexpr (RAGGED) {
+            if constexpr (WHICH == 0) { k_rows = k_left; k_left -= kBN; } else { v_rows = v_left; v_left -= kBN; }
+        }
         if constexpr (WHICH == 0) kptr += k_tile_bytes; else vptr += v_tile_bytes;
     }
+    __device__ __forceinline__ int row_of(int i) const { return min(tid0 + NT * i, G::NCH - 1) / G::CPR; }
+    __device__ __forceinline__ void blank_missing(u32x4 (&reg)[NLD], int rows) const {
+#pragma unroll
+        for (int i = 0; i < NLD; ++i)
+            if (mine(i) && row_of(i) >= rows) reg[i] = u32x4{0, 0, 0, 0};
+    }
     __device__ __forceinline__ void store_held_k(unsigned char* Ks) {
+        if (RAGGED && k_rows < kBN) blank_missing(kreg, k_rows);
 #pragma unroll
         for (int i = 0; i < NLD; ++i)
             if (mine(i)) *reinterpret_cast<u32x4*>(Ks + klo[i]) = kreg[i];
     }
     __device__ __forceinline__ void store_held_v(unsigned char* Vs) {
+        if (RAGGED && v_rows < kBN) blank_missing(vreg, v_rows);
 #pragma unroll
         for (int i = 0; i < NLD; ++i)
             if (mine(i)) *reinterpret_cast<u32x4*>(Vs + vlo[i]) = vreg[i];
