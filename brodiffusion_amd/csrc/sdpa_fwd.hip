@@ -87,7 +87,7 @@ __global__ void __launch_bounds__(kThreads4, (D > 128 ? 1 : 2)) sdpa_fwd_kernel(
         hi = p.mask_mode == MI_MASK_CAUSAL ? min(Lk, q_offset + qrow + 1) : Lk;
         if (!qvalid || hi <= lo) { lo = 0; hi = 0; }
     } else {
-        row_interval(p, b, qrow, qvalid, lo, hi);
+        row_interval(p, b, min(qrow, p.Lq - 1), q0 + wave * 32 < p.Lq, lo, hi);
     }
     const WaveExtent we = wave_extent(lo, hi);
     if (lane == 0) { red[wave] = we.lo_min; red[4 + wave] = we.hi_max; }
@@ -375,8 +375,8 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_shortkv_kernel(const SdpaDe
 // of K_t, V_{t-1} (last read in step t-1) and issues the global loads of K_{t+3}, V_{t+2}; two buffers per
 // operand suffice.
 // FORM: as in the DMA form below, without prefix; kDense and kRagged are instantiated for head_dim up to 64, where kDense
-// measures 2-3 % faster (at 80 the compiler's allocation of that instance goes wrong: twice as slow) and kRagged 17 %
-// (head_dim 40, 8 heads, 3600 tokens: 73.5 -> 61.1 us).
+// measures 2-3 % faster (at 80 the compiler's allocation of that instance goes wrong: twice as slow) and kRagged 13 %
+// (head_dim 40, 8 heads, 3600 tokens: 67.0 -> 58.5 us).
 // XTRA: key mask, logit bias and softmax denominators (see sdpa_fwd_pp_dma_kernel).
 template <typename T, int D, bool ROPE_K, int FORM = kGeneral, bool XTRA = false>
 __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_kernel(const SdpaDev p) {
@@ -410,7 +410,9 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_kernel(const SdpaDev
 
     const int n_keys = RAGGED ? visible_keys(p, b) : p.Lk;
     int lo = 0, hi = n_keys;   // DENSE: rows past the end of Q repeat its last row and are never stored
-    if constexpr (!DENSE) row_interval(p, b, qrow, qvalid, lo, hi);
+    // (rows past the end count as the last row where they share a wavefront with it: as rows without keys they put every tile
+    //  of that wavefront on the masked path; 24 heads of 128, 2500 tokens, block-causal: 83.8 -> 74.5 us)
+    if constexpr (!DENSE) row_interval(p, b, min(qrow, p.Lq - 1), q0 + wave * 32 < p.Lq, lo, hi);
     WaveExtent we{0, 0, n_keys, n_keys};
     if constexpr (!DENSE) {
         we = wave_extent(lo, hi);
@@ -629,18 +631,20 @@ __device__ __forceinline__ int swz(int row) { return 4 * (row & 3) + ((row >> 2)
 // head_dim 128 and 8 % at 72 than the general form on the same dense call.
 // FORM kRagged: every row sees the same keys, their number is free. All tiles but the last of a segment are as in kDense; that
 // one is met by scalar branches (DMA rows clamped to the last that exists, scores past it blanked). The general form clamps and
-// compares in every step, on the path that bounds this kernel (a wavefront's own chain of issue, MFMAs and softmax):
-// 24 heads of 128, 1997 tokens 65.3 -> 54.0 us, 2280 tokens + 669 cached 97.0 -> 81.6, 16 heads of 72, 3000 tokens 80.3 -> 64.6,
-// all within 4 % of the next multiple of 64 on kDense.
+// compares in every step: 24 heads of 128, 2500 tokens 77.5 -> 75.3 us, 16 heads of 72, 3600 tokens 84.0 -> 82.0.
 // PSCALE: the general form with the prefix-KV dial (factors on the rows of the cached prefix) in its softmax.
 // XTRA: the general form with a key mask (one visibility bit per key, 64-bit words per key tile built once per work group
 // in LDS behind the rings), an additive logit bias and the softmax denominators as an output (traced attention).
+// XTRA with kRagged: a key mask but no bias. The mask hides the same keys from every row (the padding of a prompt in
+// the middle of a joint sequence), so the tiles without a visible key are taken out of the walk: `vis` lists the others, and a
+// step looks up the tile that it loads. 48 query / 12 K/V heads of 128, 4608 tokens of which 435 are padding (6 of 72 tiles):
+// 520 -> 472 us; the words used to blank the scores of a hidden tile, whose MFMAs and loads ran all the same.
 template <typename T, int D, bool SPLIT, int FORM = kGeneral, bool PSCALE = false, bool XTRA = false>
 __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const SdpaDev p) {
-    constexpr bool DENSE = FORM != kGeneral, RAGGED = FORM == kRagged;
+    constexpr bool DENSE = FORM != kGeneral, RAGGED = FORM == kRagged, LISTED = XTRA && RAGGED;
     static_assert(!(SPLIT && DENSE), "the split launch clips key ranges per part");
     static_assert(!PSCALE || (!SPLIT && !DENSE), "the dial belongs to the general form");
-    static_assert(!XTRA || (!SPLIT && !DENSE && !PSCALE), "key mask, bias and denominators belong to the general form");
+    static_assert(!XTRA || (!SPLIT && FORM != kDense && !PSCALE), "key mask, bias and denominators are not in these forms");
     using G = HeadGeo<D>;
     using DG = DmaGeo<D>;
     using V8 = typename Mma<T>::v8;
@@ -715,7 +719,9 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
 
     const int n_keys = RAGGED ? visible_keys(p, b) : p.Lk;   // counts the cached prefix rows, which come first
     int lo = 0, hi = n_keys;   // DENSE: rows past the end of Q repeat its last row and are never stored
-    if constexpr (!DENSE) row_interval(p, b, qrow, qvalid, lo, hi);
+    // (rows past the end count as the last row where they share a wavefront with it: as rows without keys they put every tile
+    //  of that wavefront on the masked path; 24 heads of 128, 2500 tokens, block-causal: 83.8 -> 74.5 us)
+    if constexpr (!DENSE) row_interval(p, b, min(qrow, p.Lq - 1), q0 + wave * 32 < p.Lq, lo, hi);
     if constexpr (SPLIT) {
         lo = max(lo, kv_begin);
         hi = min(hi, kv_end);
@@ -748,10 +754,29 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
         kv_stop = __builtin_amdgcn_readfirstlane(kv_stop);
     }
     const TilePlan plan(g_lo == 0x7fffffff ? 0 : g_lo, kv_stop, p.Lp);
-    const int n_tiles = plan.n_tiles;
+    int n_tiles = plan.n_tiles;
     // XTRA: visibility words of the plan's tiles (made visible to all wavefronts by the barrier that ends the prologue)
     const unsigned long long* const kbits = (XTRA && p.key_mask) ? reinterpret_cast<const unsigned long long*>(smem + p.kbits_off) : nullptr;
     if constexpr (XTRA) build_key_bits(p, plan, b, smem + p.kbits_off, wave, lane);
+    // LISTED: tile numbers of the tiles with a visible key, in order, behind the words; every wavefront writes the whole list
+    // (the same values) and reads only what it wrote. vis_t .. vis_t3: the list's entries t .. t + 3 in step t.
+    unsigned short* const vis = LISTED ? reinterpret_cast<unsigned short*>(smem + p.kbits_off + 8 * ((p.Lk + kBN - 1) / kBN + 2)) : nullptr;
+    int vis_t = 0, vis_t1 = 0, vis_t2 = 0, vis_t3 = 0;
+    if constexpr (LISTED) {
+        __syncthreads();
+        int n = 0;
+        for (int t0 = 0; t0 < plan.n_tiles; t0 += 64) {
+            const bool on = t0 + lane < plan.n_tiles && kbits[t0 + lane] != 0ull;
+            const unsigned long long m = __ballot(on);
+            if (on) vis[n + __popcll(m & ((1ull << lane) - 1ull))] = static_cast<unsigned short>(t0 + lane);
+            n += __popcll(m);
+        }
+        n_tiles = __builtin_amdgcn_readfirstlane(n);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    auto listed = [&](int i) { return __builtin_amdgcn_readfirstlane(static_cast<int>(vis[min(i, n_tiles - 1)])); };   // n_tiles > 0
     const float* const bias_row = (XTRA && p.bias && qvalid && qrow >= p.bias_q0) ? p.bias + static_cast<long>(qrow - p.bias_q0) * p.bias_rs : nullptr;
 
     f32x16 oacc[G::VB];
@@ -770,6 +795,13 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
             reinterpret_cast<const unsigned char*>(static_cast<const T*>(p.k) + b * p.k_bs + hk * D), static_cast<unsigned>(p.k_rs) * 2u, p.Lp);
     vc.init(plan, reinterpret_cast<const unsigned char*>(static_cast<const T*>(p.vp) + b * p.vp_bs + hk * D), static_cast<unsigned>(p.vp_rs) * 2u,
             reinterpret_cast<const unsigned char*>(static_cast<const T*>(p.v) + b * p.v_bs + hk * D), static_cast<unsigned>(p.v_rs) * 2u, p.Lp);
+    auto seek = [&](TileCursor& c, int t, const void* pre, long pre_bs, const void* fresh, long fresh_bs) {   // (LISTED: one row stride for both)
+        const int j0 = plan.j0(t);
+        c.ptr = plan.in_prefix(t)
+                    ? reinterpret_cast<const unsigned char*>(static_cast<const T*>(pre) + b * pre_bs + hk * D) + static_cast<unsigned long>(j0) * c.rsb
+                    : reinterpret_cast<const unsigned char*>(static_cast<const T*>(fresh) + b * fresh_bs + hk * D) + static_cast<unsigned long>(j0 - p.Lp) * c.rsb;
+        c.rows_left = plan.limit(t) - j0;
+    };
     int drow[DG::MAXI];        // tile row this lane fetches in its m-th instruction
     unsigned dcol[DG::MAXI];   // byte offset inside that row
 #pragma unroll
@@ -795,8 +827,12 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
     auto dma = [&](const TileCursor& c, int m, int j, int lds_off) {
         unsigned voff = dcol[m];
         if constexpr (!DENSE) voff += static_cast<unsigned>(min(drow[m], min(c.rows_left, kBN) - 1)) * c.rsb;
-        // the last tile of a segment: rows past its end repeat the last one (a scalar branch, untaken for every other tile)
-        if (RAGGED && c.rows_left < kBN) voff -= static_cast<unsigned>(max(drow[m] - (c.rows_left - 1), 0)) * c.rsb;
+        // the last tile of a segment: rows past its end repeat the last one. A scalar branch that no other tile takes: the empty
+        // statement keeps the compiler from computing it for every tile and selecting
+        if (RAGGED && c.rows_left < kBN) {
+            asm volatile("" : "+v"(voff));
+            voff -= static_cast<unsigned>(max(drow[m] - (c.rows_left - 1), 0)) * c.rsb;
+        }
         const unsigned dst = lds_base + lds_off + j * 1024;
         // (the LDS base travels in m0 as a declared input: the compiler writes the register itself and knows it is taken;
         //  the s_nop is the wait state an LDS-DMA instruction needs behind a write of m0)
@@ -874,7 +910,13 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
         // XTRA: the visibility word of the tile whose softmax this wavefront runs in this step, fetched here, ahead of this
         // step's DMA instructions (an LDS read behind them would wait for them to land)
         TileExtra xt;
-        if constexpr (XTRA) {
+        if constexpr (LISTED) {
+            vis_t = vis_t1; vis_t1 = vis_t2; vis_t2 = vis_t3;
+            const unsigned long long w = kbits[grp == 1 ? vis_t : vis_t1];
+            vis_t3 = listed(t + 3);
+            xt.kw0 = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(w));
+            xt.kw1 = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(w >> 32));
+        } else if constexpr (XTRA) {
             if (kbits) {
                 const unsigned long long w = kbits[min(max(grp == 1 ? t : t + 1, 0), max(n_tiles - 1, 0))];
                 xt.kw0 = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(w));
@@ -883,7 +925,12 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
             xt.bias_cols = p.bias_cols;
         }
         auto softmax_of = [&](int tt) {
-            if constexpr (DENSE) {
+            if constexpr (LISTED) {
+                if (tt >= 0 && tt < n_tiles) {
+                    softmax_tile_rel<T, D, false, true>(sacc, pf, oacc, st, (xt.kw0 & xt.kw1) != ~0u, false, 0, 0, kBN, lh, PrefixScale(), xt);
+                    return;
+                }
+            } else if constexpr (DENSE) {
                 if (tt >= 0 && tt < n_tiles) {
                     const int rows = RAGGED ? plan.limit(tt) - plan.j0(tt) : kBN;
                     softmax_tile_rel<T, D>(sacc, pf, oacc, st, RAGGED && rows < kBN, false, 0, 0, rows, lh);
@@ -912,6 +959,12 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
         // read takes the full memory latency), so the DMA instructions of a step go where the wavefront has no
         // LDS access ahead of it for a long time: right before its softmax.
         auto issue_dma = [&]() {
+            if constexpr (LISTED) {
+                seek(kc, vis_t3, p.kp, p.kp_bs, p.k, p.k_bs);
+                seek(vc, vis_t2, p.vp, p.vp_bs, p.v, p.v_bs);
+                issued = dma_tiles(load_k, KD, load_v, VD);
+                return;
+            }
             issued = dma_tiles(load_k, KD, load_v, VD);
             if (DENSE && !RAGGED && p.Lp == 0) {
                 if (load_k) kc.ptr += kBN * kc.rsb;
@@ -1000,11 +1053,21 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
 
     if (n_tiles > 0) {
         // prologue: K_0, K_1, V_0 (the loop loads K_{t+3}, V_{t+2} from t = -1 on); cursors end at K_2, V_1
-        dma_tiles(true, 0, false, 0);
-        if (n_tiles > 1) { kc.next(); dma_tiles(true, DG::TILE, false, 0); }
-        if (n_tiles > 2) kc.next();
-        dma_tiles(false, 0, true, DG::VOFF);
-        if (n_tiles > 1) vc.next();
+        if constexpr (LISTED) {
+            vis_t2 = listed(0); vis_t3 = listed(1);     // (step -1 moves them up by one)
+            vis_t1 = vis_t2;                            // never used as tile -1, only kept inside the words
+            seek(kc, vis_t2, p.kp, p.kp_bs, p.k, p.k_bs);
+            dma_tiles(true, 0, false, 0);
+            if (n_tiles > 1) { seek(kc, vis_t3, p.kp, p.kp_bs, p.k, p.k_bs); dma_tiles(true, DG::TILE, false, 0); }
+            seek(vc, vis_t2, p.vp, p.vp_bs, p.v, p.v_bs);
+            dma_tiles(false, 0, true, DG::VOFF);
+        } else {
+            dma_tiles(true, 0, false, 0);
+            if (n_tiles > 1) { kc.next(); dma_tiles(true, DG::TILE, false, 0); }
+            if (n_tiles > 2) kc.next();
+            dma_tiles(false, 0, true, DG::VOFF);
+            if (n_tiles > 1) vc.next();
+        }
     }
     {
         // the Q tile, rotated on its way into the staging buffer behind the rings; every lane then picks the fragments of
@@ -1281,7 +1344,13 @@ int launch_d(SdpaDev p, int n_cu, hipStream_t stream) {
             if (xtra) {
                 const bool dma = dma_kernel_available<D>() && sdpa_kernel_choice() != 3;
                 if constexpr (dma_kernel_available<D>()) {
-                    if (dma) {
+                    const long listed_bytes = kbits_bytes + kbits_bytes / 4;
+                    if (dma && p.key_mask && !p.bias && same_keys_for_all_rows(p) && DmaGeo<D>::lds_bytes() + listed_bytes + 256 <= 160 * 1024) {
+                        p.kbits_off = DmaGeo<D>::lds_bytes();
+                        hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, false, kRagged, false, true>), grid, block,
+                                           DmaGeo<D>::lds_bytes() + listed_bytes, stream, p);
+                    }
+                    else if (dma) {
                         p.kbits_off = DmaGeo<D>::lds_bytes();
                         hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, false, kGeneral, false, true>), grid, block,
                                            DmaGeo<D>::lds_bytes() + kbits_bytes, stream, p);

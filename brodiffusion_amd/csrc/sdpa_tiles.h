@@ -114,7 +114,7 @@ struct TileCursor {
 //   kRagged   every query row sees the same keys [0, n) of its batch item, n any number (kv_valid_len included), prefix of any length
 enum { kGeneral = 0, kDense = 1, kRagged = 2 };
 
-// keys that every query row of batch item b sees, where no mask but kv_valid_len applies (uniform)
+// keys that every query row of batch item b sees, where no mask but kv_valid_len (and a key mask) applies (uniform)
 __device__ __forceinline__ int visible_keys(const SdpaDev& p, int b) {
     return __builtin_amdgcn_readfirstlane(p.kv_valid_len ? max(min(p.Lk, p.kv_valid_len[b]), 0) : p.Lk);
 }
@@ -307,7 +307,12 @@ struct DenseMover {
                 unsigned off = WHICH == 0 ? kgo[i] : vgo[i];
                 if constexpr (RAGGED) {
                     const int left = WHICH == 0 ? k_left : v_left;
-                    if (left < kBN) off -= static_cast<unsigned>(max(row_of(i) - (left - 1), 0)) * ((WHICH == 0 ? k_tile_bytes : v_tile_bytes) / kBN);
+                    // (a real branch: the empty statement keeps the compiler from computing this for every tile and selecting,
+                    //  15 % of the key step at head_dim 40)
+                    if (left < kBN) {
+                        asm volatile("" : "+v"(off));
+                        off -= static_cast<unsigned>(max(row_of(i) - (left - 1), 0)) * ((WHICH == 0 ? k_tile_bytes : v_tile_bytes) / kBN);
+                    }
                 }
                 if constexpr (WHICH == 0) kreg[i] = *reinterpret_cast<const u32x4*>(kptr + off);
                 else vreg[i] = *reinterpret_cast<const u32x4*>(vptr + off);
@@ -319,6 +324,7 @@ struct DenseMover {
     }
     __device__ __forceinline__ int row_of(int i) const { return min(tid0 + NT * i, G::NCH - 1) / G::CPR; }
     __device__ __forceinline__ void blank_missing(u32x4 (&reg)[NLD], int rows) const {
+        asm volatile("" : "+s"(rows));
 #pragma unroll
         for (int i = 0; i < NLD; ++i)
             if (mine(i) && row_of(i) >= rows) reg[i] = u32x4{0, 0, 0, 0};
