@@ -148,6 +148,7 @@ const float* weight(PyObject* w, PyObject* scales, at::ScalarType dt, int64_t ro
 }
 // `out` given: contiguous, `cols` wide, `numel` values; else allocated with x's leading sizes
 Tensor output(PyObject* out, const Tensor& x, int64_t cols) {
+    need(x.dim() >= 1 && x.size(-1) > 0);   // (no row count for rows without values)
     const int64_t numel = x.numel() / x.size(-1) * cols;
     if (none(out)) {
         auto sizes = x.sizes().vec();
