@@ -61,6 +61,7 @@ HOST_DIR = os.path.join(HERE, "host")
 HOST_LIB = os.path.join(LIB_DIR, "libbrodiffusion_amd_host.so")
 HOST_TEST = os.path.join(LIB_DIR, "test_host_ops")
 SPLIT_TEST = os.path.join(LIB_DIR, "test_split_geo")
+WAITING_LIB = os.path.join(LIB_DIR, "libwaiting_test.so")
 CXX = os.environ.get("CXX", "g++")
 
 
@@ -91,6 +92,11 @@ def build_host(with_test: bool = True, verbose: bool = False) -> str:
         if r.returncode != 0:
             sys.stderr.write(r.stdout + r.stderr)
             raise RuntimeError("split-geometry test build failed")
+        cmd = [*common, "-shared", os.path.join(ROOT, "tests", "cpp", "waiting_library.cpp"), "-o", WAITING_LIB]
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        if r.returncode != 0:
+            sys.stderr.write(r.stdout + r.stderr)
+            raise RuntimeError("test library build failed")
     if verbose:
         print("built", HOST_LIB)
     return HOST_LIB

@@ -89,10 +89,22 @@ int dtype_code(const Tensor& t) {
     return MI_DTYPE_F16;
 }
 void* current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
-void run(int rc, const char* op) {
+// The launches of one call, in order up to the first that is refused, without the interpreter lock: a launch waits where its
+// queue is full, and loads its kernel the first time. What they read and write is held by the caller's arguments and by the
+// Tensors of the calling function; the library's error message is one per thread.
+template <typename... F> void run(const char* op, F... launch) {
+    int rc = 0;
+    Py_BEGIN_ALLOW_THREADS
+    (void)((rc = launch(), rc == 0) && ...);
+    Py_END_ALLOW_THREADS
     if (rc == 0) return;
     PyErr_Format(PyExc_RuntimeError, "%s: %s", op, L.last_error());
     throw PyError{};
+}
+const char* name_of(PyObject* op) {
+    const char* s = PyUnicode_Check(op) ? PyUnicode_AsUTF8(op) : nullptr;
+    if (!s) { PyErr_Clear(); throw Decline{}; }
+    return s;
 }
 const float* f32(const Tensor& t) { return static_cast<const float*>(t.data_ptr()); }
 int rows32(int64_t n) { need(n >= 0 && n <= 0x7fffffff); return static_cast<int>(n); }
@@ -185,7 +197,7 @@ NATIVE(linear, 6)
     const int64_t n_out = tensor(a[0]).size(0);
     const Tensor y = output(a[3], x, n_out);
     const mi_linear_args p = linear_args(a[0], a[1], x, y, a[4], n_out);
-    run(L.linear(&p), PyUnicode_AsUTF8(a[5]));
+    run(name_of(a[5]), [&] { return L.linear(&p); });
     return given(a[3], y);
 NATIVE_END
 
@@ -196,7 +208,7 @@ NATIVE(geglu, 6)
     need(two_n % 2 == 0);
     const Tensor y = output(a[3], x, two_n / 2);
     const mi_linear_args p = linear_args(a[1], a[2], x, y, a[4], two_n / 2);
-    run(L.geglu(&p), PyUnicode_AsUTF8(a[5]));
+    run(name_of(a[5]), [&] { return L.geglu(&p); });
     return given(a[3], y);
 NATIVE_END
 
@@ -204,7 +216,12 @@ NATIVE_END
 NATIVE(add_inplace, 2)
     const Tensor &y = tensor(a[0]), &x = tensor(a[1]);
     need(y.sizes() == x.sizes() && y.scalar_type() == x.scalar_type() && y.is_contiguous() && x.is_contiguous());
-    run(L.add_inplace(y.data_ptr(), x.data_ptr(), y.numel(), dtype_code(y), current_stream()), "add_inplace_vec");
+    void* const py = y.data_ptr();
+    const void* const px = x.data_ptr();
+    const int64_t numel = y.numel();
+    const int dt = dtype_code(y);
+    void* const stream = current_stream();
+    run("add_inplace_vec", [&] { return L.add_inplace(py, px, numel, dt, stream); });
     return given(a[0], y);
 NATIVE_END
 
@@ -214,8 +231,13 @@ NATIVE(rms_norm, 4)
     need(x.dim() == 2 && x.stride(1) == 1 && g.scalar_type() == x.scalar_type() && g.numel() == x.size(1) && g.is_contiguous());
     const Tensor y = none(a[3]) ? at::empty_like(x) : tensor(a[3]);
     need(y.sizes() == x.sizes() && y.scalar_type() == x.scalar_type() && y.stride(1) == 1);
-    run(L.rms_norm(x.data_ptr(), g.data_ptr(), y.data_ptr(), rows32(x.size(0)), rows32(x.size(1)), x.stride(0), y.stride(0), static_cast<float>(number(a[2])),
-                   dtype_code(x), current_stream()), "rms_norm_rows");
+    const void *const px = x.data_ptr(), *const pg = g.data_ptr();
+    void* const py = y.data_ptr();
+    const int rows = rows32(x.size(0)), cols = rows32(x.size(1)), dt = dtype_code(x);
+    const int64_t x_rs = x.stride(0), y_rs = y.stride(0);
+    const float eps = static_cast<float>(number(a[2]));
+    void* const stream = current_stream();
+    run("rms_norm_rows", [&] { return L.rms_norm(px, pg, py, rows, cols, x_rs, y_rs, eps, dt, stream); });
     return given(a[3], y);
 NATIVE_END
 
@@ -244,7 +266,7 @@ NATIVE(rope, 9)
     p.rows = rows32(x.size(0)); p.num_heads = heads; p.head_dim = hd;
     p.x_row_stride = x.stride(0); p.out_row_stride = y.stride(0);
     p.stream = current_stream();
-    run(L.rope(&p), PyUnicode_AsUTF8(a[8]));
+    run(name_of(a[8]), [&] { return L.rope(&p); });
     return given(a[5], y);
 NATIVE_END
 
@@ -273,7 +295,7 @@ NATIVE(headnorm_rope, 10)
         p.out2 = c.data_ptr(); p.out2_rows = rows32(c.size(0)); p.out2_row_stride = c.stride(0);
     }
     p.stream = current_stream();
-    run(L.headnorm_rope(&p), "headnorm_rope");
+    run("headnorm_rope", [&] { return L.headnorm_rope(&p); });
     return given(a[7], y);
 NATIVE_END
 
@@ -301,11 +323,11 @@ void set_mask(mi_sdpa_args& p, PyObject* mask) {
         p.seg_causal[i] = truth(PyList_GET_ITEM(ca.o, i));
     }
 }
-PyObject* lend_scratch = nullptr;   // ops._own_split_scratch(device index, bytes) -> tensor
+PyObject* lend_scratch = nullptr;   // ops._own_split_scratch(device index, bytes) -> tensor of the calling thread
 
 struct Attention {   // one call; q, k, v and the output are always there
     mi_sdpa_args p;
-    Tensor out;
+    Tensor out, scratch;
     int64_t B, Lk;
     Attention(const Tensor& q, const Tensor& k, const Tensor& v, long heads, long kv_heads, PyObject* out_obj) {
         std::memset(&p, 0, sizeof(p));
@@ -355,14 +377,14 @@ struct Attention {   // one call; q, k, v and the output are always there
                     own = PyObject_CallFunction(lend_scratch, "in", static_cast<int>(out.get_device()), static_cast<Py_ssize_t>(bytes));
                     if (!own) throw PyError{};
                 }
-                const Tensor t = [&] { try { return tensor(own ? own : split_scratch); } catch (...) { Py_XDECREF(own); throw; } }();
-                Py_XDECREF(own);   // (the cache of ops.py keeps it)
-                need(t.is_contiguous());
-                p.split_scratch = t.data_ptr();
-                p.split_scratch_bytes = t.numel() * t.element_size();
+                try { scratch = tensor(own ? own : split_scratch); } catch (...) { Py_XDECREF(own); throw; }
+                Py_XDECREF(own);
+                need(scratch.is_contiguous());
+                p.split_scratch = scratch.data_ptr();
+                p.split_scratch_bytes = scratch.numel() * scratch.element_size();
             }
         }
-        run(L.sdpa(&p), op);
+        run(op, [&] { return L.sdpa(&p); });
     }
 };
 
@@ -397,7 +419,7 @@ NATIVE(sdpa, 18)
         }
     p.rope_split_half = truth(a[15]);
     if (!none(a[14])) c.rope_scratch(tensor(a[14]), q, k);
-    c.go(a[16], PyUnicode_AsUTF8(a[17]));
+    c.go(a[16], name_of(a[17]));
     return given(a[4], c.out);
 NATIVE_END
 
@@ -476,7 +498,7 @@ NATIVE(attn_block, 22)
     need(scratch.is_contiguous());
     p.scratch = scratch.data_ptr(); p.scratch_bytes = scratch.numel() * scratch.element_size();
     p.stream = current_stream();
-    run((cached ? L.kv_cached : L.qkvo)(&p), PyUnicode_AsUTF8(a[21]));
+    run(name_of(a[21]), [&] { return (cached ? L.kv_cached : L.qkvo)(&p); });
     return given(a[15], out);
 NATIVE_END
 
@@ -505,9 +527,9 @@ NATIVE(mha, 16)
     need(c.out.is_contiguous() && tensor(a[4]).dim() == 2 && tensor(a[4]).size(1) == inner);
     const Tensor y = output(a[15], c.out, n_out);
     const mi_linear_args po = linear_args(a[4], a[8], c.out, y, Py_None, n_out);
-    run(L.linear_n(p, 3), "mha_forward");
+    run("mha_forward", [&] { return L.linear_n(p, 3); });
     c.go(Py_None, "mha_forward");
-    run(L.linear(&po), "mha_forward");
+    run("mha_forward", [&] { return L.linear(&po); });
     PyObject* parts[5] = {given(a[15], y), given(a[11], qkv[0]), given(a[12], qkv[1]), given(a[13], qkv[2]), given(a[14], c.out)};
     PyObject* t = PyTuple_New(5);
     for (int i = 0; i < 5; ++i) PyTuple_SET_ITEM(t, i, parts[i]);
@@ -555,7 +577,7 @@ NATIVE(linear_attn, 10)
         if (sc.numel() > 0) { p.scratch = sc.data_ptr(); p.scratch_bytes = sc.numel() * 4; }
     }
     p.form = int32(a[9]);
-    run(L.linear_attn(&p), "linear_attention_relu_forward");
+    run("linear_attention_relu_forward", [&] { return L.linear_attn(&p); });
     return given(a[4], out);
 NATIVE_END
 
@@ -589,10 +611,14 @@ NATIVE(sana, 13)
     const Tensor y = output(a[12], x, n_out);
     const mi_linear_args po = linear_args(a[4], a[5], attn, y, Py_None, n_out);
     const char* op = "sana_self_attention";
-    run(L.linear_n(p, 3), op);
-    if (gq) run(L.rms_norm_pair(q.data_ptr(), gq, q.data_ptr(), k.data_ptr(), gk, k.data_ptr(), rows32(n), rows32(d), 0, 0, static_cast<float>(number(a[9])), dt, current_stream()), op);
-    run(L.linear_attn(&la), op);
-    run(L.linear(&po), op);
+    run(op, [&] { return L.linear_n(p, 3); });
+    if (gq) {
+        void *const pq = q.data_ptr(), *const pk = k.data_ptr(), *const stream = current_stream();
+        const float eps = static_cast<float>(number(a[9]));
+        const int rows = rows32(n), cols = rows32(d);
+        run(op, [&] { return L.rms_norm_pair(pq, gq, pq, pk, gk, pk, rows, cols, 0, 0, eps, dt, stream); });
+    }
+    run(op, [&] { return L.linear_attn(&la); }, [&] { return L.linear(&po); });
     return given(a[12], y);
 NATIVE_END
 

@@ -31,6 +31,7 @@ from __future__ import annotations
 
 import ctypes as C
 import math
+import threading
 from dataclasses import dataclass, field
 from typing import Optional, Sequence, Tuple
 
@@ -180,8 +181,8 @@ def sdpa_forward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, num_heads: i
                  prefix_k_scale: float = 1.0, prefix_v_scale: float = 1.0, prefix_k_row_scale: Optional[torch.Tensor] = None,
                  prefix_v_row_scale: Optional[torch.Tensor] = None, op: str = "sdpa_forward") -> torch.Tensor:
     """General entry: everything mi_sdpa_forward offers. Returns `out` (allocated like q if None).
-    split_scratch: None = lend the module's own scratch (grown on demand, one per device, shared by all calls of the
-    process: use one stream at a time) when the launch can use one, False = never split, a uint8 tensor = lend that."""
+    split_scratch: None = lend the module's own scratch (grown on demand, one per thread, device and stream) when the launch
+    can use one, False = never split, a uint8 tensor = lend that."""
     if logit_bias is None and lse_out is None and prefix_k_row_scale is None and prefix_v_row_scale is None and prefix_k_scale == 1.0 \
             and prefix_v_scale == 1.0:
         r = _native.sdpa(q, k, v, num_heads, out, num_kv_heads, k_prefix, v_prefix, scale, mask, kv_valid_len, key_mask, rope_q, rope_k,
@@ -309,17 +310,32 @@ def sdpa_forward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, num_heads: i
     return out
 
 
-_split_scratch_cache = {}
+class _ScratchOfThread(threading.local):
+    """Tensors by (device, stream); a new one in every thread, released with it."""
+
+    def __init__(self):
+        self.tensors = {}
+
+    def __iter__(self):
+        return iter(self.tensors)
+
+    def __getitem__(self, key):
+        return self.tensors[key]
+
+
+_split_scratch_cache = _ScratchOfThread()
 
 
 def _own_split_scratch(device, nbytes: int) -> torch.Tensor:
-    """The scratch this layer lends when the caller brings none: one per (device, current stream), grown on demand. Calls
-    on one stream run in order and may share it; calls on different streams may overlap on the GPU and must not."""
+    """The scratch this layer lends when the caller brings none: one per thread, device and current stream, grown on demand.
+    The calls of one thread on one stream run in order and may share it. Calls on different streams may overlap on the GPU; those
+    of two threads on one stream may put their launches (pieces, then merge) between each other's."""
     key = (device, _stream())
-    t = _split_scratch_cache.get(key)
+    cache = _split_scratch_cache.tensors
+    t = cache.get(key)
     if t is None or t.numel() < nbytes:
         t = torch.empty(nbytes, dtype=torch.uint8, device=device)
-        _split_scratch_cache[key] = t
+        cache[key] = t
     return t
 
 
