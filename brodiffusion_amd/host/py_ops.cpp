@@ -2,9 +2,10 @@
 // call itself. In Python one call cost 20 to 25 us of host time (attribute access on tensors, ctypes structs), more than the
 // GPU takes for a block of the U-Net's deeper levels; here it is 3 to 8, most of it the launches.
 //
-// Every function returns None, having done nothing, when a call is not plainly valid (wrong shape, dtype, device, layout, an
-// argument of another type): the Python implementation then runs, whose checks word the error. So the two agree on what is
-// valid, and the messages exist once. The library's own refusals (return value -1) are raised here.
+// Every function returns None, having launched nothing, when a call is not plainly valid (wrong shape, dtype, device, layout, an
+// argument of another type): the Python implementation then runs, whose checks word the error. So all checks of a call come
+// before its first launch, and what is taken here must be what the Python code takes (tests/test_native_calls_gpu.py makes the
+// same calls both ways). The library's own refusals (return value -1) are raised here.
 //
 // The library is not linked but bound to at import (bind): the ctypes layer and this module use the same loaded copy.
 #define PY_SSIZE_T_CLEAN
@@ -368,23 +369,20 @@ struct Attention {   // one call; q, k, v and the output are always there
         p.key_mask = f32(m);
     }
     // split_scratch: None = the scratch of ops.py for this device and stream, False = none, a tensor = that
-    void go(PyObject* split_scratch, const char* op) {
+    void lend(PyObject* split_scratch) {
+        if (split_scratch == Py_False) return;
+        const size_t bytes = L.sdpa_split_bytes(&p);
+        if (bytes == 0) return;
         PyObject* own = nullptr;
-        if (split_scratch != Py_False) {
-            const size_t bytes = L.sdpa_split_bytes(&p);
-            if (bytes > 0) {
-                if (none(split_scratch)) {
-                    own = PyObject_CallFunction(lend_scratch, "in", static_cast<int>(out.get_device()), static_cast<Py_ssize_t>(bytes));
-                    if (!own) throw PyError{};
-                }
-                try { scratch = tensor(own ? own : split_scratch); } catch (...) { Py_XDECREF(own); throw; }
-                Py_XDECREF(own);
-                need(scratch.is_contiguous());
-                p.split_scratch = scratch.data_ptr();
-                p.split_scratch_bytes = scratch.numel() * scratch.element_size();
-            }
+        if (none(split_scratch)) {
+            own = PyObject_CallFunction(lend_scratch, "in", static_cast<int>(out.get_device()), static_cast<Py_ssize_t>(bytes));
+            if (!own) throw PyError{};
         }
-        run(op, [&] { return L.sdpa(&p); });
+        try { scratch = tensor(own ? own : split_scratch); } catch (...) { Py_XDECREF(own); throw; }
+        Py_XDECREF(own);
+        need(scratch.is_contiguous());
+        p.split_scratch = scratch.data_ptr();
+        p.split_scratch_bytes = scratch.numel() * scratch.element_size();
     }
 };
 
@@ -419,7 +417,8 @@ NATIVE(sdpa, 18)
         }
     p.rope_split_half = truth(a[15]);
     if (!none(a[14])) c.rope_scratch(tensor(a[14]), q, k);
-    c.go(a[16], name_of(a[17]));
+    c.lend(a[16]);
+    run(name_of(a[17]), [&] { return L.sdpa(&p); });
     return given(a[4], c.out);
 NATIVE_END
 
@@ -437,7 +436,8 @@ NATIVE(joint, 10)
         need(kr.sizes() == k.sizes() && kr.scalar_type() == k.scalar_type());
         c.rope_scratch(kr, q, k);
     }
-    c.go(Py_None, "joint_attention");
+    c.lend(Py_None);
+    run("joint_attention", [&] { return L.sdpa(&c.p); });
     return given(a[7], c.out);
 NATIVE_END
 
@@ -527,9 +527,8 @@ NATIVE(mha, 16)
     need(c.out.is_contiguous() && tensor(a[4]).dim() == 2 && tensor(a[4]).size(1) == inner);
     const Tensor y = output(a[15], c.out, n_out);
     const mi_linear_args po = linear_args(a[4], a[8], c.out, y, Py_None, n_out);
-    run("mha_forward", [&] { return L.linear_n(p, 3); });
-    c.go(Py_None, "mha_forward");
-    run("mha_forward", [&] { return L.linear(&po); });
+    c.lend(Py_None);
+    run("mha_forward", [&] { return L.linear_n(p, 3); }, [&] { return L.sdpa(&c.p); }, [&] { return L.linear(&po); });
     PyObject* parts[5] = {given(a[15], y), given(a[11], qkv[0]), given(a[12], qkv[1]), given(a[13], qkv[2]), given(a[14], c.out)};
     PyObject* t = PyTuple_New(5);
     for (int i = 0; i < 5; ++i) PyTuple_SET_ITEM(t, i, parts[i]);
@@ -610,15 +609,11 @@ NATIVE(sana, 13)
     const int64_t n_out = tensor(a[4]).size(0);
     const Tensor y = output(a[12], x, n_out);
     const mi_linear_args po = linear_args(a[4], a[5], attn, y, Py_None, n_out);
-    const char* op = "sana_self_attention";
-    run(op, [&] { return L.linear_n(p, 3); });
-    if (gq) {
-        void *const pq = q.data_ptr(), *const pk = k.data_ptr(), *const stream = current_stream();
-        const float eps = static_cast<float>(number(a[9]));
-        const int rows = rows32(n), cols = rows32(d);
-        run(op, [&] { return L.rms_norm_pair(pq, gq, pq, pk, gk, pk, rows, cols, 0, 0, eps, dt, stream); });
-    }
-    run(op, [&] { return L.linear_attn(&la); }, [&] { return L.linear(&po); });
+    void *const pq = q.data_ptr(), *const pk = k.data_ptr(), *const stream = current_stream();
+    const float rms_eps = static_cast<float>(number(a[9]));
+    const int rows = rows32(n), cols = rows32(d);
+    auto norms = [&] { return gq ? L.rms_norm_pair(pq, gq, pq, pk, gk, pk, rows, cols, 0, 0, rms_eps, dt, stream) : 0; };
+    run("sana_self_attention", [&] { return L.linear_n(p, 3); }, norms, [&] { return L.linear_attn(&la); }, [&] { return L.linear(&po); });
     return given(a[12], y);
 NATIVE_END
 

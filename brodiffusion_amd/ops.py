@@ -56,7 +56,7 @@ class _Unbuilt:
         return getattr(module, name)
 
 
-# The calls below try the native form first (host/py_ops.cpp). It returns None, having done nothing, unless the call is plainly
+# The calls below try the native form first (host/py_ops.cpp). It returns None, having launched nothing, unless the call is plainly
 # valid; the Python code behind it then finds what is wrong, and words it.
 _native = _Unbuilt()
 
