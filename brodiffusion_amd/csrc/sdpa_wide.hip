@@ -18,8 +18,8 @@
 //   (4 rows, one 64-byte window) are both free of bank conflicts.
 //
 // A query tile is 128 rows, so a VAE mid-block has 32 (64 x 64 latent) to 128 tiles for 256 compute units: the key axis is
-// cut into as many pieces as shorten the launch (wide_split), each leaving a normalised partial output and its softmax
-// statistics in the caller's scratch, merged in a fixed order by wide_combine_kernel.
+// cut into as many pieces as shorten the launch (wide_split), each leaving its output accumulators and softmax statistics in
+// the caller's scratch, all FP32, merged in a fixed order by wide_combine_kernel: the result is rounded once.
 //
 // Masks work as everywhere (per-row visible key interval, kv_valid_len, key mask); cached prefixes, logit bias, lse output,
 // packed sequences and K rotated tile by tile are not offered at these widths (K rotated into a scratch and Q rotated on
@@ -47,8 +47,9 @@ template <int D> struct WideGeo {
     static constexpr int LDS_BYTES = 4 * TILE > STAGED ? 4 * TILE : STAGED;
     static_assert(D % 128 == 0 && TILE % 4096 == 0, "whole swizzle groups per row, whole DMA instructions per wavefront");
     static_assert(LDS_BYTES <= 160 * 1024, "one work group must fit the LDS of a compute unit");
-    // a partial result: 128 rows of D 16-bit values, then 128 references and 128 denominators
-    static constexpr long SLOT = static_cast<long>(kWideRows) * (D * 2 + 8);
+    // A partial result, FP32: the accumulators of the four wavefronts as their lanes hold them (16-byte piece ((w D / 8 + c) 64 +
+    // lane): head-dim elements 8 c + 4 lh .. + 3 of row 32 w + lq), then 128 references and 128 denominators
+    static constexpr long SLOT = static_cast<long>(kWideRows) * (D * 4 + 8);
 };
 
 // The MFMAs of this kernel are inline assembly. At head_dim 512 the output accumulator of a wavefront is exactly the 256
@@ -356,31 +357,39 @@ __global__ void __launch_bounds__(kWideThreads, 1) sdpa_wide_kernel(const SdpaDe
 
     wide_settle(x);
     const float l_tot = exchange_sum(l_sum);
-    const float inv = row_inverse(l_tot);
-    [&]<int... B>(std::integer_sequence<int, B...>) {   // accumulation registers 4 B .. 4 B + 3: head-dim elements 8 B + 4 lh ..
-        ([&] {
-            typedef T t4 __attribute__((ext_vector_type(4)));
-            const float o0 = o_get<4 * B>(), o1 = o_get<4 * B + 1>(), o2 = o_get<4 * B + 2>(), o3 = o_get<4 * B + 3>();
-            const t4 ov = {static_cast<T>(o0 * inv), static_cast<T>(o1 * inv), static_cast<T>(o2 * inv), static_cast<T>(o3 * inv)};
-            *reinterpret_cast<t4*>(smem + (wave * 32 + lq) * G::O_STRIDE + (8 * B + 4 * lh) * 2) = ov;
-        }(), ...);
-    }(std::make_integer_sequence<int, 4 * VB>{});
-    __syncthreads();
+    // accumulation registers 4 B .. 4 B + 3: head-dim elements 8 B + 4 lh ..
     if (n_split == 1) {
+        const float inv = row_inverse(l_tot);
+        [&]<int... B>(std::integer_sequence<int, B...>) {
+            ([&] {
+                typedef T t4 __attribute__((ext_vector_type(4)));
+                const float o0 = o_get<4 * B>(), o1 = o_get<4 * B + 1>(), o2 = o_get<4 * B + 2>(), o3 = o_get<4 * B + 3>();
+                const t4 ov = {static_cast<T>(o0 * inv), static_cast<T>(o1 * inv), static_cast<T>(o2 * inv), static_cast<T>(o3 * inv)};
+                *reinterpret_cast<t4*>(smem + (wave * 32 + lq) * G::O_STRIDE + (8 * B + 4 * lh) * 2) = ov;
+            }(), ...);
+        }(std::make_integer_sequence<int, 4 * VB>{});
+        __syncthreads();
         write_output<T, D, kWideThreads>(smem, o_base, p.o_rs, q0, p.Lq, kWideRows, tid);
     } else {
         unsigned char* const slot = p.split_scratch + (static_cast<long>(tile) * n_split + piece) * W::SLOT;
-        write_output<T, D, kWideThreads>(smem, reinterpret_cast<T*>(slot), D, 0, min(kWideRows, p.Lq - q0), kWideRows, tid);
-        if (lh == 0) {   // the weight of the part in the merge is l * 2^ref
-            float* const stat = reinterpret_cast<float*>(slot + static_cast<long>(kWideRows) * D * 2);
+        f32x4* const part = reinterpret_cast<f32x4*>(slot) + wave * (D / 8) * 64 + lane;
+        [&]<int... B>(std::integer_sequence<int, B...>) {
+            ([&] {
+                const float o0 = o_get<4 * B>(), o1 = o_get<4 * B + 1>(), o2 = o_get<4 * B + 2>(), o3 = o_get<4 * B + 3>();
+                part[B * 64] = f32x4{o0, o1, o2, o3};
+            }(), ...);
+        }(std::make_integer_sequence<int, 4 * VB>{});
+        if (lh == 0) {   // the weight of the part in the merge is 2^ref
+            float* const stat = reinterpret_cast<float*>(slot + static_cast<long>(kWideRows) * D * 4);
             stat[wave * 32 + lq] = -neg_ref;
             stat[kWideRows + wave * 32 + lq] = l_tot;
         }
     }
 }
 
-// out = sum_k w_k O_k / sum_k w_k with w_k = l_k 2^(ref_k - max ref) over the pieces of a query tile, in a fixed order; one
-// 16-byte piece of a row per thread, blockIdx.x = query tile.
+// out = sum_k w_k O_k / sum_k w_k l_k with w_k = 2^(ref_k - max ref) over the pieces of a query tile, in a fixed order.
+// blockIdx.x = query tile; a thread takes 8 head-dim elements of a row, 8 consecutive threads the same elements of 8 rows, so that
+// 128 bytes of a part are together on the way in and (in a wavefront) 128 bytes of a row on the way out.
 template <typename T, int D>
 __global__ void __launch_bounds__(256) wide_combine_kernel(const SdpaDev p, int n_q_tiles, int n_split) {
     using W = WideGeo<D>;
@@ -390,9 +399,10 @@ __global__ void __launch_bounds__(256) wide_combine_kernel(const SdpaDev p, int 
     const int bh = tile / n_q_tiles, q0 = (tile - bh * n_q_tiles) * kWideRows;
     const int h = bh % p.H, b = bh / p.H;
     const int idx = static_cast<int>(blockIdx.y) * 256 + static_cast<int>(threadIdx.x);
-    const int row = idx / CPR, cc = idx - row * CPR;
+    const int cc = (idx >> 3) % CPR, row = (idx >> 3) / CPR * 8 + (idx & 7);
     if (row >= kWideRows || q0 + row >= p.Lq) return;
     const unsigned char* const slots = p.split_scratch + static_cast<long>(tile) * n_split * W::SLOT;
+    const long piece0 = ((row >> 5) * CPR + cc) * 64 + (row & 31);
     // (a part without visible keys has denominator 0 and is skipped; one whose denominator is NaN is not. The bits pass
     //  through an empty asm statement because -fno-honor-nans entitles the optimiser to a comparison that is false for NaN.)
     auto empty = [](float l) {
@@ -402,42 +412,52 @@ __global__ void __launch_bounds__(256) wide_combine_kernel(const SdpaDev p, int 
     };
     float ref = kNegInf;
     for (int k = 0; k < n_split; ++k) {
-        const float* stat = reinterpret_cast<const float*>(slots + k * W::SLOT + static_cast<long>(kWideRows) * D * 2);
+        const float* stat = reinterpret_cast<const float*>(slots + k * W::SLOT + static_cast<long>(kWideRows) * D * 4);
         if (!empty(stat[kWideRows + row])) ref = fmaxf(ref, stat[row]);
     }
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    float wsum = 0.f;
+    float lsum = 0.f;
     for (int k = 0; k < n_split; ++k) {
         const unsigned char* slot = slots + k * W::SLOT;
-        const float* stat = reinterpret_cast<const float*>(slot + static_cast<long>(kWideRows) * D * 2);
+        const float* stat = reinterpret_cast<const float*>(slot + static_cast<long>(kWideRows) * D * 4);
+        const f32x4 lo = reinterpret_cast<const f32x4*>(slot)[piece0], hi = reinterpret_cast<const f32x4*>(slot)[piece0 + 32];
         const float l = stat[kWideRows + row];
         if (empty(l)) continue;
-        const float w = l * __builtin_amdgcn_exp2f(stat[row] - ref);
-        wsum += w;
-        const t8 o = *reinterpret_cast<const t8*>(slot + (static_cast<long>(row) * D + cc * 8) * 2);
+        const float w = __builtin_amdgcn_exp2f(stat[row] - ref);
+        lsum = __builtin_fmaf(w, l, lsum);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc[e] = __builtin_fmaf(w, static_cast<float>(o[e]), acc[e]);
+        for (int e = 0; e < 4; ++e) {
+            acc[e] = __builtin_fmaf(w, lo[e], acc[e]);
+            acc[4 + e] = __builtin_fmaf(w, hi[e], acc[4 + e]);
+        }
     }
-    const float inv = row_inverse(wsum);
+    const float inv = row_inverse(lsum);
     t8 out;
 #pragma unroll
     for (int e = 0; e < 8; ++e) out[e] = static_cast<T>(acc[e] * inv);
     *reinterpret_cast<t8*>(static_cast<T*>(p.o) + b * p.o_bs + static_cast<long>(q0 + row) * p.o_rs + h * D + cc * 8) = out;
 }
 
-// Pieces of the key axis: as many as minimise rounds x (steps of a piece + what a work group costs beyond its steps, about
-// kOverhead of them: Q staging, first tiles, write-out), plus the merge pass when there is one. Only unmasked calls (a valid
-// length or key mask may be on): with causal masks the tiles are unequal and fill the GPU in their own way.
+// Pieces of the key axis: as many as minimise the launch, counted in steps: rounds x (steps of a piece + kOverhead: Q staging,
+// first tiles, write-out), and for the merge kMerge plus kParts per part on every compute unit (128 x D FP32 values written and
+// read again). Fitted on MI355X to 1 .. 16 pieces of 13 lengths from 384 to 16384 tokens at each head dimension: the number
+// taken is 0.9 % slower than the best one on average, 4.3 % at worst (without kParts 3.5 and 15 %). At 512, one head, in us:
+//   1024 tokens (8 tiles)   1 piece 54.6   3 34.5   5 32.1 (taken)   8 35.4
+//   4096 (32)               1 168          4 67.2   6 63.4 (taken)   8 66.6   9 (a second round) 91.4
+//   9216 (72)               1 358          2 208    3 182 (taken)    7 210
+//   16384 (128)             1 634          2 483 (taken)             4 508
+// Only unmasked calls (a valid length or key mask may be on): with causal masks the tiles are unequal and fill the GPU in their
+// own way.
 int wide_split(const SdpaDev& p, int n_cu) {
     if (p.mask_mode != MI_MASK_NONE) return 1;
     const long tiles = static_cast<long>(p.B) * p.H * ((p.Lq + kWideRows - 1) / kWideRows);
     const int steps = (p.Lk + kWideKeys - 1) / kWideKeys;
-    constexpr int kOverhead = 6, kMerge = 4, kMaxSplit = 16, kMinSteps = 6;
+    constexpr int kOverhead = 6, kMerge = 4, kParts = 24, kMaxSplit = 16, kMinSteps = 6;
     int best = 1;
     long best_cost = 0;
     for (int s = 1; s <= kMaxSplit && (s == 1 || steps / s >= kMinSteps); ++s) {
         const long rounds = (tiles * s + n_cu - 1) / n_cu;
-        const long cost = rounds * ((steps + s - 1) / s + kOverhead) + (s > 1 ? kMerge : 0);
+        const long cost = rounds * ((steps + s - 1) / s + kOverhead) + (s > 1 ? kMerge + kParts * tiles * s / n_cu : 0);
         if (s == 1 || cost < best_cost) { best = s; best_cost = cost; }
     }
     return best;
@@ -475,7 +495,7 @@ bool sdpa_wide_head(int head_dim) { return head_dim == 256 || head_dim == 384 ||
 size_t sdpa_wide_split_scratch_bytes(const SdpaDev& p, int head_dim) {
     const int n_split = wide_split(p, device_cu_count());
     if (n_split == 1) return 0;
-    const size_t slot = static_cast<size_t>(kWideRows) * (static_cast<size_t>(head_dim) * 2 + 8);
+    const size_t slot = static_cast<size_t>(kWideRows) * (static_cast<size_t>(head_dim) * 4 + 8);
     return static_cast<size_t>(p.B) * p.H * ((p.Lq + kWideRows - 1) / kWideRows) * n_split * slot;
 }
 

@@ -140,7 +140,7 @@ def test_wide_head_rope(oracle, dtype, d, split_half):
 ])
 def test_wide_head_key_axis_in_pieces(oracle, dtype, B, H, d, Lq, Lk, valid):
     """With a scratch lent the key axis is cut into pieces whose partial results are merged: as the checker, and as the
-    launch in one piece to two units in the last place (each part is rounded once more before the merge)."""
+    launch in one piece to two units in the last place (the probabilities of a piece are rounded against its own reference)."""
     q, k, v = (randn(8541 + i, (B, n, H * d), dtype) for i, n in enumerate((Lq, Lk, Lk)))
     dq, dk, dv = (to_dev(x, dtype) for x in (q, k, v))
     kw = {} if valid is None else {"kv_valid_len": torch.tensor(valid, dtype=torch.int32, device="cuda")}
@@ -152,3 +152,16 @@ def test_wide_head_key_axis_in_pieces(oracle, dtype, B, H, d, Lq, Lk, valid):
     for b in range(B):
         n = Lk if valid is None else valid[b]
         assert_close(oracle.sdpa(q[b], k[b, :n], v[b, :n], H), to_np(pieces[b]), dtype, f"pieces d={d} batch {b}")
+
+
+@pytest.mark.parametrize("dtype,d", [("fp16", 512), ("bf16", 512), ("bf16", 384), ("fp16", 256)])
+def test_pieces_are_as_close_to_the_exact_result_as_the_whole(dtype, d):
+    """The parts of a cut launch are merged in FP32 and rounded once. Against 64 bits: the probabilities' rounding and the
+    result's make an error of sqrt(2) roundings either way; parts rounded to 16 bits before the merge would make it sqrt(3)."""
+    Lq, Lk = 256, 4096
+    q, k, v = (to_dev(randn(8561 + i, (n, d), dtype), dtype) for i, n in enumerate((Lq, Lk, Lk)))
+    exact = torch.softmax(q.double() @ k.double().t().contiguous() * d ** -0.5, dim=-1) @ v.double()
+    whole, pieces = bd.sdpa_forward(q, k, v, 1, split_scratch=False), bd.sdpa_forward(q, k, v, 1)
+    assert not torch.equal(whole, pieces), "this shape is expected to be cut"
+    error = [((x.double() - exact).norm() / exact.norm()).item() for x in (whole, pieces)]
+    assert error[1] <= 1.05 * error[0], error
