@@ -28,7 +28,7 @@ int device_cu_count();
 // rounds even when the last round fills only part of the GPU (432 tiles on 256 compute units: 2 rounds for 1.69
 // rounds of work). With the split, the tiles of the full rounds are processed whole and the tiles of the last round
 // are cut along the KEY axis into as many equal pieces as there are work-group slots; a piece covers the end of one
-// tile and the start of the next, each part leaves a normalised partial output plus its softmax statistics in a
+// tile and the start of the next, each part leaves its output accumulators and softmax statistics, all FP32, in a
 // scratch slot, and a small second kernel merges the parts of every tile. Everything is done per XCD group (work
 // groups whose id is g mod 8 share an L2): group g owns the logical tiles [g*chunk, (g+1)*chunk) and cu_g work-group
 // slots. All quantities are counted in key tiles of 64 keys ("steps"); T is the number of steps of one query tile.
@@ -51,8 +51,8 @@ struct SplitGeo {
     __host__ __device__ static int piece_begin(int c, int S, int np) { return static_cast<int>(static_cast<long>(c) * S / np); }
     // the piece that holds tail step x
     __host__ __device__ static int piece_of(int x, int S, int np) { return static_cast<int>((static_cast<long>(x + 1) * np + S - 1) / S) - 1; }
-    // bytes of one partial slot: 256 rows of head_dim 16-bit values, then 256 references and 256 denominators (FP32)
-    __host__ __device__ static long slot_bytes(int head_dim) { return 256L * head_dim * 2 + 256L * 8; }
+    // bytes of one partial slot, FP32: 256 rows of head_dim values, then 256 references and 256 denominators
+    __host__ __device__ static long slot_bytes(int head_dim) { return 256L * head_dim * 4 + 256L * 8; }
 };
 
 // Device-side view of one softmax-attention launch. Strides in elements.

@@ -1248,32 +1248,38 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
         if (p.lse && qvalid && lh == 0)
             p.lse[(static_cast<long>(b) * p.H + h) * p.Lq + qrow] = l_tot > 0.f ? __builtin_amdgcn_logf(l_tot) - st.neg_ref : __builtin_huge_valf();
     }
-    stage_output<T, D>(smem, wave * 32 + lq, lh, oacc, inv);
-    __syncthreads();
-    if constexpr (!SPLIT) {
+    if (!SPLIT || part == nullptr) {
+        stage_output<T, D>(smem, wave * 32 + lq, lh, oacc, inv);
+        __syncthreads();
         write_output<T, D, kThreads8>(smem, o_base, p.o_rs, q0, p.Lq, BM, tid);
+    } else {
+        // the accumulators of the part as the lanes hold them: 16-byte piece (wave D / 8 + c) 64 + lane is head-dim elements
+        // 8 c + 4 lh .. + 3 of row 32 wave + lq; then per row the softmax reference (log2 domain) and the denominator relative
+        // to it: the part's weight in the merge is 2^ref
+        f32x4* const slot = reinterpret_cast<f32x4*>(part) + wave * (D / 8) * 64 + lane;
+#pragma unroll
+        for (int c = 0; c < D / 8; ++c) {
+            const f32x16 block = oacc[c >> 2];
+            const int e = 4 * (c & 3);
+            slot[c * 64] = f32x4{block[e], block[e + 1], block[e + 2], block[e + 3]};
+        }
+        if (lh == 0) {
+            float* const stat = reinterpret_cast<float*>(part + static_cast<long>(BM) * D * 4);
+            stat[wave * 32 + lq] = -st.neg_ref;
+            stat[BM + wave * 32 + lq] = l_tot;
+        }
+    }
+    if constexpr (!SPLIT) {
         break;
     } else {
-        if (part == nullptr) {
-            write_output<T, D, kThreads8>(smem, o_base, p.o_rs, q0, p.Lq, BM, tid);
-        } else {
-            // normalised partial output of the part, then per row the softmax reference (log2 domain) and the
-            // denominator relative to it: the part's weight in the merge is l * 2^ref
-            write_output<T, D, kThreads8>(smem, reinterpret_cast<T*>(part), D, 0, min(BM, p.Lq - q0), BM, tid);
-            if (lh == 0) {
-                float* stat = reinterpret_cast<float*>(part + static_cast<long>(BM) * D * 2);
-                stat[wave * 32 + lq] = -st.neg_ref;
-                stat[BM + wave * 32 + lq] = l_tot;
-            }
-        }
         if (whole || seg_s >= seg_end) break;
         __syncthreads();   // the staged output is read by all threads before the next part stages its Q tile
     }
   }
 }
 
-// Merge of the parts of one split query tile: out = sum_k w_k O_k / sum_k w_k with w_k = l_k 2^(ref_k - max ref).
-// blockIdx.x = (XCD group, tail tile); tiles that were written whole are skipped.
+// Merge of the parts of one split query tile: out = sum_k w_k O_k / sum_k w_k l_k with w_k = 2^(ref_k - max ref), FP32, one
+// rounding. blockIdx.x = (XCD group, tail tile); tiles that were written whole are skipped.
 template <typename T, int D>
 __global__ void __launch_bounds__(256) sdpa_combine_kernel(const SdpaDev p) {
     typedef T t8 __attribute__((ext_vector_type(8)));
@@ -1291,13 +1297,15 @@ __global__ void __launch_bounds__(256) sdpa_combine_kernel(const SdpaDev p) {
     const int q0 = qt * BM;
     T* const o_base = static_cast<T*>(p.o) + b * p.o_bs + h * D;
     const unsigned char* slots = p.split_scratch + static_cast<long>(xg * sg.max_tail + tt) * sg.max_parts * SplitGeo::slot_bytes(D);
-    // one 16-byte piece of one row per thread; blockIdx.y walks the tile (many short work groups: the merge is a
-    // chain of two dependent loads per part, hidden by occupancy rather than by unrolling)
+    // 8 head-dim elements of one row per thread, 8 consecutive threads the same elements of 8 rows (128 bytes of a part
+    // together); blockIdx.y walks the tile (many short work groups: the merge is a chain of two dependent loads per part,
+    // hidden by occupancy rather than by unrolling)
     {
         const int idx = static_cast<int>(blockIdx.y) * 256 + static_cast<int>(threadIdx.x);
         if (idx >= BM * CPR) return;
-        const int row = idx / CPR, cc = idx - row * CPR;
+        const int cc = (idx >> 3) % CPR, row = (idx >> 3) / CPR * 8 + (idx & 7);
         if (q0 + row >= p.Lq) return;
+        const long piece0 = ((row >> 5) * CPR + cc) * 64 + (row & 31);
         // a part without visible keys has denominator 0 and is skipped; one whose denominator is NaN (a non-finite score)
         // must not be: it makes the row NaN, as it would in an unsplit launch. Hence the test on the bits.
         // (the bits pass through an empty asm statement: left visible, the optimiser turns the integer test back into a
@@ -1309,23 +1317,26 @@ __global__ void __launch_bounds__(256) sdpa_combine_kernel(const SdpaDev p) {
         };
         float ref = kNegInf;
         for (int k = 0; k < n_parts; ++k) {
-            const float* stat = reinterpret_cast<const float*>(slots + k * SplitGeo::slot_bytes(D) + static_cast<long>(BM) * D * 2);
+            const float* stat = reinterpret_cast<const float*>(slots + k * SplitGeo::slot_bytes(D) + static_cast<long>(BM) * D * 4);
             if (!empty(stat[BM + row])) ref = fmaxf(ref, stat[row]);
         }
         float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        float wsum = 0.f;
+        float lsum = 0.f;
         for (int k = 0; k < n_parts; ++k) {
             const unsigned char* slot = slots + k * SplitGeo::slot_bytes(D);
-            const float* stat = reinterpret_cast<const float*>(slot + static_cast<long>(BM) * D * 2);
+            const float* stat = reinterpret_cast<const float*>(slot + static_cast<long>(BM) * D * 4);
+            const f32x4 lo = reinterpret_cast<const f32x4*>(slot)[piece0], hi = reinterpret_cast<const f32x4*>(slot)[piece0 + 32];
             const float l = stat[BM + row];
             if (empty(l)) continue;
-            const float w = l * __builtin_amdgcn_exp2f(stat[row] - ref);
-            wsum += w;
-            const t8 o = *reinterpret_cast<const t8*>(slot + (static_cast<long>(row) * D + cc * 8) * 2);
+            const float w = __builtin_amdgcn_exp2f(stat[row] - ref);
+            lsum = __builtin_fmaf(w, l, lsum);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) acc[e] = __builtin_fmaf(w, static_cast<float>(o[e]), acc[e]);
+            for (int e = 0; e < 4; ++e) {
+                acc[e] = __builtin_fmaf(w, lo[e], acc[e]);
+                acc[4 + e] = __builtin_fmaf(w, hi[e], acc[4 + e]);
+            }
         }
-        const float inv = row_inverse(wsum);
+        const float inv = row_inverse(lsum);
         t8 out;
 #pragma unroll
         for (int e = 0; e < 8; ++e) out[e] = static_cast<T>(acc[e] * inv);

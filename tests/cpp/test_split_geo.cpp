@@ -65,7 +65,7 @@ int main() {
                 CHECK(covered_tiles == n_blocks);
                 ++cases;
             }
-    CHECK(mi::SplitGeo::slot_bytes(128) == 256L * 128 * 2 + 2048 && mi::SplitGeo::slot_bytes(72) % 16 == 0);
+    CHECK(mi::SplitGeo::slot_bytes(128) == 256L * 128 * 4 + 2048 && mi::SplitGeo::slot_bytes(72) % 16 == 0);
     if (g_failures == 0) std::printf("test_split_geo: OK (%d configurations)\n", cases);
     return g_failures == 0 ? 0 : 1;
 }

@@ -1,8 +1,8 @@
 """Key-axis split of the last round of work groups (mi_sdpa_args.split_scratch): a launch whose query tiles do not
 fill the GPU a whole number of times cuts the tiles of the last round into pieces for all compute units and merges
-the partial results. The split result must agree with the unsplit launch to rounding (each part's normalised output
-is rounded to the storage type once more before the merge: at most 2 units in the last place) and with the CPU
-checker to the usual tolerance (helpers.TOL)."""
+the partial results in FP32. The split result must agree with the unsplit launch to rounding (the probabilities of a part
+are rounded against its own reference: at most 2 units in the last place) and with the CPU checker to the usual tolerance
+(helpers.TOL)."""
 import ctypes as C
 
 import numpy as np
@@ -62,6 +62,27 @@ def test_split_matches_unsplit_and_checker(oracle, dtype, B, H, d, Lq, Lk):
     # one byte short: the library falls back to the unsplit launch
     short = bd.sdpa_forward(dq, dk, dv, H, split_scratch=scratch[: need - 16])
     assert torch.equal(short, plain)
+
+
+@pytest.mark.parametrize("dtype,H,d,L", [("bf16", 24, 128, 3328), ("fp16", 24, 128, 3328), ("bf16", 16, 72, 4352)])
+def test_split_tiles_are_as_close_to_the_exact_result_as_whole_ones(dtype, H, d, L):
+    """Against 64 bits, over the query tiles that are cut: the probabilities' rounding and the result's make an error of sqrt(2)
+    roundings either way; parts rounded to 16 bits before the merge would make it sqrt(3)."""
+    q, k, v = (to_dev(randn(8251 + i, (L, H * d), dtype), dtype) for i in range(3))
+    whole, split = bd.sdpa_forward(q, k, v, H, split_scratch=False), bd.sdpa_forward(q, k, v, H)
+    tiles = L // 256
+
+    def by_tile(x):
+        return x.view(tiles, 256, H, d).permute(2, 0, 1, 3).double()
+    cut = (by_tile(whole) != by_tile(split)).flatten(2).any(-1)       # (heads, tiles)
+    assert 0 < cut.sum().item() < H * tiles
+    errors = torch.zeros(2, dtype=torch.float64, device="cuda")
+    for h in cut.any(1).nonzero().flatten().tolist():
+        qh, kh, vh = (x[:, h * d:(h + 1) * d].double().contiguous() for x in (q, k, v))
+        exact = (torch.softmax(qh @ kh.t().contiguous() * d ** -0.5, dim=-1) @ vh).view(tiles, 256, d)[cut[h]]
+        for i, x in enumerate((whole, split)):
+            errors[i] += (by_tile(x)[h][cut[h]] - exact).square().sum()
+    assert errors[1].sqrt() <= 1.05 * errors[0].sqrt(), errors.sqrt().tolist()
 
 
 def test_split_then_smaller_call_reuses_scratch(oracle):
