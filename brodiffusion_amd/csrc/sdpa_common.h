@@ -512,7 +512,7 @@ struct RelSoftmaxState {
 };
 constexpr float kRelSumMax = 1024.f;
 
-template <typename T, int D, bool PSCALE = false, bool XTRA = false>
+template <typename T, int D, bool PSCALE = false, bool XTRA = false, bool F32SUM = false>
 __device__ __forceinline__ void softmax_tile_rel(f32x16 (&sacc)[2], typename Mma<T>::v8 (&pf)[4], f32x16 (&oacc)[HeadGeo<D>::VB],
                                                  RelSoftmaxState& st, bool masked, bool dead_row, int j0, int lo, int hi, int lh,
                                                  PrefixScale prefix = PrefixScale(), TileExtra xt = TileExtra()) {
@@ -578,8 +578,9 @@ __device__ __forceinline__ void softmax_tile_rel(f32x16 (&sacc)[2], typename Mma
     // sums exactly the values the PV product uses; measured 4 % faster at head_dim 40 and 72). From 112 on the matrix
     // pipe is the busier unit and the same change measured 6 % slower, so there the FP32 exponentials are added.
     // (not in the XTRA instances: their denominators are an output, from which the attention map is rebuilt in FP32, so they
-    // sum the exponentials before the rounding to 16 bits.)
-    constexpr bool PAIR_SUM = HeadGeo<D>::VB < 4 && !XTRA;
+    // sum the exponentials before the rounding to 16 bits; nor with F32SUM: launches below one 256-row tile per CU, where the
+    // 128-row kernel, which sums in FP32 too, is the other choice, so that the choice does not change a result's precision.)
+    constexpr bool PAIR_SUM = HeadGeo<D>::VB < 4 && !XTRA && !F32SUM;
     auto exponentiate = [&]() -> float {
         float s0 = 0.f, s1 = 0.f;
         if (PSCALE && prefix.on) {

@@ -506,7 +506,8 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_shortkv_kernel(const SdpaDe
 // measures 2-3 % faster (at 80 the compiler's allocation of that instance goes wrong: twice as slow) and kRagged 13 %
 // (head_dim 40, 8 heads, 3600 tokens: 67.0 -> 58.5 us).
 // XTRA: key mask, logit bias and softmax denominators (see sdpa_fwd_pp_dma_kernel).
-template <typename T, int D, bool ROPE_K, int FORM = kGeneral, bool XTRA = false>
+// F32SUM: see softmax_tile_rel.
+template <typename T, int D, bool ROPE_K, int FORM = kGeneral, bool XTRA = false, bool F32SUM = false>
 __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_kernel(const SdpaDev p) {
     constexpr bool DENSE = FORM != kGeneral, RAGGED = FORM == kRagged;
     static_assert(!XTRA || (!DENSE && !ROPE_K), "key mask, bias and denominators belong to the general form");
@@ -639,7 +640,7 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_kernel(const SdpaDev
             if constexpr (DENSE) {
                 if (tt >= 0 && tt < n_tiles) {
                     const int rows = RAGGED ? min(n_keys - tt * kBN, kBN) : kBN;
-                    softmax_tile_rel<T, D>(sacc, pf, oacc, st, RAGGED && rows < kBN, false, 0, 0, rows, lh);
+                    softmax_tile_rel<T, D, false, false, F32SUM>(sacc, pf, oacc, st, RAGGED && rows < kBN, false, 0, 0, rows, lh);
                     return;
                 }
             }
@@ -662,7 +663,7 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_kernel(const SdpaDev
                     xt.bias_row = biased ? bias_row : nullptr;
                     xt.bias_vec = p.bias_vec_ok && (j0 & 3) == 0 && j0 + kBN <= p.bias_cols;
                 }
-                softmax_tile_rel<T, D, false, XTRA>(sacc, pf, oacc, st, !interior, dead_row, j0, lo, min(hi, lim), lh, PrefixScale(), xt);
+                softmax_tile_rel<T, D, false, XTRA, F32SUM>(sacc, pf, oacc, st, !interior, dead_row, j0, lo, min(hi, lim), lh, PrefixScale(), xt);
             } else {
                 // nothing visible to this wavefront in that tile: the next PV pass must add zero
 #pragma unroll
@@ -767,7 +768,8 @@ __device__ __forceinline__ int swz(int row) { return 4 * (row & 3) + ((row >> 2)
 // the middle of a joint sequence), so the tiles without a visible key are taken out of the walk: `vis` lists the others, and a
 // step looks up the tile that it loads. 48 query / 12 K/V heads of 128, 4608 tokens of which 435 are padding (6 of 72 tiles):
 // 520 -> 472 us; the words used to blank the scores of a hidden tile, whose MFMAs and loads ran all the same.
-template <typename T, int D, bool SPLIT, int FORM = kGeneral, bool PSCALE = false, bool XTRA = false>
+// F32SUM: see softmax_tile_rel.
+template <typename T, int D, bool SPLIT, int FORM = kGeneral, bool PSCALE = false, bool XTRA = false, bool F32SUM = false>
 __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const SdpaDev p) {
     constexpr bool DENSE = FORM != kGeneral, RAGGED = FORM == kRagged, LISTED = XTRA && RAGGED;
     static_assert(!(SPLIT && DENSE), "the split launch clips key ranges per part");
@@ -1061,7 +1063,7 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
             } else if constexpr (DENSE) {
                 if (tt >= 0 && tt < n_tiles) {
                     const int rows = RAGGED ? plan.limit(tt) - plan.j0(tt) : kBN;
-                    softmax_tile_rel<T, D>(sacc, pf, oacc, st, RAGGED && rows < kBN, false, 0, 0, rows, lh);
+                    softmax_tile_rel<T, D, false, false, F32SUM>(sacc, pf, oacc, st, RAGGED && rows < kBN, false, 0, 0, rows, lh);
                     return;
                 }
             }
@@ -1075,7 +1077,7 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
                     xt.bias_row = biased ? bias_row : nullptr;
                     xt.bias_vec = p.bias_vec_ok && (j0 & 3) == 0 && j0 + kBN <= p.bias_cols;
                 }
-                softmax_tile_rel<T, D, PSCALE, XTRA>(sacc, pf, oacc, st, !interior, dead_row, j0, lo, min(hi, lim), lh,
+                softmax_tile_rel<T, D, PSCALE, XTRA, F32SUM>(sacc, pf, oacc, st, !interior, dead_row, j0, lo, min(hi, lim), lh,
                                                      PSCALE ? prefix_scale_of(p, plan.in_prefix(tt)) : PrefixScale(), xt);
             } else {
                 // nothing visible to this wavefront in that tile: the next PV pass must add zero
@@ -1500,26 +1502,42 @@ int launch_d(SdpaDev p, int n_cu, hipStream_t stream) {
                     hipLaunchKernelGGL((sdpa_fwd_pp_kernel<T, D, false, kGeneral, true>), grid, block, lds_bytes_8<D>() + kbits_bytes, stream, p);
                 }
             }
-            else if (rope_k) hipLaunchKernelGGL((sdpa_fwd_pp_kernel<T, D, true>), grid, block, lds_bytes_8<D>(), stream, p);
-            else if (dma_kernel_available<D>() && sdpa_kernel_choice() != 3) {
-                if constexpr (dma_kernel_available<D>()) {
-                    // whole key tiles only; a cached prefix may come first if it is whole tiles too and laid out like K / V
-                    const bool dense = p.mask_mode == MI_MASK_NONE && p.kv_valid_len == nullptr && p.Lk % kBN == 0 && !p.prefix_scaled &&
-                                       (p.Lp == 0 || (p.Lp % kBN == 0 && p.kp_rs == p.k_rs && p.vp_rs == p.v_rs));
-                    const bool ragged = same_keys_for_all_rows(p);
-                    if (dense) hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, false, kDense>), grid, block, DmaGeo<D>::lds_bytes(), stream, p);
-                    else if (ragged) hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, false, kRagged>), grid, block, DmaGeo<D>::lds_bytes(), stream, p);
-                    else if (p.prefix_scaled) hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, false, kGeneral, true>), grid, block, DmaGeo<D>::lds_bytes(), stream, p);
-                    else hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, false>), grid, block, DmaGeo<D>::lds_bytes(), stream, p);
-                }
+            else {
+                auto launch = [&](auto f32_sum) {
+                    constexpr bool F = decltype(f32_sum)::value;
+                    if (rope_k) {
+                        hipLaunchKernelGGL((sdpa_fwd_pp_kernel<T, D, true, kGeneral, false, F>), grid, block, lds_bytes_8<D>(), stream, p);
+                        return;
+                    }
+                    const bool dense = p.mask_mode == MI_MASK_NONE && p.kv_valid_len == nullptr && p.Lk % kBN == 0 && !p.prefix_scaled;
+                    if constexpr (dma_kernel_available<D>()) {
+                        if (sdpa_kernel_choice() != 3) {
+                            constexpr int lds = DmaGeo<D>::lds_bytes();
+                            // whole key tiles only; a cached prefix may come first if it is whole tiles too and laid out like K / V
+                            const bool whole = dense && (p.Lp == 0 || (p.Lp % kBN == 0 && p.kp_rs == p.k_rs && p.vp_rs == p.v_rs));
+                            if (whole) hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, false, kDense, false, false, F>), grid, block, lds, stream, p);
+                            else if (same_keys_for_all_rows(p)) hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, false, kRagged, false, false, F>), grid, block, lds, stream, p);
+                            else if (p.prefix_scaled) hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, false, kGeneral, true>), grid, block, lds, stream, p);
+                            else hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, false, kGeneral, false, false, F>), grid, block, lds, stream, p);
+                            return;
+                        }
+                    }
+                    if constexpr (D <= 64) {
+                        if (p.mask_mode == MI_MASK_NONE && p.Lp == 0) {
+                            if (dense) hipLaunchKernelGGL((sdpa_fwd_pp_kernel<T, D, false, kDense, false, F>), grid, block, lds_bytes_8<D>(), stream, p);
+                            else hipLaunchKernelGGL((sdpa_fwd_pp_kernel<T, D, false, kRagged, false, F>), grid, block, lds_bytes_8<D>(), stream, p);
+                            return;
+                        }
+                    }
+                    // (below one tile per CU only 80 and 96 come here: rows256_pay)
+                    if constexpr (!F || D > 72) hipLaunchKernelGGL((sdpa_fwd_pp_kernel<T, D, false, kGeneral, false, F>), grid, block, lds_bytes_8<D>(), stream, p);
+                };
+                // the form of the denominators (from head_dim 112 on there is one)
+                if constexpr (HeadGeo<D>::VB < 4) {
+                    if (choice == 0 && tiles256 < n_cu) launch(std::true_type{});
+                    else launch(std::false_type{});
+                } else launch(std::false_type{});
             }
-            else if (D <= 64 && p.mask_mode == MI_MASK_NONE && p.Lp == 0) {
-                if constexpr (D <= 64) {
-                    if (p.kv_valid_len == nullptr && p.Lk % kBN == 0) hipLaunchKernelGGL((sdpa_fwd_pp_kernel<T, D, false, kDense>), grid, block, lds_bytes_8<D>(), stream, p);
-                    else hipLaunchKernelGGL((sdpa_fwd_pp_kernel<T, D, false, kRagged>), grid, block, lds_bytes_8<D>(), stream, p);
-                }
-            }
-            else hipLaunchKernelGGL((sdpa_fwd_pp_kernel<T, D, false>), grid, block, lds_bytes_8<D>(), stream, p);
         }
     } else {
         if constexpr (pair_kernel_available<D>()) {
