@@ -29,7 +29,7 @@ EXPORTS = [
     "mi_malloc", "mi_free", "mi_memcpy_h2d", "mi_memcpy_d2h", "mi_memcpy_d2d_async", "mi_memset_async",
     "mi_sdpa_forward", "mi_sdpa_split_scratch_bytes", "mi_sdpa_supported", "mi_sdpa_set_kernel_choice", "mi_attention_map_avg", "mi_rope_apply", "mi_headnorm_rope", "mi_scale_rows",
     "mi_linear_attn_workspace_bytes", "mi_linear_attn_scratch_bytes", "mi_linear_attn_relu_forward", "mi_linear_attn_supported", "mi_linear_attn_relu_forward_static_scratch",
-    "mi_linear_forward", "mi_linear_forward_n", "mi_linear_geglu_forward", "mi_add_inplace", "mi_add_row_bias", "mi_rms_norm_forward", "mi_rms_norm_pair_forward", "mi_flash_attention_scratch_bytes", "mi_flash_attention_qkvo_forward",
+    "mi_linear_forward", "mi_linear_forward_n", "mi_linear_geglu_forward", "mi_add_inplace", "mi_add_row_bias", "mi_rms_norm_forward", "mi_rms_norm_pair_forward", "mi_flash_attention_scratch_bytes", "mi_attn_block_scratch_bytes", "mi_flash_attention_qkvo_forward",
     "mi_flash_attention_q_with_kv_cached_forward", "mi_flash_attention_project_kv",
 ]
 
@@ -211,6 +211,8 @@ def lib() -> C.CDLL:
         L.mi_rms_norm_pair_forward.argtypes = [C.c_void_p] * 6 + [C.c_int32, C.c_int32, C.c_int64, C.c_int64, C.c_float, C.c_int32, C.c_void_p]
         L.mi_flash_attention_scratch_bytes.argtypes = [C.c_int32] * 5
         L.mi_flash_attention_scratch_bytes.restype = C.c_size_t
+        L.mi_attn_block_scratch_bytes.argtypes = [C.POINTER(MiAttnBlockArgs)]
+        L.mi_attn_block_scratch_bytes.restype = C.c_size_t
         for name in ("mi_flash_attention_qkvo_forward", "mi_flash_attention_q_with_kv_cached_forward", "mi_flash_attention_project_kv"):
             getattr(L, name).argtypes = [C.POINTER(MiAttnBlockArgs)]
         _lib = L

@@ -49,20 +49,20 @@ LinearProblem problem(const void* x, const void* w, const void* bias, void* y, l
     return p;
 }
 
-// What the attention launch of a block of these sizes may use to cut the key axis into pieces, whichever head count its
-// channels turn out to have.
-size_t split_bytes(int batch, int q_len, int kv_len, int inner) {
-    size_t most = 0;
-    if (q_len == 0 || kv_len == 0) return 0;
-    for (int hd = 8; hd <= inner; hd += 8) {
-        if (inner % hd || !sdpa_supported(MI_DTYPE_F16, hd)) continue;
-        SdpaDev p;
-        std::memset(&p, 0, sizeof(p));
-        p.B = batch; p.H = inner / hd; p.Lq = q_len; p.Lk = kv_len;
-        const size_t n = sdpa_split_scratch_bytes(p, MI_DTYPE_F16, hd);
-        most = n > most ? n : most;
-    }
-    return most;
+// What the attention launch of a block uses to cut the key axis into pieces.
+size_t split_bytes(int batch, int q_len, int kv_len, int num_heads, int head_dim, bool causal = false, const float* key_mask = nullptr) {
+    if (q_len == 0 || kv_len == 0 || !sdpa_supported(MI_DTYPE_F16, head_dim)) return 0;
+    SdpaDev p;
+    std::memset(&p, 0, sizeof(p));
+    p.B = batch; p.H = num_heads; p.Lq = q_len; p.Lk = kv_len;
+    p.mask_mode = causal ? MI_MASK_CAUSAL : MI_MASK_NONE;
+    p.key_mask = key_mask;
+    return sdpa_split_scratch_bytes(p, MI_DTYPE_F16, head_dim);
+}
+size_t block_scratch(int batch, int q_len, int kv_len, int inner, bool with_kv, size_t split) {
+    const size_t q = round_up(static_cast<size_t>(batch) * q_len * inner * 2);
+    const size_t kv = round_up(static_cast<size_t>(batch) * kv_len * inner * 2);
+    return 2 * q + (with_kv ? 2 * kv : 0) + round_up(split);
 }
 
 // [scratch_used, scratch_bytes) of the caller's scratch is lent to the attention launch.
@@ -135,9 +135,15 @@ int mi_linear_geglu_forward(const mi_linear_args* a) {
 
 size_t mi_flash_attention_scratch_bytes(int32_t batch, int32_t q_len, int32_t kv_len, int32_t inner, int32_t with_kv) {
     if (batch <= 0 || q_len < 0 || kv_len < 0 || inner <= 0) return 0;
-    const size_t q = mi::round_up(static_cast<size_t>(batch) * q_len * inner * 2);
-    const size_t kv = mi::round_up(static_cast<size_t>(batch) * kv_len * inner * 2);
-    return 2 * q + (with_kv ? 2 * kv : 0) + mi::round_up(mi::split_bytes(batch, q_len, kv_len, inner));
+    return mi::block_scratch(batch, q_len, kv_len, inner, with_kv != 0, mi::sdpa_wide_head(inner) ? mi::split_bytes(batch, q_len, kv_len, 1, inner) : 0);
+}
+
+size_t mi_attn_block_scratch_bytes(const mi_attn_block_args* a) {
+    if (!a || a->struct_size != sizeof(mi_attn_block_args) || a->batch <= 0 || a->q_len < 0 || a->kv_len < 0 || a->inner <= 0) return 0;
+    const int kv_len = !a->ctx && !a->k ? a->q_len : a->kv_len;
+    const bool heads_ok = a->num_heads > 0 && a->inner % a->num_heads == 0;
+    return mi::block_scratch(a->batch, a->q_len, kv_len, a->inner, a->k == nullptr,
+                             heads_ok ? mi::split_bytes(a->batch, a->q_len, kv_len, a->num_heads, a->inner / a->num_heads, a->causal != 0, a->key_mask) : 0);
 }
 
 int mi_flash_attention_project_kv(const mi_attn_block_args* a) {

@@ -239,9 +239,9 @@ Tensor& thread_scratch() {
     struct BlockScratch;
     return per_stream<Tensor, BlockScratch>();
 }
-void lend_scratch(mi_attn_block_args& a, Tensor* scratch, bool with_kv) {
+void lend_scratch(mi_attn_block_args& a, Tensor* scratch) {
     Tensor& s = scratch ? *scratch : thread_scratch();
-    const std::size_t need = mi_flash_attention_scratch_bytes(a.batch, a.q_len, a.kv_len, a.inner, with_kv ? 1 : 0);
+    const std::size_t need = mi_attn_block_scratch_bytes(&a);
     if (s.data == nullptr || s.bytes() < need) s.resize(1, static_cast<int>((need + 3) / 4), Dtype::FP32, Device::GPU);
     a.scratch = s.data; a.scratch_bytes = s.bytes();
 }
@@ -302,7 +302,7 @@ void qkvo_impl(const char* op, const Tensor& X, const Tensor* Ctx, const Tensor&
     a.bk = bias_ptr(op, bk, "bk", X.dtype, Wq.rows);
     a.bv = bias_ptr(op, bv, "bv", X.dtype, Wq.rows);
     a.kv_len = S.rows; a.ctx_channels = S.cols;
-    lend_scratch(a, scratch, true);
+    lend_scratch(a, scratch);
     check(op, mi_flash_attention_qkvo_forward(&a));
 }
 void kv_cached_impl(const char* op, const Tensor& X, const Tensor& K, const Tensor& V, const Tensor& Wq, const Tensor* bq,
@@ -314,7 +314,7 @@ void kv_cached_impl(const char* op, const Tensor& X, const Tensor& K, const Tens
     if (K.dtype != X.dtype || V.dtype != X.dtype || K.cols != Wq.rows || V.cols != K.cols || V.rows != K.rows)
         fail(std::string(op) + ": K and V must be (Lk, " + std::to_string(Wq.rows) + ") of X's dtype");
     a.k = K.data; a.v = V.data; a.kv_len = K.rows;
-    lend_scratch(a, scratch, false);
+    lend_scratch(a, scratch);
     check(op, mi_flash_attention_q_with_kv_cached_forward(&a));
 }
 void project_kv_impl(const char* op, const Tensor& ctx, const Tensor& Wk, const Tensor* bk, const Tensor& Wv, const Tensor* bv,

@@ -40,7 +40,7 @@ struct Lib {
     decltype(&mi_add_inplace) add_inplace;
     decltype(&mi_rms_norm_forward) rms_norm;
     decltype(&mi_rms_norm_pair_forward) rms_norm_pair;
-    decltype(&mi_flash_attention_scratch_bytes) block_scratch_bytes;
+    decltype(&mi_attn_block_scratch_bytes) block_scratch_bytes;
     decltype(&mi_flash_attention_qkvo_forward) qkvo;
     decltype(&mi_flash_attention_q_with_kv_cached_forward) kv_cached;
     decltype(&mi_linear_attn_workspace_bytes) la_workspace_bytes;
@@ -492,9 +492,7 @@ NATIVE(attn_block, 22)
     }
     const Tensor out = output(a[15], x, c_out);
     p.out = out.data_ptr();
-    const Tensor scratch = none(a[16]) ? at::empty({static_cast<int64_t>(L.block_scratch_bytes(p.batch, p.q_len, p.kv_len, p.inner, !cached))},
-                                                   x.options().dtype(at::kByte))
-                                       : tensor(a[16]);
+    const Tensor scratch = none(a[16]) ? at::empty({static_cast<int64_t>(L.block_scratch_bytes(&p))}, x.options().dtype(at::kByte)) : tensor(a[16]);
     need(scratch.is_contiguous());
     p.scratch = scratch.data_ptr(); p.scratch_bytes = scratch.numel() * scratch.element_size();
     p.stream = current_stream();
@@ -632,7 +630,7 @@ PyObject* bind(PyObject*, PyObject* args) {
     get(L.last_error, "mi_last_error"); get(L.sdpa, "mi_sdpa_forward"); get(L.sdpa_split_bytes, "mi_sdpa_split_scratch_bytes");
     get(L.rope, "mi_rope_apply"); get(L.headnorm_rope, "mi_headnorm_rope"); get(L.linear, "mi_linear_forward"); get(L.linear_n, "mi_linear_forward_n");
     get(L.geglu, "mi_linear_geglu_forward"); get(L.add_inplace, "mi_add_inplace"); get(L.rms_norm, "mi_rms_norm_forward");
-    get(L.rms_norm_pair, "mi_rms_norm_pair_forward"); get(L.block_scratch_bytes, "mi_flash_attention_scratch_bytes");
+    get(L.rms_norm_pair, "mi_rms_norm_pair_forward"); get(L.block_scratch_bytes, "mi_attn_block_scratch_bytes");
     get(L.qkvo, "mi_flash_attention_qkvo_forward"); get(L.kv_cached, "mi_flash_attention_q_with_kv_cached_forward");
     get(L.la_workspace_bytes, "mi_linear_attn_workspace_bytes"); get(L.la_scratch_bytes, "mi_linear_attn_scratch_bytes");
     get(L.linear_attn, "mi_linear_attn_relu_forward");

@@ -533,6 +533,7 @@ def add_inplace_row_bias(Y, bias):
 
 
 def flash_attention_scratch_bytes(batch: int, q_len: int, kv_len: int, inner: int, with_kv: bool) -> int:
+    """Bytes of the `scratch` of the operators below (mi_flash_attention_scratch_bytes)."""
     return int(capi.lib().mi_flash_attention_scratch_bytes(batch, q_len, kv_len, inner, int(with_kv)))
 
 
@@ -591,9 +592,8 @@ def _attn_block(op: str, fn_name: str, X, Ctx, K, V, Wq, bq, Wk, bk, Wv, bv, Wo,
     if out.numel() != B * Lq * Cout:
         _fail(op, "out has the wrong number of rows")
     a.out = out.data_ptr()
-    need = flash_attention_scratch_bytes(B, Lq, Lk, inner, K is None)
     if scratch is None:
-        scratch = torch.empty(need, dtype=torch.uint8, device=X.device)
+        scratch = torch.empty(capi.lib().mi_attn_block_scratch_bytes(C.byref(a)), dtype=torch.uint8, device=X.device)
     if not scratch.is_contiguous():
         _fail(op, "scratch must be contiguous")
     a.scratch, a.scratch_bytes = scratch.data_ptr(), scratch.numel() * scratch.element_size()
@@ -605,7 +605,8 @@ def _attn_block(op: str, fn_name: str, X, Ctx, K, V, Wq, bq, Wk, bk, Wv, bv, Wo,
 def flash_attention_qkvo_forward(X, Ctx, Wq, bq, Wk, bk, Wv, bv, Wo, bo, d_mask, num_heads: int, causal: bool,
                                  out: Optional[torch.Tensor] = None, scratch: Optional[torch.Tensor] = None):
     """out = attention(X Wq^T + bq, S Wk^T + bk, S Wv^T + bv) Wo^T + bo with S = Ctx, or X when Ctx is None.
-    `scratch` (flash_attention_scratch_bytes(..., with_kv=True) bytes) holds the projections; None allocates it."""
+    `scratch` (flash_attention_scratch_bytes(..., with_kv=True) bytes) holds the projections; None allocates it, together with
+    what the attention launch can use to cut its key axis."""
     return _attn_block("flash_attention_qkvo_forward", "mi_flash_attention_qkvo_forward", X, Ctx, None, None,
                        Wq, bq, Wk, bk, Wv, bv, Wo, bo, d_mask, num_heads, causal, out, scratch)
 

@@ -449,8 +449,9 @@ MI_API int mi_rms_norm_pair_forward(const void* x0, const void* gain0, void* out
  *
  * Weights are (out_features, in_features) row-major, biases may be NULL. Q, K, V and the attention
  * output are rounded to `dtype` between the stages (they are tensors of that dtype in the reference too) and
- * live in `scratch`, which the caller lends: mi_flash_attention_scratch_bytes() bytes, 16-byte aligned (of
- * these only the projections are required; the rest, if lent, lets the attention launch cut its key axis into pieces).
+ * live in `scratch`, which the caller lends: mi_attn_block_scratch_bytes() or mi_flash_attention_scratch_bytes() bytes,
+ * 16-byte aligned (of these only the projections and the attention output are required; the rest, if lent, lets the attention
+ * launch cut its key axis into pieces).
  * The three projections of the qkvo form run as ONE launch, attention as one, the output projection as
  * one. Rows are batch-major: item b of x is rows [b*q_len, (b+1)*q_len); with ctx == NULL kv_len is
  * taken as q_len. head_dim = inner / num_heads must be one mi_sdpa_supported() accepts. */
@@ -484,7 +485,12 @@ typedef struct mi_attn_block_args {
     const float* wo_scales;
     void* stream;
 } mi_attn_block_args;
-/* Scratch bytes of the qkvo form (with_kv != 0) or the kv_cached form (with_kv == 0); project_kv needs none. */
+/* Scratch bytes of this call (qkvo form if k is NULL, else the kv_cached form; the scratch fields are ignored), with all that its
+ * attention launch can use. project_kv needs none. */
+MI_API size_t mi_attn_block_scratch_bytes(const mi_attn_block_args* args);
+/* The same for callers that size the scratch before they know the call: the required bytes of the qkvo form (with_kv != 0) or the
+ * kv_cached form (with_kv == 0), and what cutting the key axis takes where `inner` is the head dimension of one wide head
+ * (256, 384, 512: the VAE's mid-block). */
 MI_API size_t mi_flash_attention_scratch_bytes(int32_t batch, int32_t q_len, int32_t kv_len, int32_t inner, int32_t with_kv);
 MI_API int mi_flash_attention_qkvo_forward(const mi_attn_block_args* args);
 MI_API int mi_flash_attention_q_with_kv_cached_forward(const mi_attn_block_args* args);

@@ -15,7 +15,7 @@ API int mi_add_inplace() {
 }
 API const char* mi_last_error() { return "the gate stayed closed"; }
 API unsigned long mi_sdpa_split_scratch_bytes() { return 0; }
-API unsigned long mi_flash_attention_scratch_bytes() { return 0; }
+API unsigned long mi_attn_block_scratch_bytes() { return 0; }
 API unsigned long mi_linear_attn_workspace_bytes() { return 0; }
 API unsigned long mi_linear_attn_scratch_bytes() { return 0; }
 REFUSES(mi_sdpa_forward)

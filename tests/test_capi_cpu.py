@@ -119,6 +119,41 @@ def test_split_scratch_is_not_offered_to_calls_the_split_kernel_cannot_serve(cap
     assert lib.mi_sdpa_split_scratch_bytes(C.byref(a)) == plain
 
 
+def test_block_scratch_is_what_the_call_can_use(capi):
+    """Beyond the projections and the attention output, the scratch of a block operator is what its own attention launch cuts the
+    key axis with; without a head count only one wide head is counted. (No GPU: the planner assumes 256 compute units.)"""
+    lib = capi.lib()
+
+    def block(batch, tokens, inner, heads, **kw):
+        a = capi.MiAttnBlockArgs()
+        a.struct_size = C.sizeof(a)
+        a.dtype, a.batch, a.q_len, a.inner, a.num_heads = capi.MI_DTYPE_F16, batch, tokens, inner, heads
+        for k, v in kw.items():
+            setattr(a, k, v)
+        return lib.mi_attn_block_scratch_bytes(C.byref(a)), 4 * batch * tokens * inner * 2, lib.mi_flash_attention_scratch_bytes(batch, tokens, tokens, inner, 1)
+
+    def cut(batch, tokens, heads, head_dim):
+        a = capi.MiSdpaArgs()
+        a.struct_size = C.sizeof(a)
+        a.dtype, a.batch, a.num_heads, a.head_dim, a.q_len, a.kv_len = capi.MI_DTYPE_F16, batch, heads, head_dim, tokens, tokens
+        a.q = a.k = a.v = a.o = 0x1000              # never dereferenced
+        return (lib.mi_sdpa_split_scratch_bytes(C.byref(a)) + 255) // 256 * 256
+    # 8 heads of 160 never split; as 5 heads of 256 the same channels would
+    mine, buffers, any_heads = block(1, 1024, 1280, 8)
+    assert cut(1, 1024, 5, 256) > 0 and mine == any_heads == buffers
+    assert block(1, 1024, 1280, 5)[0] == buffers + cut(1, 1024, 5, 256)
+    # one wide head
+    mine, buffers, any_heads = block(1, 4096, 512, 1)
+    assert mine == any_heads == buffers + cut(1, 4096, 1, 512) > buffers
+    # heads of 128 whose last round is cut, and not when a mask makes the tiles unequal
+    mine, buffers, any_heads = block(1, 3328, 3072, 24)
+    assert mine == buffers + cut(1, 3328, 24, 128) > any_heads == buffers
+    assert block(1, 3328, 3072, 24, causal=1)[0] == block(1, 3328, 3072, 24, key_mask=0x1000)[0] == buffers
+    # head counts that no kernel takes
+    assert block(1, 64, 512, 3)[0] == block(1, 64, 512, 0)[0] == 4 * 64 * 512 * 2
+    assert lib.mi_attn_block_scratch_bytes(None) == 0
+
+
 def test_python_mirror_refuses_cpu_tensors():
     import torch
     import brodiffusion_amd as bd
