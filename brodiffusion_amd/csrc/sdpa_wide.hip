@@ -440,24 +440,29 @@ __global__ void __launch_bounds__(256) wide_combine_kernel(const SdpaDev p, int 
 
 // Pieces of the key axis: as many as minimise the launch, counted in steps: rounds x (steps of a piece + kOverhead: Q staging,
 // first tiles, write-out), and for the merge kMerge plus kParts per part on every compute unit (128 x D FP32 values written and
-// read again). Fitted on MI355X to 1 .. 16 pieces of 13 lengths from 384 to 16384 tokens at each head dimension: the number
-// taken is 0.9 % slower than the best one on average, 4.3 % at worst (without kParts 3.5 and 15 %). At 512, one head, in us:
-//   1024 tokens (8 tiles)   1 piece 54.6   3 34.5   5 32.1 (taken)   8 35.4
-//   4096 (32)               1 168          4 67.2   6 63.4 (taken)   8 66.6   9 (a second round) 91.4
-//   9216 (72)               1 358          2 208    3 182 (taken)    7 210
-//   16384 (128)             1 634          2 483 (taken)             4 508
+// read again), the same once more for what the parts of the launch exceed kNear by (the L2s no longer hold them). Fitted on
+// MI355X to up to 16 pieces of 45 problems (1 to 24 batch items, 300 to 16384 rows, 320 to 16384 keys) at each head dimension:
+// the number taken is 1.2 % slower than the best one on average, 10 % at worst (counting no parts: 3.1 and 21 %). At 512, us:
+//   1024 tokens (8 tiles)      1 piece 54.6   3 34.6   5 32.4           6 33.2 (taken)   8 35.4
+//   4096 (32)                  1 168          4 67.0   6 63.6 (taken)   8 67.1   9 (a second round) 91.8
+//   9216 (72)                  1 358          2 208    3 185 (taken)    7 210
+//   16384 (128)                1 638          2 493 (taken)             4 515
+//   8 x 600 (40)               1 45.7         3 38.0   4 37.2           5 40.1       3 taken
 // Only unmasked calls (a valid length or key mask may be on): with causal masks the tiles are unequal and fill the GPU in their
 // own way.
-int wide_split(const SdpaDev& p, int n_cu) {
+int wide_split(const SdpaDev& p, int head_dim, int n_cu) {
     if (p.mask_mode != MI_MASK_NONE) return 1;
     const long tiles = static_cast<long>(p.B) * p.H * ((p.Lq + kWideRows - 1) / kWideRows);
     const int steps = (p.Lk + kWideKeys - 1) / kWideKeys;
-    constexpr int kOverhead = 6, kMerge = 4, kParts = 24, kMaxSplit = 16, kMinSteps = 6;
+    constexpr int kMaxSplit = 16, kMinSteps = 5;
+    constexpr double kOverhead = 6, kMerge = 1, kParts = 16, kNear = 47e6;
     int best = 1;
-    long best_cost = 0;
+    double best_cost = 0;
     for (int s = 1; s <= kMaxSplit && (s == 1 || steps / s >= kMinSteps); ++s) {
-        const long rounds = (tiles * s + n_cu - 1) / n_cu;
-        const long cost = rounds * ((steps + s - 1) / s + kOverhead) + (s > 1 ? kMerge + kParts * tiles * s / n_cu : 0);
+        const double parts = static_cast<double>(tiles) * s, far = parts * kWideRows * head_dim * 4 - kNear;
+        const double rounds = static_cast<double>((tiles * s + n_cu - 1) / n_cu);
+        double cost = rounds * ((steps + s - 1) / s + kOverhead);
+        if (s > 1) cost += kMerge + kParts * (parts / n_cu + (far > 0 ? far / (n_cu * kWideRows * 512.0 * 4) : 0));
         if (s == 1 || cost < best_cost) { best = s; best_cost = cost; }
     }
     return best;
@@ -468,7 +473,7 @@ int launch_wide_d(const SdpaDev& p, hipStream_t stream) {
     using W = WideGeo<D>;
     const int n_q_tiles = (p.Lq + kWideRows - 1) / kWideRows;
     const long tiles = static_cast<long>(p.B) * p.H * n_q_tiles;
-    int n_split = wide_split(p, device_cu_count());
+    int n_split = wide_split(p, D, device_cu_count());
     if (p.split_scratch == nullptr || p.split_scratch_bytes < static_cast<size_t>(tiles) * n_split * W::SLOT) n_split = 1;
     const long blocks = tiles * n_split;
     if (blocks > 0x7fffff00L) return fail("mi_sdpa_forward: problem too large for one launch");
@@ -493,7 +498,7 @@ int launch_wide_d(const SdpaDev& p, hipStream_t stream) {
 bool sdpa_wide_head(int head_dim) { return head_dim == 256 || head_dim == 384 || head_dim == 512; }
 
 size_t sdpa_wide_split_scratch_bytes(const SdpaDev& p, int head_dim) {
-    const int n_split = wide_split(p, device_cu_count());
+    const int n_split = wide_split(p, head_dim, device_cu_count());
     if (n_split == 1) return 0;
     const size_t slot = static_cast<size_t>(kWideRows) * (static_cast<size_t>(head_dim) * 4 + 8);
     return static_cast<size_t>(p.B) * p.H * ((p.Lq + kWideRows - 1) / kWideRows) * n_split * slot;
