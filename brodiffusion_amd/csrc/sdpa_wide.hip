@@ -4,7 +4,8 @@
 //
 // Bound: MFMA (4 L^2 d FLOPs against 8 L d bytes). A work group is 4 wavefronts, one per SIMD, each with 32 query rows of its
 // own and all of the head dimension: at 512 the output accumulator of 32 rows is 256 registers per lane, the Q fragments
-// are 128, and one wavefront per SIMD may use 512. So no partial score ever leaves a wavefront (the earlier form dealt the
+// are 128, and one wavefront per SIMD may use 512 (that instance is still nine registers short: 40 bytes per lane of scratch, of
+// which a step reloads 4). So no partial score ever leaves a wavefront (the earlier form dealt the
 // head dimension out to the wavefronts and summed four FP32 score tiles through LDS at every step: 240 TFLOP/s at 16384
 // tokens, 2.37 ms). The key axis goes in steps of 32: with rows of up to 1 KB two stages of K and two of V are 128 KB of LDS.
 //
@@ -136,13 +137,14 @@ __global__ void __launch_bounds__(kWideThreads, 1) sdpa_wide_kernel(const SdpaDe
     const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
     const int q0 = qt * kWideRows;
     const int qrow = q0 + wave * 32 + lq;
-    const bool qvalid = qrow < p.Lq;
     const T* const q_base = static_cast<const T*>(p.q) + b * p.q_bs + h * D;
     T* const o_base = static_cast<T*>(p.o) + b * p.o_bs + h * D;
     const float* const key_mask = p.key_mask ? p.key_mask + b * p.key_mask_bs : nullptr;
 
     int lo, hi;
-    row_interval(p, b, qrow, qvalid, lo, hi);
+    // (rows past the end count as the last row where they share a wavefront with it: as rows without keys they would put every
+    //  step of that wavefront on the masked path)
+    row_interval(p, b, min(qrow, p.Lq - 1), q0 + wave * 32 < p.Lq, lo, hi);
     if (n_split > 1) {   // this work group's piece of the key axis, in whole steps
         const int steps = (p.Lk + kWideKeys - 1) / kWideKeys;
         lo = max(lo, static_cast<int>(static_cast<long>(piece) * steps / n_split) * kWideKeys);
