@@ -9,7 +9,7 @@
 // launch_linear validates a launch and hands it to the LDS-DMA kernels of linear_pipe.hip. What those do not take (contractions
 // that are no multiple of 64, operands beyond 32-bit tile offsets) runs here:
 //
-// linear_kernel: 256 threads = 4 wavefronts in a 2 x 2 arrangement over a BM x BN output tile,
+// linear_kernel: 256 threads = 4 wavefronts in a 2 x 2 arrangement over a BM x BN output tile (launch_t picks between two),
 // contraction step 64. Operand tiles go global -> registers -> LDS with 16-byte accesses, double buffered so that the
 // loads of step t+1 are in flight while step t multiplies; one barrier per step. LDS rows are 144 bytes (128 + 16): 16
 // consecutive rows start on distinct 16-byte bank groups, so the ds_read_b128 fragment reads are conflict free.
@@ -320,6 +320,19 @@ int launch_tiles(const LinearBatch& batch, int n_problems, hipStream_t st) {
 template <typename T>
 int launch_t(const LinearBatch& batch, int n_problems, hipStream_t st, bool geglu) {
     const bool w8 = batch.p[0].w_scale != nullptr;
+    // 128 tokens x 128 rows of W per tile where such tiles give every compute unit two: they read half as much per FLOP, and below
+    // that the 64-token tiles fill the GPU better. The lines are the same for 16-bit and INT8 weights, plain and GEGLU, and any
+    // contraction (us, 64-token / 128-token tiles, plain fp16):
+    //   256 tiles: 2048 x 2048 x 328 10.1 / 10.1, x 1096 24.5 / 22.5 (INT8 24.0 / 31.1)
+    //   512:       4096 x 2048 x 136 10.5 / 10.2, x 328 17.0 / 13.8, x 1096 44.7 / 29.9 (INT8 44.0 / 34.3; GEGLU 39.6 / 30.9)
+    //   2048:      8192 x 4096 x 136 32.6 / 29.5, x 1096 164 / 108, x 2056 302 / 189
+    long big = 0;
+    for (int i = 0; i < n_problems; ++i)
+        big += static_cast<long>((batch.p[i].M + 127) / 128) * ((batch.p[i].N + (geglu ? 63 : 127)) / (geglu ? 64 : 128));
+    if (big >= 2L * device_cu_count()) {
+        if (geglu) return w8 ? launch_tiles<T, 128, 128, true, true>(batch, 1, st) : launch_tiles<T, 128, 128, true>(batch, 1, st);
+        return w8 ? launch_tiles<T, 128, 128, false, true>(batch, n_problems, st) : launch_tiles<T, 128, 128>(batch, n_problems, st);
+    }
     if (geglu) return w8 ? launch_tiles<T, 64, 128, true, true>(batch, 1, st) : launch_tiles<T, 64, 128, true>(batch, 1, st);
     return w8 ? launch_tiles<T, 64, 64, false, true>(batch, n_problems, st) : launch_tiles<T, 64, 64>(batch, n_problems, st);
 }

@@ -127,3 +127,35 @@ def test_unequal_problems_in_one_launch(oracle):
     _one_ulp(oracle.linear(ctx, wv, bv), to_np(v), dtype, "V projection")
     ref = oracle.attention_qkvo(x[rows], ctx, wq, bq, wk, bk, wv, bv, wo, bo, H, dtype)
     assert_close(ref, to_np(out)[rows], dtype, "cross-attention block with unequal projections")
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("int8", [False, True], ids=["w16", "w8"])
+@pytest.mark.parametrize("geglu", [False, True], ids=["plain", "geglu"])
+@pytest.mark.parametrize("K", [72, 1096])
+def test_large_ragged_contraction(oracle, K, geglu, int8, dtype):
+    """Contractions that are no multiple of 64, with two 128 x 128 tiles per compute unit and more (33 x 17 tiles, GEGLU 33 x 33;
+    one row and one 8-feature piece in the last ones): the same bits as on the 64-row tiles that a slice of the rows takes (every
+    form accumulates in the same order), and the plain layer as the checker."""
+    M, N = 4097, 2056
+    rows = 2 * N if geglu else N
+    x, b = randn(121 + K, (M, K), dtype), randn(122, (rows,), dtype)
+    dx, db = to_dev(x, dtype), to_dev(b, dtype)
+    if int8:
+        rng = np.random.default_rng(K)
+        w = rng.integers(-128, 128, (rows, K)).astype(np.int8)
+        s = (rng.uniform(0.5, 1.5, (rows, 1)) / (74.0 * np.sqrt(K))).astype(np.float32)
+        dw, ds = torch.from_numpy(w).cuda(), torch.from_numpy(s).cuda()
+    else:
+        w, ds = _weight(oracle, 123, rows, K, dtype), None
+        dw = to_dev(w, dtype)
+
+    def run(t):
+        return bd.fused_linear_geglu(t, dw, db, W_scales=ds) if geglu else bd.linear_batched(dw, db, t, W_scales=ds)
+    y = run(dx)
+    for r0 in (0, 1000, M - 601):
+        assert torch.equal(y[r0:r0 + 601], run(dx[r0:r0 + 601].contiguous()))
+    if not geglu:
+        r = _rows(M)
+        ref = oracle.linear(x[r], w.astype(np.float32)) * s.reshape(1, -1) + b if int8 else oracle.linear(x[r], w, b)
+        _one_ulp(ref, to_np(y)[r], dtype, f"linear {M}x{N}x{K}")
