@@ -386,8 +386,10 @@ int launch_pipe(const LinearBatch& batch, int n_problems, hipStream_t st) {
 //     phi + steps lam + (m - 1) (steps tau + eps),   m = ceil(n / C) tiles on the busiest compute unit,
 // with steps = K / 64: phi what a launch of one tile per compute unit costs beyond its steps (start, first loads, write-out), lam
 // a step when the compute unit has one tile, tau and eps a step and the rest of every further tile. The constants (us) are fitted
-// to 90 problems between 32 x 1280 x 1280 and 4096 x 6720 x 2240 on MI355X, rms error 6 to 13 %; the form with the
-// smallest estimate is within 1 % of the fastest one on average, 14 % at worst. Large tiles need fewer bytes per FLOP
+// to problems between 32 x 1280 x 1280 and 4096 x 6720 x 2240 on MI355X. Every form timed again on 232 problems (32 to 8192 rows, nine
+// layers of the supported models): rms error 6 to 17 % by form, 23 % for the 128 x 128 tiles of two stages and the GEGLU ones of
+// 128 tokens, whose few-tile launches are overestimated; the form taken is 0.1 (INT8 0.9, GEGLU 0.7) % slower than the fastest
+// one on average, 11 % at worst. Large tiles need fewer bytes per FLOP
 // (a step of 128 x 128 moves 32 KB for 0.5 us of a saturated compute unit), small ones fill the GPU: 128 x 1280 x 1280
 // takes 6 us with 80 tiles of 64 x 32, 8 with 20 of 128 x 64, 16 with 10 of 256 x 128; 1024 x 2240 x 2240 takes 18 us
 // with 144 tiles of 128 x 128, 24 with 288 of 128 x 64, 50 with 36 of 256 x 256.

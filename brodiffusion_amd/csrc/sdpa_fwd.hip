@@ -539,8 +539,7 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_kernel(const SdpaDev
 
     const int n_keys = RAGGED ? visible_keys(p, b) : p.Lk;
     int lo = 0, hi = n_keys;   // DENSE: rows past the end of Q repeat its last row and are never stored
-    // (rows past the end count as the last row where they share a wavefront with it: as rows without keys they put every tile
-    //  of that wavefront on the masked path; 24 heads of 128, 2500 tokens, block-causal: 83.8 -> 74.5 us)
+    // (rows past the end: as in sdpa_fwd_pp_dma_kernel)
     if constexpr (!DENSE) row_interval(p, b, min(qrow, p.Lq - 1), q0 + wave * 32 < p.Lq, lo, hi);
     WaveExtent we{0, 0, n_keys, n_keys};
     if constexpr (!DENSE) {
@@ -1358,7 +1357,7 @@ bool plan_split(SdpaDev& p, int n_cu) {
     p.split = SplitGeo{};
     if constexpr (!dma_kernel_available<D>()) return false;
     if (p.mask_mode != MI_MASK_NONE || p.kv_valid_len || p.key_mask || p.Lp > 0 || p.cos_k || p.cu_q) return false;
-    // the logit bias and the softmax denominators exist in the 128-row kernel only
+    // (the split form neither adds a logit bias nor writes the softmax denominators)
     if (p.bias != nullptr || p.lse != nullptr) return false;
     if (n_cu < 8 || n_cu % 8 != 0 || sdpa_kernel_choice() == 1 || sdpa_kernel_choice() == 3) return false;
     const long tiles = static_cast<long>(p.B) * p.H * ((p.Lq + 255) / 256);
@@ -1396,14 +1395,17 @@ bool same_keys_for_all_rows(const SdpaDev& p) {
 // 128-row tiles. With a 256-row tile or more per CU the former always. Below that the 128-row kernel keeps more CUs busy, but
 // each of them runs one wavefront per SIMD whose softmax nothing hides, and from the 257th work group on two share a CU
 // anyway ("crowded"); a CU with eight wavefronts needs 2/3 of the time per row and key, and costs about 1.5 us more to start
-// (rings, two-part Q staging). The lines are where the two sides met (us, 128-row / 256-row, one head count each):
-//   128, no mask:      T = 4 11.7 / 12.5, 6 14.9 / 15.0, 8 18.5 / 17.6, 16 31.3 / 27.2, 32 (192 tiles) 74 / 52; cross, 3 key
-//                      tiles, 216 query tiles 15.2 / 14.5, 96 query tiles 11.2 / 12.6
-//   72, no mask:       T = 4 11.5 / 11.3, cross with 4: 12.2 / 12.5, 9 19.5 / 17.7, 36 (144 tiles) 72 / 50
-//   40 and 64:         faster from one key tile on (6.1 / 5.7; 1024 tokens 24.4 / 18.1)
-//   128, 72 masked:    T = 8 18.8 / 19.6 and 18.0 / 17.7, 16 31.4 / 29.8 and 30.3 / 27.3, 32 (192 tiles, block-causal) 79 / 54
-//   80, 96, 112:       crowded only: 144 tiles of 80 72 / 64, 192 of 96 98 / 92, 128 of 80 102 / 114; masked never (96: 70 / 79)
-//   K rotated by tile: crowded only: 144 tiles 72 / 57, 120 tiles 40 / 41
+// (rings, two-part Q staging). The lines are where the two sides meet (us, 128-row / 256-row, 8 heads of 40 and 80, 16 of 64, 72
+// and 96, 24 of 128; over a sweep of 156 such calls the side taken is at most 7 % slower than the other, 0.6 % on average):
+//   128, no mask:      T = 4 11.5 / 12.5, 5 13.3 / 13.9, 8 18.0 / 17.3, 16 30.8 / 26.9, 32 (192 tiles) 74.7 / 52.7; cross, 3 key
+//                      tiles, 216 query tiles 15.0 / 14.6, 96 query tiles 11.1 / 12.7
+//   72, no mask:       T = 4 11.4 / 10.8, 5 12.9 / 12.0, cross with 2 9.2 / 10.1, with 5 13.4 / 13.5, 16 29.3 / 23.6, 36 (144
+//                      tiles) 70.4 / 45.7
+//   40 and 64:         equal or faster from one key tile on (6.4 / 5.7 and 5.7 / 5.7; 1024 tokens 24.3 / 18.5 and 24.1 / 19.2)
+//   128, 72 masked:    T = 8 18.2 / 19.4 and 17.7 / 17.8, 16 31.0 / 29.7 and 29.6 / 27.1, 32 (192 tiles, block-causal) 79.1 / 54.8
+//   80, 96, 112:       crowded only: 144 tiles of 96 69.1 / 56.2, 192 tiles 92.2 / 74.1, 128 of 80 100 / 111; masked never (96,
+//                      160 tiles: 58.7 / 60.7)
+//   K rotated by tile: crowded only: 128, 144 tiles 70.9 / 55.9, 96 tiles 40.7 / 39.0; 40, 40 tiles 35.3 / 36.9
 template <int D>
 bool rows256_pay(const SdpaDev& p, int n_cu, bool xtra) {
     const long heads = static_cast<long>(p.B) * p.H;

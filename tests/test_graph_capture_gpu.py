@@ -42,7 +42,7 @@ def test_graph_replays_equal_eager():
     # a linear layer large enough for the 256 x 256-tile kernel
     xl, wl, bl = rnd(4608, 1024), rnd(3072, 1024) / 32, rnd(3072)
     o_big = torch.empty(4608, 3072, dtype=torch.bfloat16, device=dev)
-    # the tile-walking GEMM forms: FF1 + GEGLU with 128-token tiles (at least two per compute unit) and a long contraction
+    # FF1 + GEGLU with at least two tiles per compute unit, and a long contraction
     # over few tiles (FF2)
     xr = rnd(4096, C, dt=torch.float16)
     wr, br = rnd(2 * 1280, C, dt=torch.float16) / C ** 0.5, rnd(2 * 1280, dt=torch.float16)

@@ -98,7 +98,7 @@ def test_large_linear_agrees_with_small_tile_kernel():
     w = (torch.randn(3072, 1024, generator=g) / 32).to(dt).cuda()
     b = torch.randn(3072, generator=g).to(dt).cuda()
     big = bd.linear_batched(w, b, x)                 # 18 x 12 tiles of 256 x 256: the large kernel
-    small = bd.linear_batched(w, b, x[:2048])        # 8 x 12 tiles: the 128 x 128 kernel
+    small = bd.linear_batched(w, b, x[:2048])        # 8 x 12 of them: smaller tiles
     assert torch.equal(big[:2048], small)
 
 

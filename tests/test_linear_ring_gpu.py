@@ -1,6 +1,5 @@
-"""The projection GEMM in its tile-walking form (in_features a multiple of 320 and at least 640, problems too small for the
-128 x 128 and 256 x 256 tile kernels: the FF2 and attention projections of the U-Net's deeper levels), against the CPU
-checker on the same seeded inputs: the real shapes, ragged token and feature counts, no bias, operands that are slices of
+"""The projection GEMM on the FF2 and attention projections of the U-Net's deeper levels (long contractions over few tiles: the
+forms with LDS-DMA rings of 64 x 32 to 128 x 128 tiles), against the CPU checker on the same seeded inputs: the real shapes, ragged token and feature counts, no bias, operands that are slices of
 wider buffers, three problems of different sizes in one launch. Bound: FP32 accumulation and one rounding (one unit in the
 last place of the result's magnitude, as in tests/test_attn_block_gpu.py); the checker follows y = x w^T + b of
 bt::linear_batched (src/unet_blocks.cpp:238-240)."""
@@ -33,7 +32,7 @@ def _one_ulp(ref, got, dtype, what):
     (8192, 320, 1280, True),      # FF2 of the 64 x 64 level
     (512, 1280, 1280, True),      # an attention projection of the 16 x 16 level
     (77, 1280, 640, False),       # fewer tokens than one tile, no bias
-    (1000, 328, 960, True),       # 40 of 64 tokens and 8 of 64 features in the last tiles; three groups of five steps
+    (1000, 328, 960, True),       # 40 of 64 tokens and 8 of 64 features in the last tiles; fifteen stages
     (3, 8, 640, False)])          # a corner of one tile
 def test_ring_linear_matches_checker(oracle, dtype, M, N, K, bias):
     x = randn(51 + M, (M, K), dtype)
@@ -66,8 +65,8 @@ def test_ring_linear_with_strides(oracle):
 
 
 def test_three_projections_in_one_launch(oracle):
-    """The Q, K and V projections of a self-attention block at C = 640 share a launch (three problems, one grid row
-    each): flash_attention_qkvo_forward against the checker's block (src/unet_blocks.cpp:255-273)."""
+    """The Q, K and V projections of a self-attention block at C = 640 share a launch (three problems, their tiles
+    in one row): flash_attention_qkvo_forward against the checker's block (src/unet_blocks.cpp:255-273)."""
     dtype, B, N, Cc, H = "fp16", 2, 300, 640, 8
     x = randn(71, (B, N, Cc), dtype)
     ws = [_weight(oracle, 72 + i, Cc, Cc, dtype) for i in range(4)]

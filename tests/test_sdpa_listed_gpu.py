@@ -1,5 +1,6 @@
-"""Key masks and block-causal calls on the 256-row kernel: tiles without a visible key are taken out of the walk, and query tiles
-that lie in one segment run the form without masks. Masks that hide whole tiles in any place, all keys, or single keys."""
+"""Key masks and block-causal calls on the 256-row kernel. Key masks: tiles without a visible key are taken out of the walk; masks
+that hide whole tiles in any place, all keys, or single keys. Block-causal: query tiles of 256 rows inside a segment, across the
+border of two, and behind a causal one, all on the general form."""
 import numpy as np
 import pytest
 import torch
@@ -55,7 +56,6 @@ def test_every_key_hidden_and_a_hidden_nan(oracle, rows256):
     assert_close(oracle.sdpa(q, k, v, H, key_mask=m[1]), to_np(out[1]), dtype)
 
 
-# query tiles of 256 rows that lie inside a segment, across the border of two, and behind a causal one
 @pytest.mark.parametrize("d", [72, 128])
 @pytest.mark.parametrize("prefix", [0, 100])
 @pytest.mark.parametrize("ends,causal", [([256, 700, 1300], [1, 0, 0]), ([93, 300, 1300], [1, 0, 0]), ([257, 512, 1300], [0, 1, 0]), ([100, 1300], [0, 0]), ([40, 1300], [0, 1])])
