@@ -324,18 +324,22 @@ class _ScratchOfThread(threading.local):
 
 
 _split_scratch_cache = _ScratchOfThread()
+_captured_scratch = {}      # by address: what captured graphs use; they may be replayed at any time
 
 
 def _own_split_scratch(device, nbytes: int) -> torch.Tensor:
     """The scratch this layer lends when the caller brings none: one per thread, device and current stream, grown on demand.
     The calls of one thread on one stream run in order and may share it. Calls on different streams may overlap on the GPU; those
-    of two threads on one stream may put their launches (pieces, then merge) between each other's."""
+    of two threads on one stream may put their launches (pieces, then merge) between each other's. One that a graph was captured
+    with is kept when the thread ends or its next call needs a larger one."""
     key = (device, _stream())
     cache = _split_scratch_cache.tensors
     t = cache.get(key)
     if t is None or t.numel() < nbytes:
         t = torch.empty(nbytes, dtype=torch.uint8, device=device)
         cache[key] = t
+    if torch.cuda.is_current_stream_capturing():
+        _captured_scratch[t.data_ptr()] = t
     return t
 
 

@@ -70,6 +70,35 @@ def test_threads_on_one_stream_have_scratch_of_their_own():
         assert len(got) == 6 and all(torch.equal(g, ref) for g in got)
 
 
+def test_scratch_of_a_captured_call_outlives_its_thread():
+    """A split launch captured in a thread that then ends: its replay must not write into memory that somebody else has got since."""
+    H, L = 24, 3328
+    q, k, v = (rand(L, H * 128) for _ in range(3))
+    expected, out = bd.sdpa_forward(q, k, v, H), torch.empty_like(q)
+    stream, graph, size = torch.cuda.Stream(), torch.cuda.CUDAGraph(), []
+
+    def work():
+        with torch.cuda.stream(stream):
+            for _ in range(2):
+                bd.sdpa_forward(q, k, v, H, out=out)
+            stream.synchronize()
+            with torch.cuda.graph(graph, stream=stream):
+                bd.sdpa_forward(q, k, v, H, out=out)
+            size.append(max(ops._split_scratch_cache[key].numel() for key in ops._split_scratch_cache))
+    t = threading.Thread(target=work)
+    t.start()
+    t.join()
+    with torch.cuda.stream(stream):
+        others = [torch.full((size[0],), 0x5A, dtype=torch.uint8, device="cuda") for _ in range(3)]
+    torch.cuda.synchronize()
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, expected)
+        assert all((x == 0x5A).all() for x in others)
+
+
 def test_a_declined_call_has_launched_nothing():
     """Arguments that only the last steps of a call use are read before the first: nothing reaches a library that refuses every
     launch (tests/cpp/waiting_library.cpp)."""
