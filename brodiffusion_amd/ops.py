@@ -536,8 +536,17 @@ def add_inplace_row_bias(Y, bias):
     return Y
 
 
-def flash_attention_scratch_bytes(batch: int, q_len: int, kv_len: int, inner: int, with_kv: bool) -> int:
-    """Bytes of the `scratch` of the operators below (mi_flash_attention_scratch_bytes)."""
+def flash_attention_scratch_bytes(batch: int, q_len: int, kv_len: int, inner: int, with_kv: bool, num_heads: int = 0) -> int:
+    """Bytes of the `scratch` of the operators below (mi_flash_attention_scratch_bytes); with num_heads also what an unmasked call
+    with that many heads can use to cut its key axis (mi_attn_block_scratch_bytes)."""
+    if num_heads > 0:
+        a = capi.MiAttnBlockArgs()
+        a.struct_size = C.sizeof(a)
+        a.dtype = capi.MI_DTYPE_BF16
+        a.batch, a.q_len, a.kv_len, a.inner, a.num_heads = batch, q_len, kv_len, inner, num_heads
+        a.ctx = 1                                  # (only whether there are separate keys is read)
+        a.k = None if with_kv else 1
+        return int(capi.lib().mi_attn_block_scratch_bytes(C.byref(a)))
     return int(capi.lib().mi_flash_attention_scratch_bytes(batch, q_len, kv_len, inner, int(with_kv)))
 
 

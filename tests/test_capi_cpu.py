@@ -152,6 +152,12 @@ def test_block_scratch_is_what_the_call_can_use(capi):
     # head counts that no kernel takes
     assert block(1, 64, 512, 3)[0] == block(1, 64, 512, 0)[0] == 4 * 64 * 512 * 2
     assert lib.mi_attn_block_scratch_bytes(None) == 0
+    # the Python function: without a head count and with one
+    import brodiffusion_amd as bd
+    assert bd.flash_attention_scratch_bytes(1, 3328, 3328, 3072, True) == 4 * 3328 * 3072 * 2
+    assert bd.flash_attention_scratch_bytes(1, 3328, 3328, 3072, True, 24) == 4 * 3328 * 3072 * 2 + cut(1, 3328, 24, 128)
+    assert bd.flash_attention_scratch_bytes(1, 3328, 3328, 3072, False, num_heads=24) == 2 * 3328 * 3072 * 2 + cut(1, 3328, 24, 128)
+    assert bd.flash_attention_scratch_bytes(2, 64, 77, 1280, True, 8) == bd.flash_attention_scratch_bytes(2, 64, 77, 1280, True)
 
 
 def test_python_mirror_refuses_cpu_tensors():
