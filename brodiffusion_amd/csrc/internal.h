@@ -106,6 +106,10 @@ bool sdpa_wide_head(int head_dim);
 size_t sdpa_wide_split_scratch_bytes(const SdpaDev& p, int head_dim);
 int launch_sdpa_wide(const SdpaDev& p, int dtype, int head_dim, hipStream_t stream);
 
+// Calls with few query rows or few keys, and more (sdpa_small.hip): whether they take a call at kernel choice 0, and the launch.
+bool sdpa_small_takes(const SdpaDev& p, int head_dim);
+int launch_sdpa_small(const SdpaDev& p, int dtype, int head_dim, hipStream_t stream);
+
 // Device-side view of the head-averaged attention map launch (batch 1).
 struct MapDev {
     const void* q; const void* k;

@@ -1,9 +1,9 @@
-// Flash-style softmax attention forward for gfx950 (MI355X), hand-written. Five kernels share the building blocks of
-// sdpa_common.h; launch_d picks one per call:
+// Flash-style softmax attention forward for gfx950 (MI355X), hand-written. Four kernels share the building blocks of
+// sdpa_common.h; launch_d picks one per call that sdpa_small.hip does not take:
 //
 //   sdpa_fwd_kernel         4 wavefronts = 128 query rows per work group, K/V tiles through registers into padded LDS,
-//                           double buffered. Few keys or few work groups (rows256_pay), head_dim 160, packed
-//                           variable-length sequences, extras together with the prefix dial or tile-wise K rotation.
+//                           double buffered. Few keys or few work groups (rows256_pay) with extras or masks, packed
+//                           variable-length sequences, head_dim 160 with any of these, extras together with the prefix dial or tile-wise K rotation.
 //   sdpa_fwd_pp_kernel      8 wavefronts = 256 query rows, 2 wavefronts per SIMD, one work-group barrier per key tile:
 //                           between two barriers every wavefront runs the MFMA stream (O += V^T P of tile t, then
 //                           S = K Q^T of tile t+1) and one softmax, in opposite order in the two groups of four, so the
@@ -11,7 +11,6 @@
 //   sdpa_fwd_pp_dma_kernel  the same schedule with K/V tiles moved global -> LDS by DMA (head_dim 72 and 128), optionally
 //                           with the last, partly filled round of work groups cut along the key axis (SPLIT) and merged
 //                           by sdpa_combine_kernel.
-//   sdpa_fwd_pair_kernel    8 wavefronts for 128 query rows, two key tiles at a time: few query tiles (head_dim 80, 96, 112).
 //   sdpa_shortkv_kernel     short key sequences (cross attention): K and V of a head stay in LDS, a work group walks
 //                           several query tiles, no barrier in the key loop.
 //
@@ -176,133 +175,6 @@ __global__ void __launch_bounds__(kThreads4, (D > 128 ? 1 : 2)) sdpa_fwd_kernel(
     stage_output<T, D>(smem, wave * 32 + lq, lh, oacc, inv);
     __syncthreads();
     write_output<T, D, kThreads4>(smem, o_base, p.o_rs, q0, Lq, BM, tid);
-}
-
-// ───────────────────────── few query tiles: two key tiles at a time ─────────────────────────
-// The middle levels of a U-Net (32 x 32 tokens, 8 heads of 80) are 64 work groups of 128 rows for 256 CUs, each a serial walk
-// over its keys. Here a work group has 8 wavefronts for those rows: 0 to 3 take the even key tiles, 4 to 7 the odd ones, and the
-// two halves are merged through LDS in FP32. Half the steps, and two wavefronts per SIMD that cover each other's softmax.
-// Two pairs of tiles are 92 to 140 KB of LDS (head_dim 160 does not fit), so the form pays while no CU would get two groups.
-// 8 heads of 80: 1024 tokens 29.2 -> 23.1 us, 2048 tokens of batch 2 53.1 -> 41.3, 231 keys 11.9 -> 10.6; 16 heads of 112, 960
-// tokens 32.0 -> 25.2. (64-row groups of 4 wavefronts, twice as many: 24.1 and 52.9 us on the first two.)
-template <int D> constexpr int lds_bytes_pair() { return 4 * (HeadGeo<D>::K_BYTES + HeadGeo<D>::V_BYTES); }
-template <int D> constexpr bool pair_kernel_available() { return D == 80 || D == 96 || D == 112; }
-
-template <typename T, int D>
-__global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pair_kernel(const SdpaDev p) {
-    using G = HeadGeo<D>;
-    using V8 = typename Mma<T>::v8;
-    constexpr int BM = 128, TILE = G::K_BYTES + G::V_BYTES, STAGE = 2 * TILE;
-    constexpr int PART = (G::VB * 16 + 2) * 64 * 4;   // what a wavefront hands over: output, maximum and denominator of its lanes
-    constexpr int OUT = 4 * PART;
-    static_assert(OUT + BM * G::O_STRIDE <= lds_bytes_pair<D>() && lds_bytes_pair<D>() <= 160 * 1024 - 64, "LDS");
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    __shared__ int red[16];
-
-    int qt, bh;
-    if (!block_to_tile(p, qt, bh)) return;
-    const int h = bh % p.H, b = bh / p.H;
-    const int tid = threadIdx.x;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int half = wave >> 2, rows = 32 * (wave & 3);
-    const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
-    const int q0 = qt * BM;
-    const int qrow = q0 + rows + lq;
-    const int hk = h / p.kv_group;
-    const T* const q_base = static_cast<const T*>(p.q) + b * p.q_bs + h * D;
-    T* const o_base = static_cast<T*>(p.o) + b * p.o_bs + h * D;
-
-    int lo, hi;
-    row_interval(p, b, min(qrow, p.Lq - 1), q0 + rows < p.Lq, lo, hi);
-    const WaveExtent we = wave_extent(lo, hi);
-    if (lane == 0) { red[wave] = we.lo_min; red[8 + wave] = we.hi_max; }
-    V8 qf[G::KC];
-    stage_q_tile<T, D, kThreads8, BM>(smem, p, q_base, q0, tid);
-    __syncthreads();
-    read_q_frags<T, D>(qf, smem, rows + lq, lh);
-    __syncthreads();
-    zero_pads<D, kThreads8>(smem, smem + G::K_BYTES, TILE, TILE, 4, tid);
-    __syncthreads();
-    const int g_lo = __builtin_amdgcn_readfirstlane(min(min(red[0], red[1]), min(red[2], red[3])));
-    const int kv_stop = __builtin_amdgcn_readfirstlane(max(max(red[8], red[9]), max(red[10], red[11])));
-    const TilePlan plan(g_lo == 0x7fffffff ? 0 : g_lo, kv_stop, p.Lp);
-    const int n_tiles = plan.n_tiles;
-
-    f32x16 oacc[G::VB];
-#pragma unroll
-    for (int vb = 0; vb < G::VB; ++vb)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) oacc[vb][e] = 0.f;
-    SoftmaxState st;
-    const float cl2 = p.scale_log2;
-    const float lazy_raw = kLazyLog2 / cl2;
-
-    using Mover = TileMover<T, D, kThreads8, false>;
-    auto mover = [&]() {
-        return Mover{p, plan,
-                     reinterpret_cast<const unsigned char*>(static_cast<const T*>(p.k) + b * p.k_bs + hk * D),
-                     reinterpret_cast<const unsigned char*>(static_cast<const T*>(p.v) + b * p.v_bs + hk * D),
-                     reinterpret_cast<const unsigned char*>(static_cast<const T*>(p.kp) + b * p.kp_bs + hk * D),
-                     reinterpret_cast<const unsigned char*>(static_cast<const T*>(p.vp) + b * p.vp_bs + hk * D), tid, {}, {}, 1.f};
-    };
-    Mover even = mover(), odd = mover();
-    auto issue = [&](int t) {
-        if (t < n_tiles) { even.template issue<0>(t); even.template issue<1>(t); }
-        if (t + 1 < n_tiles) { odd.template issue<0>(t + 1); odd.template issue<1>(t + 1); }
-    };
-    auto store = [&](int t, unsigned char* to) {
-        if (t < n_tiles) { even.store_k(t, to); even.store_v(t, to + G::K_BYTES); }
-        if (t + 1 < n_tiles) { odd.store_k(t + 1, to + TILE); odd.store_v(t + 1, to + TILE + G::K_BYTES); }
-    };
-    issue(0);
-    store(0, smem);
-    issue(2);
-    __syncthreads();
-    for (int t0 = 0; t0 < n_tiles; t0 += 2) {
-        const unsigned char* Ks = smem + ((t0 >> 1) & 1) * STAGE + half * TILE;
-        const unsigned char* Vs = Ks + G::K_BYTES;
-        const int t = t0 + half;
-        if (t < n_tiles) {
-            const int j0 = plan.j0(t), lim = plan.limit(t);
-            if (j0 < we.hi_max && j0 + kBN > we.lo_min) {
-                f32x16 sacc[2];
-                V8 pf[4];
-                mfma_stream<T, D, false, true>(Vs, Ks, pf, qf, oacc, sacc, lane);
-                const bool interior = (j0 >= we.lo_max) && (j0 + kBN <= min(we.hi_min, lim));
-                softmax_tile<T, D>(sacc, pf, oacc, st, cl2, lazy_raw, !interior, j0, lo, min(hi, lim), lh, nullptr);
-                mfma_stream<T, D, true, false>(Vs, Ks, pf, qf, oacc, sacc, lane);
-            }
-        }
-        store(t0 + 2, smem + (((t0 >> 1) + 1) & 1) * STAGE);
-        issue(t0 + 4);
-        __syncthreads();
-    }
-
-    // merge: the odd half hands its FP32 state over, weights 2^(maximum - larger maximum) as in the online softmax
-    float* const part = reinterpret_cast<float*>(smem + (wave & 3) * PART) + lane;
-    if (half == 1) {
-#pragma unroll
-        for (int vb = 0; vb < G::VB; ++vb)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) part[(vb * 16 + e) * 64] = oacc[vb][e];
-        part[G::VB * 16 * 64] = st.m;
-        part[(G::VB * 16 + 1) * 64] = st.l;
-    }
-    __syncthreads();
-    if (half == 0) {
-        const float m1 = part[G::VB * 16 * 64], l1 = part[(G::VB * 16 + 1) * 64];
-        const float m = fmaxf(st.m, m1);
-        const float mc = m == kNegInf ? 0.f : m * cl2;
-        const float a0 = __builtin_amdgcn_exp2f(st.m * cl2 - mc), a1 = __builtin_amdgcn_exp2f(m1 * cl2 - mc);   // 0 from -inf
-        const float inv = row_inverse(exchange_sum(st.l * a0 + l1 * a1));
-#pragma unroll
-        for (int vb = 0; vb < G::VB; ++vb)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) oacc[vb][e] = oacc[vb][e] * a0 + part[(vb * 16 + e) * 64] * a1;
-        stage_output<T, D>(smem + OUT, rows + lq, lh, oacc, inv);
-    }
-    __syncthreads();
-    write_output<T, D, kThreads8>(smem + OUT, o_base, p.o_rs, q0, p.Lq, BM, tid);
 }
 
 // ───────────────────────── short key sequences (cross attention) ─────────────────────────
@@ -1391,7 +1263,7 @@ bool same_keys_for_all_rows(const SdpaDev& p) {
     return p.mask_mode == MI_MASK_NONE && !p.prefix_scaled && (p.Lp == 0 || (p.kp_rs == p.k_rs && p.vp_rs == p.v_rs));
 }
 
-// Whether a launch runs on 256-row tiles (8 wavefronts, two per SIMD, softmax of one under the MFMAs of the other) or on
+// Whether a launch that sdpa_small.hip leaves here runs on 256-row tiles (8 wavefronts, two per SIMD, softmax of one under the MFMAs of the other) or on
 // 128-row tiles. With a 256-row tile or more per CU the former always. Below that the 128-row kernel keeps more CUs busy, but
 // each of them runs one wavefront per SIMD whose softmax nothing hides, and from the 257th work group on two share a CU
 // anyway ("crowded"); a CU with eight wavefronts needs 2/3 of the time per row and key, and costs about 1.5 us more to start
@@ -1542,18 +1414,6 @@ int launch_d(SdpaDev p, int n_cu, hipStream_t stream) {
             }
         }
     } else {
-        if constexpr (pair_kernel_available<D>()) {
-            // from 4 key tiles on (16 heads of 96, 256 tokens: 10.7 -> 10.3 us) and while no CU gets two groups (the LDS holds one)
-            const long tiles128 = static_cast<long>(p.B) * p.H * ((p.Lq + 127) / 128);
-            if (choice == 0 && !xtra && !rope_k && !p.prefix_scaled && tiles128 <= n_cu && n_kt >= 4) {
-                p.n_q_tiles = (p.Lq + 127) / 128;
-                p.n_blocks = static_cast<int>(tiles128);
-                hipLaunchKernelGGL((sdpa_fwd_pair_kernel<T, D>), dim3(grid_blocks(p)), dim3(kThreads8), lds_bytes_pair<D>(), stream, p);
-                const hipError_t e = hipGetLastError();
-                if (e != hipSuccess) return fail("sdpa_fwd launch: %s", hipGetErrorString(e));
-                return 0;
-            }
-        }
         p.n_q_tiles = (p.Lq + 127) / 128;
         p.n_blocks = p.B * p.H * p.n_q_tiles;
         const dim3 grid(grid_blocks(p)), block(kThreads4);
@@ -1605,6 +1465,8 @@ size_t sdpa_split_scratch_bytes(const SdpaDev& p, int dtype, int head_dim) {
 
 int launch_sdpa(const SdpaDev& p, int dtype, int head_dim, hipStream_t stream) {
     if (sdpa_wide_head(head_dim)) return launch_sdpa_wide(p, dtype, head_dim, stream);
+    if ((dtype == MI_DTYPE_BF16 || dtype == MI_DTYPE_F16) && sdpa_kernel_choice() == 0 && sdpa_small_takes(p, head_dim))
+        return launch_sdpa_small(p, dtype, head_dim, stream);
     const int n_cu = device_cu_count();
     if (dtype == MI_DTYPE_BF16) return launch_t<__bf16>(p, head_dim, n_cu, stream);
     if (dtype == MI_DTYPE_F16) return launch_t<_Float16>(p, head_dim, n_cu, stream);

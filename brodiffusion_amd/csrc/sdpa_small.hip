@@ -1,0 +1,439 @@
+// Softmax attention for calls that are latency before they are anything else (few query rows, or few keys), and for the head
+// dimensions that the 256-row kernels of sdpa_fwd.hip serve badly.
+//
+// Such a call is a chain: operands -> LDS -> scores -> softmax -> values -> out. The 128-row kernel makes it long (three barriers
+// and a staging pass before the first key tile is even requested, then 64-key tiles one after the other on one wavefront per SIMD)
+// and leaves most of the GPU out of it: 64 tokens of 8 heads of 160 took 8.5 us on 16 work groups, an empty launch takes 2.3.
+// Here a work group is R x S wavefronts for 32 R query rows: wavefront (r, s) has rows 32 r .. 32 r + 31 and the 32-key blocks
+// s, s + S, ..., so that S blocks are worked on at a time, and the S partial results of a row are merged through LDS in FP32.
+//   * Every operand of the first block is requested before anything is waited for: query rows straight into MFMA operand
+//     registers, keys and values by LDS DMA. No barrier stands in front of the first product where R = 1.
+//   * A block sits in LDS as panels of 32 keys x 64 bytes (32 head-dim elements), deposited by DMA instructions of 16 keys x 64
+//     bytes. All panels of a row share one address (the panel is a scalar offset), the fragments of K and V are read from two
+//     addresses each plus immediates, and an XOR of the 16-byte piece with (key / 4) % 4 spreads 16 rows over all banks for the K
+//     reads (four rows are 256 bytes) and leaves the V transpose reads on theirs.
+//   * The fragments of a block are all read into registers before it is multiplied. Then its LDS is free, and the next block's
+//     DMA runs under the products and the softmax of this one: one buffer, no ring. (Two and three buffers measured the same: an
+//     LDS read issued behind a DMA load waits for that load. What hides the rest is other wavefronts, and a small footprint lets
+//     more of them in.)
+// What bounds it: the latency of a block's DMA per step with few rows, the VALU with many.
+// Measured (fp16, 8 heads; before: the 128-row kernel, for 80 in pairs of tiles, for 40 and 72 the 256-row kernels), us:
+//   self, tokens x head_dim: 64 x 160 8.5 -> 6.1, 256 x 160 14.5 -> 8.0, 1024 x 160 37.3 -> 16.6; 512 x 80 14.4 -> 6.9, 2048 x 80
+//   39.7 -> 25.0; 1024 x 40 18.0 -> 9.0, 2048 x 40 31 -> 18.4; 16 heads of 72, 1024 23.3 -> 14.6; 24 of 128, 512 16.9 -> 11.3
+//   77 keys, queries x head_dim: 64 x 160 10.7 -> 6.6, 1024 x 80 8.8 -> 5.3, 4096 x 40 8.1 -> 6.0
+#include "sdpa_tiles.h"
+
+namespace mi {
+namespace {
+
+using namespace sdpa;
+
+constexpr int kKB = 32;        // keys of a block
+constexpr int kMaxWaves = 8;
+constexpr int kMaxLds = 160 * 1024 - 64;
+
+template <int D> struct SmallGeo {
+    using G = HeadGeo<D>;
+    static constexpr int NP = G::VB;                            // panels of 32 head-dim elements
+    static constexpr int PANEL = kKB * 64;                      // bytes of 32 keys of a panel
+    static constexpr int OPER = NP * PANEL, BLOCK = 2 * OPER;   // K or V of a block; both
+    static constexpr int P_STRIDE = D * 4 + 16;                 // bytes of one row of a partial output
+    static constexpr int PART = 32 * P_STRIDE + 2 * 32 * 4;     // a wavefront's partial output, maxima and denominators
+};
+
+template <typename T, int D, int R>
+__global__ void __launch_bounds__(64 * kMaxWaves, D <= 64 ? 4 : D <= 80 ? 3 : 2) sdpa_small_kernel(const SdpaDev p, int S) {
+    using G = HeadGeo<D>;
+    using SG = SmallGeo<D>;
+    using V8 = typename Mma<T>::v8;
+    typedef T t8 __attribute__((ext_vector_type(8)));
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    __shared__ int red[2 * R];
+
+    const int logical = logical_block(p.n_blocks);
+    if (logical < 0) return;
+    const int qt = logical % p.n_q_tiles, bh = logical / p.n_q_tiles;
+    const int h = bh % p.H, b = bh / p.H;
+    const int hk = h / p.kv_group;
+    const int tid = threadIdx.x, NT = 64 * R * S;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = wave % R, s = wave / R;
+    const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
+    const int q0 = qt * (32 * R);
+
+    // ── requests: this lane's query row with its RoPE entries, then the first block of keys and values ──
+    const bool rope = p.cos_q != nullptr && !p.rope_split;
+    u32x4 qraw[G::KC];
+    f32x4 cs[G::KC], sn[G::KC];
+    const int qrow = min(q0 + 32 * r + lq, p.Lq - 1);
+    const T* const q_row = static_cast<const T*>(p.q) + b * p.q_bs + h * D + static_cast<long>(qrow) * p.q_rs;
+#pragma unroll
+    for (int c = 0; c < G::KC; ++c) qraw[c] = *reinterpret_cast<const u32x4*>(q_row + min(16 * c + 8 * lh, D - 8));
+    if (rope) {
+#pragma unroll
+        for (int c = 0; c < G::KC; ++c) {
+            const long at = static_cast<long>(qrow) * (D / 2) + min(16 * c + 8 * lh, D - 8) / 2;
+            cs[c] = *reinterpret_cast<const f32x4*>(p.cos_q + at);
+            sn[c] = *reinterpret_cast<const f32x4*>(p.sin_q + at);
+        }
+    }
+    // Visible keys [lo, hi) of this lane's row, and the blocks of the work group: those of the cached prefix, then those of the fresh
+    // keys, from the first to the last that one of its rows sees; none straddles the two.
+    int n_keys = p.Lk;
+    if (p.kv_valid_len) n_keys = __builtin_amdgcn_readfirstlane(max(min(n_keys, p.kv_valid_len[b]), 0));
+    int lo = 0, hi = n_keys, first_key = 0, stop_key = n_keys;
+    WaveExtent we{0, 0, n_keys, n_keys};
+    if (p.mask_mode != MI_MASK_NONE) {
+        row_interval(p, b, min(q0 + 32 * r + lq, p.Lq - 1), q0 + 32 * r < p.Lq, lo, hi);
+        we = wave_extent(lo, hi);
+        first_key = we.lo_min; stop_key = we.hi_max;
+        if (R > 1) {
+            if (lane == 0) { red[r] = we.lo_min; red[R + r] = we.hi_max; }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < R; ++i) { first_key = min(first_key, red[i]); stop_key = max(stop_key, red[R + i]); }
+            first_key = __builtin_amdgcn_readfirstlane(first_key);
+            stop_key = __builtin_amdgcn_readfirstlane(stop_key);
+        }
+        if (first_key >= stop_key) first_key = stop_key = 0;
+    }
+    const int n_pre = min(p.Lp, stop_key), n_fresh = max(stop_key - p.Lp, 0);     // keys of the two segments up to the last visible one
+    const int pre0 = first_key / kKB, fresh0 = max(first_key - p.Lp, 0) / kKB;
+    const int pre_blocks = max((n_pre + kKB - 1) / kKB - pre0, 0);
+    const int n_blocks = pre_blocks + (n_fresh + kKB - 1) / kKB - fresh0;      // this wavefront takes blocks s, s + S, ...
+
+    // ── DMA duty: a block is 2 operands x 2 groups of 16 keys x NP panels; the R wavefronts that share it take 4 / R
+    //    (operand, group) pairs each ──
+    constexpr int PAIRS = 4 / R;
+    const unsigned lds_base = static_cast<unsigned>(reinterpret_cast<size_t>((__attribute__((address_space(3))) unsigned char*)smem));
+    const int prow = lane >> 2, pch = (lane & 3) ^ ((prow >> 2) & 3);
+    const unsigned last_cut = static_cast<unsigned>(max(pch - (G::CPR - 1 - 4 * (SG::NP - 1)), 0)) * 16u;   // chunks past the row's end repeat its last one
+    auto load_block = [&](int blk) {
+        const bool pre = blk < pre_blocks;
+        const int row0 = (pre ? pre0 + blk : fresh0 + blk - pre_blocks) * kKB, last = (pre ? n_pre : n_fresh) - 1;   // rows past the end repeat the last one
+#pragma unroll
+        for (int i = 0; i < PAIRS; ++i) {
+            const int pair = r * PAIRS + i, op = pair >> 1, g = pair & 1;
+            const void* const t = op ? (pre ? p.vp : p.v) : (pre ? p.kp : p.k);
+            const long bs = op ? (pre ? p.vp_bs : p.v_bs) : (pre ? p.kp_bs : p.k_bs), rs = op ? (pre ? p.vp_rs : p.v_rs) : (pre ? p.kp_rs : p.k_rs);
+            const unsigned char* const base = reinterpret_cast<const unsigned char*>(static_cast<const T*>(t) + b * bs + hk * D);
+            const unsigned off = static_cast<unsigned>(min(row0 + 16 * g + prow, last)) * (static_cast<unsigned>(rs) * 2u) + static_cast<unsigned>(pch) * 16u;
+            const unsigned dst = lds_base + s * SG::BLOCK + op * SG::OPER + g * 1024;
+            // (inline assembly: for the builtin the compiler would wait for the load in front of every later LDS read; the LDS base
+            //  travels in m0, and the s_nop is the wait state an LDS-DMA instruction needs behind a write of m0)
+#pragma unroll
+            for (int pn = 0; pn < SG::NP; ++pn)
+                asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(pn == SG::NP - 1 ? off - last_cut : off), "s"(base + pn * 64),
+                             "{m0}"(dst + pn * SG::PANEL) : "memory");
+        }
+    };
+    if (s < n_blocks) load_block(s);
+
+    if (p.cos_q != nullptr && p.rope_split) {
+        // pairs of two halves: four elements at a time lie in one half (head_dim / 2 is a multiple of 4), their partners and table
+        // entries are fetched here
+        typedef T t4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+        for (int c = 0; c < G::KC; ++c) {
+            t8 x = __builtin_bit_cast(t8, qraw[c]);
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+                const int d = min(16 * c + 8 * lh, D - 8) + 4 * g;
+                const bool upper = d >= D / 2;
+                const int pair = upper ? d - D / 2 : d;
+                const t4 other = *reinterpret_cast<const t4*>(q_row + (upper ? pair : d + D / 2));
+                const f32x4 c4 = *reinterpret_cast<const f32x4*>(p.cos_q + static_cast<long>(qrow) * (D / 2) + pair);
+                const f32x4 s4 = *reinterpret_cast<const f32x4*>(p.sin_q + static_cast<long>(qrow) * (D / 2) + pair);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float own = static_cast<float>(x[4 * g + e]), oth = static_cast<float>(other[e]);
+                    const float re = rope_re(own, oth, c4[e], s4[e]), im = rope_im(oth, own, c4[e], s4[e]);
+                    x[4 * g + e] = static_cast<T>(upper ? im : re);
+                }
+            }
+            qraw[c] = __builtin_bit_cast(u32x4, x);
+        }
+    }
+    V8 qf[G::KC];
+#pragma unroll
+    for (int c = 0; c < G::KC; ++c) {
+        u32x4 v = qraw[c];
+        if (rope) v = rope_chunk<T>(v, cs[c], sn[c]);
+        // (the pad of the head dimension: the upper lane half of the last fragment)
+        if (G::DK > D && c == G::KC - 1 && lh) v = u32x4{0, 0, 0, 0};
+        qf[c] = __builtin_bit_cast(V8, v);
+    }
+    const unsigned pad_keep = lh ? 0u : ~0u;
+    f32x16 oacc[G::VB];
+#pragma unroll
+    for (int vb = 0; vb < G::VB; ++vb)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) oacc[vb][e] = 0.f;
+    float m = kNegInf, mc = 0.f, l = 0.f;
+    bool started = false;      // a block has been accumulated
+    const float cl2 = p.scale_log2;
+    const float lazy_raw = kLazyLog2 / cl2;
+    const int trow = (lane & 15) >> 2, j4 = lane & 3, g1 = (lane >> 4) & 1;
+    unsigned kaddr[2], vaddr[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        kaddr[i] = lq * 64 + (((2 * i + lh) ^ ((lq >> 2) & 3)) << 4);
+        vaddr[i] = SG::OPER + (4 * lh + 8 * i + trow) * 64 + (((2 * g1 + (j4 >> 1)) ^ (lh + 2 * i)) << 4) + 8 * (j4 & 1);
+    }
+
+    const int n_steps = (n_blocks + S - 1) / S;
+    for (int t = 0; t < n_steps; ++t) {
+        const int blk = t * S + s;
+        const bool pre = blk < pre_blocks;
+        const int row0 = (pre ? pre0 + blk : fresh0 + blk - pre_blocks) * kKB, j0 = pre ? row0 : p.Lp + row0;
+        const int rows = (pre ? n_pre : n_fresh) - row0;      // keys of the block
+        const bool mine = blk < n_blocks && j0 < we.hi_max && j0 + kKB > we.lo_min;
+        const unsigned char* const buf = smem + s * SG::BLOCK;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (R > 1) __syncthreads();
+        V8 kf[G::KC], vf[2][G::VB];
+        if (mine) {
+#pragma unroll
+            for (int c = 0; c < G::KC; ++c) kf[c] = *reinterpret_cast<const V8*>(buf + kaddr[c & 1] + (c >> 1) * SG::PANEL);
+#pragma unroll
+            for (int c4 = 0; c4 < 2; ++c4)
+#pragma unroll
+                for (int vb = 0; vb < G::VB; ++vb) {
+                    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(buf + vaddr[0] + vb * SG::PANEL + c4 * 1024));
+                    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(buf + vaddr[1] + vb * SG::PANEL + c4 * 1024));
+                    vf[c4][vb] = __builtin_bit_cast(V8, s16x8(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7)));
+                }
+        }
+        if (t + 1 < n_steps) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if (R > 1) __syncthreads();
+            if (blk + S < n_blocks) load_block(blk + S);
+        }
+        if (mine) {
+            f32x16 sacc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int c = 0; c < G::KC; ++c) {
+                u32x4 a = __builtin_bit_cast(u32x4, kf[c]);
+                if (G::DK > D && c == G::KC - 1) a &= pad_keep;
+                sacc = Mma<T>::run(__builtin_bit_cast(V8, a), qf[c], sacc);
+            }
+            if (j0 < we.lo_max || j0 + min(rows, kKB) > we.hi_min || rows < kKB) {
+                const int x0 = j0 + 4 * lh - lo, top = min(hi, j0 + rows) - 1 - lo;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    const float score = sacc[e];
+                    sacc[e] = blank_outside(score, x0 + 8 * (e >> 2) + (e & 3), top);
+                }
+            }
+            if (rows < kKB) {
+                // value rows of zeros past the end (they repeat the last row, which may hold infinities)
+                const int top = rows - 1 - 4 * lh;
+#pragma unroll
+                for (int c4 = 0; c4 < 2; ++c4) {
+                    u32x4 keep;
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) {
+                        const int key = 16 * c4 + 8 * (w >> 1) + 2 * (w & 1);   // and the one after it
+                        keep[w] = (key <= top ? 0xffffu : 0u) | (key + 1 <= top ? 0xffff0000u : 0u);
+                    }
+#pragma unroll
+                    for (int vb = 0; vb < G::VB; ++vb) vf[c4][vb] = __builtin_bit_cast(V8, __builtin_bit_cast(u32x4, vf[c4][vb]) & keep);
+                }
+            }
+            float mloc = sacc[0];
+#pragma unroll
+            for (int e = 1; e < 16; ++e) mloc = fmaxf(mloc, sacc[e]);
+            mloc = exchange_max(mloc);
+            if (__any(mloc > m + lazy_raw)) {
+                const float m_new = fmaxf(m, mloc);
+                const float mc_new = (m_new == kNegInf) ? 0.f : m_new * cl2;
+                if (started) {
+                    const float alpha = __builtin_amdgcn_exp2f(m * cl2 - mc_new);
+                    l *= alpha;
+#pragma unroll
+                    for (int vb = 0; vb < G::VB; ++vb)
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) oacc[vb][e] *= alpha;
+                }
+                m = m_new;
+                mc = mc_new;
+            }
+            started = true;
+            V8 pf[2];
+            float l0 = 0.f, l1 = 0.f;
+#pragma unroll
+            for (int c4 = 0; c4 < 2; ++c4)
+#pragma unroll
+                for (int i = 0; i < 8; i += 2) {
+                    const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[8 * c4 + i], cl2, -mc));
+                    const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[8 * c4 + i + 1], cl2, -mc));
+                    l0 += p0;
+                    l1 += p1;
+                    pf[c4][i] = static_cast<T>(p0);
+                    pf[c4][i + 1] = static_cast<T>(p1);
+                }
+            l += l0 + l1;
+#pragma unroll
+            for (int c4 = 0; c4 < 2; ++c4)
+#pragma unroll
+                for (int vb = 0; vb < G::VB; ++vb) oacc[vb] = Mma<T>::run(vf[c4][vb], pf[c4], oacc[vb]);
+        }
+    }
+    __syncthreads();     // the blocks are used up
+    const float l_tot = exchange_sum(l);
+    T* const o_base = static_cast<T*>(p.o) + b * p.o_bs + h * D;
+    if (S == 1) {
+        // every wavefront has all keys of its rows
+        stage_output<T, D>(smem, 32 * r + lq, lh, oacc, row_inverse(l_tot));
+        __syncthreads();
+        write_output<T, D, 64 * R>(smem, o_base, p.o_rs, q0, p.Lq, 32 * R, tid);
+        return;
+    }
+    // ── partial outputs, maxima and denominators to LDS, FP32; then every thread merges 16-byte pieces of output rows ──
+    {
+        unsigned char* const part = smem + (s * R + r) * SG::PART;
+        unsigned char* const row = part + lq * SG::P_STRIDE;
+#pragma unroll
+        for (int vb = 0; vb < G::VB; ++vb)
+#pragma unroll
+            for (int bb = 0; bb < 4; ++bb) {
+                const int d0 = 32 * vb + 8 * bb + 4 * lh;
+                if (32 * vb + 8 * bb < D) {
+                    const f32x16 acc = oacc[vb];
+                    *reinterpret_cast<f32x4*>(row + d0 * 4) = f32x4{acc[4 * bb], acc[4 * bb + 1], acc[4 * bb + 2], acc[4 * bb + 3]};
+                }
+            }
+        float* const stat = reinterpret_cast<float*>(part + 32 * SG::P_STRIDE);
+        if (lh == 0) { stat[lq] = m; stat[32 + lq] = l_tot; }
+    }
+    __syncthreads();
+    for (int idx = tid; idx < 32 * R * G::CPR; idx += NT) {
+        const int row = idx / G::CPR, cc = idx - row * G::CPR;
+        if (q0 + row >= p.Lq) break;
+        const unsigned char* const part = smem + (row >> 5) * SG::PART;
+        const int lr = row & 31;
+        float mm = kNegInf;
+        for (int k = 0; k < S; ++k) mm = fmaxf(mm, reinterpret_cast<const float*>(part + k * R * SG::PART + 32 * SG::P_STRIDE)[lr]);
+        const float mmc = mm == kNegInf ? 0.f : mm * cl2;
+        float lsum = 0.f;
+        f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = {0.f, 0.f, 0.f, 0.f};
+        for (int k = 0; k < S; ++k) {
+            const unsigned char* const pk = part + k * R * SG::PART;
+            const float* const stat = reinterpret_cast<const float*>(pk + 32 * SG::P_STRIDE);
+            const float w = __builtin_amdgcn_exp2f(stat[lr] * cl2 - mmc);
+            lsum = __builtin_fmaf(w, stat[32 + lr], lsum);
+            const f32x4 a = *reinterpret_cast<const f32x4*>(pk + lr * SG::P_STRIDE + cc * 32);
+            const f32x4 c = *reinterpret_cast<const f32x4*>(pk + lr * SG::P_STRIDE + cc * 32 + 16);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                lo[e] = __builtin_fmaf(w, a[e], lo[e]);
+                hi[e] = __builtin_fmaf(w, c[e], hi[e]);
+            }
+        }
+        const float inv = row_inverse(lsum);
+        t8 out;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            out[e] = static_cast<T>(lo[e] * inv);
+            out[4 + e] = static_cast<T>(hi[e] * inv);
+        }
+        *reinterpret_cast<t8*>(o_base + static_cast<long>(q0 + row) * p.o_rs + cc * 8) = out;
+    }
+}
+
+// 32-key blocks of a call (those of the prefix and of the fresh keys apart)
+int key_blocks(const SdpaDev& p) { return (p.Lp + kKB - 1) / kKB + (p.Lk - p.Lp + kKB - 1) / kKB; }
+
+// Whether a call comes here, and with how many row groups and at most how many wavefronts to a work group.
+//
+// Calls without extras (key mask, logit bias, denominators), tile-wise K rotation, the prefix dial or packed sequences. The lines
+// are from 8 head dimensions x 64 to 8192 units (32 query rows of a head) x 1 to 256 key blocks of 8 fp16 heads, every R and two S
+// against the kernel that took the call before (us, before / here; n = compute units). Masked calls (causal, windowed, block-causal;
+// 8 dimensions x 64 to 1008 units) take 0.35 to 0.98 of the time up to 4 n units, except windowed ones of 80 to 112 above 3 n (1008
+// units, window 256: 96 15.9 / 17.3); beyond 4 n they are left where their longest tiles start first.
+//   units <= n       R = 1: 256 units, 5, 32 and 128 blocks: 40 8.4 / 4.8, 18.2 / 8.9, 56 / 25; 72 10.5 / 5.4, 23 / 10.2, 73 / 27; 128
+//                    10.5 / 6.7, 25.7 / 12, 79 / 30; 160 13.4 / 7.9, 37 / 16.5, 134 / 43
+//   units <= 2 n     R = 2: 512 units, 5, 32 and 128 blocks: 40 8.5 / 5.5, 18 / 11, 56 / 32; 80 10.5 / 6.5, 23 / 15, 73 / 40; 128 10.8 /
+//                    7.9, 26 / 18, 79 / 51
+//   units <= 4 n     R = 4: 1024 units, 5, 32 and 128 blocks: 40 8.9 / 6.7, 19 / 17, 57 / 54 (R = 2: 6.9, 17, 52: taken from 48 blocks
+//                    on up to head_dim 64, where two such groups share a CU); 72 11.2 / 7.7, 24 / 21, 73 / 65; 128 11.4 / 8.8, 27 / 25,
+//                    84 / 82. One wavefront per 32 rows up to 8 blocks (6 up to head_dim 64), then two: 72, 768 units, 5 blocks 7.4 and
+//                    8.2, 8 blocks 9.2 and 9.5, 16 blocks 14.1 and 13.0
+//   more             R = 4, S = 1: 160 at any size (1400 units, 8 blocks 28 / 17; 4096 units, 32 blocks 152 / 96). The others below one
+//                    256-row tile per CU (8 n units) while the keys are few: 1400 units, 5 and 8 blocks 40 9.2 / 7.6, 9.5 / 9.5; 72 12.5 /
+//                    9.5, 12.3 / 11.8, 16 blocks 16.6 / 18; 128 13.6 / 11.2, 14.5 / 14.1. Above it short keys have a kernel of their own,
+//                    and of the long ones 80, 96 and 112 come here, which the 256-row kernel serves without its special forms: 4096 units,
+//                    16, 32 and 64 blocks 80 45 / 35, 73 / 62, 134 / 115; 96 45 / 37, 70 / 64, 120 / 119; 112 50 / 44, 79 / 76, 136 / 142
+struct SmallPlan { int R = 0, waves = 0; };
+SmallPlan plan_small(const SdpaDev& p, int D, int n_cu) {
+    if (p.key_mask || p.bias || p.lse || p.cu_q || p.cos_k || p.prefix_scaled) return {};
+    // row offsets inside K and V are 32-bit
+    const long most = (1L << 31) - 1;
+    if (p.Lk * p.k_rs * 2 > most || p.Lk * p.v_rs * 2 > most || (p.Lp > 0 && (p.Lp * p.kp_rs * 2 > most || p.Lp * p.vp_rs * 2 > most))) return {};
+    const long heads = static_cast<long>(p.B) * p.H, units = heads * ((p.Lq + 31) / 32);
+    const int nb = key_blocks(p);
+    const bool masked = p.mask_mode != MI_MASK_NONE;
+    if (masked && (units > 4L * n_cu || (p.window > 0 && units > 3L * n_cu && D >= 80 && D <= 112))) return {};
+    if (units <= n_cu) return {1, kMaxWaves};
+    if (units <= 2L * n_cu) return {2, kMaxWaves};
+    if (units <= 4L * n_cu) {
+        if (D <= 64 && nb >= 48) return {2, kMaxWaves};
+        return {4, nb <= (D <= 64 ? 6 : 8) ? 4 : kMaxWaves};
+    }
+    const SmallPlan whole{4, 4};
+    if (D == 160) return whole;
+    const bool long_keys = D == 80 || (D == 96 && nb <= 64) || (D == 112 && nb <= 32);
+    if (heads * ((p.Lq + 255) / 256) < n_cu) return nb <= (D <= 64 ? 6 : 8) || (long_keys && nb <= (D == 80 ? 64 : 24)) ? whole : SmallPlan{};
+    return long_keys && nb > 10 ? whole : SmallPlan{};
+}
+
+template <typename T, int D, int R>
+int launch_small(SdpaDev p, int most_waves, hipStream_t stream) {
+    using SG = SmallGeo<D>;
+    const int n_kb = key_blocks(p);
+    int S = max(1, min(min(n_kb, most_waves / R), kMaxLds / max(SG::BLOCK, R * SG::PART)));
+    const int steps = (n_kb + S - 1) / S;
+    S = max(1, (n_kb + steps - 1) / max(steps, 1));      // as few wavefronts as take that many steps
+    const int lds = S == 1 ? max(SG::BLOCK, 32 * R * HeadGeo<D>::O_STRIDE) : S * max(SG::BLOCK, R * SG::PART);
+    p.n_q_tiles = (p.Lq + 32 * R - 1) / (32 * R);
+    p.n_blocks = p.B * p.H * p.n_q_tiles;
+    hipLaunchKernelGGL((sdpa_small_kernel<T, D, R>), dim3((p.n_blocks + 7) / 8 * 8), dim3(64 * R * S), lds, stream, p, S);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail("sdpa_fwd launch: %s", hipGetErrorString(e));
+    return 0;
+}
+
+template <typename T, int D>
+int launch_small_r(const SdpaDev& p, const SmallPlan& plan, hipStream_t stream) {
+    switch (plan.R) {
+        case 1: return launch_small<T, D, 1>(p, plan.waves, stream);
+        case 2: return launch_small<T, D, 2>(p, plan.waves, stream);
+        default: return launch_small<T, D, 4>(p, plan.waves, stream);
+    }
+}
+
+template <typename T>
+int launch_small_t(const SdpaDev& p, int head_dim, const SmallPlan& plan, hipStream_t stream) {
+    switch (head_dim) {
+        case 40: return launch_small_r<T, 40>(p, plan, stream);
+        case 64: return launch_small_r<T, 64>(p, plan, stream);
+        case 72: return launch_small_r<T, 72>(p, plan, stream);
+        case 80: return launch_small_r<T, 80>(p, plan, stream);
+        case 96: return launch_small_r<T, 96>(p, plan, stream);
+        case 112: return launch_small_r<T, 112>(p, plan, stream);
+        case 128: return launch_small_r<T, 128>(p, plan, stream);
+        default: return launch_small_r<T, 160>(p, plan, stream);
+    }
+}
+
+}  // namespace
+
+int launch_sdpa_small(const SdpaDev& p, int dtype, int head_dim, hipStream_t stream) {
+    const SmallPlan plan = plan_small(p, head_dim, device_cu_count());
+    if (dtype == MI_DTYPE_BF16) return launch_small_t<__bf16>(p, head_dim, plan, stream);
+    return launch_small_t<_Float16>(p, head_dim, plan, stream);
+}
+
+bool sdpa_small_takes(const SdpaDev& p, int head_dim) { return plan_small(p, head_dim, device_cu_count()).R != 0; }
+
+}  // namespace mi

@@ -1,6 +1,6 @@
-"""Launches with at most one 128-row query tile per compute unit at head_dim 80, 96 and 112: two halves of a work group take the
-even and the odd key tiles and merge. Key counts around the pairs of tiles, rows around the query tile, masks that leave one
-half without keys, a partial prefix, and scores far apart between the halves."""
+"""Launches with at most one 128-row query tile per compute unit at head_dim 80, 96 and 112: the wavefronts of a work group take
+key blocks in turn and merge. Key counts around the pairs of tiles, rows around the query tile, masks that leave some
+of them without keys, a partial prefix, and scores far apart between them."""
 import numpy as np
 import pytest
 import torch
