@@ -106,8 +106,11 @@ bool sdpa_wide_head(int head_dim);
 size_t sdpa_wide_split_scratch_bytes(const SdpaDev& p, int head_dim);
 int launch_sdpa_wide(const SdpaDev& p, int dtype, int head_dim, hipStream_t stream);
 
-// Calls with few query rows or few keys, and more (sdpa_small.hip): whether they take a call at kernel choice 0, and the launch.
+// Calls with few query rows (sdpa_small.hip) and unmasked ones of some sizes (sdpa_flow.hip): whether the kernel takes a call at kernel
+// choice 0, and the launch.
 bool sdpa_small_takes(const SdpaDev& p, int head_dim);
+bool sdpa_flow_takes(const SdpaDev& p, int head_dim, int n_cu);
+int launch_sdpa_flow(const SdpaDev& p, int dtype, int head_dim, hipStream_t stream);
 int launch_sdpa_small(const SdpaDev& p, int dtype, int head_dim, hipStream_t stream);
 
 // Device-side view of the head-averaged attention map launch (batch 1).

@@ -1,5 +1,5 @@
 // Flash-style softmax attention forward for gfx950 (MI355X), hand-written. Four kernels share the building blocks of
-// sdpa_common.h; launch_d picks one per call that sdpa_small.hip does not take:
+// sdpa_common.h; launch_d picks one per call that sdpa_small.hip and sdpa_flow.hip do not take:
 //
 //   sdpa_fwd_kernel         4 wavefronts = 128 query rows per work group, K/V tiles through registers into padded LDS,
 //                           double buffered. Few keys or few work groups (rows256_pay) with extras or masks, packed
@@ -1228,6 +1228,7 @@ template <int D>
 bool plan_split(SdpaDev& p, int n_cu) {
     p.split = SplitGeo{};
     if constexpr (!dma_kernel_available<D>()) return false;
+    if (sdpa_kernel_choice() == 0 && sdpa_flow_takes(p, D, n_cu)) return false;
     if (p.mask_mode != MI_MASK_NONE || p.kv_valid_len || p.key_mask || p.Lp > 0 || p.cos_k || p.cu_q) return false;
     // (the split form neither adds a logit bias nor writes the softmax denominators)
     if (p.bias != nullptr || p.lse != nullptr) return false;
@@ -1263,7 +1264,7 @@ bool same_keys_for_all_rows(const SdpaDev& p) {
     return p.mask_mode == MI_MASK_NONE && !p.prefix_scaled && (p.Lp == 0 || (p.kp_rs == p.k_rs && p.vp_rs == p.v_rs));
 }
 
-// Whether a launch that sdpa_small.hip leaves here runs on 256-row tiles (8 wavefronts, two per SIMD, softmax of one under the MFMAs of the other) or on
+// Whether a launch that comes here runs on 256-row tiles (8 wavefronts, two per SIMD, softmax of one under the MFMAs of the other) or on
 // 128-row tiles. With a 256-row tile or more per CU the former always. Below that the 128-row kernel keeps more CUs busy, but
 // each of them runs one wavefront per SIMD whose softmax nothing hides, and from the 257th work group on two share a CU
 // anyway ("crowded"); a CU with eight wavefronts needs 2/3 of the time per row and key, and costs about 1.5 us more to start
@@ -1306,6 +1307,14 @@ int launch_d(SdpaDev p, int n_cu, hipStream_t stream) {
         if (e != hipSuccess) return fail("sdpa_fwd launch: %s", hipGetErrorString(e));
         return 0;
     }
+    const int choice = sdpa_kernel_choice();
+    const long tiles256 = static_cast<long>(p.B) * p.H * ((p.Lq + 255) / 256);
+    // short key sequences whose K and V fit in LDS next to a query tile: one work group walks several query tiles
+    const int n_kt = (p.Lk + kBN - 1) / kBN;
+    const bool short_keys = D <= 128 && choice == 0 && p.mask_mode == MI_MASK_NONE && p.bias == nullptr && p.lse == nullptr && p.Lp == 0 && !rope_k &&
+                            p.cos_q == nullptr && n_kt >= 1 && n_kt <= shortkv_max_tiles<(D <= 128 ? D : 128)>() && tiles256 >= n_cu &&
+                            shortkv_lds_bytes<D>(n_kt, p.key_mask != nullptr) <= 160 * 1024;
+    if (choice == 0 && !short_keys && sdpa_flow_takes(p, D, n_cu)) return launch_sdpa_flow(p, std::is_same_v<T, __bf16> ? MI_DTYPE_BF16 : MI_DTYPE_F16, D, stream);
     if constexpr (dma_kernel_available<D>()) {
         if (p.split_scratch != nullptr && plan_split<D>(p, n_cu) &&
             p.split_scratch_bytes >= static_cast<size_t>(8) * p.split.max_tail * p.split.max_parts * SplitGeo::slot_bytes(D)) {
@@ -1323,8 +1332,6 @@ int launch_d(SdpaDev p, int n_cu, hipStream_t stream) {
         p.split = SplitGeo{};
     }
     // head_dim above 128 does not fit two wavefronts per SIMD and stays on the 128-row kernel
-    const long tiles256 = static_cast<long>(p.B) * p.H * ((p.Lq + 255) / 256);
-    const int choice = sdpa_kernel_choice();
     // calls with a key mask, a logit bias or a request for the softmax denominators take the XTRA instances of the 256-row
     // kernels (visibility words of all key tiles in LDS behind the tile buffers), unless K is rotated tile by tile, the
     // prefix-KV dial is on as well, or the key sequence is too long for the words to fit: then the 128-row kernel
@@ -1334,11 +1341,7 @@ int launch_d(SdpaDev p, int n_cu, hipStream_t stream) {
     // calls with the prefix-KV dial stay on the 128-row kernel unless the DMA kernel (which has an instance for it) takes them
     const bool dial_ok = !p.prefix_scaled || (dma_kernel_available<D>() && !rope_k && choice != 3);
     const bool pingpong = D <= 128 && xtra_ok && dial_ok && (choice >= 2 || (choice == 0 && rows256_pay<D>(p, n_cu, xtra)));
-    // short key sequences whose K and V fit in LDS next to a query tile: one work group walks several query tiles
-    const int n_kt = (p.Lk + kBN - 1) / kBN;
-    if (D <= 128 && choice == 0 && p.mask_mode == MI_MASK_NONE && p.bias == nullptr && p.lse == nullptr &&
-        p.Lp == 0 && !rope_k && p.cos_q == nullptr && n_kt >= 1 && n_kt <= shortkv_max_tiles<(D <= 128 ? D : 128)>() && tiles256 >= n_cu &&
-        shortkv_lds_bytes<D>(n_kt, p.key_mask != nullptr) <= 160 * 1024) {
+    if (short_keys) {
         if constexpr (D <= 128) {
             p.n_q_tiles = (p.Lq + 255) / 256;
             const int n_strip = static_cast<int>(tiles256 / n_cu);   // 256 query rows per work group and round: about one work group per CU

@@ -1,5 +1,4 @@
-// Softmax attention for calls that are latency before they are anything else (few query rows, or few keys), and for the head
-// dimensions that the 256-row kernels of sdpa_fwd.hip serve badly.
+// Softmax attention for calls with few query rows: latency before they are anything else.
 //
 // Such a call is a chain: operands -> LDS -> scores -> softmax -> values -> out. The 128-row kernel makes it long (three barriers
 // and a staging pass before the first key tile is even requested, then 64-key tiles one after the other on one wavefront per SIMD)
@@ -8,15 +7,12 @@
 // s, s + S, ..., so that S blocks are worked on at a time, and the S partial results of a row are merged through LDS in FP32.
 //   * Every operand of the first block is requested before anything is waited for: query rows straight into MFMA operand
 //     registers, keys and values by LDS DMA. No barrier stands in front of the first product where R = 1.
-//   * A block sits in LDS as panels of 32 keys x 64 bytes (32 head-dim elements), deposited by DMA instructions of 16 keys x 64
-//     bytes. All panels of a row share one address (the panel is a scalar offset), the fragments of K and V are read from two
-//     addresses each plus immediates, and an XOR of the 16-byte piece with (key / 4) % 4 spreads 16 rows over all banks for the K
-//     reads (four rows are 256 bytes) and leaves the V transpose reads on theirs.
+//   * A block sits in LDS as panels (PanelReads): all panels of a row share one address (the panel is a scalar offset), and the
+//     fragments of K and V are read from two addresses each plus immediates.
 //   * The fragments of a block are all read into registers before it is multiplied. Then its LDS is free, and the next block's
-//     DMA runs under the products and the softmax of this one: one buffer, no ring. (Two and three buffers measured the same: an
-//     LDS read issued behind a DMA load waits for that load. What hides the rest is other wavefronts, and a small footprint lets
-//     more of them in.)
-// What bounds it: the latency of a block's DMA per step with few rows, the VALU with many.
+//     DMA runs under the products and the softmax of this one: one buffer, no ring. (Two and three buffers measured the same;
+//     a small footprint lets more wavefronts in.)
+// What bounds it: the latency of a block's DMA per step.
 // Measured (fp16, 8 heads; before: the 128-row kernel, for 80 in pairs of tiles, for 40 and 72 the 256-row kernels), us:
 //   self, tokens x head_dim: 64 x 160 8.5 -> 6.1, 256 x 160 14.5 -> 8.0, 1024 x 160 37.3 -> 16.6; 512 x 80 14.4 -> 6.9, 2048 x 80
 //   39.7 -> 25.0; 1024 x 40 18.0 -> 9.0, 2048 x 40 31 -> 18.4; 16 heads of 72, 1024 23.3 -> 14.6; 24 of 128, 512 16.9 -> 11.3
@@ -62,21 +58,8 @@ __global__ void __launch_bounds__(64 * kMaxWaves, D <= 64 ? 4 : D <= 80 ? 3 : 2)
     const int q0 = qt * (32 * R);
 
     // ── requests: this lane's query row with its RoPE entries, then the first block of keys and values ──
-    const bool rope = p.cos_q != nullptr && !p.rope_split;
-    u32x4 qraw[G::KC];
-    f32x4 cs[G::KC], sn[G::KC];
-    const int qrow = min(q0 + 32 * r + lq, p.Lq - 1);
-    const T* const q_row = static_cast<const T*>(p.q) + b * p.q_bs + h * D + static_cast<long>(qrow) * p.q_rs;
-#pragma unroll
-    for (int c = 0; c < G::KC; ++c) qraw[c] = *reinterpret_cast<const u32x4*>(q_row + min(16 * c + 8 * lh, D - 8));
-    if (rope) {
-#pragma unroll
-        for (int c = 0; c < G::KC; ++c) {
-            const long at = static_cast<long>(qrow) * (D / 2) + min(16 * c + 8 * lh, D - 8) / 2;
-            cs[c] = *reinterpret_cast<const f32x4*>(p.cos_q + at);
-            sn[c] = *reinterpret_cast<const f32x4*>(p.sin_q + at);
-        }
-    }
+    QRowFrags<T, D> qr;
+    qr.issue(p, b, h, min(q0 + 32 * r + lq, p.Lq - 1), lh);
     // Visible keys [lo, hi) of this lane's row, and the blocks of the work group: those of the cached prefix, then those of the fresh
     // keys, from the first to the last that one of its rows sees; none straddles the two.
     int n_keys = p.Lk;
@@ -129,40 +112,8 @@ __global__ void __launch_bounds__(64 * kMaxWaves, D <= 64 ? 4 : D <= 80 ? 3 : 2)
     };
     if (s < n_blocks) load_block(s);
 
-    if (p.cos_q != nullptr && p.rope_split) {
-        // pairs of two halves: four elements at a time lie in one half (head_dim / 2 is a multiple of 4), their partners and table
-        // entries are fetched here
-        typedef T t4 __attribute__((ext_vector_type(4)));
-#pragma unroll
-        for (int c = 0; c < G::KC; ++c) {
-            t8 x = __builtin_bit_cast(t8, qraw[c]);
-#pragma unroll
-            for (int g = 0; g < 2; ++g) {
-                const int d = min(16 * c + 8 * lh, D - 8) + 4 * g;
-                const bool upper = d >= D / 2;
-                const int pair = upper ? d - D / 2 : d;
-                const t4 other = *reinterpret_cast<const t4*>(q_row + (upper ? pair : d + D / 2));
-                const f32x4 c4 = *reinterpret_cast<const f32x4*>(p.cos_q + static_cast<long>(qrow) * (D / 2) + pair);
-                const f32x4 s4 = *reinterpret_cast<const f32x4*>(p.sin_q + static_cast<long>(qrow) * (D / 2) + pair);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float own = static_cast<float>(x[4 * g + e]), oth = static_cast<float>(other[e]);
-                    const float re = rope_re(own, oth, c4[e], s4[e]), im = rope_im(oth, own, c4[e], s4[e]);
-                    x[4 * g + e] = static_cast<T>(upper ? im : re);
-                }
-            }
-            qraw[c] = __builtin_bit_cast(u32x4, x);
-        }
-    }
     V8 qf[G::KC];
-#pragma unroll
-    for (int c = 0; c < G::KC; ++c) {
-        u32x4 v = qraw[c];
-        if (rope) v = rope_chunk<T>(v, cs[c], sn[c]);
-        // (the pad of the head dimension: the upper lane half of the last fragment)
-        if (G::DK > D && c == G::KC - 1 && lh) v = u32x4{0, 0, 0, 0};
-        qf[c] = __builtin_bit_cast(V8, v);
-    }
+    qr.finish(p, lh, qf);
     const unsigned pad_keep = lh ? 0u : ~0u;
     f32x16 oacc[G::VB];
 #pragma unroll
@@ -173,13 +124,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves, D <= 64 ? 4 : D <= 80 ? 3 : 2)
     bool started = false;      // a block has been accumulated
     const float cl2 = p.scale_log2;
     const float lazy_raw = kLazyLog2 / cl2;
-    const int trow = (lane & 15) >> 2, j4 = lane & 3, g1 = (lane >> 4) & 1;
-    unsigned kaddr[2], vaddr[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        kaddr[i] = lq * 64 + (((2 * i + lh) ^ ((lq >> 2) & 3)) << 4);
-        vaddr[i] = SG::OPER + (4 * lh + 8 * i + trow) * 64 + (((2 * g1 + (j4 >> 1)) ^ (lh + 2 * i)) << 4) + 8 * (j4 & 1);
-    }
+    const PanelReads at(lane);
 
     const int n_steps = (n_blocks + S - 1) / S;
     for (int t = 0; t < n_steps; ++t) {
@@ -194,15 +139,11 @@ __global__ void __launch_bounds__(64 * kMaxWaves, D <= 64 ? 4 : D <= 80 ? 3 : 2)
         V8 kf[G::KC], vf[2][G::VB];
         if (mine) {
 #pragma unroll
-            for (int c = 0; c < G::KC; ++c) kf[c] = *reinterpret_cast<const V8*>(buf + kaddr[c & 1] + (c >> 1) * SG::PANEL);
+            for (int c = 0; c < G::KC; ++c) kf[c] = *reinterpret_cast<const V8*>(buf + at.k[c & 1] + (c >> 1) * SG::PANEL);
 #pragma unroll
             for (int c4 = 0; c4 < 2; ++c4)
 #pragma unroll
-                for (int vb = 0; vb < G::VB; ++vb) {
-                    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(buf + vaddr[0] + vb * SG::PANEL + c4 * 1024));
-                    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(buf + vaddr[1] + vb * SG::PANEL + c4 * 1024));
-                    vf[c4][vb] = __builtin_bit_cast(V8, s16x8(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7)));
-                }
+                for (int vb = 0; vb < G::VB; ++vb) vf[c4][vb] = at.template v_frag<T>(buf + SG::OPER + vb * SG::PANEL + c4 * 1024);
         }
         if (t + 1 < n_steps) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -355,36 +296,21 @@ int key_blocks(const SdpaDev& p) { return (p.Lp + kKB - 1) / kKB + (p.Lk - p.Lp 
 //                    10.5 / 6.7, 25.7 / 12, 79 / 30; 160 13.4 / 7.9, 37 / 16.5, 134 / 43
 //   units <= 2 n     R = 2: 512 units, 5, 32 and 128 blocks: 40 8.5 / 5.5, 18 / 11, 56 / 32; 80 10.5 / 6.5, 23 / 15, 73 / 40; 128 10.8 /
 //                    7.9, 26 / 18, 79 / 51
-//   units <= 4 n     R = 4: 1024 units, 5, 32 and 128 blocks: 40 8.9 / 6.7, 19 / 17, 57 / 54 (R = 2: 6.9, 17, 52: taken from 48 blocks
-//                    on up to head_dim 64, where two such groups share a CU); 72 11.2 / 7.7, 24 / 21, 73 / 65; 128 11.4 / 8.8, 27 / 25,
-//                    84 / 82. One wavefront per 32 rows up to 8 blocks (6 up to head_dim 64), then two: 72, 768 units, 5 blocks 7.4 and
-//                    8.2, 8 blocks 9.2 and 9.5, 16 blocks 14.1 and 13.0
-//   more             R = 4, S = 1: 160 at any size (1400 units, 8 blocks 28 / 17; 4096 units, 32 blocks 152 / 96). The others below one
-//                    256-row tile per CU (8 n units) while the keys are few: 1400 units, 5 and 8 blocks 40 9.2 / 7.6, 9.5 / 9.5; 72 12.5 /
-//                    9.5, 12.3 / 11.8, 16 blocks 16.6 / 18; 128 13.6 / 11.2, 14.5 / 14.1. Above it short keys have a kernel of their own,
-//                    and of the long ones 80, 96 and 112 come here, which the 256-row kernel serves without its special forms: 4096 units,
-//                    16, 32 and 64 blocks 80 45 / 35, 73 / 62, 134 / 115; 96 45 / 37, 70 / 64, 120 / 119; 112 50 / 44, 79 / 76, 136 / 142
+//   units <= 4 n     unmasked calls go to sdpa_flow.hip, but for many keys at 64 (R = 2, two groups to a CU: 1024 units, 64 and 128
+//                    blocks 33 / 30, 65 / 53; there 32, 60). Masked ones: R = 4, one wavefront per 32 rows up to 8 blocks (6 up to
+//                    head_dim 64), then two: 72, 768 units, 5 blocks 7.4 and 8.2, 8 blocks 9.2 and 9.5, 16 blocks 14.1 and 13.0
 struct SmallPlan { int R = 0, waves = 0; };
 SmallPlan plan_small(const SdpaDev& p, int D, int n_cu) {
-    if (p.key_mask || p.bias || p.lse || p.cu_q || p.cos_k || p.prefix_scaled) return {};
-    // row offsets inside K and V are 32-bit
-    const long most = (1L << 31) - 1;
-    if (p.Lk * p.k_rs * 2 > most || p.Lk * p.v_rs * 2 > most || (p.Lp > 0 && (p.Lp * p.kp_rs * 2 > most || p.Lp * p.vp_rs * 2 > most))) return {};
-    const long heads = static_cast<long>(p.B) * p.H, units = heads * ((p.Lq + 31) / 32);
+    if (p.key_mask || p.bias || p.lse || p.cu_q || p.cos_k || p.prefix_scaled || !offsets_fit_32_bits(p)) return {};
+    const long units = static_cast<long>(p.B) * p.H * ((p.Lq + 31) / 32);
     const int nb = key_blocks(p);
     const bool masked = p.mask_mode != MI_MASK_NONE;
-    if (masked && (units > 4L * n_cu || (p.window > 0 && units > 3L * n_cu && D >= 80 && D <= 112))) return {};
     if (units <= n_cu) return {1, kMaxWaves};
     if (units <= 2L * n_cu) return {2, kMaxWaves};
-    if (units <= 4L * n_cu) {
-        if (D <= 64 && nb >= 48) return {2, kMaxWaves};
-        return {4, nb <= (D <= 64 ? 6 : 8) ? 4 : kMaxWaves};
-    }
-    const SmallPlan whole{4, 4};
-    if (D == 160) return whole;
-    const bool long_keys = D == 80 || (D == 96 && nb <= 64) || (D == 112 && nb <= 32);
-    if (heads * ((p.Lq + 255) / 256) < n_cu) return nb <= (D <= 64 ? 6 : 8) || (long_keys && nb <= (D == 80 ? 64 : 24)) ? whole : SmallPlan{};
-    return long_keys && nb > 10 ? whole : SmallPlan{};
+    if (units > 4L * n_cu) return {};
+    if (!masked) return D == 64 && nb >= 48 ? SmallPlan{2, kMaxWaves} : SmallPlan{};
+    if (p.window > 0 && units > 3L * n_cu && D >= 80 && D <= 112) return {};
+    return {4, nb <= (D <= 64 ? 6 : 8) ? 4 : kMaxWaves};
 }
 
 template <typename T, int D, int R>

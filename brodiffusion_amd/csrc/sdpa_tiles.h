@@ -373,6 +373,98 @@ __device__ __forceinline__ void write_output(const unsigned char* Os, T* o_base,
     }
 }
 
+// A lane's own query row straight from memory into the MFMA operand registers, rotated on the way (kernels whose wavefronts do
+// not share query rows): requested by `issue`, rotated and picked up by `finish`, so that a kernel can request its first keys in
+// between. Same arithmetic and single rounding as the staged forms of sdpa_common.h.
+template <typename T, int D>
+struct QRowFrags {
+    using G = HeadGeo<D>;
+    using V8 = typename Mma<T>::v8;
+    const T* row;
+    int qrow;
+    u32x4 raw[G::KC];
+    f32x4 cs[G::KC], sn[G::KC];
+    __device__ __forceinline__ void issue(const SdpaDev& p, int b, int h, int qrow_, int lh) {
+        qrow = qrow_;
+        row = static_cast<const T*>(p.q) + b * p.q_bs + h * D + static_cast<long>(qrow) * p.q_rs;
+#pragma unroll
+        for (int c = 0; c < G::KC; ++c) raw[c] = *reinterpret_cast<const u32x4*>(row + min(16 * c + 8 * lh, D - 8));
+        if (p.cos_q != nullptr && !p.rope_split) {
+#pragma unroll
+            for (int c = 0; c < G::KC; ++c) {
+                const long at = static_cast<long>(qrow) * (D / 2) + min(16 * c + 8 * lh, D - 8) / 2;
+                cs[c] = *reinterpret_cast<const f32x4*>(p.cos_q + at);
+                sn[c] = *reinterpret_cast<const f32x4*>(p.sin_q + at);
+            }
+        }
+    }
+    __device__ __forceinline__ void finish(const SdpaDev& p, int lh, V8 (&qf)[G::KC]) {
+        typedef T t4 __attribute__((ext_vector_type(4)));
+        typedef T t8 __attribute__((ext_vector_type(8)));
+        if (p.cos_q != nullptr && p.rope_split) {
+            // pairs of two halves: four elements at a time lie in one half (head_dim / 2 is a multiple of 4), their partners and
+            // table entries are fetched here
+#pragma unroll
+            for (int c = 0; c < G::KC; ++c) {
+                t8 x = __builtin_bit_cast(t8, raw[c]);
+#pragma unroll
+                for (int g = 0; g < 2; ++g) {
+                    const int d = min(16 * c + 8 * lh, D - 8) + 4 * g;
+                    const bool upper = d >= D / 2;
+                    const int pair = upper ? d - D / 2 : d;
+                    const t4 other = *reinterpret_cast<const t4*>(row + (upper ? pair : d + D / 2));
+                    const f32x4 c4 = *reinterpret_cast<const f32x4*>(p.cos_q + static_cast<long>(qrow) * (D / 2) + pair);
+                    const f32x4 s4 = *reinterpret_cast<const f32x4*>(p.sin_q + static_cast<long>(qrow) * (D / 2) + pair);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float own = static_cast<float>(x[4 * g + e]), oth = static_cast<float>(other[e]);
+                        const float re = rope_re(own, oth, c4[e], s4[e]), im = rope_im(oth, own, c4[e], s4[e]);
+                        x[4 * g + e] = static_cast<T>(upper ? im : re);
+                    }
+                }
+                raw[c] = __builtin_bit_cast(u32x4, x);
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < G::KC; ++c) {
+            u32x4 v = raw[c];
+            if (p.cos_q != nullptr && !p.rope_split) v = rope_chunk<T>(v, cs[c], sn[c]);
+            // (the pad of the head dimension: the upper lane half of the last fragment)
+            if (G::DK > D && c == G::KC - 1 && lh) v = u32x4{0, 0, 0, 0};
+            qf[c] = __builtin_bit_cast(V8, v);
+        }
+    }
+};
+
+// Row offsets inside K, V and the cached prefix fit 32 bits (kernels that add a 32-bit lane offset to a base per head).
+inline bool offsets_fit_32_bits(const SdpaDev& p) {
+    const long most = (1L << 31) - 1;
+    return p.Lk * p.k_rs * 2 <= most && p.Lk * p.v_rs * 2 <= most && (p.Lp == 0 || (p.Lp * p.kp_rs * 2 <= most && p.Lp * p.vp_rs * 2 <= most));
+}
+
+// Keys and values as panels of 32 keys x 64 bytes (32 head-dim elements): what sdpa_small.hip and sdpa_flow.hip keep in LDS. A DMA
+// instruction deposits 16 keys x 64 bytes (lane: key lane / 4, 16-byte piece lane % 4), and piece c of key k lies at position
+// c ^ (k / 4) % 4, which puts the same piece of 16 consecutive keys (K reads) on all banks and leaves the V transpose reads (4 keys
+// x 64 bytes) on theirs. Read offsets inside a panel of K (fragment c of 16 elements: panel c / 2) and of V (fragment of 16 keys
+// c4 of a block and panel vb: + 1024 c4, two halves); 245 and 209 of the 256 bytes per clock that an LDS serves.
+struct PanelReads {
+    unsigned k[2], v[2];
+    __device__ __forceinline__ explicit PanelReads(int lane) {
+        const int lq = lane & 31, lh = lane >> 5, trow = (lane & 15) >> 2, j4 = lane & 3, g1 = (lane >> 4) & 1;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            k[i] = lq * 64 + (((2 * i + lh) ^ ((lq >> 2) & 3)) << 4);
+            v[i] = (4 * lh + 8 * i + trow) * 64 + (((2 * g1 + (j4 >> 1)) ^ (lh + 2 * i)) << 4) + 8 * (j4 & 1);
+        }
+    }
+    template <typename T>
+    __device__ __forceinline__ typename Mma<T>::v8 v_frag(const unsigned char* panel) const {
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(panel + v[0]));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(panel + v[1]));
+        return __builtin_bit_cast(typename Mma<T>::v8, s16x8(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7)));
+    }
+};
+
 constexpr int kThreads8 = 512;
 template <int D> constexpr int lds_bytes_8() {
     using G = HeadGeo<D>;

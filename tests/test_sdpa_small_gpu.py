@@ -29,18 +29,6 @@ def test_rows_and_keys(oracle, dtype, d, H, Lq, Lk):
     assert_close(oracle.sdpa(q, k, v, H, rows=rows)[rows], to_np(out)[rows], dtype, f"{H} x {Lq} rows, {Lk} keys")
 
 
-# past four units per compute unit: wavefronts that have all keys of their rows (160 always; 80 with keys that the short-key kernel
-# does not take; the others below one 256-row tile per compute unit)
-@pytest.mark.parametrize("dtype,d,H,Lq,Lk", [("fp16", 160, 17, 1953, 300), ("fp16", 160, 24, 2800, 33), ("fp16", 80, 24, 2800, 353),
-                                             ("bf16", 96, 24, 2800, 353), ("bf16", 112, 24, 2800, 353), ("bf16", 128, 17, 2047, 250),
-                                             ("bf16", 72, 17, 2047, 77), ("fp16", 40, 17, 2047, 190)])
-def test_whole_rows(oracle, dtype, d, H, Lq, Lk):
-    q, k, v = randn(9611, (Lq, H * d), dtype), randn(9612, (Lk, H * d), dtype), randn(9613, (Lk, H * d), dtype)
-    out = bd.sdpa_forward(to_dev(q, dtype), to_dev(k, dtype), to_dev(v, dtype), H)
-    rows = sampled(Lq)
-    assert_close(oracle.sdpa(q, k, v, H, rows=rows)[rows], to_np(out)[rows], dtype, f"{H} x {Lq} rows, {Lk} keys")
-
-
 @pytest.mark.parametrize("dtype,d", DIMS)
 @pytest.mark.parametrize("H,Lq", [(3, 40), (9, 993), (16, 1285)])
 @pytest.mark.parametrize("Lp,Lk", [(1, 64), (31, 1), (33, 130), (64, 33), (300, 95)])
