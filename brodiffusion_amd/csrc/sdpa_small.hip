@@ -12,11 +12,14 @@
 //   * The fragments of a block are all read into registers before it is multiplied. Then its LDS is free, and the next block's
 //     DMA runs under the products and the softmax of this one: one buffer, no ring. (Two and three buffers measured the same;
 //     a small footprint lets more wavefronts in.)
-// What bounds it: the latency of a block's DMA per step.
+//   * The parts meet in LDS scaled already: a wavefront first learns the maxima and sums of the others (256 B each), scales its own
+//     registers and writes them, so that the last pass is loads and additions, in straight code for its number of parts.
+// What bounds it: a chain of latencies. Of 9500 clocks of a work group of 64 x 160: 1300 to the first request, 2200 until its data are in
+// LDS, 1600 for the one block, 1900 for scaling and writing the parts, 1600 for their sum and the write-out (4400 before it was straight).
 // Measured (fp16, 8 heads; before: the 128-row kernel, for 80 in pairs of tiles, for 40 and 72 the 256-row kernels), us:
-//   self, tokens x head_dim: 64 x 160 8.5 -> 6.1, 256 x 160 14.5 -> 8.0, 1024 x 160 37.3 -> 16.6; 512 x 80 14.4 -> 6.9, 2048 x 80
-//   39.7 -> 25.0; 1024 x 40 18.0 -> 9.0, 2048 x 40 31 -> 18.4; 16 heads of 72, 1024 23.3 -> 14.6; 24 of 128, 512 16.9 -> 11.3
-//   77 keys, queries x head_dim: 64 x 160 10.7 -> 6.6, 1024 x 80 8.8 -> 5.3, 4096 x 40 8.1 -> 6.0
+//   self, tokens x head_dim: 64 x 160 8.5 -> 5.0, 256 x 160 14.6 -> 7.0, 1024 x 160 37.4 -> 15.4; 512 x 80 14.4 -> 6.9, 2048 x 80
+//   39.8 -> 22.2; 1024 x 40 18.1 -> 8.5
+//   77 keys, queries x head_dim: 64 x 160 10.7 -> 5.7, 1024 x 80 8.9 -> 4.8, 4096 x 40 8.1 -> 6.3
 #include "sdpa_tiles.h"
 
 namespace mi {
@@ -34,11 +37,26 @@ template <int D> struct SmallGeo {
     static constexpr int PANEL = kKB * 64;                      // bytes of 32 keys of a panel
     static constexpr int OPER = NP * PANEL, BLOCK = 2 * OPER;   // K or V of a block; both
     static constexpr int P_STRIDE = D * 4 + 16;                 // bytes of one row of a partial output
-    static constexpr int PART = 32 * P_STRIDE + 2 * 32 * 4;     // a wavefront's partial output, maxima and denominators
+    static constexpr int PART = 32 * P_STRIDE;                  // a wavefront's part of the output
 };
 
-template <typename T, int D, int R>
-__global__ void __launch_bounds__(64 * kMaxWaves, D <= 64 ? 4 : D <= 80 ? 3 : 2) sdpa_small_kernel(const SdpaDev p, int S) {
+// What the unmasked kernel needs, side by side: read one by one from the launch view, at ten places of the prologue, the arguments of a
+// short call were seven scalar-load latencies in a row in front of its first key (64 x 160, with the straight sum: 6.7 -> 5.0 us).
+struct SmallArgs {
+    const void* q; const void* k; const void* v; const void* kp; const void* vp; void* o;
+    const int* kv_valid_len; const float* cos_q; const float* sin_q;
+    long q_rs, q_bs, o_bs, k_bs, v_bs, kp_bs, vp_bs;                  // elements
+    unsigned k_rsb, v_rsb, kp_rsb, vp_rsb, o_rsb;                     // bytes
+    int Lq, Lk, Lp, n_blocks, n_q_tiles, H, kv_group, S, rope_split;
+    unsigned inv_tiles, inv_heads, inv_group;                         // 2^32 / divisor, rounded up (exact while dividend x divisor < 2^32)
+    float scale_log2;
+};
+struct NoMask {};
+__device__ __forceinline__ int quotient(int x, int d, unsigned inv) { return d == 1 ? x : static_cast<int>(__umulhi(static_cast<unsigned>(x), inv)); }
+
+template <typename T, int D, int R, bool MASKED>
+__global__ void __launch_bounds__(64 * kMaxWaves, D <= 64 ? 4 : D <= 80 ? 3 : 2)
+    sdpa_small_kernel(const SmallArgs p, const std::conditional_t<MASKED, SdpaDev, NoMask> mask) {
     using G = HeadGeo<D>;
     using SG = SmallGeo<D>;
     using V8 = typename Mma<T>::v8;
@@ -46,11 +64,16 @@ __global__ void __launch_bounds__(64 * kMaxWaves, D <= 64 ? 4 : D <= 80 ? 3 : 2)
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     __shared__ int red[2 * R];
 
+    // (all arguments requested here, in a few wide loads)
+    asm volatile("" : : "s"(p.q), "s"(p.k), "s"(p.v), "s"(p.q_rs), "s"(p.q_bs), "s"(p.k_bs), "s"(p.v_bs), "s"(p.k_rsb), "s"(p.v_rsb), "s"(p.Lq), "s"(p.Lk),
+                 "s"(p.n_blocks), "s"(p.n_q_tiles), "s"(p.H), "s"(p.kv_group), "s"(p.S), "s"(p.inv_tiles), "s"(p.inv_heads), "s"(p.inv_group), "s"(p.kv_valid_len),
+                 "s"(p.cos_q), "s"(p.Lp), "s"(p.o), "s"(p.o_bs), "s"(p.o_rsb), "s"(p.scale_log2));
     const int logical = logical_block(p.n_blocks);
     if (logical < 0) return;
-    const int qt = logical % p.n_q_tiles, bh = logical / p.n_q_tiles;
-    const int h = bh % p.H, b = bh / p.H;
-    const int hk = h / p.kv_group;
+    const int S = p.S;
+    const int bh = quotient(logical, p.n_q_tiles, p.inv_tiles), qt = logical - bh * p.n_q_tiles;
+    const int b = quotient(bh, p.H, p.inv_heads), h = bh - b * p.H;
+    const int hk = quotient(h, p.kv_group, p.inv_group);
     const int tid = threadIdx.x, NT = 64 * R * S;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = wave % R, s = wave / R;
@@ -66,8 +89,8 @@ __global__ void __launch_bounds__(64 * kMaxWaves, D <= 64 ? 4 : D <= 80 ? 3 : 2)
     if (p.kv_valid_len) n_keys = __builtin_amdgcn_readfirstlane(max(min(n_keys, p.kv_valid_len[b]), 0));
     int lo = 0, hi = n_keys, first_key = 0, stop_key = n_keys;
     WaveExtent we{0, 0, n_keys, n_keys};
-    if (p.mask_mode != MI_MASK_NONE) {
-        row_interval(p, b, min(q0 + 32 * r + lq, p.Lq - 1), q0 + 32 * r < p.Lq, lo, hi);
+    if constexpr (MASKED) {
+        row_interval(mask, b, min(q0 + 32 * r + lq, p.Lq - 1), q0 + 32 * r < p.Lq, lo, hi);
         we = wave_extent(lo, hi);
         first_key = we.lo_min; stop_key = we.hi_max;
         if (R > 1) {
@@ -81,7 +104,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves, D <= 64 ? 4 : D <= 80 ? 3 : 2)
         if (first_key >= stop_key) first_key = stop_key = 0;
     }
     const int n_pre = min(p.Lp, stop_key), n_fresh = max(stop_key - p.Lp, 0);     // keys of the two segments up to the last visible one
-    const int pre0 = first_key / kKB, fresh0 = max(first_key - p.Lp, 0) / kKB;
+    const int pre0 = MASKED ? first_key / kKB : 0, fresh0 = MASKED ? max(first_key - p.Lp, 0) / kKB : 0;
     const int pre_blocks = max((n_pre + kKB - 1) / kKB - pre0, 0);
     const int n_blocks = pre_blocks + (n_fresh + kKB - 1) / kKB - fresh0;      // this wavefront takes blocks s, s + S, ...
 
@@ -98,9 +121,10 @@ __global__ void __launch_bounds__(64 * kMaxWaves, D <= 64 ? 4 : D <= 80 ? 3 : 2)
         for (int i = 0; i < PAIRS; ++i) {
             const int pair = r * PAIRS + i, op = pair >> 1, g = pair & 1;
             const void* const t = op ? (pre ? p.vp : p.v) : (pre ? p.kp : p.k);
-            const long bs = op ? (pre ? p.vp_bs : p.v_bs) : (pre ? p.kp_bs : p.k_bs), rs = op ? (pre ? p.vp_rs : p.v_rs) : (pre ? p.kp_rs : p.k_rs);
+            const long bs = op ? (pre ? p.vp_bs : p.v_bs) : (pre ? p.kp_bs : p.k_bs);
+            const unsigned rsb = op ? (pre ? p.vp_rsb : p.v_rsb) : (pre ? p.kp_rsb : p.k_rsb);
             const unsigned char* const base = reinterpret_cast<const unsigned char*>(static_cast<const T*>(t) + b * bs + hk * D);
-            const unsigned off = static_cast<unsigned>(min(row0 + 16 * g + prow, last)) * (static_cast<unsigned>(rs) * 2u) + static_cast<unsigned>(pch) * 16u;
+            const unsigned off = static_cast<unsigned>(min(row0 + 16 * g + prow, last)) * rsb + static_cast<unsigned>(pch) * 16u;
             const unsigned dst = lds_base + s * SG::BLOCK + op * SG::OPER + g * 1024;
             // (inline assembly: for the builtin the compiler would wait for the load in front of every later LDS read; the LDS base
             //  travels in m0, and the s_nop is the wait state an LDS-DMA instruction needs behind a write of m0)
@@ -132,7 +156,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves, D <= 64 ? 4 : D <= 80 ? 3 : 2)
         const bool pre = blk < pre_blocks;
         const int row0 = (pre ? pre0 + blk : fresh0 + blk - pre_blocks) * kKB, j0 = pre ? row0 : p.Lp + row0;
         const int rows = (pre ? n_pre : n_fresh) - row0;      // keys of the block
-        const bool mine = blk < n_blocks && j0 < we.hi_max && j0 + kKB > we.lo_min;
+        const bool mine = blk < n_blocks && (!MASKED || (j0 < we.hi_max && j0 + kKB > we.lo_min));
         const unsigned char* const buf = smem + s * SG::BLOCK;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         if (R > 1) __syncthreads();
@@ -158,7 +182,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves, D <= 64 ? 4 : D <= 80 ? 3 : 2)
                 if (G::DK > D && c == G::KC - 1) a &= pad_keep;
                 sacc = Mma<T>::run(__builtin_bit_cast(V8, a), qf[c], sacc);
             }
-            if (j0 < we.lo_max || j0 + min(rows, kKB) > we.hi_min || rows < kKB) {
+            if (rows < kKB || (MASKED && (j0 < we.lo_max || j0 + kKB > we.hi_min))) {
                 const int x0 = j0 + 4 * lh - lo, top = min(hi, j0 + rows) - 1 - lo;
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
@@ -220,20 +244,41 @@ __global__ void __launch_bounds__(64 * kMaxWaves, D <= 64 ? 4 : D <= 80 ? 3 : 2)
                 for (int vb = 0; vb < G::VB; ++vb) oacc[vb] = Mma<T>::run(vf[c4][vb], pf[c4], oacc[vb]);
         }
     }
-    __syncthreads();     // the blocks are used up
-    const float l_tot = exchange_sum(l);
+    float l_tot = exchange_sum(l);
     T* const o_base = static_cast<T*>(p.o) + b * p.o_bs + h * D;
     if (S == 1) {
         // every wavefront has all keys of its rows
+        __syncthreads();     // the blocks are used up
         stage_output<T, D>(smem, 32 * r + lq, lh, oacc, row_inverse(l_tot));
         __syncthreads();
-        write_output<T, D, 64 * R>(smem, o_base, p.o_rs, q0, p.Lq, 32 * R, tid);
+        write_output<T, D, 64 * R>(smem, o_base, static_cast<long>(p.o_rsb / 2), q0, p.Lq, 32 * R, tid);
         return;
     }
-    // ── partial outputs, maxima and denominators to LDS, FP32; then every thread merges 16-byte pieces of output rows ──
+    // ── merge: maxima and denominators first, so that every wavefront scales its own part by 2^(maximum - row's maximum) / row's
+    //    denominator; then the parts, FP32, whose sum is the result. (Merged piece by piece from unscaled parts, with the weights
+    //    formed anew for each, this took as long as all the rest of a short call.) ──
+    float* const stat = reinterpret_cast<float*>(smem + S * max(SG::BLOCK, R * SG::PART));      // [s][r][maximum, denominator][32]
+    if (lh == 0) {
+        stat[(s * R + r) * 64 + lq] = m;
+        stat[(s * R + r) * 64 + 32 + lq] = l_tot;
+    }
+    __syncthreads();         // (also: the blocks are used up)
+    float ms[kMaxWaves / R], ls[kMaxWaves / R];
+#pragma unroll
+    for (int k = 0; k < kMaxWaves / R; ++k) {
+        ms[k] = k < S ? stat[(k * R + r) * 64 + lq] : kNegInf;
+        ls[k] = k < S ? stat[(k * R + r) * 64 + 32 + lq] : 0.f;
+    }
+    float top = ms[0];
+#pragma unroll
+    for (int k = 1; k < kMaxWaves / R; ++k) top = fmaxf(top, ms[k]);
+    const float topc = top == kNegInf ? 0.f : top * cl2;
+    float lsum = 0.f;
+#pragma unroll
+    for (int k = 0; k < kMaxWaves / R; ++k) lsum = __builtin_fmaf(__builtin_amdgcn_exp2f(ms[k] * cl2 - topc), ls[k], lsum);     // 0 from -inf
+    const float factor = __builtin_amdgcn_exp2f(m * cl2 - topc) * row_inverse(lsum);
     {
-        unsigned char* const part = smem + (s * R + r) * SG::PART;
-        unsigned char* const row = part + lq * SG::P_STRIDE;
+        unsigned char* const row = smem + (s * R + r) * SG::PART + lq * SG::P_STRIDE;
 #pragma unroll
         for (int vb = 0; vb < G::VB; ++vb)
 #pragma unroll
@@ -241,45 +286,39 @@ __global__ void __launch_bounds__(64 * kMaxWaves, D <= 64 ? 4 : D <= 80 ? 3 : 2)
                 const int d0 = 32 * vb + 8 * bb + 4 * lh;
                 if (32 * vb + 8 * bb < D) {
                     const f32x16 acc = oacc[vb];
-                    *reinterpret_cast<f32x4*>(row + d0 * 4) = f32x4{acc[4 * bb], acc[4 * bb + 1], acc[4 * bb + 2], acc[4 * bb + 3]};
+                    *reinterpret_cast<f32x4*>(row + d0 * 4) = f32x4{acc[4 * bb] * factor, acc[4 * bb + 1] * factor, acc[4 * bb + 2] * factor, acc[4 * bb + 3] * factor};
                 }
             }
-        float* const stat = reinterpret_cast<float*>(part + 32 * SG::P_STRIDE);
-        if (lh == 0) { stat[lq] = m; stat[32 + lq] = l_tot; }
     }
     __syncthreads();
-    for (int idx = tid; idx < 32 * R * G::CPR; idx += NT) {
-        const int row = idx / G::CPR, cc = idx - row * G::CPR;
-        if (q0 + row >= p.Lq) break;
-        const unsigned char* const part = smem + (row >> 5) * SG::PART;
-        const int lr = row & 31;
-        float mm = kNegInf;
-        for (int k = 0; k < S; ++k) mm = fmaxf(mm, reinterpret_cast<const float*>(part + k * R * SG::PART + 32 * SG::P_STRIDE)[lr]);
-        const float mmc = mm == kNegInf ? 0.f : mm * cl2;
-        float lsum = 0.f;
-        f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = {0.f, 0.f, 0.f, 0.f};
-        for (int k = 0; k < S; ++k) {
-            const unsigned char* const pk = part + k * R * SG::PART;
-            const float* const stat = reinterpret_cast<const float*>(pk + 32 * SG::P_STRIDE);
-            const float w = __builtin_amdgcn_exp2f(stat[lr] * cl2 - mmc);
-            lsum = __builtin_fmaf(w, stat[32 + lr], lsum);
-            const f32x4 a = *reinterpret_cast<const f32x4*>(pk + lr * SG::P_STRIDE + cc * 32);
-            const f32x4 c = *reinterpret_cast<const f32x4*>(pk + lr * SG::P_STRIDE + cc * 32 + 16);
+    // (one straight piece of code per number of parts: with a branch per part in one loop for all, a pass took 900 clocks)
+    unsigned char* const o_rows = reinterpret_cast<unsigned char*>(o_base) + static_cast<unsigned long>(q0) * p.o_rsb;
+    const int n_rows = min(p.Lq - q0, 32 * R);
+    auto sum_parts = [&](auto count) {
+        constexpr int N = decltype(count)::value;
+        for (int idx = tid; idx < n_rows * G::CPR; idx += NT) {
+            const unsigned row = static_cast<unsigned>(idx) / G::CPR, cc = static_cast<unsigned>(idx) % G::CPR;
+            const unsigned char* const part = smem + (row >> 5) * SG::PART + (row & 31) * SG::P_STRIDE + cc * 32;
+            f32x4 lo[N], hi[N];
+#pragma unroll
+            for (int k = 0; k < N; ++k) {
+                lo[k] = *reinterpret_cast<const f32x4*>(part + k * R * SG::PART);
+                hi[k] = *reinterpret_cast<const f32x4*>(part + k * R * SG::PART + 16);
+            }
+#pragma unroll
+            for (int k = 1; k < N; ++k) { lo[0] += lo[k]; hi[0] += hi[k]; }
+            t8 out;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                lo[e] = __builtin_fmaf(w, a[e], lo[e]);
-                hi[e] = __builtin_fmaf(w, c[e], hi[e]);
+                out[e] = static_cast<T>(lo[0][e]);
+                out[4 + e] = static_cast<T>(hi[0][e]);
             }
+            *reinterpret_cast<t8*>(o_rows + static_cast<unsigned long>(row) * p.o_rsb + cc * 16) = out;
         }
-        const float inv = row_inverse(lsum);
-        t8 out;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            out[e] = static_cast<T>(lo[e] * inv);
-            out[4 + e] = static_cast<T>(hi[e] * inv);
-        }
-        *reinterpret_cast<t8*>(o_base + static_cast<long>(q0 + row) * p.o_rs + cc * 8) = out;
-    }
+    };
+    [&]<int... I>(std::integer_sequence<int, I...>) {
+        ([&] { if (S == I + 2) sum_parts(std::integral_constant<int, I + 2>{}); }(), ...);
+    }(std::make_integer_sequence<int, kMaxWaves / R - 1>{});
 }
 
 // 32-key blocks of a call (those of the prefix and of the fresh keys apart)
@@ -301,7 +340,7 @@ int key_blocks(const SdpaDev& p) { return (p.Lp + kKB - 1) / kKB + (p.Lk - p.Lp 
 //                    head_dim 64), then two: 72, 768 units, 5 blocks 7.4 and 8.2, 8 blocks 9.2 and 9.5, 16 blocks 14.1 and 13.0
 struct SmallPlan { int R = 0, waves = 0; };
 SmallPlan plan_small(const SdpaDev& p, int D, int n_cu) {
-    if (p.key_mask || p.bias || p.lse || p.cu_q || p.cos_k || p.prefix_scaled || !offsets_fit_32_bits(p)) return {};
+    if (p.key_mask || p.bias || p.lse || p.cu_q || p.cos_k || p.prefix_scaled || !offsets_fit_32_bits(p) || p.o_rs < 0 || p.o_rs >= (1L << 30)) return {};
     const long units = static_cast<long>(p.B) * p.H * ((p.Lq + 31) / 32);
     const int nb = key_blocks(p);
     const bool masked = p.mask_mode != MI_MASK_NONE;
@@ -313,17 +352,29 @@ SmallPlan plan_small(const SdpaDev& p, int D, int n_cu) {
     return {4, nb <= (D <= 64 ? 6 : 8) ? 4 : kMaxWaves};
 }
 
-template <typename T, int D, int R>
-int launch_small(SdpaDev p, int most_waves, hipStream_t stream) {
+template <typename T, int D, int R, bool MASKED>
+int launch_small(const SdpaDev& p, int most_waves, hipStream_t stream) {
     using SG = SmallGeo<D>;
     const int n_kb = key_blocks(p);
-    int S = max(1, min(min(n_kb, most_waves / R), kMaxLds / max(SG::BLOCK, R * SG::PART)));
+    int S = max(1, min(min(n_kb, most_waves / R), kMaxLds / (max(SG::BLOCK, R * SG::PART) + 256 * R)));
     const int steps = (n_kb + S - 1) / S;
     S = max(1, (n_kb + steps - 1) / max(steps, 1));      // as few wavefronts as take that many steps
-    const int lds = S == 1 ? max(SG::BLOCK, 32 * R * HeadGeo<D>::O_STRIDE) : S * max(SG::BLOCK, R * SG::PART);
-    p.n_q_tiles = (p.Lq + 32 * R - 1) / (32 * R);
-    p.n_blocks = p.B * p.H * p.n_q_tiles;
-    hipLaunchKernelGGL((sdpa_small_kernel<T, D, R>), dim3((p.n_blocks + 7) / 8 * 8), dim3(64 * R * S), lds, stream, p, S);
+    const int lds = S == 1 ? max(SG::BLOCK, 32 * R * HeadGeo<D>::O_STRIDE) : S * (max(SG::BLOCK, R * SG::PART) + 256 * R);
+    SmallArgs a{};
+    a.q = p.q; a.k = p.k; a.v = p.v; a.kp = p.kp; a.vp = p.vp; a.o = p.o;
+    a.kv_valid_len = p.kv_valid_len; a.cos_q = p.cos_q; a.sin_q = p.sin_q; a.rope_split = p.rope_split;
+    a.q_rs = p.q_rs; a.q_bs = p.q_bs; a.o_bs = p.o_bs; a.k_bs = p.k_bs; a.v_bs = p.v_bs; a.kp_bs = p.kp_bs; a.vp_bs = p.vp_bs;
+    a.k_rsb = static_cast<unsigned>(p.k_rs) * 2u; a.v_rsb = static_cast<unsigned>(p.v_rs) * 2u;
+    a.o_rsb = static_cast<unsigned>(p.o_rs) * 2u;
+    a.kp_rsb = static_cast<unsigned>(p.kp_rs) * 2u; a.vp_rsb = static_cast<unsigned>(p.vp_rs) * 2u;
+    a.Lq = p.Lq; a.Lk = p.Lk; a.Lp = p.Lp; a.H = p.H; a.kv_group = p.kv_group; a.S = S; a.scale_log2 = p.scale_log2;
+    a.n_q_tiles = (p.Lq + 32 * R - 1) / (32 * R);
+    a.n_blocks = p.B * p.H * a.n_q_tiles;
+    auto inverse = [](int d) { return static_cast<unsigned>(((1ull << 32) + d - 1) / static_cast<unsigned>(d)); };      // (not used for 1)
+    a.inv_tiles = inverse(a.n_q_tiles); a.inv_heads = inverse(a.H); a.inv_group = inverse(a.kv_group);
+    const dim3 grid((a.n_blocks + 7) / 8 * 8), block(64 * R * S);
+    if constexpr (MASKED) hipLaunchKernelGGL((sdpa_small_kernel<T, D, R, true>), grid, block, lds, stream, a, p);
+    else hipLaunchKernelGGL((sdpa_small_kernel<T, D, R, false>), grid, block, lds, stream, a, NoMask{});
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail("sdpa_fwd launch: %s", hipGetErrorString(e));
     return 0;
@@ -331,10 +382,11 @@ int launch_small(SdpaDev p, int most_waves, hipStream_t stream) {
 
 template <typename T, int D>
 int launch_small_r(const SdpaDev& p, const SmallPlan& plan, hipStream_t stream) {
+    if (p.mask_mode == MI_MASK_NONE) return plan.R == 1 ? launch_small<T, D, 1, false>(p, plan.waves, stream) : launch_small<T, D, 2, false>(p, plan.waves, stream);
     switch (plan.R) {
-        case 1: return launch_small<T, D, 1>(p, plan.waves, stream);
-        case 2: return launch_small<T, D, 2>(p, plan.waves, stream);
-        default: return launch_small<T, D, 4>(p, plan.waves, stream);
+        case 1: return launch_small<T, D, 1, true>(p, plan.waves, stream);
+        case 2: return launch_small<T, D, 2, true>(p, plan.waves, stream);
+        default: return launch_small<T, D, 4, true>(p, plan.waves, stream);
     }
 }
 

@@ -384,7 +384,9 @@ struct QRowFrags {
     int qrow;
     u32x4 raw[G::KC];
     f32x4 cs[G::KC], sn[G::KC];
-    __device__ __forceinline__ void issue(const SdpaDev& p, int b, int h, int qrow_, int lh) {
+    // (P: SdpaDev, or kernel arguments with the same names for Q and its tables)
+    template <typename P>
+    __device__ __forceinline__ void issue(const P& p, int b, int h, int qrow_, int lh) {
         qrow = qrow_;
         row = static_cast<const T*>(p.q) + b * p.q_bs + h * D + static_cast<long>(qrow) * p.q_rs;
 #pragma unroll
@@ -398,7 +400,8 @@ struct QRowFrags {
             }
         }
     }
-    __device__ __forceinline__ void finish(const SdpaDev& p, int lh, V8 (&qf)[G::KC]) {
+    template <typename P>
+    __device__ __forceinline__ void finish(const P& p, int lh, V8 (&qf)[G::KC]) {
         typedef T t4 __attribute__((ext_vector_type(4)));
         typedef T t8 __attribute__((ext_vector_type(8)));
         if (p.cos_q != nullptr && p.rope_split) {
