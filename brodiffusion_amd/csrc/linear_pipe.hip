@@ -18,9 +18,14 @@
 // on an otherwise empty compute unit, 0.4 dealt out. The accumulation order is the same in every form (and in linear_dma.hip):
 // a problem gives the same bits whichever one takes it, alone or in a launch with others.
 //
-// Measured (fp16 / bf16, one launch; before: 64 x 64 tiles through registers, one step ahead): 4096 x 1152 x 1152 30 -> 19 us,
-// three of them 90 -> 45; 1024 x 2240 x 2240 30 -> 18, three 90 -> 38; 2048 x 640 x 640 8.4 -> 6.7 (INT8 weights 11.5 -> 7.5);
-// 128 x 1280 x 1280 8.2 -> 6.0; GEGLU 3072 x 640 -> 2 x 2560 39 -> 33, INT8 54 -> 37.
+// Around the steps, a work group's fixed part (clocks of a 128 x 128 tile of 35 steps, 32 000 in all; before -> now): to the first DMA
+// instruction 1900 -> 1250 (PipeArgs), first stage landed 2900, bias and last barrier 950 -> 390 (the bias is requested ahead of the
+// loop), tile staged 1000, stored 1300 -> 570 (all pieces read before the first is stored).
+//
+// Measured (fp16 / bf16, one launch, us; first: 64 x 64 tiles through registers, one step ahead; then: this pipeline with the fixed part
+// as it was; now): 4096 x 1152 x 1152 30 / 18.2 / 17.6; 1024 x 2240 x 2240 30 / 17.5 / 17.0, three of them 90 / 36.0 / 35.4;
+// 2048 x 640 x 640 8.4 / 6.9 / 6.1 (INT8 weights 11.5 / 7.8 / 6.7); 128 x 1280 x 1280 8.2 / 6.4 / 5.7; GEGLU 3072 x 640 -> 2 x 2560
+// 39 / 32.0 / 30.7; 16384 x 512 x 512 - / 15.1 / 14.3, three - / 42.3 / 37.3.
 #include <cmath>
 #include <type_traits>
 #include <utility>
@@ -32,7 +37,27 @@ namespace gemm {
 namespace {
 
 constexpr int kBK = 64;   // contraction elements per stage
-struct PanelWidths { int w[kMaxLinearProblems]; };   // per problem: columns of tiles walked together
+// A launch as the kernel reads it. A problem is two cache lines, all of which are asked for before the first is used, and what a work
+// group divides by to find its tile comes with an inverse: with the launch view and plain divisions the first DMA instruction stood
+// behind four scalar-load latencies and four divisions (1900 clocks, 700 of them gone).
+struct alignas(64) PipeProblem {
+    const void* x; const void* w; const void* bias; void* y; const float* w_scale;
+    int M, N, K, panel_tiles, width, last_width, n_panels;            // tiles of a whole panel, columns of tiles of a panel and of the last one
+    unsigned ldx_b, ldw_b, inv_panel, inv_width, inv_last;            // row strides in bytes; floor(2^32 / divisor)
+    long ldy_b;
+};
+struct PipeArgs {
+    PipeProblem p[kMaxLinearProblems];
+    int first[kMaxLinearProblems];       // first tile of a problem
+    int n_tiles, chunk;
+};
+// x / d and x % d for x < 2^32; inv = floor(2^32 / d), one less for d = 1: the estimate is at most one short
+struct DivMod { int q, r; };
+__device__ __forceinline__ DivMod div_mod(int x, int d, unsigned inv) {
+    unsigned q = __umulhi(static_cast<unsigned>(x), inv), r = static_cast<unsigned>(x) - q * d;
+    if (r >= static_cast<unsigned>(d)) { ++q; r -= d; }
+    return {static_cast<int>(q), static_cast<int>(r)};
+}
 
 template <typename T, bool W8, bool GEGLU, int WM, int WN, int TM, int TN, int S>
 struct PipeGeo {
@@ -80,7 +105,7 @@ template <> __device__ __forceinline__ bf16x8 widen<__bf16>(u32x2 raw) {
 }
 
 template <typename T, bool W8, bool GEGLU, int WM, int WN, int TM, int TN, int S>
-__global__ void __launch_bounds__(64 * WM * WN, 2) linear_pipe_kernel(const LinearBatch batch, int n_problems, const PanelWidths panels) {
+__global__ void __launch_bounds__(64 * WM * WN, 2) linear_pipe_kernel(const PipeArgs args) {
     using G = PipeGeo<T, W8, GEGLU, WM, WN, TM, TN, S>;
     using M = Mma<T>;
     using V8 = typename M::v8;
@@ -92,20 +117,17 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) linear_pipe_kernel(const Line
     // contiguous run of it. A problem's tiles are numbered panel by panel (panels.w columns of tiles, row by row), so that a
     // run is about as many rows of X as rows of W: what a run touches comes from the last-level cache, which serves a
     // compute unit 28 bytes per ns when all of them ask, once, and from then on from the L2 at 95.
-    auto tiles_of = [&](int i) { return ((batch.p[i].M + BM - 1) / BM) * ((batch.p[i].N + BN_OUT - 1) / BN_OUT); };
-    const int n0_tiles = tiles_of(0), n1_tiles = n_problems > 1 ? tiles_of(1) : 0, n2_tiles = n_problems > 2 ? tiles_of(2) : 0;
-    const int n_tiles = n0_tiles + n1_tiles + n2_tiles;
-    const int chunk = (n_tiles + 7) >> 3;
-    int tile = (static_cast<int>(blockIdx.x) & 7) * chunk + (static_cast<int>(blockIdx.x) >> 3);
-    if (tile >= n_tiles) return;
-    int pi = 0;
-    if (tile >= n0_tiles) { tile -= n0_tiles; pi = 1; if (tile >= n1_tiles) { tile -= n1_tiles; pi = 2; } }
-    const LinearProblem& p = batch.p[__builtin_amdgcn_readfirstlane(pi)];
-    const int tiles_n = (p.N + BN_OUT - 1) / BN_OUT, tiles_m = (p.M + BM - 1) / BM;
-    const int pw = panels.w[__builtin_amdgcn_readfirstlane(pi)];
-    const int panel = tile / (tiles_m * pw), in_panel = tile - panel * tiles_m * pw;
-    const int w_here = min(pw, tiles_n - panel * pw);
-    const int m0 = (in_panel / w_here) * BM, n0 = (panel * pw + in_panel % w_here) * BN_OUT;
+#pragma unroll
+    for (int i = 0; i < kMaxLinearProblems; ++i) asm volatile("" : : "s"(args.p[i].x), "s"(args.p[i].ldx_b));
+    asm volatile("" : : "s"(args.first[1]), "s"(args.first[2]), "s"(args.n_tiles), "s"(args.chunk));
+    int tile = (static_cast<int>(blockIdx.x) & 7) * args.chunk + (static_cast<int>(blockIdx.x) >> 3);
+    if (tile >= args.n_tiles) return;
+    const int pi = (tile >= args.first[1] ? 1 : 0) + (tile >= args.first[2] ? 1 : 0);
+    const PipeProblem& p = args.p[pi];
+    const DivMod in_problem = div_mod(tile - args.first[pi], p.panel_tiles, p.inv_panel);
+    const bool last = in_problem.q == p.n_panels - 1;
+    const DivMod in_panel = div_mod(in_problem.r, last ? p.last_width : p.width, last ? p.inv_last : p.inv_width);
+    const int m0 = in_panel.q * BM, n0 = (in_problem.q * p.width + in_panel.r) * BN_OUT;
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -119,13 +141,13 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) linear_pipe_kernel(const Line
         return reinterpret_cast<const unsigned char*>(static_cast<unsigned long>(hi) << 32 | lo);
     };
     // ── DMA duty: X instructions wave + NW m (8 rows of 128 bytes each), W instructions likewise (INT8: 16 rows of 64) ──
-    const unsigned char* xg = uniform(static_cast<const unsigned char*>(p.x) + static_cast<long>(m0) * p.ldx * 2);
-    const unsigned char* wg = uniform(static_cast<const unsigned char*>(p.w) + (GEGLU ? 0L : static_cast<long>(n0) * p.ldw * (W8 ? 1 : 2)));
+    const unsigned char* xg = uniform(static_cast<const unsigned char*>(p.x) + static_cast<long>(m0) * p.ldx_b);
+    const unsigned char* wg = uniform(static_cast<const unsigned char*>(p.w) + (GEGLU ? 0L : static_cast<long>(n0) * p.ldw_b));
     unsigned xoff[G::MX], woff[G::MW];
 #pragma unroll
     for (int u = 0; u < G::MX; ++u) {
         const int r = 8 * (wave + G::NW * u) + (lane >> 3);
-        xoff[u] = static_cast<unsigned>(min(r, p.M - 1 - m0)) * (static_cast<unsigned>(p.ldx) * 2u) + ((lane & 7) ^ ((r >> 1) & 7)) * 16u;
+        xoff[u] = static_cast<unsigned>(min(r, p.M - 1 - m0)) * p.ldx_b + ((lane & 7) ^ ((r >> 1) & 7)) * 16u;
     }
 #pragma unroll
     for (int u = 0; u < G::MW; ++u) {
@@ -133,7 +155,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) linear_pipe_kernel(const Line
         const unsigned piece = W8 ? (lane & 3) ^ ((r >> 2) & 3) : (lane & 7) ^ ((r >> 1) & 7);
         // GEGLU: 32-row groups of the tile alternate between the value and the gate rows of the same features
         const int row = GEGLU ? min(n0 + 32 * (r >> 6) + (r & 31), p.N - 1) + ((r >> 5) & 1) * p.N : min(r, p.N - 1 - n0);
-        woff[u] = static_cast<unsigned>(row) * (static_cast<unsigned>(p.ldw) * (W8 ? 1u : 2u)) + piece * 16u;
+        woff[u] = static_cast<unsigned>(row) * p.ldw_b + piece * 16u;
     }
     const unsigned lds_base = static_cast<unsigned>(reinterpret_cast<size_t>((__attribute__((address_space(3))) unsigned char*)lds));
     // (the LDS destination travels in m0; the s_nop is the wait state an LDS-DMA instruction needs behind a write of m0)
@@ -159,6 +181,27 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) linear_pipe_kernel(const Line
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         }
     };
+
+    // The bias (and scale) of this lane's features, requested ahead of the first DMA: behind the loop its latency was 700 to 1800 clocks.
+    // (N is a multiple of 8, so 4 features are in or out together; those past the end are not stored.)
+    typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+    const T* const bias = static_cast<const T*>(p.bias);
+    V4 braw[TN][4];
+    f32x4_a4 sraw[W8 ? TN : 1][4];
+    auto feature = [&](int a, int g) { return min(n0 + (GEGLU ? wn : wn * TN + a) * 32 + 8 * g + 4 * lh, p.N - 4) + (GEGLU ? a * p.N : 0); };
+#pragma unroll
+    for (int a = 0; a < TN; ++a)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            if constexpr (W8) sraw[a][g] = *reinterpret_cast<const f32x4_a4*>(p.w_scale + feature(a, g));
+            braw[a][g] = V4{};
+        }
+    if (bias != nullptr) {
+#pragma unroll
+        for (int a = 0; a < TN; ++a)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) braw[a][g] = *reinterpret_cast<const V4*>(bias + feature(a, g));
+    }
 
     // ── fragment reads: a stage is four chunks of 16 contraction elements, read two at a time ──
     unsigned xaddr[4], waddr[4];
@@ -270,20 +313,6 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) linear_pipe_kernel(const Line
         for (++t; t < n; ++t) step(std::false_type{}, std::false_type{}, t);
     }
 
-    // the bias of this lane's features, requested ahead of the barrier
-    const T* const bias = static_cast<const T*>(p.bias);
-    V4 braw[TN][4];
-#pragma unroll
-    for (int a = 0; a < TN; ++a)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const int feat = GEGLU ? n0 + wn * 32 + 8 * g + 4 * lh : n0 + (wn * TN + a) * 32 + 8 * g + 4 * lh;
-            const bool there = bias != nullptr && feat < p.N;
-            const V4 raw = *reinterpret_cast<const V4*>(there ? bias + feat + (GEGLU ? a * p.N : 0) : static_cast<const T*>(p.w));
-            const V4 zero = {static_cast<T>(0.f), static_cast<T>(0.f), static_cast<T>(0.f), static_cast<T>(0.f)};
-            braw[a][g] = there ? raw : zero;
-        }
-
     __syncthreads();   // the ring is used up
     // ── epilogue: acc[a][b][4g + i] is feature n0 + (wn TN + a) 32 + 8g + 4 lh + i of token m0 + (wm TM + b) 32 + lq; the tile
     //    leaves through LDS as 16-byte pieces of rows of Y ──
@@ -291,13 +320,6 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) linear_pipe_kernel(const Line
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             const int feat = wn * 32 + 8 * g + 4 * lh;
-            float sv[4] = {1.f, 1.f, 1.f, 1.f}, sg[4] = {1.f, 1.f, 1.f, 1.f};
-            if constexpr (W8) {
-                if (n0 + feat < p.N) {   // N is a multiple of 8, so the 4 features are in or out together
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) { sv[i] = p.w_scale[n0 + feat + i]; sg[i] = p.w_scale[p.N + n0 + feat + i]; }
-                }
-            }
 #pragma unroll
             for (int b = 0; b < TM; ++b) {
                     V4 o;
@@ -306,8 +328,8 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) linear_pipe_kernel(const Line
                         const float bv = static_cast<float>(braw[0][g][i]), bg = static_cast<float>(braw[1][g][i]);
                         float val, gate;
                         if constexpr (W8) {   // the two halves are rounded where the reference's 16-bit intermediate would
-                            val = static_cast<float>(static_cast<T>(scaled_acc(acc[0][b][4 * g + i], sv[i], bv)));
-                            gate = static_cast<float>(static_cast<T>(scaled_acc(acc[1][b][4 * g + i], sg[i], bg)));
+                            val = static_cast<float>(static_cast<T>(scaled_acc(acc[0][b][4 * g + i], sraw[0][g][i], bv)));
+                            gate = static_cast<float>(static_cast<T>(scaled_acc(acc[1][b][4 * g + i], sraw[1][g][i], bg)));
                         } else {
                             val = acc[0][b][4 * g + i] + bv;
                             gate = acc[1][b][4 * g + i] + bg;
@@ -323,20 +345,13 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) linear_pipe_kernel(const Line
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const int feat = (wn * TN + a) * 32 + 8 * g + 4 * lh;
-                float sc[4] = {1.f, 1.f, 1.f, 1.f};
-                if constexpr (W8) {
-                    if (n0 + feat < p.N) {
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) sc[i] = p.w_scale[n0 + feat + i];
-                    }
-                }
 #pragma unroll
                 for (int b = 0; b < TM; ++b) {
                         V4 o;
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
                             const float bv = static_cast<float>(braw[a][g][i]);
-                            if constexpr (W8) o[i] = static_cast<T>(scaled_acc(acc[a][b][4 * g + i], sc[i], bv));
+                            if constexpr (W8) o[i] = static_cast<T>(scaled_acc(acc[a][b][4 * g + i], sraw[a][g][i], bv));
                             else o[i] = static_cast<T>(acc[a][b][4 * g + i] + bv);
                         }
                         *reinterpret_cast<V4*>(lds + ((wm * TM + b) * 32 + lq) * G::OUT_ROW + feat * 2) = o;
@@ -344,28 +359,32 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) linear_pipe_kernel(const Line
             }
     }
     __syncthreads();
-    unsigned char* const yg = static_cast<unsigned char*>(p.y);
     constexpr int PPR = BN_OUT / 8;   // 16-byte pieces per staged row
+    constexpr int PIECES = BM * PPR / G::NT, RSTEP = G::NT / PPR;
+    static_assert(BM * PPR % G::NT == 0 && G::NT % PPR == 0, "the same pieces for every thread, one below the other");
+    const int row = tid / PPR, piece = tid % PPR;
+    unsigned char* const yg = static_cast<unsigned char*>(p.y) + static_cast<long>(m0 + row) * p.ldy_b + (n0 + piece * 8) * 2L;
+    u32x4 out[PIECES];
 #pragma unroll
-    for (int idx = tid; idx < BM * PPR; idx += G::NT) {
-        const int row = idx / PPR, piece = idx % PPR;
-        if (m0 + row < p.M && n0 + piece * 8 < p.N)
-            *reinterpret_cast<u32x4*>(yg + (static_cast<long>(m0 + row) * p.ldy + n0 + piece * 8) * 2) =
-                *reinterpret_cast<const u32x4*>(lds + row * G::OUT_ROW + piece * 16);
+    for (int i = 0; i < PIECES; ++i) out[i] = *reinterpret_cast<const u32x4*>(lds + (row + i * RSTEP) * G::OUT_ROW + piece * 16);
+    // (whole tiles without a branch: one per piece, each with its own read and wait, took 300 clocks a piece)
+    if (m0 + BM <= p.M && n0 + BN_OUT <= p.N) {
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) *reinterpret_cast<u32x4*>(yg + i * RSTEP * p.ldy_b) = out[i];
+    } else if (n0 + piece * 8 < p.N) {
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i)
+            if (m0 + row + i * RSTEP < p.M) *reinterpret_cast<u32x4*>(yg + i * RSTEP * p.ldy_b) = out[i];
     }
 }
 
 template <typename T, bool W8, bool GEGLU, int WM, int WN, int TM, int TN, int S>
 int launch_pipe(const LinearBatch& batch, int n_problems, hipStream_t st) {
     using G = PipeGeo<T, W8, GEGLU, WM, WN, TM, TN, S>;
+    auto tiles_m = [&](int i) { return (batch.p[i].M + G::BM - 1) / G::BM; };
+    auto tiles_n = [&](int i) { return (batch.p[i].N + G::BN_OUT - 1) / G::BN_OUT; };
     long tiles = 0;
-    for (int i = 0; i < n_problems; ++i)
-        tiles += static_cast<long>((batch.p[i].M + G::BM - 1) / G::BM) * ((batch.p[i].N + G::BN_OUT - 1) / G::BN_OUT);
-    PanelWidths panels{};
-    for (int i = 0; i < n_problems; ++i) {
-        const int tiles_n = (batch.p[i].N + G::BN_OUT - 1) / G::BN_OUT;
-        panels.w[i] = min(tiles_n, max(1, static_cast<int>(std::sqrt(static_cast<double>(tiles) / 8 * G::BM / G::BN) + 0.5)));
-    }
+    for (int i = 0; i < n_problems; ++i) tiles += static_cast<long>(tiles_m(i)) * tiles_n(i);
     if (tiles > 0x7ffffff0L) return fail("linear: problem too large for one launch");
     if (G::LDS > 64 * 1024) {
         static thread_local bool raised = false;
@@ -375,8 +394,27 @@ int launch_pipe(const LinearBatch& batch, int n_problems, hipStream_t st) {
             raised = true;
         }
     }
-    hipLaunchKernelGGL((linear_pipe_kernel<T, W8, GEGLU, WM, WN, TM, TN, S>), dim3(static_cast<unsigned>((tiles + 7) / 8 * 8)), dim3(G::NT), G::LDS, st,
-                       batch, n_problems, panels);
+    auto inverse = [](int d) { return d == 1 ? 0xffffffffu : static_cast<unsigned>((1ull << 32) / static_cast<unsigned>(d)); };
+    PipeArgs args{};
+    args.n_tiles = static_cast<int>(tiles);
+    args.chunk = (args.n_tiles + 7) / 8;
+    int first = 0;
+    for (int i = 0; i < kMaxLinearProblems; ++i) {
+        args.first[i] = i < n_problems ? first : 0x7fffffff;
+        if (i >= n_problems) continue;
+        const LinearProblem& b = batch.p[i];
+        PipeProblem& p = args.p[i];
+        p.x = b.x; p.w = b.w; p.bias = b.bias; p.y = b.y; p.w_scale = b.w_scale;
+        p.M = b.M; p.N = b.N; p.K = b.K;
+        p.ldx_b = static_cast<unsigned>(b.ldx) * 2u; p.ldw_b = static_cast<unsigned>(b.ldw) * (W8 ? 1u : 2u); p.ldy_b = b.ldy * 2;
+        p.width = min(tiles_n(i), max(1, static_cast<int>(std::sqrt(static_cast<double>(tiles) / 8 * G::BM / G::BN) + 0.5)));
+        p.n_panels = (tiles_n(i) + p.width - 1) / p.width;
+        p.last_width = tiles_n(i) - (p.n_panels - 1) * p.width;
+        p.panel_tiles = tiles_m(i) * p.width;
+        p.inv_panel = inverse(p.panel_tiles); p.inv_width = inverse(p.width); p.inv_last = inverse(p.last_width);
+        first += tiles_m(i) * tiles_n(i);
+    }
+    hipLaunchKernelGGL((linear_pipe_kernel<T, W8, GEGLU, WM, WN, TM, TN, S>), dim3(static_cast<unsigned>((tiles + 7) / 8 * 8)), dim3(G::NT), G::LDS, st, args);
     MI_HIP_CHECK(hipGetLastError());
     return 0;
 }

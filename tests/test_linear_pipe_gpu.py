@@ -90,3 +90,15 @@ def test_pipe_three_unequal_problems_in_one_launch(oracle):
     out = bd.flash_attention_qkvo_forward(x, ctx, wq, None, wk, None, wv, None, wo, None, None, H, False)
     q, k, v = bd.linear_batched(wq, None, x), bd.linear_batched(wk, None, ctx), bd.linear_batched(wv, None, ctx)
     assert torch.equal(bd.linear_batched(wo, None, bd.flash_attention_forward(q, k, v, None, H, False)), out)
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 40, 64), (300, 1288, 640), (257, 200, 1280)])
+def test_pipe_scales_start_at_any_float(oracle, M, N, K):
+    """The scales are read four at a time: rows 1 .. N of a longer scale vector (4-byte alignment), N off every tile width, no bias.
+    Same bits as from a vector of their own."""
+    x = to_dev(randn(121 + M, (M, K), "fp16"), "fp16")
+    w, s = (torch.from_numpy(a).cuda() for a in _int8(122 + N, N, K))
+    longer = torch.full((N + 2, 1), float("nan"), device="cuda")
+    longer[1:-1] = s
+    assert longer[1:-1].data_ptr() % 16 == 4
+    assert torch.equal(bd.linear_forward_batched_int8w_fp16(w, longer[1:-1], None, x), bd.linear_forward_batched_int8w_fp16(w, s, None, x))
