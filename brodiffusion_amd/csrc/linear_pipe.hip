@@ -18,14 +18,20 @@
 // on an otherwise empty compute unit, 0.4 dealt out. The accumulation order is the same in every form (and in linear_dma.hip):
 // a problem gives the same bits whichever one takes it, alone or in a launch with others.
 //
+// With NL > 0 the work group has NL further wavefronts that do nothing but load (a whole stage behind the barrier that frees its slot)
+// and the others nothing but read and multiply: an LDS-DMA instruction keeps its wavefront from issuing for 33 clocks, the products of
+// 64 contraction elements of a 32 x 32 block take 128. Steps of the small tiles become 10 to 20 % shorter, a 32 x 32 tile on one
+// multiplying wavefront possible at all.
+//
 // Around the steps, a work group's fixed part (clocks of a 128 x 128 tile of 35 steps, 32 000 in all; before -> now): to the first DMA
 // instruction 1900 -> 1250 (PipeArgs), first stage landed 2900, bias and last barrier 950 -> 390 (the bias is requested ahead of the
 // loop), tile staged 1000, stored 1300 -> 570 (all pieces read before the first is stored).
 //
 // Measured (fp16 / bf16, one launch, us; first: 64 x 64 tiles through registers, one step ahead; then: this pipeline with the fixed part
-// as it was; now): 4096 x 1152 x 1152 30 / 18.2 / 17.6; 1024 x 2240 x 2240 30 / 17.5 / 17.0, three of them 90 / 36.0 / 35.4;
-// 2048 x 640 x 640 8.4 / 6.9 / 6.1 (INT8 weights 11.5 / 7.8 / 6.7); 128 x 1280 x 1280 8.2 / 6.4 / 5.7; GEGLU 3072 x 640 -> 2 x 2560
-// 39 / 32.0 / 30.7; 16384 x 512 x 512 - / 15.1 / 14.3, three - / 42.3 / 37.3.
+// as it was; now, with the tiles that the rule below takes): 4096 x 1152 x 1152 30 / 16.9 / 14.5 to 17.3 (192 x 128 tiles; it differs
+// from GPU to GPU); 1024 x 2240 x 2240 30 / 16.3 / 16.1; 2048 x 640 x 640 8.4 / 6.9 / 6.0 (INT8 weights 11.5 / 7.8 / 6.4);
+// 128 x 1280 x 1280 8.2 / 6.4 / 4.6 (INT8 - / 8.2 / 5.7), three of them - / 6.9 / 5.7 (INT8 - / 8.7 / 6.7); 256 x 1152 x 1152 - / 6.2 / 5.0;
+// 3072 x 640 x 2560 - / 17.4 / 15.8; GEGLU 3072 x 640 -> 2 x 2560 39 / 32.0 / 29; three of 16384 x 512 x 512 - / 42.3 / 36.
 #include <cmath>
 #include <type_traits>
 #include <utility>
@@ -59,18 +65,19 @@ __device__ __forceinline__ DivMod div_mod(int x, int d, unsigned inv) {
     return {static_cast<int>(q), static_cast<int>(r)};
 }
 
-template <typename T, bool W8, bool GEGLU, int WM, int WN, int TM, int TN, int S>
+template <typename T, bool W8, bool GEGLU, int WM, int WN, int TM, int TN, int S, int NL>
 struct PipeGeo {
     static constexpr int NW = WM * WN, NT = 64 * NW;
     static constexpr int BM = WM * TM * 32, BN = WN * TN * 32;
     static constexpr int BN_OUT = GEGLU ? BN / 2 : BN;
     static constexpr int WROW = W8 ? 64 : 128;                    // bytes of a W row in a stage
     static constexpr int X_BYTES = BM * 128, W_BYTES = BN * WROW, STAGE = X_BYTES + W_BYTES;
-    static constexpr int MX = X_BYTES / 1024 / NW, MW = W_BYTES / 1024 / NW;   // DMA instructions per wavefront and stage
+    static constexpr int LW = NL ? NL : NW;                       // wavefronts that load
+    static constexpr int MX = X_BYTES / 1024 / LW, MW = W_BYTES / 1024 / LW;   // DMA instructions of such a one per stage
     static constexpr int MI = MX + MW;
     static constexpr int OUT_ROW = BN_OUT * 2 + 16;
     static constexpr int LDS = S * STAGE > BM * OUT_ROW ? S * STAGE : BM * OUT_ROW;
-    static_assert(MX * NW * 1024 == X_BYTES && MW * NW * 1024 == W_BYTES, "the same DMA duty for every wavefront");
+    static_assert(MX * LW * 1024 == X_BYTES && MW * LW * 1024 == W_BYTES, "the same DMA duty for every loading wavefront");
     static_assert(!GEGLU || TN == 2, "the GEGLU form pairs the two feature blocks of a wavefront");
     static_assert(LDS <= 160 * 1024, "LDS of a compute unit");
     static_assert((S - 1) * MI < 64, "outstanding loads fit the counter");
@@ -104,9 +111,9 @@ template <> __device__ __forceinline__ bf16x8 widen<__bf16>(u32x2 raw) {
     return __builtin_bit_cast(bf16x8, r);
 }
 
-template <typename T, bool W8, bool GEGLU, int WM, int WN, int TM, int TN, int S>
-__global__ void __launch_bounds__(64 * WM * WN, 2) linear_pipe_kernel(const PipeArgs args) {
-    using G = PipeGeo<T, W8, GEGLU, WM, WN, TM, TN, S>;
+template <typename T, bool W8, bool GEGLU, int WM, int WN, int TM, int TN, int S, int NL>
+__global__ void __launch_bounds__(64 * (WM * WN + NL), 2) linear_pipe_kernel(const PipeArgs args) {
+    using G = PipeGeo<T, W8, GEGLU, WM, WN, TM, TN, S, NL>;
     using M = Mma<T>;
     using V8 = typename M::v8;
     using V4 = typename M::v4;
@@ -134,24 +141,25 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) linear_pipe_kernel(const Pipe
     const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
     const int wm = wave % WM, wn = wave / WM;
 
+    const int lw = NL ? wave - G::NW : wave;     // (NL: the loading wavefronts come last)
     // a pointer that is the same for the whole wavefront, in scalar registers
     auto uniform = [](const unsigned char* q) {
         const unsigned long u = reinterpret_cast<unsigned long>(q);
         const unsigned lo = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(u)), hi = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(u >> 32));
         return reinterpret_cast<const unsigned char*>(static_cast<unsigned long>(hi) << 32 | lo);
     };
-    // ── DMA duty: X instructions wave + NW m (8 rows of 128 bytes each), W instructions likewise (INT8: 16 rows of 64) ──
+    // ── DMA duty: X instructions lw + LW m (8 rows of 128 bytes each), W instructions likewise (INT8: 16 rows of 64) ──
     const unsigned char* xg = uniform(static_cast<const unsigned char*>(p.x) + static_cast<long>(m0) * p.ldx_b);
     const unsigned char* wg = uniform(static_cast<const unsigned char*>(p.w) + (GEGLU ? 0L : static_cast<long>(n0) * p.ldw_b));
     unsigned xoff[G::MX], woff[G::MW];
 #pragma unroll
     for (int u = 0; u < G::MX; ++u) {
-        const int r = 8 * (wave + G::NW * u) + (lane >> 3);
+        const int r = 8 * (lw + G::LW * u) + (lane >> 3);
         xoff[u] = static_cast<unsigned>(min(r, p.M - 1 - m0)) * p.ldx_b + ((lane & 7) ^ ((r >> 1) & 7)) * 16u;
     }
 #pragma unroll
     for (int u = 0; u < G::MW; ++u) {
-        const int r = W8 ? 16 * (wave + G::NW * u) + (lane >> 2) : 8 * (wave + G::NW * u) + (lane >> 3);
+        const int r = W8 ? 16 * (lw + G::LW * u) + (lane >> 2) : 8 * (lw + G::LW * u) + (lane >> 3);
         const unsigned piece = W8 ? (lane & 3) ^ ((r >> 2) & 3) : (lane & 7) ^ ((r >> 1) & 7);
         // GEGLU: 32-row groups of the tile alternate between the value and the gate rows of the same features
         const int row = GEGLU ? min(n0 + 32 * (r >> 6) + (r & 31), p.N - 1) + ((r >> 5) & 1) * p.N : min(r, p.N - 1 - n0);
@@ -164,8 +172,8 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) linear_pipe_kernel(const Pipe
     };
     // pieces [J0, J1) of this wavefront's share of a stage; xg / wg stand on that stage
     auto dma_piece = [&](int j, unsigned slot) {
-        if (j < G::MX) dma(xoff[j < G::MX ? j : 0], xg, lds_base + slot + (wave + G::NW * j) * 1024);
-        else dma(woff[j < G::MX ? 0 : j - G::MX], wg, lds_base + slot + G::X_BYTES + (wave + G::NW * (j - G::MX)) * 1024);
+        if (j < G::MX) dma(xoff[j < G::MX ? j : 0], xg, lds_base + slot + (lw + G::LW * j) * 1024);
+        else dma(woff[j < G::MX ? 0 : j - G::MX], wg, lds_base + slot + G::X_BYTES + (lw + G::LW * (j - G::MX)) * 1024);
     };
     auto next_stage = [&]() {
         xg += kBK * 2;
@@ -287,7 +295,48 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) linear_pipe_kernel(const Pipe
         prev = cur;
         cur = nxt;
     };
-    if (n < S) {   // everything fits the ring
+    if constexpr (NL > 0) {
+        const int ahead = n < S ? n : S;
+        if (wave >= G::NW) {
+            unsigned slot = 0;
+            auto load_stage = [&]() {
+#pragma unroll
+                for (int j = 0; j < MI; ++j) dma_piece(j, slot);
+                next_stage();
+                slot = slot + G::STAGE == S * G::STAGE ? 0u : slot + G::STAGE;
+            };
+            for (int s = 0; s < ahead; ++s) load_stage();
+            if (ahead == S) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"((S - 1) * MI) : "memory");
+            else wait_barrier(ahead - 1);
+            int t = 0;
+            for (; t < n - S; ++t) {       // stage t + 1 has landed, the slot of stage t is free
+                wait_barrier(S - 2);
+                load_stage();
+            }
+            for (; t < n - 1; ++t) wait_barrier(n - 2 - t);
+            __syncthreads();
+            __syncthreads();
+            return;
+        }
+        asm volatile("s_barrier" ::: "memory");      // stage 0 has landed
+        read_half(Half0{}, 0);
+        for (int t = 0; t < n - 1; ++t) {
+            const unsigned nxt = cur + G::STAGE == S * G::STAGE ? 0u : cur + G::STAGE;
+            read_half(Half1{}, cur);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply_half(Half0{}, Half0{}, Half0{}, 0u);
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // stage t is in registers
+            read_half(Half0{}, nxt);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply_half(Half1{}, Half0{}, Half0{}, 0u);
+            __builtin_amdgcn_sched_barrier(0);
+            cur = nxt;
+        }
+        read_half(Half1{}, cur);
+        multiply_half(Half0{}, Half0{}, Half0{}, 0u);
+        multiply_half(Half1{}, Half0{}, Half0{}, 0u);
+    } else if (n < S) {   // everything fits the ring
         for (int s = 0; s < n; ++s) {
 #pragma unroll
             for (int j = 0; j < MI; ++j) dma_piece(j, s * G::STAGE);
@@ -378,9 +427,9 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) linear_pipe_kernel(const Pipe
     }
 }
 
-template <typename T, bool W8, bool GEGLU, int WM, int WN, int TM, int TN, int S>
+template <typename T, bool W8, bool GEGLU, int WM, int WN, int TM, int TN, int S, int NL>
 int launch_pipe(const LinearBatch& batch, int n_problems, hipStream_t st) {
-    using G = PipeGeo<T, W8, GEGLU, WM, WN, TM, TN, S>;
+    using G = PipeGeo<T, W8, GEGLU, WM, WN, TM, TN, S, NL>;
     auto tiles_m = [&](int i) { return (batch.p[i].M + G::BM - 1) / G::BM; };
     auto tiles_n = [&](int i) { return (batch.p[i].N + G::BN_OUT - 1) / G::BN_OUT; };
     long tiles = 0;
@@ -389,7 +438,7 @@ int launch_pipe(const LinearBatch& batch, int n_problems, hipStream_t st) {
     if (G::LDS > 64 * 1024) {
         static thread_local bool raised = false;
         if (!raised) {
-            MI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&linear_pipe_kernel<T, W8, GEGLU, WM, WN, TM, TN, S>),
+            MI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&linear_pipe_kernel<T, W8, GEGLU, WM, WN, TM, TN, S, NL>),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS));
             raised = true;
         }
@@ -414,7 +463,7 @@ int launch_pipe(const LinearBatch& batch, int n_problems, hipStream_t st) {
         p.inv_panel = inverse(p.panel_tiles); p.inv_width = inverse(p.width); p.inv_last = inverse(p.last_width);
         first += tiles_m(i) * tiles_n(i);
     }
-    hipLaunchKernelGGL((linear_pipe_kernel<T, W8, GEGLU, WM, WN, TM, TN, S>), dim3(static_cast<unsigned>((tiles + 7) / 8 * 8)), dim3(G::NT), G::LDS, st, args);
+    hipLaunchKernelGGL((linear_pipe_kernel<T, W8, GEGLU, WM, WN, TM, TN, S, NL>), dim3(static_cast<unsigned>((tiles + 7) / 8 * 8)), dim3(G::NT + 64 * NL), G::LDS, st, args);
     MI_HIP_CHECK(hipGetLastError());
     return 0;
 }
@@ -424,28 +473,36 @@ int launch_pipe(const LinearBatch& batch, int n_problems, hipStream_t st) {
 //     phi + steps lam + (m - 1) (steps tau + eps),   m = ceil(n / C) tiles on the busiest compute unit,
 // with steps = K / 64: phi what a launch of one tile per compute unit costs beyond its steps (start, first loads, write-out), lam
 // a step when the compute unit has one tile, tau and eps a step and the rest of every further tile. The constants (us) are fitted
-// to problems between 32 x 1280 x 1280 and 4096 x 6720 x 2240 on MI355X. Every form timed again on 232 problems (32 to 8192 rows, nine
-// layers of the supported models): rms error 6 to 17 % by form, 23 % for the 128 x 128 tiles of two stages and the GEGLU ones of
-// 128 tokens, whose few-tile launches are overestimated; the form taken is 0.1 (INT8 0.9, GEGLU 0.7) % slower than the fastest
-// one on average, 11 % at worst. Large tiles need fewer bytes per FLOP
-// (a step of 128 x 128 moves 32 KB for 0.5 us of a saturated compute unit), small ones fill the GPU: 128 x 1280 x 1280
-// takes 6 us with 80 tiles of 64 x 32, 8 with 20 of 128 x 64, 16 with 10 of 256 x 128; 1024 x 2240 x 2240 takes 18 us
-// with 144 tiles of 128 x 128, 24 with 288 of 128 x 64, 50 with 36 of 256 x 256.
+// on MI355X to 350 problems (32 to 16384 rows, eleven layers of the supported models, one or three of a launch; 16-bit: jointly with a
+// term for the bytes of the operands, the same for every form). The form taken is 1.0 (INT8 0.7, GEGLU 1.3, GEGLU of INT8 0.9) % slower
+// than the fastest one on average; at worst 30 %, where the fastest one's own time differs by as much from one set of buffers to the
+// next (6144 x 320 x 320, three of them). Large tiles need fewer bytes per FLOP: a compute unit takes 1 KB from its L2 in 16 to 24
+// clocks, so a step of 128 x 128 (32 KB) takes 600 to 700 where its products take 512, one of 128 x 64 (24 KB) 450 to 650 where they take
+// 256. Small ones fill the GPU: 128 x 1280 x 1280 takes 4.6 us with 160 tiles of 32 x 32, 5.3 with 80 of 64 x 32, 8.6 with 20 of
+// 128 x 64; 1024 x 2240 x 2240 takes 16 us with 144 tiles of 128 x 128, 22 with 280 of 128 x 64, 50 with 36 of 256 x 256.
+// Loading wavefronts (see the top) pay where the products of a step are short. They are no help where a compute unit holds two work
+// groups of large register use: GEGLU 3072 x 640 -> 2 x 2560 31 -> 36 us, three of 16384 x 512 x 512 37 -> 44.
 struct Form {
     int bm, bn_out;
     float phi, lam, tau, eps;
 };
-enum { k64x32, k64x64, k128x64, k128x128, k128x128_2, k256x128, k256x256, kPlainForms };
-constexpr Form kPlain[kPlainForms] = {
-    {64, 32, 2.8f, 0.164f, 0.129f, 0.5f},   {64, 64, 2.8f, 0.199f, 0.197f, 0.9f},   {128, 64, 3.5f, 0.289f, 0.319f, 1.2f}, {128, 128, 4.6f, 0.350f, 0.556f, 3.8f},
-    {128, 128, 3.9f, 0.617f, 0.380f, 3.5f}, {256, 128, 5.7f, 0.613f, 0.920f, 7.0f}, {256, 256, 8.3f, 1.216f, 1.888f, 8.6f}};
-// INT8 weights: the widening makes small steps dearer and the large tiles no better (the 256-row forms are not built)
-constexpr Form kPlainW8[] = {
-    {64, 32, 1e9f, 0.f, 0.f, 0.f},          {64, 64, 3.1f, 0.257f, 0.149f, 1.1f},   {128, 64, 4.2f, 0.315f, 0.237f, 1.7f}, {128, 128, 5.3f, 0.370f, 0.609f, 3.6f},
-    {128, 128, 4.9f, 0.644f, 0.390f, 2.3f}, {256, 128, 1e9f, 0.f, 0.f, 0.f},        {256, 256, 1e9f, 0.f, 0.f, 0.f}};
-enum { kG64x64, kG128x64, kG256x64, kGegluForms };   // output features; the W tile holds twice as many rows
-constexpr Form kGeglu[kGegluForms] = {{64, 64, 3.2f, 0.378f, 0.282f, 1.8f}, {128, 64, 5.9f, 0.628f, 0.217f, 4.5f}, {256, 64, 7.5f, 0.674f, 0.957f, 7.7f}};
-constexpr Form kGegluW8[kGegluForms] = {{64, 64, 4.2f, 0.427f, 0.298f, 2.0f}, {128, 64, 6.5f, 0.682f, 0.384f, 3.3f}, {256, 64, 8.2f, 0.866f, 1.007f, 8.2f}};
+enum { k32x32, k64x32, k64x64, k128x64_load, k128x64, k128x128, k128x128_2, k192x128, k256x128, k256x256, kPlainForms };
+constexpr Form kPlain[kPlainForms] = {{32, 32, 2.46f, 0.091f, 0.058f, 0.22f},   {64, 32, 2.60f, 0.111f, 0.126f, 0.34f},   {64, 64, 2.52f, 0.154f, 0.190f, 0.42f},
+                                      {128, 64, 2.53f, 0.250f, 0.322f, 0.76f},  {128, 64, 2.57f, 0.274f, 0.322f, 0.59f},  {128, 128, 3.95f, 0.356f, 0.529f, 3.18f},
+                                      {128, 128, 3.19f, 0.515f, 0.465f, 1.20f}, {192, 128, 4.67f, 0.511f, 0.727f, 4.11f}, {256, 128, 5.03f, 0.656f, 0.839f, 6.17f},
+                                      {256, 256, 8.05f, 1.379f, 1.789f, 6.40f}};
+// INT8 weights: the widening makes small steps dearer and the large tiles no better (those above 128 x 128 are not built)
+enum { k8_32x32, k8_64x64, k8_128x64, k8_128x128, k8_128x128_2, kPlainW8Forms };
+constexpr Form kPlainW8[kPlainW8Forms] = {{32, 32, 2.47f, 0.155f, 0.049f, 0.33f},
+                                          {64, 64, 2.75f, 0.209f, 0.187f, 0.80f},
+                                          {128, 64, 3.03f, 0.325f, 0.286f, 1.43f},
+                                          {128, 128, 4.03f, 0.420f, 0.562f, 3.98f},
+                                          {128, 128, 2.89f, 0.658f, 0.382f, 3.13f}};
+enum { kG64x64, kG128x64_2, kG128x64, kG256x64, kGegluForms };   // output features; the W tile holds twice as many rows
+constexpr Form kGeglu[kGegluForms] = {{64, 64, 2.65f, 0.377f, 0.330f, 1.20f}, {128, 64, 3.66f, 0.648f, 0.496f, 2.09f}, {128, 64, 4.41f, 0.442f, 0.588f, 4.08f},
+                                      {256, 64, 5.99f, 0.800f, 0.834f, 8.98f}};
+enum { kG8_64x64, kG8_128x64_2, kG8_256x64, kGegluW8Forms };
+constexpr Form kGegluW8[kGegluW8Forms] = {{64, 64, 3.92f, 0.315f, 0.302f, 1.17f}, {128, 64, 3.92f, 0.653f, 0.429f, 2.93f}, {256, 64, 7.90f, 0.816f, 1.031f, 6.53f}};
 
 // 256 x 256 tiles take contractions from 512 on (below, their prologue is most of the launch).
 int pick_form(const Form* forms, int n_forms, const LinearBatch& batch, int n_problems) {
@@ -471,28 +528,40 @@ int pick_form(const Form* forms, int n_forms, const LinearBatch& batch, int n_pr
 template <typename T>
 int launch_form(const LinearBatch& b, int n, bool geglu, int dtype, hipStream_t st) {
     const bool w8 = b.p[0].w_scale != nullptr;
+    if (geglu && w8) {
+        switch (pick_form(kGegluW8, kGegluW8Forms, b, n)) {
+            case kG8_64x64: return launch_pipe<T, true, true, 2, 2, 1, 2, 3, 0>(b, n, st);
+            case kG8_128x64_2: return launch_pipe<T, true, true, 2, 2, 2, 2, 2, 0>(b, n, st);
+            default: return launch_pipe<T, true, true, 4, 2, 2, 2, 3, 0>(b, n, st);
+        }
+    }
     if (geglu) {
-        switch (pick_form(w8 ? kGegluW8 : kGeglu, kGegluForms, b, n)) {
-            case kG64x64: return w8 ? launch_pipe<T, true, true, 2, 2, 1, 2, 3>(b, n, st) : launch_pipe<T, false, true, 2, 2, 1, 2, 3>(b, n, st);
-            case kG128x64: return w8 ? launch_pipe<T, true, true, 2, 2, 2, 2, 2>(b, n, st) : launch_pipe<T, false, true, 2, 2, 2, 2, 2>(b, n, st);
-            default: return w8 ? launch_pipe<T, true, true, 4, 2, 2, 2, 3>(b, n, st) : launch_pipe<T, false, true, 4, 2, 2, 2, 3>(b, n, st);
+        switch (pick_form(kGeglu, kGegluForms, b, n)) {
+            case kG64x64: return launch_pipe<T, false, true, 2, 2, 1, 2, 3, 4>(b, n, st);
+            case kG128x64_2: return launch_pipe<T, false, true, 2, 2, 2, 2, 2, 0>(b, n, st);
+            case kG128x64: return launch_pipe<T, false, true, 2, 2, 2, 2, 3, 4>(b, n, st);
+            default: return launch_pipe<T, false, true, 4, 2, 2, 2, 3, 0>(b, n, st);
         }
     }
     if (w8) {
-        switch (pick_form(kPlainW8, kPlainForms, b, n)) {
-            case k64x64: return launch_pipe<T, true, false, 2, 2, 1, 1, 4>(b, n, st);
-            case k128x64: return launch_pipe<T, true, false, 2, 2, 2, 1, 3>(b, n, st);
-            case k128x128: return launch_pipe<T, true, false, 2, 4, 2, 1, 4>(b, n, st);
-            default: return launch_pipe<T, true, false, 2, 2, 2, 2, 2>(b, n, st);
+        switch (pick_form(kPlainW8, kPlainW8Forms, b, n)) {
+            case k8_32x32: return launch_pipe<T, true, false, 1, 1, 1, 1, 6, 2>(b, n, st);
+            case k8_64x64: return launch_pipe<T, true, false, 2, 2, 1, 1, 4, 4>(b, n, st);
+            case k8_128x64: return launch_pipe<T, true, false, 2, 2, 2, 1, 3, 4>(b, n, st);
+            case k8_128x128: return launch_pipe<T, true, false, 2, 4, 2, 1, 4, 0>(b, n, st);
+            default: return launch_pipe<T, true, false, 2, 2, 2, 2, 2, 0>(b, n, st);
         }
     }
     switch (pick_form(kPlain, kPlainForms, b, n)) {
-        case k64x32: return launch_pipe<T, false, false, 2, 1, 1, 1, 4>(b, n, st);
-        case k64x64: return launch_pipe<T, false, false, 2, 2, 1, 1, 4>(b, n, st);
-        case k128x64: return launch_pipe<T, false, false, 2, 2, 2, 1, 3>(b, n, st);
-        case k128x128: return launch_pipe<T, false, false, 2, 4, 2, 1, 4>(b, n, st);
-        case k128x128_2: return launch_pipe<T, false, false, 2, 2, 2, 2, 2>(b, n, st);
-        case k256x128: return launch_pipe<T, false, false, 4, 2, 2, 2, 3>(b, n, st);
+        case k32x32: return launch_pipe<T, false, false, 1, 1, 1, 1, 6, 2>(b, n, st);
+        case k64x32: return launch_pipe<T, false, false, 2, 1, 1, 1, 6, 2>(b, n, st);
+        case k64x64: return launch_pipe<T, false, false, 2, 2, 1, 1, 4, 4>(b, n, st);
+        case k128x64_load: return launch_pipe<T, false, false, 2, 2, 2, 1, 3, 4>(b, n, st);
+        case k128x64: return launch_pipe<T, false, false, 2, 2, 2, 1, 3, 0>(b, n, st);
+        case k128x128: return launch_pipe<T, false, false, 2, 2, 2, 2, 3, 4>(b, n, st);
+        case k128x128_2: return launch_pipe<T, false, false, 2, 2, 2, 2, 2, 0>(b, n, st);
+        case k192x128: return launch_pipe<T, false, false, 2, 4, 3, 1, 4, 0>(b, n, st);
+        case k256x128: return launch_pipe<T, false, false, 4, 2, 2, 2, 3, 0>(b, n, st);
         default: return launch_linear_dma(b, n, dtype, st);
     }
 }

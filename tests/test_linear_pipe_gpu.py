@@ -92,6 +92,24 @@ def test_pipe_three_unequal_problems_in_one_launch(oracle):
     assert torch.equal(bd.linear_batched(wo, None, bd.flash_attention_forward(q, k, v, None, H, False)), out)
 
 
+RINGS = [(33, 40, 320), (33, 40, 384), (31, 8, 448),               # 32 x 32 tiles, ring of 6: one stage fewer, as many, one more
+         (257, 1096, 320), (257, 1096, 384), (257, 1096, 448),      # 64 x 32, 6
+         (513, 1288, 192), (513, 1288, 256), (513, 1288, 320),      # 64 x 64, 4
+         (2049, 648, 128), (2049, 648, 192), (2049, 648, 256),      # 128 x 64, 3
+         (4609, 1160, 192), (4000, 1032, 256), (4000, 1032, 320)]   # 192 x 128, 4 (its own wavefronts load)
+
+
+@pytest.mark.parametrize("int8", [False, True], ids=["w16", "w8"])
+@pytest.mark.parametrize("M,N,K", RINGS)
+def test_pipe_loading_wavefronts_around_the_ring(oracle, int8, M, N, K):
+    (test_pipe_linear_int8_matches_checker if int8 else test_pipe_linear_matches_checker)(oracle, "fp16", M, N, K)
+
+
+@pytest.mark.parametrize("M,N,K", [(129, 200, 192), (1030, 1288, 256), (1030, 1288, 320), (2049, 1032, 128)])
+def test_pipe_geglu_loading_wavefronts(oracle, M, N, K):
+    test_pipe_geglu_is_the_linear_layer_and_the_gate(oracle, "bf16", False, M, N, K)
+
+
 @pytest.mark.parametrize("M,N,K", [(65, 40, 64), (300, 1288, 640), (257, 200, 1280)])
 def test_pipe_scales_start_at_any_float(oracle, M, N, K):
     """The scales are read four at a time: rows 1 .. N of a longer scale vector (4-byte alignment), N off every tile width, no bias.
