@@ -50,10 +50,47 @@ __global__ void __launch_bounds__(256) add_row_bias_kernel(T* y, const T* bias, 
     }
 }
 
-// RMS normalisation of whole rows: one work group per row (grid-stride over rows), the row held in registers between
+// RMS normalisation of whole rows of more than 4096 columns: one work group per row (grid-stride over rows), the row held in registers between
 // the sum of squares and the scaling (up to kRmsChunks 16-byte chunks per thread), FP32 arithmetic, one rounding.
 // blockIdx.y: which of up to two tensors (q and k of one call site share a launch: 1024 x 2240 twice, 7 -> 4 us).
 template <typename T> struct RmsOperands { const T* x; const T* gain; T* out; };
+// Rows of up to 4096 columns: a wavefront per row with N chunks per lane, no LDS and no barrier; the gain is requested together with
+// the row. (With a work group per row a row of 2240 columns left most lanes of its second pass empty and met at two barriers:
+// 256, 1024 and 4096 rows of 2240 3.2 -> 2.9, 4.1 -> 3.4 and 10.5 -> 6.4 us.)
+template <typename T, int N>
+__global__ void __launch_bounds__(256) rms_norm_wave_kernel(RmsOperands<T> a, RmsOperands<T> b, int rows, int cols, long x_rs, long o_rs, float eps) {
+    const RmsOperands<T>& op = blockIdx.y == 0 ? a : b;
+    typedef T t8 __attribute__((ext_vector_type(8)));
+    const int cpr = cols / 8, lane = threadIdx.x & 63;
+    for (long r = blockIdx.x * 4L + (threadIdx.x >> 6); r < rows; r += gridDim.x * 4L) {
+        u32x4 v[N], g[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] = *reinterpret_cast<const u32x4*>(op.x + r * x_rs + min(lane + 64 * i, cpr - 1) * 8);
+#pragma unroll
+        for (int i = 0; i < N; ++i) g[i] = *reinterpret_cast<const u32x4*>(op.gain + min(lane + 64 * i, cpr - 1) * 8);
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const t8 x8 = __builtin_bit_cast(t8, v[i]);
+            float s = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) { const float f = static_cast<float>(x8[e]); s = __builtin_fmaf(f, f, s); }
+            if (i < N - 1 || lane + 64 * i < cpr) ss += s;
+        }
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) ss += __shfl_xor(ss, off);
+        const float inv = __builtin_amdgcn_rsqf(ss / static_cast<float>(cols) + eps);
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const t8 x8 = __builtin_bit_cast(t8, v[i]), g8 = __builtin_bit_cast(t8, g[i]);
+            t8 o;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[e] = static_cast<T>(static_cast<float>(x8[e]) * inv * static_cast<float>(g8[e]));
+            if (i < N - 1 || lane + 64 * i < cpr) *reinterpret_cast<u32x4*>(op.out + r * o_rs + (lane + 64 * i) * 8) = __builtin_bit_cast(u32x4, o);
+        }
+    }
+}
+
 constexpr int kRmsChunks = 8;   // 256 threads x 8 chunks x 8 elements = rows of up to 16384 columns
 template <typename T>
 __global__ void __launch_bounds__(256) rms_norm_rows_kernel(RmsOperands<T> a, RmsOperands<T> b, int rows, int cols, long x_rs, long o_rs, float eps) {
@@ -119,7 +156,14 @@ int rms_norm_n(const char* op, int n, const void* x0, const void* gain0, void* o
         using T = decltype(tag);
         const RmsOperands<T> a{static_cast<const T*>(x0), static_cast<const T*>(gain0), static_cast<T*>(out0)};
         const RmsOperands<T> b{static_cast<const T*>(x1), static_cast<const T*>(gain1), static_cast<T*>(out1)};
-        hipLaunchKernelGGL(rms_norm_rows_kernel<T>, grid, dim3(256), 0, resolve_stream(stream), a, b, rows, cols, x_rs, o_rs, eps);
+        hipStream_t st = resolve_stream(stream);
+        const dim3 wave_grid(static_cast<unsigned>((rows + 3L) / 4 < (1 << 16) ? (rows + 3L) / 4 : (1 << 16)), n);
+#define MI_RMS_CASE(N) case N: hipLaunchKernelGGL((rms_norm_wave_kernel<T, N>), wave_grid, dim3(256), 0, st, a, b, rows, cols, x_rs, o_rs, eps); break;
+        switch ((cols / 8 + 63) / 64) {
+            MI_RMS_CASE(1) MI_RMS_CASE(2) MI_RMS_CASE(3) MI_RMS_CASE(4) MI_RMS_CASE(5) MI_RMS_CASE(6) MI_RMS_CASE(7) MI_RMS_CASE(8)
+            default: hipLaunchKernelGGL(rms_norm_rows_kernel<T>, grid, dim3(256), 0, st, a, b, rows, cols, x_rs, o_rs, eps);
+        }
+#undef MI_RMS_CASE
     };
     if (dtype == MI_DTYPE_BF16) launch(__bf16{});
     else if (dtype == MI_DTYPE_F16) launch(_Float16{});

@@ -2,6 +2,8 @@
 // Bandwidth-bound elementwise pass (one read and one write of x); used where the rotated
 // tensor itself must exist in HBM (the prefix cache keeps post-RoPE K). Attention calls
 // apply the rotation while loading Q and K instead.
+#include <type_traits>
+
 #include "internal.h"
 
 namespace mi {
@@ -9,6 +11,38 @@ namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+// How the kernels with 4 heads to a thread deal rows out: a block takes rb rows, t = 0 .. rb * units of them 16-byte chunk
+// positions (a unit: one chunk position of 4 heads). Row, chunk and address then come from 32-bit multiplications by inverses;
+// dividing a 64-bit index by the number of units cost more than everything between the loads and the stores
+// (24 heads of 128, us: head norm 300 rows 3.5 -> 2.7, 1997 5.3 -> 4.6, 4608 9.9 -> 9.4; with the rotation 3.7 -> 2.8, 5.7 -> 4.9,
+// 10.7 -> 9.8; rotation alone 4608 10.1 -> 9.7; a copy of 4608 rows takes 9.1). In the head norm the sums of squares also
+// left the LDS permutation network for DPP moves.
+struct RowUnits {
+    int units, rb, threads;      // of a row; rows and threads of a block
+    unsigned inv;                // ceil(2^32 / units): t / units exactly for t * units < 2^32
+    long blocks;
+    RowUnits(long rows, int units_) : units(units_), rb(1), inv(0xffffffffu / static_cast<unsigned>(units_) + 1u) {
+        // the number of rows that leaves the fewest lanes of the block's last wavefront empty
+        for (int n = 2, best = (units + 63) / 64 * 64 - units; n * units <= 256; ++n)
+            if (const int empty = (n * units + 63) / 64 * 64 - n * units; empty * rb <= best * n) { rb = n; best = empty; }
+        threads = rb * units < 256 ? (rb * units + 63) / 64 * 64 : 256;
+        blocks = (rows + rb - 1) / rb;
+    }
+    unsigned grid() const { return static_cast<unsigned>(blocks < (1 << 20) ? blocks : (1 << 20)); }
+};
+
+// sum over groups of N neighbouring lanes (N = 4, 8 or 16, all of them active), in every lane of the group; the order of a butterfly
+template <int N> __device__ __forceinline__ float group_sum(float v) {
+    auto moved = [](float f, auto ctrl) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, f), decltype(ctrl)::value, 0xf, 0xf, false));
+    };
+    v += moved(v, std::integral_constant<int, 0xB1>{});                        // quad_perm [1, 0, 3, 2]
+    v += moved(v, std::integral_constant<int, 0x4E>{});                        // quad_perm [2, 3, 0, 1]
+    if constexpr (N >= 8) v += moved(v, std::integral_constant<int, 0x141>{});  // row_half_mirror: the other quad of 8
+    if constexpr (N >= 16) v += moved(v, std::integral_constant<int, 0x140>{}); // row_mirror: the other half of 16
+    return v;
+}
 
 // Adjacent pairs (x[2p], x[2p+1]): one thread rotates one 16-byte chunk = 4 pairs.
 template <typename T>
@@ -41,39 +75,41 @@ __global__ void __launch_bounds__(256) rope_adjacent_kernel(const T* __restrict_
 
 // Adjacent pairs with one table for all heads: a thread rotates the same 16-byte chunk position of 4 heads of a row, so the
 // chunk's table entries are fetched once for the four and 4 data loads are in flight per thread. The heads of a thread
-// are n_hg apart (h = j * n_hg + hg), so that for each j the lanes of a wavefront touch consecutive heads, i.e. one
+// are H / 4 apart, so that for each of the four the lanes of a wavefront touch consecutive heads, i.e. one
 // contiguous piece of the row. Same arithmetic per element as the kernel above.
 template <typename T>
-__global__ void __launch_bounds__(256) rope_adjacent_heads_kernel(const T* __restrict__ x, T* __restrict__ out,
-                                                                  const float* __restrict__ cs, const float* __restrict__ sn,
-                                                                  int rows, int H, int d, long x_rs, long o_rs) {
+__global__ void __launch_bounds__(256) rope_adjacent_heads_kernel(const T* x, T* out, const float* __restrict__ cs, const float* __restrict__ sn, int rows,
+                                                                  int d, long x_rs, long o_rs, RowUnits ru, unsigned inv_cpd) {
     typedef T t8 __attribute__((ext_vector_type(8)));
     constexpr int HB = 4;
-    const int cpd = d / 8, n_hg = H / HB;
-    const long total = static_cast<long>(rows) * n_hg * cpd;
-    for (long idx = blockIdx.x * 256L + threadIdx.x; idx < total; idx += gridDim.x * 256L) {
-        const long t = idx / cpd;
-        const int dcq = static_cast<int>(idx - t * cpd);
-        const long r = t / n_hg;
-        const int hg = static_cast<int>(t - r * n_hg);
-        const f32x4 cv = *reinterpret_cast<const f32x4*>(cs + r * (d / 2) + dcq * 4);
-        const f32x4 sv = *reinterpret_cast<const f32x4*>(sn + r * (d / 2) + dcq * 4);
-        u32x4 raw[HB];
+    const int cpd = d / 8, n = ru.rb * ru.units;
+    const long quarter = ru.units * 8L;
+    for (long block = blockIdx.x; block < ru.blocks; block += gridDim.x)
+        for (int t = threadIdx.x; t < n; t += blockDim.x) {
+            const int rr = static_cast<int>(__umulhi(t, ru.inv)), u = t - rr * ru.units;
+            const long r = block * ru.rb + rr;
+            if (r >= rows) break;
+            const int dcq = u - static_cast<int>(__umulhi(u, inv_cpd)) * cpd;
+            const T* const xr = x + r * x_rs + u * 8;
+            u32x4 raw[HB];
 #pragma unroll
-        for (int j = 0; j < HB; ++j) raw[j] = *reinterpret_cast<const u32x4*>(x + r * x_rs + (j * n_hg + hg) * d + dcq * 8);
+            for (int j = 0; j < HB; ++j) raw[j] = *reinterpret_cast<const u32x4*>(xr + j * quarter);
+            const f32x4 cv = *reinterpret_cast<const f32x4*>(cs + r * (d / 2) + dcq * 4);
+            const f32x4 sv = *reinterpret_cast<const f32x4*>(sn + r * (d / 2) + dcq * 4);
+            T* const o = out + r * o_rs + u * 8;
 #pragma unroll
-        for (int j = 0; j < HB; ++j) {
-            t8 v = __builtin_bit_cast(t8, raw[j]);
+            for (int j = 0; j < HB; ++j) {
+                t8 v = __builtin_bit_cast(t8, raw[j]);
 #pragma unroll
-            for (int p = 0; p < 4; ++p) {
-                const float a = static_cast<float>(v[2 * p]);
-                const float b = static_cast<float>(v[2 * p + 1]);
-                v[2 * p] = static_cast<T>(rope_re(a, b, cv[p], sv[p]));
-                v[2 * p + 1] = static_cast<T>(rope_im(a, b, cv[p], sv[p]));
+                for (int p = 0; p < 4; ++p) {
+                    const float a = static_cast<float>(v[2 * p]);
+                    const float b = static_cast<float>(v[2 * p + 1]);
+                    v[2 * p] = static_cast<T>(rope_re(a, b, cv[p], sv[p]));
+                    v[2 * p + 1] = static_cast<T>(rope_im(a, b, cv[p], sv[p]));
+                }
+                *reinterpret_cast<u32x4*>(o + j * quarter) = __builtin_bit_cast(u32x4, v);
             }
-            *reinterpret_cast<u32x4*>(out + r * o_rs + (j * n_hg + hg) * d + dcq * 8) = __builtin_bit_cast(u32x4, v);
         }
-    }
 }
 
 // Split-half pairs (x[p], x[p + d/2]): one thread per pair (d/2 need not be a multiple of 8).
@@ -194,77 +230,76 @@ __global__ void __launch_bounds__(256) headnorm_rope_kernel(const T* x, T* out, 
     }
 }
 
-// The same for head counts that are multiples of 4: a thread takes one chunk position of 4 heads of a row (heads n_hg
+// The same for head counts that are multiples of 4: a thread takes one chunk position of 4 heads of a row (heads H / 4
 // apart, so that for each of the four the lanes of a wavefront touch one contiguous piece of the row), with one fetch of
 // the gain and table entries and one index computation for the four, and 4 loads in flight. Same arithmetic per element.
-template <typename T, int CPR>
-__global__ void __launch_bounds__(256) headnorm_rope_heads_kernel(const T* x, T* out, T* out2,
-                                                                  const T* __restrict__ gain, const float* __restrict__ cs,
-                                                                  const float* __restrict__ sn, int rows, int H, float eps,
-                                                                  long x_rs, long o_rs, long o2_rs, int out2_rows, int split_half) {
+// kRot: 0 no rotation, 1 adjacent pairs, 2 split-half pairs.
+template <typename T, int CPR, int kRot>
+__global__ void __launch_bounds__(256) headnorm_rope_heads_kernel(const T* x, T* out, T* out2, const T* __restrict__ gain, const float* __restrict__ cs,
+                                                                  const float* __restrict__ sn, int rows, float eps, long x_rs, long o_rs, long o2_rs,
+                                                                  int out2_rows, RowUnits ru) {
     typedef T t8 __attribute__((ext_vector_type(8)));
     constexpr int d = CPR * 8, HB = 4;
-    const int n_hg = H / HB;
-    const long total = static_cast<long>(rows) * n_hg * CPR;
-    for (long idx = blockIdx.x * 256L + threadIdx.x; idx < total; idx += gridDim.x * 256L) {
-        const long t = idx / CPR;
-        const int cq = static_cast<int>(idx - t * CPR);
-        const long r = t / n_hg;
-        const int hg = static_cast<int>(t - r * n_hg);
-        const int dc = cq * 8;
-        u32x4 raw[HB];
+    const int n = ru.rb * ru.units;
+    const long quarter = ru.units * 8L;
+    for (long block = blockIdx.x; block < ru.blocks; block += gridDim.x)
+        for (int t = threadIdx.x; t < n; t += blockDim.x) {
+            const int rr = static_cast<int>(__umulhi(t, ru.inv)), u = t - rr * ru.units;
+            const long r = block * ru.rb + rr;
+            if (r >= rows) break;      // (whole heads: the lanes of a sum stay together)
+            const int dc = u % CPR * 8;
+            const bool upper = dc >= d / 2;
+            const T* const xr = x + r * x_rs + u * 8;
+            u32x4 raw[HB];
 #pragma unroll
-        for (int j = 0; j < HB; ++j) raw[j] = *reinterpret_cast<const u32x4*>(x + r * x_rs + (j * n_hg + hg) * d + dc);
-        const t8 g = __builtin_bit_cast(t8, *reinterpret_cast<const u32x4*>(gain + dc));
-        f32x4 c0 = {0.f, 0.f, 0.f, 0.f}, c1 = c0, s0 = c0, s1 = c0;
-        const bool upper = dc >= d / 2;
-        if (cs != nullptr && split_half) {
-            const int pp = upper ? dc - d / 2 : dc;
-            c0 = *reinterpret_cast<const f32x4*>(cs + r * (d / 2) + pp);
-            c1 = *reinterpret_cast<const f32x4*>(cs + r * (d / 2) + pp + 4);
-            s0 = *reinterpret_cast<const f32x4*>(sn + r * (d / 2) + pp);
-            s1 = *reinterpret_cast<const f32x4*>(sn + r * (d / 2) + pp + 4);
-        } else if (cs != nullptr) {
-            c0 = *reinterpret_cast<const f32x4*>(cs + r * (d / 2) + dc / 2);
-            s0 = *reinterpret_cast<const f32x4*>(sn + r * (d / 2) + dc / 2);
-        }
-#pragma unroll
-        for (int j = 0; j < HB; ++j) {
-            const t8 v = __builtin_bit_cast(t8, raw[j]);
-            float f[8];
-            float ss = 0.f;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) { f[e] = static_cast<float>(v[e]); ss = __builtin_fmaf(f[e], f[e], ss); }
-#pragma unroll
-            for (int off = 1; off < CPR; off <<= 1) ss += __shfl_xor(ss, off);
-            const float inv = __builtin_amdgcn_rsqf(ss * (1.0f / d) + eps);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) f[e] = f[e] * inv * static_cast<float>(g[e]);
-            t8 o;
-            if (cs != nullptr && split_half) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float other = __shfl_xor(f[e], CPR / 2);
-                    const float a = upper ? other : f[e], b = upper ? f[e] : other;
-                    const float c = e < 4 ? c0[e & 3] : c1[e & 3], sv = e < 4 ? s0[e & 3] : s1[e & 3];
-                    o[e] = static_cast<T>(upper ? rope_im(a, b, c, sv) : rope_re(a, b, c, sv));
-                }
-            } else if (cs != nullptr) {
-#pragma unroll
-                for (int p = 0; p < 4; ++p) {
-                    o[2 * p] = static_cast<T>(rope_re(f[2 * p], f[2 * p + 1], c0[p], s0[p]));
-                    o[2 * p + 1] = static_cast<T>(rope_im(f[2 * p], f[2 * p + 1], c0[p], s0[p]));
-                }
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) o[e] = static_cast<T>(f[e]);
+            for (int j = 0; j < HB; ++j) raw[j] = *reinterpret_cast<const u32x4*>(xr + j * quarter);
+            const t8 g = __builtin_bit_cast(t8, *reinterpret_cast<const u32x4*>(gain + dc));
+            f32x4 c0, c1, s0, s1;
+            if constexpr (kRot == 2) {
+                const int pp = upper ? dc - d / 2 : dc;
+                c0 = *reinterpret_cast<const f32x4*>(cs + r * (d / 2) + pp);
+                c1 = *reinterpret_cast<const f32x4*>(cs + r * (d / 2) + pp + 4);
+                s0 = *reinterpret_cast<const f32x4*>(sn + r * (d / 2) + pp);
+                s1 = *reinterpret_cast<const f32x4*>(sn + r * (d / 2) + pp + 4);
+            } else if constexpr (kRot == 1) {
+                c0 = *reinterpret_cast<const f32x4*>(cs + r * (d / 2) + dc / 2);
+                s0 = *reinterpret_cast<const f32x4*>(sn + r * (d / 2) + dc / 2);
             }
-            const u32x4 bits = __builtin_bit_cast(u32x4, o);
-            const long col = static_cast<long>(j * n_hg + hg) * d + dc;
-            *reinterpret_cast<u32x4*>(out + r * o_rs + col) = bits;
-            if (r < out2_rows) *reinterpret_cast<u32x4*>(out2 + r * o2_rs + col) = bits;
+            T* const o_row = out + r * o_rs + u * 8;
+#pragma unroll
+            for (int j = 0; j < HB; ++j) {
+                const t8 v = __builtin_bit_cast(t8, raw[j]);
+                float f[8];
+                float ss = 0.f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) { f[e] = static_cast<float>(v[e]); ss = __builtin_fmaf(f[e], f[e], ss); }
+                const float inv = __builtin_amdgcn_rsqf(group_sum<CPR>(ss) * (1.0f / d) + eps);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) f[e] = f[e] * inv * static_cast<float>(g[e]);
+                t8 o;
+                if constexpr (kRot == 2) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const float other = __shfl_xor(f[e], CPR / 2);
+                        const float a = upper ? other : f[e], b = upper ? f[e] : other;
+                        const float c = e < 4 ? c0[e & 3] : c1[e & 3], sv = e < 4 ? s0[e & 3] : s1[e & 3];
+                        o[e] = static_cast<T>(upper ? rope_im(a, b, c, sv) : rope_re(a, b, c, sv));
+                    }
+                } else if constexpr (kRot == 1) {
+#pragma unroll
+                    for (int p = 0; p < 4; ++p) {
+                        o[2 * p] = static_cast<T>(rope_re(f[2 * p], f[2 * p + 1], c0[p], s0[p]));
+                        o[2 * p + 1] = static_cast<T>(rope_im(f[2 * p], f[2 * p + 1], c0[p], s0[p]));
+                    }
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) o[e] = static_cast<T>(f[e]);
+                }
+                const u32x4 bits = __builtin_bit_cast(u32x4, o);
+                *reinterpret_cast<u32x4*>(o_row + j * quarter) = bits;
+                if (r < out2_rows) *reinterpret_cast<u32x4*>(out2 + r * o2_rs + u * 8 + j * quarter) = bits;
+            }
         }
-    }
 }
 
 // out[r][c] = x[r][c] * scale * (row_scale ? row_scale[r] : 1): one thread per 16-byte chunk.
@@ -296,12 +331,15 @@ int launch_headnorm(const mi_headnorm_rope_args* a, long x_rs, long o_rs, long o
     const T* g = static_cast<const T*>(a->gain);
     const int r2 = a->out2 ? a->out2_rows : 0;
     const bool four = a->num_heads % 4 == 0;
-    const long blocks4 = (blocks + 3) / 4;
+    auto launch_four = [&](auto kernel, int cpr) {
+        const RowUnits ru(a->rows, a->num_heads / 4 * cpr);
+        hipLaunchKernelGGL(kernel, dim3(ru.grid()), dim3(ru.threads), 0, st, x, o, o2, g, a->cos, a->sin, a->rows, a->eps, x_rs, o_rs, o2_rs, r2, ru);
+    };
 #define MI_HEADNORM_CASE(CPR)                                                                                          \
     case CPR * 8:                                                                                                      \
-        if (four)                                                                                                      \
-            hipLaunchKernelGGL((headnorm_rope_heads_kernel<T, CPR>), dim3(blocks4), dim3(256), 0, st, x, o, o2, g, a->cos, \
-                               a->sin, a->rows, a->num_heads, a->eps, x_rs, o_rs, o2_rs, r2, a->split_half);           \
+        if (four && !a->cos) launch_four(headnorm_rope_heads_kernel<T, CPR, 0>, CPR);                                  \
+        else if (four && !a->split_half) launch_four(headnorm_rope_heads_kernel<T, CPR, 1>, CPR);                      \
+        else if (four) launch_four(headnorm_rope_heads_kernel<T, CPR, 2>, CPR);                                        \
         else                                                                                                           \
             hipLaunchKernelGGL((headnorm_rope_kernel<T, CPR>), dim3(blocks), dim3(256), 0, st, x, o, o2, g, a->cos,    \
                                a->sin, a->rows, a->num_heads, a->eps, x_rs, o_rs, o2_rs, r2, a->split_half);           \
@@ -337,11 +375,11 @@ int launch(const mi_rope_args* a, long x_rs, long o_rs, hipStream_t st) {
     } else if (a->split_half) {
         hipLaunchKernelGGL(rope_split_kernel<T>, dim3(blocks), dim3(256), 0, st, x, o, a->cos, a->sin, a->rows,
                            a->num_heads, a->head_dim, x_rs, o_rs, a->per_head);
-    } else if (!a->per_head && a->num_heads % 4 == 0) {
-        long hb = (work / 4 + 255) / 256;
-        if (hb > 256 * 32) hb = 256 * 32;
-        hipLaunchKernelGGL(rope_adjacent_heads_kernel<T>, dim3(hb), dim3(256), 0, st, x, o, a->cos, a->sin, a->rows,
-                           a->num_heads, a->head_dim, x_rs, o_rs);
+    } else if (!a->per_head && a->num_heads % 4 == 0 && a->head_dim > 8 && static_cast<long>(a->num_heads) * a->head_dim * a->head_dim < (1L << 31)) {
+        // (the inverses hold: units * (d / 8) < 2^23; below two chunks to a head there is nothing to divide)
+        const RowUnits ru(a->rows, a->num_heads / 4 * (a->head_dim / 8));
+        hipLaunchKernelGGL(rope_adjacent_heads_kernel<T>, dim3(ru.grid()), dim3(ru.threads), 0, st, x, o, a->cos, a->sin, a->rows, a->head_dim, x_rs, o_rs,
+                           ru, 0xffffffffu / static_cast<unsigned>(a->head_dim / 8) + 1u);
     } else {
         hipLaunchKernelGGL(rope_adjacent_kernel<T>, dim3(blocks), dim3(256), 0, st, x, o, a->cos, a->sin, a->rows,
                            a->num_heads, a->head_dim, x_rs, o_rs, a->per_head);

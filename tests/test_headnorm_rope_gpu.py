@@ -112,3 +112,35 @@ def test_prefix_dial_equals_scaled_keys_and_values(oracle):
     v = np.concatenate([oracle.round_to(vp * np.float32(1.25), dtype), vf])
     assert_close(oracle.sdpa(q, k, v, H), to_np(out), dtype, "prefix dial")
     assert not torch.equal(out, bd.sdpa_forward(dq, dkf, dvf, H, k_prefix=dkp, v_prefix=dvp))
+
+
+@pytest.mark.parametrize("split_half", [False, True])
+@pytest.mark.parametrize("L,H,d", [(1, 4, 32), (257, 4, 32), (5, 12, 64), (1024, 20, 128), (3, 64, 128), (7, 68, 128), (130, 160, 64)])
+def test_four_heads_per_thread(oracle, split_half, L, H, d):
+    """Rows per block from one to many, rows of whole and of part wavefronts, rows longer than a block; in place; first rows copied out.
+    Against the checker, and bit for bit against the kernels with one chunk per thread (a tensor of one head more)."""
+    dtype = "bf16"
+    x = randn(9300 + L, (L, (H + 1) * d), dtype)
+    gain = oracle.round_to(1.0 + 0.2 * randn(9301, (d,), "fp32"), dtype)
+    ang = np.linspace(0.0, 7.0, L * d // 2, dtype=np.float32).reshape(L, d // 2)
+    cos, sin = np.cos(ang), np.sin(ang)
+    wide, dg = to_dev(x, dtype), to_dev(gain, dtype)
+    dcos, dsin = torch.from_numpy(cos).cuda(), torch.from_numpy(sin).cuda()
+    for normed in (True, False):
+        def call(t, heads, **kw):
+            if normed:
+                return bd.headnorm_rope(t, dg, 1e-6, dcos, dsin, d, heads, split_half=split_half, **kw)
+            return bd.rope_apply(t, dcos, dsin, d, heads, split_half=split_half, **kw)
+        one = call(wide, H + 1)
+        four = call(wide[:, :H * d].contiguous(), H)
+        assert torch.equal(four, one[:, :H * d])
+        exact = oracle.headnorm_rope(x[:, :H * d], gain, 1e-6, cos, sin, H, d) if normed and not split_half else None
+        if exact is not None:
+            unit = 2.0 ** -8
+            assert np.all(np.abs(to_np(four) - exact) <= unit * np.maximum(np.abs(exact), 2.0 ** -6) * 1.02 + 1e-6)
+    buf = wide[:, :H * d].contiguous()
+    cache = torch.full((L, H * d), 9.0, device="cuda", dtype=buf.dtype)
+    first = (L + 1) // 2
+    want = bd.headnorm_rope(buf, dg, 1e-6, dcos, dsin, d, H, split_half=split_half)
+    bd.headnorm_rope(buf, dg, 1e-6, dcos, dsin, d, H, split_half=split_half, out=buf, cache_out=cache[:first])
+    assert torch.equal(buf, want) and torch.equal(cache[:first], want[:first]) and (cache[first:] == 9).all()

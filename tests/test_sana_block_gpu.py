@@ -84,7 +84,8 @@ def test_sana_identity_seam_inject(oracle):
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "fp16"])
-@pytest.mark.parametrize("rows,cols", [(300, 2240), (7, 8), (64, 4096), (3, 16384)])
+@pytest.mark.parametrize("rows,cols", [(300, 2240), (7, 8), (64, 4096), (3, 16384),
+                                       (1, 504), (5, 512), (6, 520), (9, 4088), (2, 4104)])   # around whole chunks per lane; the last a row too wide for one wavefront
 def test_rms_norm_rows(oracle, dtype, rows, cols):
     x = oracle.round_to(randn(9950 + cols, (rows, cols), dtype) * 3.0, dtype)
     g = oracle.round_to(1.0 + 0.3 * randn(9951, (cols,), "fp32"), dtype)
