@@ -109,6 +109,7 @@ int launch_sdpa_wide(const SdpaDev& p, int dtype, int head_dim, hipStream_t stre
 // Calls with few query rows (sdpa_small.hip) and unmasked ones of some sizes (sdpa_flow.hip): whether the kernel takes a call at kernel
 // choice 0, and the launch.
 bool sdpa_small_takes(const SdpaDev& p, int head_dim);
+bool sdpa_flow_runs(const SdpaDev& p);
 bool sdpa_flow_takes(const SdpaDev& p, int head_dim, int n_cu);
 int launch_sdpa_flow(const SdpaDev& p, int dtype, int head_dim, hipStream_t stream);
 int launch_sdpa_small(const SdpaDev& p, int dtype, int head_dim, hipStream_t stream);

@@ -298,8 +298,13 @@ int launch_flow_t(const SdpaDev& p, int head_dim, hipStream_t stream) {
 //                     units, 10 blocks 10.8 / 10.1
 //   64                up to 4 n units and 47 blocks (1024 units, 32 blocks 19.6 / 18.1), few keys, a last round up to half full (2304 units,
 //                     64 blocks 72 / 55; 3072 72 / 63)
+// (Calls whose keys fit LDS: launch_d asks sdpa_flow_runs and shortkv_pays instead.)
+bool sdpa_flow_runs(const SdpaDev& p) {
+    return !(p.mask_mode != MI_MASK_NONE || p.key_mask || p.bias || p.lse || p.cu_q || p.cos_k || p.prefix_scaled) && offsets_fit_32_bits(p);
+}
+
 bool sdpa_flow_takes(const SdpaDev& p, int head_dim, int n_cu) {
-    if (p.mask_mode != MI_MASK_NONE || p.key_mask || p.bias || p.lse || p.cu_q || p.cos_k || p.prefix_scaled || !offsets_fit_32_bits(p)) return false;
+    if (!sdpa_flow_runs(p)) return false;
     const long heads = static_cast<long>(p.B) * p.H, units = heads * ((p.Lq + 31) / 32), tiles = heads * ((p.Lq + 255) / 256), last = tiles % n_cu;
     const int blocks = (p.Lp + 31) / 32 + (p.Lk - p.Lp + 31) / 32;
     const bool full = tiles >= n_cu, half_round = tiles > n_cu && last > 0 && 2 * last <= n_cu;

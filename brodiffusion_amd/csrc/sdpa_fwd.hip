@@ -1296,6 +1296,35 @@ bool rows256_pay(const SdpaDev& p, int n_cu, bool xtra) {
     return plain && crowded && T >= 16;
 }
 
+// How many 256-row tiles of a head a work group of the short-key kernel walks, and the tiles that the busiest CU then has. The fewest
+// of the latter; among equals the most tiles per group (each group loads the head's keys once). Rounding tiles per CU down instead
+// gave a second, nearly empty round of groups as long as the first: with 2.5 to 7.5 tiles per CU 20 to 60 % of the launch.
+struct ShortPlan { int tiles = 1; long busiest = 0; };
+ShortPlan plan_short(long heads, int q_tiles, int n_cu) {
+    ShortPlan best;
+    auto consider = [&](int n) {
+        const long groups = heads * ((q_tiles + n - 1) / n), busiest = (groups + n_cu - 1) / n_cu * n;
+        if (best.busiest == 0 || busiest <= best.busiest) best = {n, busiest};
+    };
+    for (int n = 1; n <= min(q_tiles, 16); ++n) consider(n);
+    const int per_head = max(1, static_cast<int>(n_cu / heads));      // groups of a head that one round holds
+    const int one_round = (q_tiles + per_head - 1) / per_head;
+    if (one_round > 16) consider(one_round);
+    return best;
+}
+
+// Whether a call whose keys fit LDS is faster on the short-key kernel than on sdpa_flow.hip, which deals rows out finer and takes time
+// in proportion to the rows, where the short-key kernel takes that of whole rounds of 256-row tiles per CU; it is the better one
+// from a round that is nearly full on, the more so the more rounds share one load of the keys (us, short-key / flow, 16 heads of 40
+// and 72, 77 keys: 1.06 tiles per CU 12.6 / 9.3 and 15.9 / 11.8, 1.5 12.8 / 9.8 and 16.6 / 12.6, 2 11.8 / 11.8 and 15.3 / 16.5, 2.5
+// (as 3) 15.6 / 14.9 and 19.8 / 19.8, 3 15.6 / 17.3 and 19.8 / 22.9, 4 18.9 / 23.0 and 24.2 / 28.7; 154 keys 1.5 15.9 / 11.2). 112: 1 16.8 /
+// 12.5, 8 74.7 / 67.9. 128 stays here, where it gives the same bits as the 128-row kernel (1.5 tiles per CU 20.6 / 17.2).
+template <int D>
+bool shortkv_pays(const ShortPlan& plan, long tiles256, int n_cu) {
+    if (D == 112) return false;
+    return D == 128 || plan.busiest >= 4 || 16 * tiles256 >= 15 * plan.busiest * n_cu;
+}
+
 template <typename T, int D>
 int launch_d(SdpaDev p, int n_cu, hipStream_t stream) {
     const bool rope_k = p.cos_k != nullptr;
@@ -1314,7 +1343,9 @@ int launch_d(SdpaDev p, int n_cu, hipStream_t stream) {
     const bool short_keys = D <= 128 && choice == 0 && p.mask_mode == MI_MASK_NONE && p.bias == nullptr && p.lse == nullptr && p.Lp == 0 && !rope_k &&
                             p.cos_q == nullptr && n_kt >= 1 && n_kt <= shortkv_max_tiles<(D <= 128 ? D : 128)>() && tiles256 >= n_cu &&
                             shortkv_lds_bytes<D>(n_kt, p.key_mask != nullptr) <= 160 * 1024;
-    if (choice == 0 && !short_keys && sdpa_flow_takes(p, D, n_cu)) return launch_sdpa_flow(p, std::is_same_v<T, __bf16> ? MI_DTYPE_BF16 : MI_DTYPE_F16, D, stream);
+    const ShortPlan short_plan = short_keys ? plan_short(static_cast<long>(p.B) * p.H, (p.Lq + 255) / 256, n_cu) : ShortPlan{};
+    const bool flow = short_keys ? sdpa_flow_runs(p) && !shortkv_pays<D>(short_plan, tiles256, n_cu) : choice == 0 && sdpa_flow_takes(p, D, n_cu);
+    if (flow) return launch_sdpa_flow(p, std::is_same_v<T, __bf16> ? MI_DTYPE_BF16 : MI_DTYPE_F16, D, stream);
     if constexpr (dma_kernel_available<D>()) {
         if (p.split_scratch != nullptr && plan_split<D>(p, n_cu) &&
             p.split_scratch_bytes >= static_cast<size_t>(8) * p.split.max_tail * p.split.max_parts * SplitGeo::slot_bytes(D)) {
@@ -1344,7 +1375,7 @@ int launch_d(SdpaDev p, int n_cu, hipStream_t stream) {
     if (short_keys) {
         if constexpr (D <= 128) {
             p.n_q_tiles = (p.Lq + 255) / 256;
-            const int n_strip = static_cast<int>(tiles256 / n_cu);   // 256 query rows per work group and round: about one work group per CU
+            const int n_strip = short_plan.tiles;
             const int strips_per_head = (p.n_q_tiles + n_strip - 1) / n_strip;
             p.n_blocks = p.B * p.H * strips_per_head;
             hipLaunchKernelGGL((sdpa_shortkv_kernel<T, D>), dim3(grid_blocks(p)), dim3(kThreads8), shortkv_lds_bytes<D>(n_kt, p.key_mask != nullptr), stream, p,

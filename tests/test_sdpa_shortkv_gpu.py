@@ -83,3 +83,39 @@ def test_shortkv_key_mask(oracle, dtype, B, H, d, Lq, Lk):
     for b, n in enumerate((Lk - 20, 70)):
         ref = oracle.sdpa(q[b], k[b, :n], v[b, :n], H, key_mask=m[b, :n], rows=rows)
         assert_close(ref[rows], to_np(out[b])[rows], dtype, f"short-kv key mask + valid length, batch {b}")
+
+
+@pytest.mark.parametrize("B,H,d,Lq,Lk,mask", [
+    (1, 16, 72, 256 * 17, 77, False),        # just above a round: the kernel for finer tiles
+    (1, 16, 40, 256 * 29 + 1, 128, False),   # last round not full enough / just full enough to stay
+    (1, 16, 40, 256 * 30 + 1, 128, False),
+    (1, 16, 80, 256 * 45 + 3, 65, False),    # three tiles to a work group
+    (3, 100, 40, 300, 33, False),            # more heads than compute units
+    (1, 150, 64, 1200, 50, True),            # fewest tiles for the busiest one, not fewest work groups
+    (1, 5, 40, 256 * 1000 + 9, 20, False),   # more than 16 tiles to a work group
+    (1, 16, 72, 256 * 25, 77, True),         # uneven rounds with a key mask: always the short-key kernel
+    (1, 16, 112, 256 * 17, 77, False),
+])
+def test_shortkv_rounds(oracle, B, H, d, Lq, Lk, mask):
+    """Query sets of uneven rounds: the plan of tiles per work group, and the calls that leave for finer tiles."""
+    dtype = "bf16"
+    g = torch.Generator(device="cuda").manual_seed(Lq)
+    dq = torch.randn(B, Lq, H * d, device="cuda", generator=g).to(torch.bfloat16)
+    k, v = randn(9751, (B, Lk, H * d), dtype), randn(9752, (B, Lk, H * d), dtype)
+    dk, dv = to_dev(k, dtype), to_dev(v, dtype)
+    km = None
+    if mask:
+        km = torch.ones(B, Lk, device="cuda")
+        km[:, 3:9] = 0
+    out = bd.sdpa_forward(dq, dk, dv, H, key_mask=km)
+    want = rows128(dq, dk, dv, H, key_mask=km)
+    if mask:
+        assert torch.equal(out, want)
+    diff = (out.float() - want.float()).norm() / want.float().norm()
+    assert diff <= 5e-3                                            # two correct roundings of P and O to bf16
+    rows = np.unique(np.concatenate([np.arange(0, Lq, max(1, Lq // 12)), [Lq - 1]])).astype(np.int32)
+    some = torch.from_numpy(rows.astype(np.int64)).cuda()
+    for b in range(B):
+        keep = np.ones(Lk, bool) if km is None else km[b].cpu().numpy() > 0
+        ref = oracle.sdpa(to_np(dq[b][some]), k[b][keep], v[b][keep], H)
+        assert_close(ref, to_np(out[b][some]), dtype, f"batch {b}")
