@@ -11,6 +11,7 @@
 //                 zero pad), or comes from the K fragments against an all-ones operand where the
 //                 head dimension leaves no pad. No atomics anywhere: results are bit-reproducible.
 //   reduce kernel: adds the partial states of the token chunks into the state, in a fixed order.
+//   sum-apply kernel: takes the place of the two for short calls, see there.
 //   apply kernel: S is staged in LDS as 16-bit A operand, relu(Q) rows are B operands; the denominator
 //                 is an exact FP32 dot of z with the lane's own Q values plus one exchange between
 //                 lanes l and l^32.
@@ -495,6 +496,152 @@ __global__ void __launch_bounds__(kThreads) linattn_apply_kernel(const LinDev p)
         if constexpr (G::DP > D) {
             // the results overwrote the zero pad chunks of the tile (value channels D..DP-1 are zero anyway: the pad
             // rows of S are zero), nothing to restore
+        }
+        __syncthreads();
+    }
+}
+
+// ── apply straight from the partial states: no reduction launch ──
+// A group takes a chunk of tokens and one slice of 32 value channels of a head. It adds up its slice of the partial states (and z) in the
+// order of the reduction kernel while its first Q rows are on their way, and multiplies as the kernel above does: same bits. The
+// groups of a head's first chunk also leave the sums in the workspace. Every group of a slice reads its part of all partial
+// states, which is cheap where a reduction launch would be mostly latency: 20 heads of 112, us for the call, with a reduction launch / without: 256
+// tokens 12.8 / 9.9, 1024 18.6 / 16.1, 4096 31.8 / 30.9, 5184 34.5 / 35.2; 16 of 72, 1024 13.9 / 10.4, 4096 21.3 / 20.6; 40 of 112, 2048
+// 30.6 / 30.0, 4096 41 / 45: Q is read once per slice, so the line is drawn at a number of tokens of all heads times further slices.
+constexpr int kSumThreads = 256;
+template <typename T, int D>
+__global__ void __launch_bounds__(kSumThreads) linattn_sum_apply_kernel(const LinDev p) {
+    using G = LGeo<D>;
+    using V8 = typename Mma<T>::v8;
+    constexpr int TM = 128;                       // tokens per tile
+    constexpr int NQ = (TM * G::CPR + kSumThreads - 1) / kSumThreads;
+    __shared__ __attribute__((aligned(16))) unsigned char Ss[32 * G::S_STRIDE];
+    __shared__ __attribute__((aligned(16))) unsigned char Qs[TM * G::S_STRIDE];
+    __shared__ __attribute__((aligned(16))) float Zs[G::DP];
+
+    int bh, piece;
+    if (!lin_block(p, bh, piece)) return;
+    const int chunk = piece / G::NB, slice = piece - chunk * G::NB;      // (the slices of a chunk next to each other: they share its Q rows)
+    const int b = bh / p.H, h = bh % p.H;
+    const int n_begin = chunk * p.tokens_per_group;
+    const int n_end = min(p.N, n_begin + p.tokens_per_group);
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int lq = lane & 31, lh = lane >> 5;
+    const T* const q_base = static_cast<const T*>(p.q) + b * p.q_bs + h * D;
+    T* const o_base = static_cast<T*>(p.o) + b * p.o_bs + h * D + 32 * slice;
+    const int last = n_end - 1;
+    const int rows = min(32, D - 32 * slice);     // value channels of the slice
+
+    u32x4 qreg[NQ];
+    auto issue_q = [&](int n0) {
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) {
+            const int idx = min(tid + kSumThreads * i, TM * G::CPR - 1);
+            const int row = idx / G::CPR, cc = idx - row * G::CPR;
+            qreg[i] = *reinterpret_cast<const u32x4*>(q_base + static_cast<long>(min(n0 + row, last)) * p.q_rs + cc * 8);
+        }
+    };
+    issue_q(n_begin);
+    {
+        // quads of the slice's rows, then those of z; every part's are requested before the first is added
+        constexpr int QPR = D / 4, NS = (33 * QPR + kSumThreads - 1) / kSumThreads;
+        const float* const part = p.part + static_cast<long>(bh) * p.n_part * G::WS_FLOATS;
+        f32x4 v[kMaxStateSplit][NS];
+        int off[NS];
+#pragma unroll
+        for (int t = 0; t < NS; ++t) {
+            const int idx = tid + kSumThreads * t, i = idx / QPR, j = (idx - i * QPR) * 4;
+            off[t] = i < 32 ? min(32 * slice + i, D - 1) * D + j : D * D + min(j, D - 4);
+        }
+#pragma unroll
+        for (int c = 0; c < kMaxStateSplit; ++c)
+            if (c < p.n_part) {
+#pragma unroll
+                for (int t = 0; t < NS; ++t) v[c][t] = *reinterpret_cast<const f32x4*>(part + c * G::WS_FLOATS + off[t]);
+            }
+#pragma unroll
+        for (int c = 1; c < kMaxStateSplit; ++c)
+            if (c < p.n_part) {
+#pragma unroll
+                for (int t = 0; t < NS; ++t) v[0][t] += v[c][t];
+            }
+        typedef T t4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+        for (int t = 0; t < NS; ++t) {
+            const int idx = tid + kSumThreads * t, i = idx / QPR, j = (idx - i * QPR) * 4;
+            if (i < 32) {
+                t4 tv;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) tv[e] = i < rows ? static_cast<T>(v[0][t][e]) : static_cast<T>(0.f);
+                *reinterpret_cast<t4*>(Ss + i * G::S_STRIDE + j * 2) = tv;
+            } else if (i == 32) *reinterpret_cast<f32x4*>(Zs + j) = v[0][t];
+            if (chunk == 0 && (i < rows || (i == 32 && slice == 0)))
+                *reinterpret_cast<f32x4*>(p.ws + static_cast<long>(bh) * G::WS_FLOATS + off[t]) = v[0][t];
+        }
+    }
+    if constexpr (G::DP > D) {  // pad columns of S, z and the Q tile stay zero
+        constexpr int PC = (G::DP - D) / 8;
+        for (int i = tid; i < 32 * PC; i += kSumThreads) *reinterpret_cast<u32x4*>(Ss + (i / PC) * G::S_STRIDE + D * 2 + (i % PC) * 16) = u32x4{0, 0, 0, 0};
+        for (int i = tid; i < TM * PC; i += kSumThreads) *reinterpret_cast<u32x4*>(Qs + (i / PC) * G::S_STRIDE + D * 2 + (i % PC) * 16) = u32x4{0, 0, 0, 0};
+        if (tid < G::DP - D) Zs[D + tid] = 0.f;
+    }
+
+    for (int n0 = n_begin; n0 < n_end; n0 += TM) {
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) {
+            const int idx = tid + kSumThreads * i;
+            const int row = idx / G::CPR, cc = idx - row * G::CPR;
+            if (idx < TM * G::CPR) *reinterpret_cast<u32x4*>(Qs + row * G::S_STRIDE + cc * 16) = relu8<T>(qreg[i]);
+        }
+        __syncthreads();
+        if (n0 + TM < n_end) issue_q(n0 + TM);
+
+        const int trow = wave * 32 + lq;          // this lane's token within the tile
+        V8 qf[G::KC];
+        float den = 0.f;
+#pragma unroll
+        for (int c = 0; c < G::KC; ++c) {
+            const int d0 = 16 * c + 8 * lh;
+            qf[c] = __builtin_bit_cast(V8, *reinterpret_cast<const u32x4*>(Qs + trow * G::S_STRIDE + d0 * 2));
+            const f32x4 z0 = *reinterpret_cast<const f32x4*>(Zs + d0);
+            const f32x4 z1 = *reinterpret_cast<const f32x4*>(Zs + d0 + 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                den = __builtin_fmaf(z0[e], static_cast<float>(qf[c][e]), den);
+                den = __builtin_fmaf(z1[e], static_cast<float>(qf[c][4 + e]), den);
+            }
+        }
+        {
+            const int di = __builtin_bit_cast(int, den);
+            const i32x2 r = __builtin_amdgcn_permlane32_swap(di, di, false, false);
+            const int r0 = r[0], r1 = r[1];
+            den = __builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1);
+        }
+        const float rs = __builtin_amdgcn_rsqf(den + p.eps);
+        const float recip = rs * rs;
+        f32x16 acc;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+#pragma unroll
+        for (int c = 0; c < G::KC; ++c) {
+            const u32x4 a = *reinterpret_cast<const u32x4*>(Ss + lq * G::S_STRIDE + (16 * c + 8 * lh) * 2);
+            acc = Mma<T>::run(__builtin_bit_cast(V8, a), qf[c], acc);
+        }
+        // (a wavefront's rows are its own: they take its results without a barrier)
+#pragma unroll
+        for (int bb = 0; bb < 4; ++bb) {
+            typedef T t4 __attribute__((ext_vector_type(4)));
+            t4 ov;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) ov[e] = static_cast<T>(acc[4 * bb + e] * recip);
+            *reinterpret_cast<t4*>(Qs + trow * G::S_STRIDE + (8 * bb + 4 * lh) * 2) = ov;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < TM * 4 / kSumThreads; ++i) {
+            const int idx = tid + kSumThreads * i, row = idx >> 2, cc = idx & 3;
+            if (cc * 8 < rows && n0 + row <= last)
+                *reinterpret_cast<u32x4*>(o_base + static_cast<long>(n0 + row) * p.o_rs + cc * 8) = *reinterpret_cast<const u32x4*>(Qs + row * G::S_STRIDE + cc * 16);
         }
         __syncthreads();
     }
@@ -1136,12 +1283,14 @@ int launch_d(LinDev p, bool accumulate, int max_split, int n_cu, hipStream_t st)
         using FG = FusedGeo<D>;
         const int groups = BH * FG::NS;
         const bool fits = !accumulate && static_cast<long>(BH) * FG::NS < (1L << 24);
-        // Picked by size (measured, 256 compute units): with one slice per head (head_dim 32) nothing is read twice and the
-        // single launch wins at every length once its work groups cover a quarter of the GPU; with several slices every
+        // Picked by size (measured, 256 compute units; us, several launches / one): with one slice per head (head_dim 32) nothing is
+        // read twice, but a work group streams all tokens of its head (20 heads, 512 tokens 6.2 / 5.6, 777 6.7 / 7.2, 4096 10.5 /
+        // 25.4; 70 heads, 1024 9.2 / 8.8, 1500 10.5 / 11.8, 4096 18.7 / 26.3; 140 heads, 4096 30.9 / 28.9); with several slices every
         // work group pulls all of K and Q through its own compute unit's L2 port (about 50 GB/s each), which costs more
-        // than the two extra launches from about 2000 tokens on (head_dim 112, 40 heads: 13.6 against 18.5 us at 512
-        // tokens, 20.5 against 23.4 at 1024, 32 against 31 at 2048, 55 against 42 at 4096).
-        const bool by_size = fits && (FG::NS == 1 ? 4 * groups >= n_cu : (2 * groups >= n_cu && p.N <= kFusedMaxTokens));
+        // than the extra launches beyond 1024 tokens (head_dim 112, 40 heads: 14.7 / 12.9 at 512 tokens, 20.5 / 20.4 at
+        // 1024, 30 / 32 at 2048, 45 / 55 at 4096).
+        const bool few = FG::NS == 1 && (p.N <= 512 || (4 * groups >= n_cu && p.N <= kFusedMaxTokens));
+        const bool by_size = fits && (few || (2 * groups >= n_cu && (FG::NS == 1 || p.N <= kFusedMaxTokens)));
         if (fits && (p.form == MI_LINEAR_ATTN_FORM_ONE_LAUNCH || (p.form == MI_LINEAR_ATTN_FORM_BY_SIZE && by_size))) {
             static thread_local bool raised = false;
             if (!raised) {
@@ -1156,16 +1305,19 @@ int launch_d(LinDev p, bool accumulate, int max_split, int n_cu, hipStream_t st)
             return 0;
         }
     }
+    bool sums_parts = false;      // the apply pass adds the partial states up itself
     // State pass. The tokens of a head are split over enough groups to keep most CUs streaming, if the caller lent a
-    // scratch for the partial states; each group needs a few tiles to amortise its prologue and epilogue.
+    // scratch for the partial states.
     {
         LinDev ps = p;
         const int tiles = (ps.N + kStateTile - 1) / kStateTile;
-        // the largest split that still gives every group a CU of its own and at least two tiles (40 heads on 256 CUs: 6;
+        // the largest split that still gives every group a CU of its own and at least one or two tiles (40 heads on 256 CUs: 6;
         // two groups per CU measured slower, a power of two leaves a third of the CUs idle)
         int split = 1;
+        // (without a reduction launch one tile: 20 heads of 112, 256 tokens 12.8 / 9.9, 1024 16.4 / 16.1; with one, 256 tokens 12.8 / 13.9)
+        const bool may_sum = !accumulate && max_split > 0 && static_cast<long>(BH) * p.N * (G::NB - 1) <= 840L * n_cu;
         for (int s2 = 2; s2 <= max_split; ++s2)
-            if (BH * s2 <= n_cu && tiles / s2 >= 2) split = s2;
+            if (BH * s2 <= n_cu && tiles / s2 >= (may_sum ? 1 : 2)) split = s2;
         ps.tokens_per_group = ((tiles + split - 1) / split) * kStateTile;
         ps.n_chunks = (ps.N + ps.tokens_per_group - 1) / ps.tokens_per_group;
         ps.n_blocks = BH * ps.n_chunks;
@@ -1175,7 +1327,9 @@ int launch_d(LinDev p, bool accumulate, int max_split, int n_cu, hipStream_t st)
         ps.add_to_state = (!partials && accumulate) ? 1 : 0;
         hipLaunchKernelGGL((linattn_state_kernel<T, D>), dim3(((ps.n_blocks + 7) / 8) * 8), dim3(kStateThreads),
                            StateGeo<D>::LDS_BYTES, st, ps);
-        if (partials) {
+        sums_parts = partials && may_sum;
+        if (sums_parts) { p.part = ps.part; p.n_part = ps.n_part; }
+        else if (partials) {
             const long ws4 = G::WS_FLOATS / 4, total4 = static_cast<long>(BH) * ws4;   // D is a multiple of 8: whole 16-byte pieces
             const int blocks = static_cast<int>(std::min<long>((total4 + 255) / 256, 2048));
             hipLaunchKernelGGL(linattn_reduce_kernel, dim3(blocks), dim3(256), 0, st, p.ws, p.part, ps.n_part, ws4, total4,
@@ -1190,6 +1344,18 @@ int launch_d(LinDev p, bool accumulate, int max_split, int n_cu, hipStream_t st)
         q.n_blocks = BH * q.n_chunks;
         return dim3(((q.n_blocks + 7) / 8) * 8);
     };
+    if (sums_parts) {
+        // (two groups per CU; three: 20 heads of 112, 1024 tokens 16.4 -> 17.6, 4096 31 -> 34)
+        const int tiles = (p.N + 127) / 128;
+        const int per_bh = std::max(1, 2 * n_cu / (BH * G::NB));
+        p.tokens_per_group = 128 * ((tiles + per_bh - 1) / per_bh);
+        p.n_chunks = G::NB * ((p.N + p.tokens_per_group - 1) / p.tokens_per_group);
+        p.n_blocks = BH * p.n_chunks;
+        hipLaunchKernelGGL((linattn_sum_apply_kernel<T, D>), dim3(((p.n_blocks + 7) / 8) * 8), dim3(kSumThreads), 0, st, p);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return fail("mi_linear_attn_relu_forward launch: %s", hipGetErrorString(e));
+        return 0;
+    }
     {
         const int tiles = (p.N + 127) / 128;
         const int per_bh = std::max(1, 2 * n_cu / BH);

@@ -352,7 +352,8 @@ typedef struct mi_linear_attn_args {
     void* scratch;          /* device, 16-byte aligned, or NULL */
     size_t scratch_bytes;
     int32_t form;           /* MI_LINEAR_ATTN_FORM_BY_SIZE (0): the library picks. _THREE_LAUNCHES: state per token chunk, reduction
-                               of the partial states (in `scratch`), apply. _ONE_LAUNCH: the state split along its value channels,
+                               of the partial states (in `scratch`), apply; the last two are one launch where that is faster, with
+                               the same bits. _ONE_LAUNCH: the state split along its value channels,
                                every work group streams K, its slice of V, then Q, and writes its slice of O; no scratch is used.
                                A call that accumulates onto a state always takes the three launches */
     int32_t layout;         /* MI_LAYOUT_TOKEN_MAJOR (0): q, k, v, o are (batch, n_tokens, heads*head_dim), a row per token, as

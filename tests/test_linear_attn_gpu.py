@@ -217,3 +217,25 @@ def test_rope_apply_perhead_and_inplace(oracle):
     assert np.max(np.abs(to_np(out) - ref)) <= 2.0 ** -8 * max(1.0, np.abs(ref).max())
     bd.rope_apply_perhead(dx, torch.from_numpy(cos).cuda(), torch.from_numpy(sin).cuda(), d, H, out=dx)
     assert torch.equal(dx, out)
+
+
+@pytest.mark.parametrize("B,H,d,N", [(1, 20, 112, 129), (1, 20, 112, 1024), (1, 3, 112, 2300), (2, 5, 72, 700), (1, 2, 64, 257), (1, 4, 128, 900), (3, 1, 32, 1100),
+                                     (1, 20, 112, 3584), (1, 20, 112, 3585)])
+def test_linear_attention_sums_partial_states_on_apply(oracle, B, H, d, N):
+    """The apply pass that adds the partial states up itself (no reduction launch): token chunks of one and several tiles, ragged last
+    chunks, narrow last slices, both sides of the rule's line; output and captured state, and the same again from run to run."""
+    dtype = "bf16"
+    q, k, v = (randn(5100 + i + N, (B, N, H * d), dtype) for i in range(3))
+    dq, dk, dv = (to_dev(t, dtype) for t in (q, k, v))
+    ws = torch.full((B * H * (d * d + d),), float("nan"), dtype=torch.float32, device="cuda")
+    wide = torch.full((B, N, H * d + 8), 7.0, dtype=torch.bfloat16, device="cuda")
+    out = bd.linear_attention_relu_forward(dq, dk, dv, H, out=wide[:, :, :H * d], workspace=ws, form=1)
+    assert (wide[:, :, H * d:] == 7).all()
+    wsn = to_np(ws).reshape(B, H, d * d + d)
+    for b in range(B):
+        ref, S, z = oracle.linear_attn_relu(q[b], k[b], v[b], H, return_state=True)
+        assert_close(ref, to_np(out[b]), dtype, f"out b={b}")
+        assert np.max(np.abs(wsn[b, :, :d * d].reshape(H, d, d) - S)) <= 1e-4 * max(1.0, np.max(np.abs(S)))
+        assert np.max(np.abs(wsn[b, :, d * d:] - z)) <= 1e-4 * max(1.0, np.max(np.abs(z)))
+    ws2 = torch.empty_like(ws)
+    assert torch.equal(bd.linear_attention_relu_forward(dq, dk, dv, H, workspace=ws2, form=1), out) and torch.equal(ws2, ws)
