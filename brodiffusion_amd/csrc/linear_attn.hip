@@ -1289,7 +1289,7 @@ int launch_d(LinDev p, bool accumulate, int max_split, int n_cu, hipStream_t st)
         // work group pulls all of K and Q through its own compute unit's L2 port (about 50 GB/s each), which costs more
         // than the extra launches beyond 1024 tokens (head_dim 112, 40 heads: 14.7 / 12.9 at 512 tokens, 20.5 / 20.4 at
         // 1024, 30 / 32 at 2048, 45 / 55 at 4096).
-        const bool few = FG::NS == 1 && (p.N <= 512 || (4 * groups >= n_cu && p.N <= kFusedMaxTokens));
+        const bool few = FG::NS == 1 && (p.N <= 512 || (4 * groups >= n_cu && (p.N <= kFusedMaxTokens || max_split < 2)));   // (or no scratch to split with)
         const bool by_size = fits && (few || (2 * groups >= n_cu && (FG::NS == 1 || p.N <= kFusedMaxTokens)));
         if (fits && (p.form == MI_LINEAR_ATTN_FORM_ONE_LAUNCH || (p.form == MI_LINEAR_ATTN_FORM_BY_SIZE && by_size))) {
             static thread_local bool raised = false;
