@@ -2,6 +2,7 @@
 // projection GEMM (linear.hip) and the softmax-attention kernels behind the C ABI. Three launches for the whole block:
 // Q/K/V projections (one grid), attention, output projection. Nothing is allocated; intermediates live in the
 // caller's scratch.
+#include <cmath>
 #include <cstring>
 
 #include "internal.h"
@@ -63,6 +64,21 @@ size_t block_scratch(int batch, int q_len, int kv_len, int inner, bool with_kv, 
     const size_t q = round_up(static_cast<size_t>(batch) * q_len * inner * 2);
     const size_t kv = round_up(static_cast<size_t>(batch) * kv_len * inner * 2);
     return 2 * q + (with_kv ? 2 * kv : 0) + round_up(split);
+}
+
+// The attention launch of a block with cached keys as a launch view: enough for sdpa_projected_takes and its launch.
+SdpaDev cached_view(const mi_attn_block_args* a, const BlockDims& d, void* o) {
+    SdpaDev p;
+    std::memset(&p, 0, sizeof(p));
+    p.k = a->k; p.v = a->v; p.o = o;
+    p.B = a->batch; p.H = a->num_heads; p.Lq = a->q_len; p.Lk = a->kv_len; p.kv_group = 1;
+    p.q_rs = p.k_rs = p.v_rs = p.o_rs = a->inner;
+    p.q_bs = p.o_bs = static_cast<long>(a->q_len) * a->inner;
+    p.k_bs = p.v_bs = static_cast<long>(a->kv_len) * a->inner;
+    p.scale_log2 = 1.0f / std::sqrt(static_cast<float>(d.head_dim)) * 1.4426950408889634f;
+    p.mask_mode = a->causal ? MI_MASK_CAUSAL : MI_MASK_NONE;
+    p.key_mask = a->key_mask;
+    return p;
 }
 
 // [scratch_used, scratch_bytes) of the caller's scratch is lent to the attention launch.
@@ -214,8 +230,13 @@ int mi_flash_attention_q_with_kv_cached_forward(const mi_attn_block_args* a) {
     mi::LinearBatch b;
     std::memset(&b, 0, sizeof(b));
     b.p[0] = mi::problem(a->x, a->wq, a->bq, sq, d.q_rows, a->inner, a->channels, a->wq_scales);
-    if (mi::launch_linear(b, 1, a->dtype, st) != 0) return -1;
-    if (mi::attend(a, d, sq, a->k, a->v, sa, a->kv_len, need) != 0) return -1;
+    const mi::SdpaDev view = mi::cached_view(a, d, sa);
+    if (mi::sdpa_projected_takes(view, b.p[0], d.head_dim)) {
+        if (mi::launch_sdpa_projected(view, b.p[0], a->dtype, d.head_dim, st) != 0) return -1;
+    } else {
+        if (mi::launch_linear(b, 1, a->dtype, st) != 0) return -1;
+        if (mi::attend(a, d, sq, a->k, a->v, sa, a->kv_len, need) != 0) return -1;
+    }
     std::memset(&b, 0, sizeof(b));
     b.p[0] = mi::problem(sa, a->wo, a->bo, a->out, d.q_rows, a->out_channels, a->inner, a->wo_scales);
     return mi::launch_linear(b, 1, a->dtype, st);

@@ -145,4 +145,9 @@ bool linear_pipe_takes(const LinearBatch& batch, int n_problems, bool geglu);
 int launch_linear_pipe(const LinearBatch& batch, int n_problems, int dtype, bool geglu, hipStream_t stream);
 int launch_linear_dma(const LinearBatch& batch, int n_problems, int dtype, hipStream_t stream);
 
+// Cross-attention to cached keys with its query projection in the same launch (sdpa_small.hip): p.q is not read, q projects batch * Lq
+// rows to H * head_dim columns (q.y is not written).
+bool sdpa_projected_takes(const SdpaDev& p, const LinearProblem& q, int head_dim);
+int launch_sdpa_projected(const SdpaDev& p, const LinearProblem& q, int dtype, int head_dim, hipStream_t stream);
+
 }  // namespace mi

@@ -83,34 +83,6 @@ struct PipeGeo {
     static_assert((S - 1) * MI < 64, "outstanding loads fit the counter");
 };
 
-// 8 INT8 weights -> 8 values of T, exactly
-template <typename T> __device__ __forceinline__ typename Mma<T>::v8 widen(u32x2 raw);
-template <> __device__ __forceinline__ f16x8 widen<_Float16>(u32x2 raw) {
-    // u = w + 128 as the low byte of 1024 + u (0x6400 | u), minus 1152
-    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-    const f16x2 off = {static_cast<_Float16>(1152.f), static_cast<_Float16>(1152.f)};
-    u32x4 r;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const unsigned u = raw[i] ^ 0x80808080u;
-        const unsigned lo = __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u), hi = __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u);
-        r[2 * i] = __builtin_bit_cast(unsigned, __builtin_bit_cast(f16x2, lo) - off);
-        r[2 * i + 1] = __builtin_bit_cast(unsigned, __builtin_bit_cast(f16x2, hi) - off);
-    }
-    return __builtin_bit_cast(f16x8, r);
-}
-template <> __device__ __forceinline__ bf16x8 widen<__bf16>(u32x2 raw) {
-    // |w| <= 128 has at most 8 significant bits: the upper half of the FP32 value is the bf16 value
-    u32x4 r;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const unsigned pair = i & 1 ? raw[i >> 1] >> 16 : raw[i >> 1];
-        const float a = static_cast<float>(static_cast<signed char>(pair & 0xffu)), b = static_cast<float>(static_cast<signed char>((pair >> 8) & 0xffu));
-        r[i] = __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, b), __builtin_bit_cast(unsigned, a), 0x07060302u);
-    }
-    return __builtin_bit_cast(bf16x8, r);
-}
-
 template <typename T, bool W8, bool GEGLU, int WM, int WN, int TM, int TN, int S, int NL>
 __global__ void __launch_bounds__(64 * (WM * WN + NL), 2) linear_pipe_kernel(const PipeArgs args) {
     using G = PipeGeo<T, W8, GEGLU, WM, WN, TM, TN, S, NL>;

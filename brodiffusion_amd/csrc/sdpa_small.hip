@@ -20,6 +20,10 @@
 //   self, tokens x head_dim: 64 x 160 8.5 -> 5.0, 256 x 160 14.6 -> 7.0, 1024 x 160 37.4 -> 15.4; 512 x 80 14.4 -> 6.9, 2048 x 80
 //   39.8 -> 22.2; 1024 x 40 18.1 -> 8.5
 //   77 keys, queries x head_dim: 64 x 160 10.7 -> 5.7, 1024 x 80 8.9 -> 4.8, 4096 x 40 8.1 -> 6.3
+//
+// The instances with PROJ also form their query rows (project_rows): the cached cross-attention of a block, whose query projection
+// is as short as the attention behind it and, as a launch of its own, mostly start, first loads and write-out.
+#include "linear_math.h"
 #include "sdpa_tiles.h"
 
 namespace mi {
@@ -52,13 +56,179 @@ struct SmallArgs {
     float scale_log2;
 };
 struct NoMask {};
-__device__ __forceinline__ int quotient(int x, int d, unsigned inv) { return d == 1 ? x : static_cast<int>(__umulhi(static_cast<unsigned>(x), inv)); }
 
-template <typename T, int D, int R, bool MASKED>
-__global__ void __launch_bounds__(64 * kMaxWaves, D <= 64 ? 4 : D <= 80 ? 3 : 2)
-    sdpa_small_kernel(const SmallArgs p, const std::conditional_t<MASKED, SdpaDev, NoMask> mask) {
+// The query projection inside the kernel (project_rows): x (rows of a batch item, contraction elements), w (H D, contraction).
+struct ProjArgs {
+    const void* x; const void* w; const void* bias; const float* w_scale;
+    long x_bsb;                          // bytes between batch items of x
+    unsigned x_rsb, w_rsb; int n_steps;  // steps of 64 contraction elements
+};
+constexpr int kProjS = 3;                // wavefronts to a row group of 32, and steps of a round of the projection
+// PROJ: 0 none, 1 16-bit weights, 2 INT8 weights. LDS: two buffers of kProjS stages each (64 rows of X, D rows of W of 64 contraction elements), the
+// projected rows, the key blocks; the parts of the output will lie where the stages were.
+template <int D, int PROJ> struct ProjGeo {
     using G = HeadGeo<D>;
     using SG = SmallGeo<D>;
+    static constexpr int WROW = PROJ == 2 ? 64 : 128;                       // bytes of a W row in a stage
+    static constexpr int MX = 8, MW = (D * WROW + 1023) / 1024;             // DMA instructions per stage
+    static constexpr int X_BYTES = 8192, STAGE = X_BYTES + MW * 1024;
+    static constexpr int Q_AT = 2 * kProjS * STAGE;                      // the projected rows
+    static constexpr int cmax(int a, int b) { return a > b ? a : b; }
+    static constexpr int BLOCKS_AT = PROJ ? (cmax(Q_AT + 64 * G::O_STRIDE, kProjS * (cmax(SG::BLOCK, 2 * SG::PART) + 512)) + 1023) / 1024 * 1024 : 0;
+    static constexpr int LDS = BLOCKS_AT + kProjS * SG::BLOCK;
+    static_assert(!PROJ || LDS <= 160 * 1024, "LDS of a compute unit");
+    static_assert(!PROJ || kProjS * SG::BLOCK >= 4096, "fragments of W rows past the last stage's end stay inside");
+};
+__device__ __forceinline__ int quotient(int x, int d, unsigned inv) { return d == 1 ? x : static_cast<int>(__umulhi(static_cast<unsigned>(x), inv)); }
+
+// Rows q0 .. q0 + 63 of x times the D rows of W of head h, into the MFMA operand registers of the score product, rounded once to T as
+// the projection launch rounds them, in its order of additions: same bits. Wavefronts 0 to 2 multiply, 32 features of all 64 rows each
+// (two chains of products on one fragment of W, which INT8 weights are widened into once); wavefronts 3 to 5 load: an LDS-DMA
+// instruction keeps its wavefront from issuing for as long as a product takes. A round is 3 steps of 64 contraction elements, one per
+// loading wavefront; round i + 2 goes into the buffer of round i once its fragments are in registers, and last come the first key
+// blocks (request_keys), which land under the write-out of the rows.
+template <typename T, int D, int PROJ, typename Keys>
+__device__ __forceinline__ void project_rows(const ProjArgs& a, int b, int h, int q0, int Lq, int wave, int lane, unsigned char* smem, unsigned lds_base,
+                                             Keys request_keys, bool has_keys, typename Mma<T>::v8 (&qf)[HeadGeo<D>::KC]) {
+    using G = HeadGeo<D>;
+    using SG = SmallGeo<D>;
+    using PG = ProjGeo<D, PROJ>;
+    using V8 = typename Mma<T>::v8;
+    constexpr bool W8 = PROJ == 2;
+    constexpr int KEY_LOADS = 2 * SG::NP;       // DMA instructions of request_keys
+    const int lq = lane & 31, lh = lane >> 5;
+    const int n = a.n_steps, rounds = (n + kProjS - 1) / kProjS;
+    auto meet = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+    if (wave >= kProjS) {
+        const int k = wave - kProjS;
+        const unsigned char* const xg = static_cast<const unsigned char*>(a.x) + b * a.x_bsb + static_cast<long>(q0) * a.x_rsb;
+        const unsigned char* const wg = static_cast<const unsigned char*>(a.w) + static_cast<long>(h) * D * a.w_rsb;
+        unsigned xoff[PG::MX], woff[PG::MW];
+#pragma unroll
+        for (int u = 0; u < PG::MX; ++u) {
+            const int row = 8 * u + (lane >> 3);
+            xoff[u] = static_cast<unsigned>(min(row, Lq - 1 - q0)) * a.x_rsb + ((lane & 7) ^ ((row >> 1) & 7)) * 16u;
+        }
+#pragma unroll
+        for (int u = 0; u < PG::MW; ++u) {
+            const int row = W8 ? 16 * u + (lane >> 2) : 8 * u + (lane >> 3);
+            woff[u] = static_cast<unsigned>(min(row, D - 1)) * a.w_rsb + (W8 ? (lane & 3) ^ ((row >> 2) & 3) : (lane & 7) ^ ((row >> 1) & 7)) * 16u;
+        }
+        auto dma = [&](unsigned voff, const unsigned char* base, unsigned dst) {
+            asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(base), "{m0}"(dst) : "memory");
+        };
+        auto request = [&](int i) {      // this wavefront's stage of round i; behind the last round its keys
+            const int t = kProjS * i + k;
+            if (i == rounds) request_keys();
+            else if (i < rounds && t < n) {
+                const unsigned dst = lds_base + ((i & 1) * kProjS + k) * PG::STAGE;
+#pragma unroll
+                for (int u = 0; u < PG::MX; ++u) dma(xoff[u], xg + t * 128L, dst + u * 1024);
+#pragma unroll
+                for (int u = 0; u < PG::MW; ++u) dma(woff[u], wg + t * static_cast<long>(PG::WROW), dst + PG::X_BYTES + u * 1024);
+            }
+        };
+        request(0);
+        request(1);
+        for (int i = 0; i < rounds; ++i) {
+            // the stage of round i has landed: at most what was requested after it is in flight
+            if (i + 1 < rounds && kProjS * (i + 1) + k < n) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(PG::MX + PG::MW) : "memory");
+            else if (i + 1 == rounds && has_keys) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(KEY_LOADS) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            meet();
+            meet();
+            request(i + 2);
+        }
+    } else {
+        f32x16 acc[2];
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[r][e] = 0.f;
+        const bool has_features = wave < G::VB;
+        // bias and scales of this lane's features, requested here: behind the loop their latency would stand alone
+        typedef T t4 __attribute__((ext_vector_type(4)));
+        typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+        t4 bias[4];
+        f32x4_a4 scale[W8 ? 4 : 1];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int feat = h * D + min(32 * wave + 8 * g + 4 * lh, D - 4);
+            bias[g] = t4{};
+            if (a.bias) bias[g] = *reinterpret_cast<const t4*>(static_cast<const T*>(a.bias) + feat);
+            if constexpr (W8) scale[g] = *reinterpret_cast<const f32x4_a4*>(a.w_scale + feat);
+        }
+        for (int i = 0; i < rounds; ++i) {
+            meet();          // the stages of round i are there
+            const unsigned char* const st = smem + (i & 1) * kProjS * PG::STAGE;
+            using WRaw = std::conditional_t<W8, gemm::u32x2, V8>;
+            V8 xf[kProjS][4][2];
+            WRaw wf[kProjS][4];
+            // (stages past the last step hold something else: their fragments are read, not multiplied)
+            if (has_features) {
+#pragma unroll
+                for (int k = 0; k < kProjS; ++k)
+#pragma unroll
+                    for (int kk = 0; kk < 4; ++kk) {
+                        const int swz = ((2 * kk + lh) ^ ((lq >> 1) & 7)) << 4;
+#pragma unroll
+                        for (int r = 0; r < 2; ++r) xf[k][kk][r] = *reinterpret_cast<const V8*>(st + k * PG::STAGE + r * 4096 + lq * 128 + swz);
+                        wf[k][kk] = *reinterpret_cast<const WRaw*>(st + k * PG::STAGE + PG::X_BYTES + wave * 32 * PG::WROW +
+                                                                   (W8 ? lq * 64 + ((kk ^ ((lq >> 2) & 3)) << 4) + 8 * lh : lq * 128 + swz));
+                    }
+            }
+            auto multiply = [&](int k) {
+                if (!has_features || kProjS * i + k >= n) return;
+#pragma unroll
+                for (int kk = 0; kk < 4; ++kk) {
+                    V8 w;
+                    if constexpr (W8) w = gemm::widen<T>(wf[k][kk]);
+                    else w = wf[k][kk];
+#pragma unroll
+                    for (int r = 0; r < 2; ++r) acc[r] = Mma<T>::run(w, xf[k][kk][r], acc[r]);
+                }
+            };
+            multiply(0);     // (while the fragments of the other two steps arrive)
+            multiply(1);
+            meet();          // everybody holds its fragments: the buffer is free
+            if (i == rounds - 1) request_keys();
+            multiply(2);
+        }
+        // acc[r][4 g + e] is feature 32 wave + 8 g + 4 lh + e of row 32 r + lq
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int feat = 32 * wave + 8 * g + 4 * lh;
+            if (feat < D) {
+#pragma unroll
+                for (int r = 0; r < 2; ++r) {
+                    const f32x16 v = acc[r];
+                    t4 out;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        if constexpr (W8) out[e] = static_cast<T>(gemm::scaled_acc(v[4 * g + e], scale[g][e], static_cast<float>(bias[g][e])));
+                        else out[e] = static_cast<T>(v[4 * g + e] + static_cast<float>(bias[g][e]));
+                    }
+                    *reinterpret_cast<t4*>(smem + PG::Q_AT + (32 * r + lq) * G::O_STRIDE + feat * 2) = out;
+                }
+            }
+        }
+    }
+    meet();
+#pragma unroll
+    for (int c = 0; c < G::KC; ++c) {
+        u32x4 q = *reinterpret_cast<const u32x4*>(smem + PG::Q_AT + (32 * (wave & 1) + lq) * G::O_STRIDE + (2 * c + lh) * 16);
+        if (G::DK > D && c == G::KC - 1 && lh) q = u32x4{0, 0, 0, 0};
+        qf[c] = __builtin_bit_cast(V8, q);
+    }
+    meet();          // (the parts of the output will lie where the rows are)
+}
+
+template <typename T, int D, int R, bool MASKED, int PROJ>
+__global__ void __launch_bounds__(64 * kMaxWaves, PROJ ? 2 : D <= 64 ? 4 : D <= 80 ? 3 : 2)
+    sdpa_small_kernel(const SmallArgs p, const std::conditional_t<MASKED, SdpaDev, std::conditional_t<PROJ != 0, ProjArgs, NoMask>> ext) {
+    using G = HeadGeo<D>;
+    using SG = SmallGeo<D>;
+    using PG = ProjGeo<D, PROJ>;
     using V8 = typename Mma<T>::v8;
     typedef T t8 __attribute__((ext_vector_type(8)));
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -82,7 +252,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves, D <= 64 ? 4 : D <= 80 ? 3 : 2)
 
     // ── requests: this lane's query row with its RoPE entries, then the first block of keys and values ──
     QRowFrags<T, D> qr;
-    qr.issue(p, b, h, min(q0 + 32 * r + lq, p.Lq - 1), lh);
+    if constexpr (PROJ == 0) qr.issue(p, b, h, min(q0 + 32 * r + lq, p.Lq - 1), lh);
     // Visible keys [lo, hi) of this lane's row, and the blocks of the work group: those of the cached prefix, then those of the fresh
     // keys, from the first to the last that one of its rows sees; none straddles the two.
     int n_keys = p.Lk;
@@ -90,7 +260,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves, D <= 64 ? 4 : D <= 80 ? 3 : 2)
     int lo = 0, hi = n_keys, first_key = 0, stop_key = n_keys;
     WaveExtent we{0, 0, n_keys, n_keys};
     if constexpr (MASKED) {
-        row_interval(mask, b, min(q0 + 32 * r + lq, p.Lq - 1), q0 + 32 * r < p.Lq, lo, hi);
+        row_interval(ext, b, min(q0 + 32 * r + lq, p.Lq - 1), q0 + 32 * r < p.Lq, lo, hi);
         we = wave_extent(lo, hi);
         first_key = we.lo_min; stop_key = we.hi_max;
         if (R > 1) {
@@ -125,7 +295,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves, D <= 64 ? 4 : D <= 80 ? 3 : 2)
             const unsigned rsb = op ? (pre ? p.vp_rsb : p.v_rsb) : (pre ? p.kp_rsb : p.k_rsb);
             const unsigned char* const base = reinterpret_cast<const unsigned char*>(static_cast<const T*>(t) + b * bs + hk * D);
             const unsigned off = static_cast<unsigned>(min(row0 + 16 * g + prow, last)) * rsb + static_cast<unsigned>(pch) * 16u;
-            const unsigned dst = lds_base + s * SG::BLOCK + op * SG::OPER + g * 1024;
+            const unsigned dst = lds_base + PG::BLOCKS_AT + s * SG::BLOCK + op * SG::OPER + g * 1024;
             // (inline assembly: for the builtin the compiler would wait for the load in front of every later LDS read; the LDS base
             //  travels in m0, and the s_nop is the wait state an LDS-DMA instruction needs behind a write of m0)
 #pragma unroll
@@ -134,10 +304,11 @@ __global__ void __launch_bounds__(64 * kMaxWaves, D <= 64 ? 4 : D <= 80 ? 3 : 2)
                              "{m0}"(dst + pn * SG::PANEL) : "memory");
         }
     };
-    if (s < n_blocks) load_block(s);
-
     V8 qf[G::KC];
-    qr.finish(p, lh, qf);
+    if constexpr (PROJ == 0) {
+        if (s < n_blocks) load_block(s);
+        qr.finish(p, lh, qf);
+    } else project_rows<T, D, PROJ>(ext, b, h, q0, p.Lq, wave, lane, smem, lds_base, [&] { if (s < n_blocks) load_block(s); }, s < n_blocks, qf);
     const unsigned pad_keep = lh ? 0u : ~0u;
     f32x16 oacc[G::VB];
 #pragma unroll
@@ -157,7 +328,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves, D <= 64 ? 4 : D <= 80 ? 3 : 2)
         const int row0 = (pre ? pre0 + blk : fresh0 + blk - pre_blocks) * kKB, j0 = pre ? row0 : p.Lp + row0;
         const int rows = (pre ? n_pre : n_fresh) - row0;      // keys of the block
         const bool mine = blk < n_blocks && (!MASKED || (j0 < we.hi_max && j0 + kKB > we.lo_min));
-        const unsigned char* const buf = smem + s * SG::BLOCK;
+        const unsigned char* const buf = smem + PG::BLOCKS_AT + s * SG::BLOCK;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         if (R > 1) __syncthreads();
         V8 kf[G::KC], vf[2][G::VB];
@@ -352,14 +523,7 @@ SmallPlan plan_small(const SdpaDev& p, int D, int n_cu) {
     return {4, nb <= (D <= 64 ? 6 : 8) ? 4 : kMaxWaves};
 }
 
-template <typename T, int D, int R, bool MASKED>
-int launch_small(const SdpaDev& p, int most_waves, hipStream_t stream) {
-    using SG = SmallGeo<D>;
-    const int n_kb = key_blocks(p);
-    int S = max(1, min(min(n_kb, most_waves / R), kMaxLds / (max(SG::BLOCK, R * SG::PART) + 256 * R)));
-    const int steps = (n_kb + S - 1) / S;
-    S = max(1, (n_kb + steps - 1) / max(steps, 1));      // as few wavefronts as take that many steps
-    const int lds = S == 1 ? max(SG::BLOCK, 32 * R * HeadGeo<D>::O_STRIDE) : S * (max(SG::BLOCK, R * SG::PART) + 256 * R);
+SmallArgs small_args(const SdpaDev& p, int R, int S) {
     SmallArgs a{};
     a.q = p.q; a.k = p.k; a.v = p.v; a.kp = p.kp; a.vp = p.vp; a.o = p.o;
     a.kv_valid_len = p.kv_valid_len; a.cos_q = p.cos_q; a.sin_q = p.sin_q; a.rope_split = p.rope_split;
@@ -372,9 +536,21 @@ int launch_small(const SdpaDev& p, int most_waves, hipStream_t stream) {
     a.n_blocks = p.B * p.H * a.n_q_tiles;
     auto inverse = [](int d) { return static_cast<unsigned>(((1ull << 32) + d - 1) / static_cast<unsigned>(d)); };      // (not used for 1)
     a.inv_tiles = inverse(a.n_q_tiles); a.inv_heads = inverse(a.H); a.inv_group = inverse(a.kv_group);
+    return a;
+}
+
+template <typename T, int D, int R, bool MASKED>
+int launch_small(const SdpaDev& p, int most_waves, hipStream_t stream) {
+    using SG = SmallGeo<D>;
+    const int n_kb = key_blocks(p);
+    int S = max(1, min(min(n_kb, most_waves / R), kMaxLds / (max(SG::BLOCK, R * SG::PART) + 256 * R)));
+    const int steps = (n_kb + S - 1) / S;
+    S = max(1, (n_kb + steps - 1) / max(steps, 1));      // as few wavefronts as take that many steps
+    const int lds = S == 1 ? max(SG::BLOCK, 32 * R * HeadGeo<D>::O_STRIDE) : S * (max(SG::BLOCK, R * SG::PART) + 256 * R);
+    SmallArgs a = small_args(p, R, S);
     const dim3 grid((a.n_blocks + 7) / 8 * 8), block(64 * R * S);
-    if constexpr (MASKED) hipLaunchKernelGGL((sdpa_small_kernel<T, D, R, true>), grid, block, lds, stream, a, p);
-    else hipLaunchKernelGGL((sdpa_small_kernel<T, D, R, false>), grid, block, lds, stream, a, NoMask{});
+    if constexpr (MASKED) hipLaunchKernelGGL((sdpa_small_kernel<T, D, R, true, 0>), grid, block, lds, stream, a, p);
+    else hipLaunchKernelGGL((sdpa_small_kernel<T, D, R, false, 0>), grid, block, lds, stream, a, NoMask{});
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail("sdpa_fwd launch: %s", hipGetErrorString(e));
     return 0;
@@ -404,7 +580,55 @@ int launch_small_t(const SdpaDev& p, int head_dim, const SmallPlan& plan, hipStr
     }
 }
 
+// ── cached cross-attention with its query projection in one launch ──
+template <typename T, int D, int PROJ>
+int launch_projected(const SdpaDev& p, const ProjArgs& proj, hipStream_t stream) {
+    using PG = ProjGeo<D, PROJ>;
+    static thread_local bool raised = false;
+    if (!raised) {
+        MI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&sdpa_small_kernel<T, D, 2, false, PROJ>), hipFuncAttributeMaxDynamicSharedMemorySize, PG::LDS));
+        raised = true;
+    }
+    const SmallArgs a = small_args(p, 2, kProjS);
+    hipLaunchKernelGGL((sdpa_small_kernel<T, D, 2, false, PROJ>), dim3((a.n_blocks + 7) / 8 * 8), dim3(64 * 2 * kProjS), PG::LDS, stream, a, proj);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail("sdpa_fwd launch: %s", hipGetErrorString(e));
+    return 0;
+}
+template <typename T>
+int launch_projected_t(const SdpaDev& p, const ProjArgs& proj, int head_dim, hipStream_t stream) {
+    if (head_dim == 40) return proj.w_scale ? launch_projected<T, 40, 2>(p, proj, stream) : launch_projected<T, 40, 1>(p, proj, stream);
+    return proj.w_scale ? launch_projected<T, 80, 2>(p, proj, stream) : launch_projected<T, 80, 1>(p, proj, stream);
+}
+
 }  // namespace
+
+// Where one launch less is worth the rows of x that every head projects for itself: up to a work group of 64 rows per compute unit (8
+// heads, 77 keys, 16-bit weights, the whole block with its output projection in us, before / here: 40 of 320 channels, 8 groups 10.2 /
+// 9.6, 256 13.8 / 11.7, 480 16.1 / 17.0; 80 of 640, 8 groups 11.7 / 12.7, 128 15.0 / 15.0, 144 15.9 / 15.0, 256 19.3 / 17.2, 480 26.2 /
+// 27.0; INT8 weights: 40, 256 14.3 / 12.1, 80, 256 20.8 / 18.0; 231 keys 15.6 / 13.5 and 22.5 / 19.7). Not measured, so not taken: more
+// than 640 channels or 256 keys.
+bool sdpa_projected_takes(const SdpaDev& p, const LinearProblem& q, int head_dim) {
+    if (head_dim != 40 && head_dim != 80) return false;
+    if (sdpa_kernel_choice() != 0 || p.Lk < 1 || !sdpa_flow_runs(p) || p.kv_valid_len || p.cos_q || p.Lp != 0 || p.o_rs >= (1L << 30)) return false;
+    // the projection's own conditions (launch_linear checks the rest, with its messages, when a call goes there)
+    const uintptr_t al = reinterpret_cast<uintptr_t>(q.x) | reinterpret_cast<uintptr_t>(q.w) | reinterpret_cast<uintptr_t>(q.bias) | reinterpret_cast<uintptr_t>(p.k) |
+                         reinterpret_cast<uintptr_t>(p.v) | reinterpret_cast<uintptr_t>(p.o);
+    if ((al & 15u) || (reinterpret_cast<uintptr_t>(q.w_scale) & 3u) || q.K <= 0 || q.K % 64 != 0 || q.N % 8 != 0 || q.ldx % 8 != 0 || q.ldw % 16 != 0) return false;
+    if (static_cast<long>(q.ldx) * 2 * 64 >= (1L << 31) || static_cast<long>(q.ldw) * 2 * 80 >= (1L << 31)) return false;
+    const long groups = static_cast<long>(p.B) * p.H * ((p.Lq + 63) / 64);
+    const int n_cu = device_cu_count();
+    return groups <= n_cu && (head_dim == 40 || 2 * groups > n_cu) && q.K <= 640 && key_blocks(p) <= 8;
+}
+
+int launch_sdpa_projected(const SdpaDev& p, const LinearProblem& q, int dtype, int head_dim, hipStream_t stream) {
+    ProjArgs a{};
+    a.x = q.x; a.w = q.w; a.bias = q.bias; a.w_scale = q.w_scale;
+    a.x_bsb = static_cast<long>(p.Lq) * q.ldx * 2;
+    a.x_rsb = static_cast<unsigned>(q.ldx) * 2u; a.w_rsb = static_cast<unsigned>(q.ldw) * (q.w_scale ? 1u : 2u); a.n_steps = q.K / 64;
+    if (dtype == MI_DTYPE_BF16) return launch_projected_t<__bf16>(p, a, head_dim, stream);
+    return launch_projected_t<_Float16>(p, a, head_dim, stream);
+}
 
 int launch_sdpa_small(const SdpaDev& p, int dtype, int head_dim, hipStream_t stream) {
     const SmallPlan plan = plan_small(p, head_dim, device_cu_count());
