@@ -29,7 +29,7 @@
 //
 // Measured (fp16 / bf16, one launch, us; first: 64 x 64 tiles through registers, one step ahead; then: this pipeline with the fixed part
 // as it was; now, with the tiles that the rule below takes): 4096 x 1152 x 1152 30 / 16.9 / 14.5 to 17.3 (192 x 128 tiles; it differs
-// from GPU to GPU); 1024 x 2240 x 2240 30 / 16.3 / 16.1; 2048 x 640 x 640 8.4 / 6.9 / 6.0 (INT8 weights 11.5 / 7.8 / 6.4);
+// from GPU to GPU); 1024 x 2240 x 2240 30 / 16.3 / 14.8; 2048 x 640 x 640 8.4 / 6.9 / 6.0 (INT8 weights 11.5 / 7.8 / 6.4);
 // 128 x 1280 x 1280 8.2 / 6.4 / 4.6 (INT8 - / 8.2 / 5.7), three of them - / 6.9 / 5.7 (INT8 - / 8.7 / 6.7); 256 x 1152 x 1152 - / 6.2 / 5.0;
 // 3072 x 640 x 2560 - / 17.4 / 15.8; GEGLU 3072 x 640 -> 2 x 2560 39 / 32.0 / 29; three of 16384 x 512 x 512 - / 42.3 / 36.
 #include <cmath>
@@ -451,18 +451,21 @@ int launch_pipe(const LinearBatch& batch, int n_problems, hipStream_t st) {
 // next (6144 x 320 x 320, three of them). Large tiles need fewer bytes per FLOP: a compute unit takes 1 KB from its L2 in 16 to 24
 // clocks, so a step of 128 x 128 (32 KB) takes 600 to 700 where its products take 512, one of 128 x 64 (24 KB) 450 to 650 where they take
 // 256. Small ones fill the GPU: 128 x 1280 x 1280 takes 4.6 us with 160 tiles of 32 x 32, 5.3 with 80 of 64 x 32, 8.6 with 20 of
-// 128 x 64; 1024 x 2240 x 2240 takes 16 us with 144 tiles of 128 x 128, 22 with 280 of 128 x 64, 50 with 36 of 256 x 256.
+// 128 x 64; 1024 x 2240 x 2240 takes 15 us with 192 tiles of 128 x 96, 22 with 280 of 128 x 64, 50 with 36 of 256 x 256.
+// The tiles 96 features wide (constants from 17 problems of their own) are for the counts between: 1024 x 2240 x 2240 16.7 -> 14.8 us on
+// 192 tiles of 128 x 96, 2048 x 1152 x 1152 10.3 -> 9.0, 2048 x 640 x 2560 15.0 -> 12.6 on 224 of 64 x 96. Wavefronts that own 128 x 64
+// or 96 x 64 instead of 64 x 64 (a quarter fewer LDS reads) gave nothing: 1024 x 6720 x 2240 32.8 -> 32.9.
 // Loading wavefronts (see the top) pay where the products of a step are short. They are no help where a compute unit holds two work
 // groups of large register use: GEGLU 3072 x 640 -> 2 x 2560 31 -> 36 us, three of 16384 x 512 x 512 37 -> 44.
 struct Form {
     int bm, bn_out;
     float phi, lam, tau, eps;
 };
-enum { k32x32, k64x32, k64x64, k128x64_load, k128x64, k128x128, k128x128_2, k192x128, k256x128, k256x256, kPlainForms };
+enum { k32x32, k64x32, k64x64, k64x96, k128x64_load, k128x64, k128x96, k128x128, k128x128_2, k192x128, k256x128, k256x256, kPlainForms };
 constexpr Form kPlain[kPlainForms] = {{32, 32, 2.46f, 0.091f, 0.058f, 0.22f},   {64, 32, 2.60f, 0.111f, 0.126f, 0.34f},   {64, 64, 2.52f, 0.154f, 0.190f, 0.42f},
-                                      {128, 64, 2.53f, 0.250f, 0.322f, 0.76f},  {128, 64, 2.57f, 0.274f, 0.322f, 0.59f},  {128, 128, 3.95f, 0.356f, 0.529f, 3.18f},
-                                      {128, 128, 3.19f, 0.515f, 0.465f, 1.20f}, {192, 128, 4.67f, 0.511f, 0.727f, 4.11f}, {256, 128, 5.03f, 0.656f, 0.839f, 6.17f},
-                                      {256, 256, 8.05f, 1.379f, 1.789f, 6.40f}};
+                                      {64, 96, 3.10f, 0.225f, 0.240f, 1.50f},   {128, 64, 2.53f, 0.250f, 0.322f, 0.76f},  {128, 64, 2.57f, 0.274f, 0.322f, 0.59f},
+                                      {128, 96, 3.50f, 0.318f, 0.360f, 2.30f},  {128, 128, 3.95f, 0.356f, 0.529f, 3.18f}, {128, 128, 3.19f, 0.515f, 0.465f, 1.20f},
+                                      {192, 128, 4.67f, 0.511f, 0.727f, 4.11f}, {256, 128, 5.03f, 0.656f, 0.839f, 6.17f}, {256, 256, 8.05f, 1.379f, 1.789f, 6.40f}};
 // INT8 weights: the widening makes small steps dearer and the large tiles no better (those above 128 x 128 are not built)
 enum { k8_32x32, k8_64x64, k8_128x64, k8_128x128, k8_128x128_2, kPlainW8Forms };
 constexpr Form kPlainW8[kPlainW8Forms] = {{32, 32, 2.47f, 0.155f, 0.049f, 0.33f},
@@ -528,7 +531,9 @@ int launch_form(const LinearBatch& b, int n, bool geglu, int dtype, hipStream_t 
         case k32x32: return launch_pipe<T, false, false, 1, 1, 1, 1, 6, 2>(b, n, st);
         case k64x32: return launch_pipe<T, false, false, 2, 1, 1, 1, 6, 2>(b, n, st);
         case k64x64: return launch_pipe<T, false, false, 2, 2, 1, 1, 4, 4>(b, n, st);
+        case k64x96: return launch_pipe<T, false, false, 2, 3, 1, 1, 5, 4>(b, n, st);
         case k128x64_load: return launch_pipe<T, false, false, 2, 2, 2, 1, 3, 4>(b, n, st);
+        case k128x96: return launch_pipe<T, false, false, 2, 3, 2, 1, 4, 4>(b, n, st);
         case k128x64: return launch_pipe<T, false, false, 2, 2, 2, 1, 3, 0>(b, n, st);
         case k128x128: return launch_pipe<T, false, false, 2, 2, 2, 2, 3, 4>(b, n, st);
         case k128x128_2: return launch_pipe<T, false, false, 2, 2, 2, 2, 2, 0>(b, n, st);

@@ -120,3 +120,18 @@ def test_pipe_scales_start_at_any_float(oracle, M, N, K):
     longer[1:-1] = s
     assert longer[1:-1].data_ptr() % 16 == 4
     assert torch.equal(bd.linear_forward_batched_int8w_fp16(w, longer[1:-1], None, x), bd.linear_forward_batched_int8w_fp16(w, s, None, x))
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("M,N,K", [(1024, 2240, 2240), (962, 2184, 2240), (2048, 1152, 1152), (2048, 640, 2560), (1985, 616, 2560), (1999, 584, 2624)])
+def test_tiles_96_features_wide(oracle, dtype, M, N, K):
+    """128 x 96 and 64 x 96 tiles, whole and with a last column of 72, 40 and 8 features and ragged last rows; the row behind stays."""
+    x = randn(8600 + M, (M, K), dtype)
+    w = _weight(oracle, 8601 + N, N, K, dtype)
+    b = oracle.round_to(0.3 * randn(8602, (N,), "fp32"), dtype)
+    got = bd.linear_batched(to_dev(w, dtype), to_dev(b, dtype), to_dev(x, dtype))
+    rows = _rows(M)
+    _one_ulp(oracle.linear(x[rows], w, b), to_np(got)[rows], dtype, "plain")
+    out = torch.full((M + 1, N), 7.0, dtype=got.dtype, device="cuda")
+    bd.linear_batched(to_dev(w, dtype), to_dev(b, dtype), to_dev(x, dtype), out[:M])
+    assert torch.equal(out[:M], got) and (out[M:] == 7).all()
