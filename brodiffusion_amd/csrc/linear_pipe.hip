@@ -29,7 +29,7 @@
 //
 // Measured (fp16 / bf16, one launch, us; first: 64 x 64 tiles through registers, one step ahead; then: this pipeline with the fixed part
 // as it was; now, with the tiles that the rule below takes): 4096 x 1152 x 1152 30 / 16.9 / 14.5 to 17.3 (192 x 128 tiles; it differs
-// from GPU to GPU); 1024 x 2240 x 2240 30 / 16.3 / 14.8; 2048 x 640 x 640 8.4 / 6.9 / 6.0 (INT8 weights 11.5 / 7.8 / 6.4);
+// from GPU to GPU); 1024 x 2240 x 2240 30 / 16.3 / 14.8; 2048 x 640 x 640 8.4 / 6.9 / 6.0 (INT8 weights 11.5 / 7.8 / 5.8);
 // 128 x 1280 x 1280 8.2 / 6.4 / 4.6 (INT8 - / 8.2 / 5.7), three of them - / 6.9 / 5.7 (INT8 - / 8.7 / 6.7); 256 x 1152 x 1152 - / 6.2 / 5.0;
 // 3072 x 640 x 2560 - / 17.4 / 15.8; GEGLU 3072 x 640 -> 2 x 2560 39 / 32.0 / 29; three of 16384 x 512 x 512 - / 42.3 / 36.
 #include <cmath>
@@ -453,7 +453,8 @@ int launch_pipe(const LinearBatch& batch, int n_problems, hipStream_t st) {
 // 256. Small ones fill the GPU: 128 x 1280 x 1280 takes 4.6 us with 160 tiles of 32 x 32, 5.3 with 80 of 64 x 32, 8.6 with 20 of
 // 128 x 64; 1024 x 2240 x 2240 takes 15 us with 192 tiles of 128 x 96, 22 with 280 of 128 x 64, 50 with 36 of 256 x 256.
 // The tiles 96 features wide (constants from 17 problems of their own) are for the counts between: 1024 x 2240 x 2240 16.7 -> 14.8 us on
-// 192 tiles of 128 x 96, 2048 x 1152 x 1152 10.3 -> 9.0, 2048 x 640 x 2560 15.0 -> 12.6 on 224 of 64 x 96. Wavefronts that own 128 x 64
+// 192 tiles of 128 x 96, 2048 x 1152 x 1152 10.3 -> 9.0, 2048 x 640 x 2560 15.0 -> 12.6 on 224 of 64 x 96; INT8
+// 2048 x 640 x 640 6.4 -> 5.8, 1024 x 1280 x 1280 9.4 -> 8.2, 4096 x 640 x 640 8.7 -> 7.7. Wavefronts that own 128 x 64
 // or 96 x 64 instead of 64 x 64 (a quarter fewer LDS reads) gave nothing: 1024 x 6720 x 2240 32.8 -> 32.9.
 // Loading wavefronts (see the top) pay where the products of a step are short. They are no help where a compute unit holds two work
 // groups of large register use: GEGLU 3072 x 640 -> 2 x 2560 31 -> 36 us, three of 16384 x 512 x 512 37 -> 44.
@@ -467,10 +468,12 @@ constexpr Form kPlain[kPlainForms] = {{32, 32, 2.46f, 0.091f, 0.058f, 0.22f},   
                                       {128, 96, 3.50f, 0.318f, 0.360f, 2.30f},  {128, 128, 3.95f, 0.356f, 0.529f, 3.18f}, {128, 128, 3.19f, 0.515f, 0.465f, 1.20f},
                                       {192, 128, 4.67f, 0.511f, 0.727f, 4.11f}, {256, 128, 5.03f, 0.656f, 0.839f, 6.17f}, {256, 256, 8.05f, 1.379f, 1.789f, 6.40f}};
 // INT8 weights: the widening makes small steps dearer and the large tiles no better (those above 128 x 128 are not built)
-enum { k8_32x32, k8_64x64, k8_128x64, k8_128x128, k8_128x128_2, kPlainW8Forms };
+enum { k8_32x32, k8_64x64, k8_64x96, k8_128x64, k8_128x96, k8_128x128, k8_128x128_2, kPlainW8Forms };
 constexpr Form kPlainW8[kPlainW8Forms] = {{32, 32, 2.47f, 0.155f, 0.049f, 0.33f},
                                           {64, 64, 2.75f, 0.209f, 0.187f, 0.80f},
+                                          {64, 96, 3.30f, 0.245f, 0.235f, 0.90f},
                                           {128, 64, 3.03f, 0.325f, 0.286f, 1.43f},
+                                          {128, 96, 4.00f, 0.350f, 0.360f, 1.50f},
                                           {128, 128, 4.03f, 0.420f, 0.562f, 3.98f},
                                           {128, 128, 2.89f, 0.658f, 0.382f, 3.13f}};
 enum { kG64x64, kG128x64_2, kG128x64, kG256x64, kGegluForms };   // output features; the W tile holds twice as many rows
@@ -522,7 +525,9 @@ int launch_form(const LinearBatch& b, int n, bool geglu, int dtype, hipStream_t 
         switch (pick_form(kPlainW8, kPlainW8Forms, b, n)) {
             case k8_32x32: return launch_pipe<T, true, false, 1, 1, 1, 1, 6, 2>(b, n, st);
             case k8_64x64: return launch_pipe<T, true, false, 2, 2, 1, 1, 4, 4>(b, n, st);
+            case k8_64x96: return launch_pipe<T, true, false, 2, 3, 1, 1, 5, 2>(b, n, st);
             case k8_128x64: return launch_pipe<T, true, false, 2, 2, 2, 1, 3, 4>(b, n, st);
+            case k8_128x96: return launch_pipe<T, true, false, 2, 3, 2, 1, 3, 2>(b, n, st);
             case k8_128x128: return launch_pipe<T, true, false, 2, 4, 2, 1, 4, 0>(b, n, st);
             default: return launch_pipe<T, true, false, 2, 2, 2, 2, 2, 0>(b, n, st);
         }

@@ -135,3 +135,15 @@ def test_tiles_96_features_wide(oracle, dtype, M, N, K):
     out = torch.full((M + 1, N), 7.0, dtype=got.dtype, device="cuda")
     bd.linear_batched(to_dev(w, dtype), to_dev(b, dtype), to_dev(x, dtype), out[:M])
     assert torch.equal(out[:M], got) and (out[M:] == 7).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(2048, 640, 640), (1985, 616, 640), (2000, 584, 64), (4096, 640, 640), (4037, 600, 704), (8192, 320, 128)])
+def test_int8_tiles_96_features_wide(oracle, M, N, K):
+    x = randn(8700 + M, (M, K), "fp16")
+    w, s = _int8(8701 + N, N, K)
+    b = oracle.round_to(0.3 * randn(8702, (N,), "fp32"), "fp16")
+    out = torch.full((M + 1, N), 7.0, dtype=torch.float16, device="cuda")
+    bd.linear_forward_batched_int8w_fp16(torch.from_numpy(w).cuda(), torch.from_numpy(s).cuda(), to_dev(b, "fp16"), to_dev(x, "fp16"), out[:M])
+    rows = _rows(M)
+    _one_ulp(oracle.linear(x[rows], w.astype(np.float32) * s, b), to_np(out)[rows], "fp16", "int8")
+    assert (out[M:] == 7).all()
