@@ -452,8 +452,9 @@ int launch_pipe(const LinearBatch& batch, int n_problems, hipStream_t st) {
 // clocks, so a step of 128 x 128 (32 KB) takes 600 to 700 where its products take 512, one of 128 x 64 (24 KB) 450 to 650 where they take
 // 256. Small ones fill the GPU: 128 x 1280 x 1280 takes 4.6 us with 160 tiles of 32 x 32, 5.3 with 80 of 64 x 32, 8.6 with 20 of
 // 128 x 64; 1024 x 2240 x 2240 takes 15 us with 192 tiles of 128 x 96, 22 with 280 of 128 x 64, 50 with 36 of 256 x 256.
-// The tiles 96 features wide (constants from 17 problems of their own) are for the counts between: 1024 x 2240 x 2240 16.7 -> 14.8 us on
-// 192 tiles of 128 x 96, 2048 x 1152 x 1152 10.3 -> 9.0, 2048 x 640 x 2560 15.0 -> 12.6 on 224 of 64 x 96; INT8
+// The tiles 96 features wide and the GEGLU tile of 192 x 128 (constants from 17 problems of their own) are for the counts between: 1024 x 2240 x 2240 16.7 -> 14.8 us on
+// 192 tiles of 128 x 96, 2048 x 1152 x 1152 10.3 -> 9.0, 2048 x 640 x 2560 15.0 -> 12.6 on 224 of 64 x 96; GEGLU 2048 x 640 ->
+// 2 x 2560 21.9 -> 19.1 and 1024 x 1280 -> 2 x 5120 37.3 -> 31.6 (INT8 24.1 -> 22.2, 40.9 -> 35.1) on 220 and 240 of 192 x 128; INT8
 // 2048 x 640 x 640 6.4 -> 5.8, 1024 x 1280 x 1280 9.4 -> 8.2, 4096 x 640 x 640 8.7 -> 7.7. Wavefronts that own 128 x 64
 // or 96 x 64 instead of 64 x 64 (a quarter fewer LDS reads) gave nothing: 1024 x 6720 x 2240 32.8 -> 32.9.
 // Loading wavefronts (see the top) pay where the products of a step are short. They are no help where a compute unit holds two work
@@ -476,11 +477,12 @@ constexpr Form kPlainW8[kPlainW8Forms] = {{32, 32, 2.47f, 0.155f, 0.049f, 0.33f}
                                           {128, 96, 4.00f, 0.350f, 0.360f, 1.50f},
                                           {128, 128, 4.03f, 0.420f, 0.562f, 3.98f},
                                           {128, 128, 2.89f, 0.658f, 0.382f, 3.13f}};
-enum { kG64x64, kG128x64_2, kG128x64, kG256x64, kGegluForms };   // output features; the W tile holds twice as many rows
+enum { kG64x64, kG128x64_2, kG128x64, kG256x64, kG192x128, kGegluForms };   // output features; the W tile holds twice as many rows
 constexpr Form kGeglu[kGegluForms] = {{64, 64, 2.65f, 0.377f, 0.330f, 1.20f}, {128, 64, 3.66f, 0.648f, 0.496f, 2.09f}, {128, 64, 4.41f, 0.442f, 0.588f, 4.08f},
-                                      {256, 64, 5.99f, 0.800f, 0.834f, 8.98f}};
-enum { kG8_64x64, kG8_128x64_2, kG8_256x64, kGegluW8Forms };
-constexpr Form kGegluW8[kGegluW8Forms] = {{64, 64, 3.92f, 0.315f, 0.302f, 1.17f}, {128, 64, 3.92f, 0.653f, 0.429f, 2.93f}, {256, 64, 7.90f, 0.816f, 1.031f, 6.53f}};
+                                      {256, 64, 5.99f, 0.800f, 0.834f, 8.98f}, {192, 128, 7.00f, 1.200f, 1.250f, 7.00f}};
+enum { kG8_64x64, kG8_128x64_2, kG8_256x64, kG8_192x128, kGegluW8Forms };
+constexpr Form kGegluW8[kGegluW8Forms] = {{64, 64, 3.92f, 0.315f, 0.302f, 1.17f}, {128, 64, 3.92f, 0.653f, 0.429f, 2.93f}, {256, 64, 7.90f, 0.816f, 1.031f, 6.53f},
+                                          {192, 128, 9.30f, 1.290f, 1.500f, 5.50f}};
 
 // 256 x 256 tiles take contractions from 512 on (below, their prologue is most of the launch).
 int pick_form(const Form* forms, int n_forms, const LinearBatch& batch, int n_problems) {
@@ -510,6 +512,7 @@ int launch_form(const LinearBatch& b, int n, bool geglu, int dtype, hipStream_t 
         switch (pick_form(kGegluW8, kGegluW8Forms, b, n)) {
             case kG8_64x64: return launch_pipe<T, true, true, 2, 2, 1, 2, 3, 0>(b, n, st);
             case kG8_128x64_2: return launch_pipe<T, true, true, 2, 2, 2, 2, 2, 0>(b, n, st);
+            case kG8_192x128: return launch_pipe<T, true, true, 2, 4, 3, 2, 3, 0>(b, n, st);
             default: return launch_pipe<T, true, true, 4, 2, 2, 2, 3, 0>(b, n, st);
         }
     }
@@ -518,6 +521,7 @@ int launch_form(const LinearBatch& b, int n, bool geglu, int dtype, hipStream_t 
             case kG64x64: return launch_pipe<T, false, true, 2, 2, 1, 2, 3, 4>(b, n, st);
             case kG128x64_2: return launch_pipe<T, false, true, 2, 2, 2, 2, 2, 0>(b, n, st);
             case kG128x64: return launch_pipe<T, false, true, 2, 2, 2, 2, 3, 4>(b, n, st);
+            case kG192x128: return launch_pipe<T, false, true, 2, 4, 3, 2, 2, 0>(b, n, st);
             default: return launch_pipe<T, false, true, 4, 2, 2, 2, 3, 0>(b, n, st);
         }
     }

@@ -147,3 +147,22 @@ def test_int8_tiles_96_features_wide(oracle, M, N, K):
     rows = _rows(M)
     _one_ulp(oracle.linear(x[rows], w.astype(np.float32) * s, b), to_np(out)[rows], "fp16", "int8")
     assert (out[M:] == 7).all()
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("M,N,K", [(2048, 2560, 640), (1985, 2536, 640), (1024, 5120, 1280)])
+def test_geglu_tiles_192_rows(oracle, dtype, M, N, K):
+    """192 x 128 GEGLU tiles, whole and ragged, against the checker's layer with exact GELU on FP32 halves."""
+    x = randn(8800 + M, (M, K), dtype)
+    w = _weight(oracle, 8801 + N, 2 * N, K, dtype)
+    b = oracle.round_to(0.3 * randn(8802, (2 * N,), "fp32"), dtype)
+    out = torch.full((M + 1, N), 7.0, dtype=to_dev(b, dtype).dtype, device="cuda")
+    bd.fused_linear_geglu(to_dev(x, dtype), to_dev(w, dtype), to_dev(b, dtype), out[:M])
+    rows = _rows(M)
+    _one_ulp(oracle.geglu_exact(oracle.linear(x[rows], w, b)), to_np(out)[rows], dtype, "geglu")
+    assert (out[M:] == 7).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(2048, 2560, 640), (1985, 2536, 640)])
+def test_int8_geglu_tiles_192_rows(oracle, M, N, K):
+    test_pipe_geglu_is_the_linear_layer_and_the_gate(oracle, "fp16", True, M, N, K)
