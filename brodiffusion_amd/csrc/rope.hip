@@ -20,12 +20,13 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 // left the LDS permutation network for DPP moves.
 struct RowUnits {
     int units, rb, threads;      // of a row; rows and threads of a block
-    unsigned inv;                // ceil(2^32 / units): t / units exactly for t * units < 2^32
+    unsigned inv;                // ceil(2^32 / units): t / units exactly for t * units < 2^32 (0, and no division, with one row to a block)
     long blocks;
     RowUnits(long rows, int units_) : units(units_), rb(1), inv(0xffffffffu / static_cast<unsigned>(units_) + 1u) {
         // the number of rows that leaves the fewest lanes of the block's last wavefront empty
         for (int n = 2, best = (units + 63) / 64 * 64 - units; n * units <= 256; ++n)
             if (const int empty = (n * units + 63) / 64 * 64 - n * units; empty * rb <= best * n) { rb = n; best = empty; }
+        if (rb == 1) inv = 0;
         threads = rb * units < 256 ? (rb * units + 63) / 64 * 64 : 256;
         blocks = (rows + rb - 1) / rb;
     }
@@ -330,7 +331,7 @@ int launch_headnorm(const mi_headnorm_rope_args* a, long x_rs, long o_rs, long o
     T* o2 = static_cast<T*>(a->out2);
     const T* g = static_cast<const T*>(a->gain);
     const int r2 = a->out2 ? a->out2_rows : 0;
-    const bool four = a->num_heads % 4 == 0;
+    const bool four = a->num_heads % 4 == 0 && static_cast<long>(a->num_heads) * a->head_dim < (1L << 30);
     auto launch_four = [&](auto kernel, int cpr) {
         const RowUnits ru(a->rows, a->num_heads / 4 * cpr);
         hipLaunchKernelGGL(kernel, dim3(ru.grid()), dim3(ru.threads), 0, st, x, o, o2, g, a->cos, a->sin, a->rows, a->eps, x_rs, o_rs, o2_rs, r2, ru);

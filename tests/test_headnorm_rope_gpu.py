@@ -115,7 +115,8 @@ def test_prefix_dial_equals_scaled_keys_and_values(oracle):
 
 
 @pytest.mark.parametrize("split_half", [False, True])
-@pytest.mark.parametrize("L,H,d", [(1, 4, 32), (257, 4, 32), (5, 12, 64), (1024, 20, 128), (3, 64, 128), (7, 68, 128), (130, 160, 64)])
+@pytest.mark.parametrize("L,H,d", [(1, 4, 32), (257, 4, 32), (5, 12, 64), (1024, 20, 128), (3, 64, 128), (7, 68, 128), (130, 160, 64),
+                                   (3, 20000, 128)])      # more chunk positions to a row than a 32-bit inverse divides by
 def test_four_heads_per_thread(oracle, split_half, L, H, d):
     """Rows per block from one to many, rows of whole and of part wavefronts, rows longer than a block; in place; first rows copied out.
     Against the checker, and bit for bit against the kernels with one chunk per thread (a tensor of one head more)."""
