@@ -127,6 +127,24 @@ struct MapDev {
 };
 int launch_attention_map(const MapDev& p, int dtype, int head_dim, hipStream_t stream);
 
+// Whether two 16-bit operands of `batch` items of `rows` rows of `len` elements (row strides of at least a row, any batch strides, in
+// elements) can share an element. Column slices of one buffer share none; where strides differ, overlapping address ranges count.
+inline bool operands_overlap(const void* a, long a_rs, long a_bs, const void* b, long b_rs, long b_bs, long batch, long rows, long len) {
+    auto reach = [&](long rs, long bs, long& first, long& last) {
+        const long items = (batch - 1) * bs;
+        first = items < 0 ? items : 0;
+        last = (items > 0 ? items : 0) + (rows - 1) * rs + len;
+    };
+    long a0, a1, b0, b1;
+    reach(a_rs, a_bs, a0, a1);
+    reach(b_rs, b_bs, b0, b1);
+    const long apart = (static_cast<long>(reinterpret_cast<intptr_t>(a)) - static_cast<long>(reinterpret_cast<intptr_t>(b))) / 2;      // elements from b to a
+    if (apart + a0 >= b1 || apart + a1 <= b0) return false;
+    if (a_rs != b_rs || (batch > 1 && (a_bs % a_rs != 0 || b_bs % a_rs != 0))) return true;
+    const long column = (apart % a_rs + a_rs) % a_rs;      // a's first column among b's
+    return column < len || column > a_rs - len;
+}
+
 // One Y = X W^T + bias problem: X (M, K), W (N, K), Y (M, N), bias (N) or null; strides in elements.
 struct LinearProblem {
     const void* x; const void* w; const void* bias; void* y;

@@ -89,6 +89,7 @@ struct LinDev {
     int n_blocks;   // work groups with work = B * H * n_chunks
     int form;       // MI_LINEAR_ATTN_FORM_*
     int channel_major;   // operands are (heads * head_dim, tokens) per batch item; row strides are between channel rows
+    bool o_over_q, o_over_k;   // O shares memory with Q or with K (host only)
 };
 constexpr int kFusedMaxTokens = 1024;   // up to here the one-launch form is taken for sliced heads when the kernel is picked by size
 
@@ -1282,7 +1283,8 @@ int launch_d(LinDev p, bool accumulate, int max_split, int n_cu, hipStream_t st)
     {
         using FG = FusedGeo<D>;
         const int groups = BH * FG::NS;
-        const bool fits = !accumulate && static_cast<long>(BH) * FG::NS < (1L << 24);
+        // (nor where O lies on Q, whose last unit several wavefronts fetch and write, or, with several slices, on the K that the others read)
+        const bool fits = !accumulate && static_cast<long>(BH) * FG::NS < (1L << 24) && !p.o_over_q && (FG::NS == 1 || !p.o_over_k);
         // Picked by size (measured, 256 compute units; us, several launches / one): with one slice per head (head_dim 32) nothing is
         // read twice, but a work group streams all tokens of its head (20 heads, 512 tokens 6.2 / 5.6, 777 6.7 / 7.2, 4096 10.5 /
         // 25.4; 70 heads, 1024 9.2 / 8.8, 1500 10.5 / 11.8, 4096 18.7 / 26.3; 140 heads, 4096 30.9 / 28.9); with several slices every
@@ -1315,7 +1317,9 @@ int launch_d(LinDev p, bool accumulate, int max_split, int n_cu, hipStream_t st)
         // two groups per CU measured slower, a power of two leaves a third of the CUs idle)
         int split = 1;
         // (without a reduction launch one tile: 20 heads of 112, 256 tokens 12.8 / 9.9, 1024 16.4 / 16.1; with one, 256 tokens 12.8 / 13.9)
-        const bool may_sum = !accumulate && max_split > 0 && static_cast<long>(BH) * p.N * (G::NB - 1) <= 840L * n_cu;
+        // (its slices of a head each read whole rows of Q and write their columns of O: not where O is Q, whose rows the apply kernel
+        //  reads and writes in one group)
+        const bool may_sum = !accumulate && max_split > 0 && static_cast<long>(BH) * p.N * (G::NB - 1) <= 840L * n_cu && (G::NB == 1 || !p.o_over_q);
         for (int s2 = 2; s2 <= max_split; ++s2)
             if (BH * s2 <= n_cu && tiles / s2 >= (may_sum ? 1 : 2)) split = s2;
         ps.tokens_per_group = ((tiles + split - 1) / split) * kStateTile;
@@ -1435,6 +1439,8 @@ int linear_attn_forward(const mi_linear_attn_args* a, const char* op, void* part
     const uintptr_t al = reinterpret_cast<uintptr_t>(a->q) | reinterpret_cast<uintptr_t>(a->k) | reinterpret_cast<uintptr_t>(a->v) |
                          reinterpret_cast<uintptr_t>(a->o) | reinterpret_cast<uintptr_t>(a->workspace);
     if (al & 15u) return fail("%s: pointers must be 16-byte aligned", op);
+    p.o_over_q = operands_overlap(p.o, p.o_rs, p.o_bs, p.q, p.q_rs, p.q_bs, p.B, n_rows, row_len);
+    p.o_over_k = operands_overlap(p.o, p.o_rs, p.o_bs, p.k, p.k_rs, p.k_bs, p.B, n_rows, row_len);
     p.eps = a->eps;
     p.ws = static_cast<float*>(a->workspace);
     p.part = max_split > 0 ? static_cast<float*>(part) : nullptr; p.n_part = 0; p.add_to_state = 0;

@@ -329,7 +329,9 @@ MI_API int mi_scale_rows(const mi_scale_rows_args* args);
  * `scratch` (optional, FP32, up to mi_linear_attn_scratch_bytes) lets the state pass split the
  * tokens of a head over several work groups, one partial state each, summed by a small
  * reduction: several times faster at image sizes. Without it one work group streams all
- * tokens of a (batch, head). Results are deterministic either way (no atomics). */
+ * tokens of a (batch, head). Results are deterministic either way (no atomics).
+ * Token-major, `o` may be q, k or v itself (same pointer and strides); otherwise, and always with channel-major operands, it
+ * must not share memory with them. */
 typedef struct mi_linear_attn_args {
     uint32_t struct_size;
     int32_t dtype;
@@ -355,7 +357,8 @@ typedef struct mi_linear_attn_args {
                                of the partial states (in `scratch`), apply; the last two are one launch where that is faster, with
                                the same bits. _ONE_LAUNCH: the state split along its value channels,
                                every work group streams K, its slice of V, then Q, and writes its slice of O; no scratch is used.
-                               A call that accumulates onto a state always takes the three launches */
+                               A call that accumulates onto a state always takes the three launches, and one whose O shares memory
+                               with Q or K never the single one */
     int32_t layout;         /* MI_LAYOUT_TOKEN_MAJOR (0): q, k, v, o are (batch, n_tokens, heads*head_dim), a row per token, as
                                everywhere in this header. MI_LAYOUT_CHANNEL_MAJOR: (batch, heads*head_dim, n_tokens), a row per
                                channel, head h in rows [h*head_dim, (h+1)*head_dim) — the layout in which the reference keeps

@@ -2,6 +2,7 @@
 // The device code and the host planner share these formulas; here they are checked by brute force against their
 // definition: the pieces of a group tile its tail steps exactly once, piece_of() inverts piece_begin(), the parts of
 // a tile are numbered 0 .. n-1 without gaps and never exceed max_parts as the planner computes it.
+// Also whether two operands share memory (operands_overlap, csrc/internal.h), against their elements.
 // Compiled for the host by hipcc (the header pulls in the HIP runtime declarations); runs without a GPU.
 #include <cstdio>
 #include <vector>
@@ -14,8 +15,38 @@ static int g_failures = 0;
         if (!(cond)) { std::printf("CHECK failed %s:%d: %s\n", __FILE__, __LINE__, #cond); ++g_failures; } \
     } while (0)
 
+// operands_overlap against the elements themselves, on small operands at every offset in one buffer
+static void check_operands_overlap() {
+    static char buffer[2 * 4096];
+    for (long batch : {1, 2})
+        for (long rows : {1, 3})
+            for (long len : {4, 8})
+                for (long a_rs : {8, 12, 24})
+                    for (long b_rs : {8, 24})
+                        for (long a_items : {-2, 1, 4})
+                            for (long odd : {0, 4})
+                                for (long at = 0; at < 256; at += 4) {
+                                    const long a_bs = a_items * rows * a_rs + odd, b_bs = rows * b_rs, origin = 1024;
+                                    std::vector<bool> of_b(4096);
+                                    for (long i = 0; i < batch; ++i)
+                                        for (long r = 0; r < rows; ++r)
+                                            for (long c = 0; c < len; ++c) of_b[origin + i * b_bs + r * b_rs + c] = true;
+                                    bool shared = false;
+                                    for (long i = 0; i < batch; ++i)
+                                        for (long r = 0; r < rows; ++r)
+                                            for (long c = 0; c < len; ++c) shared |= of_b[origin - 128 + at + i * a_bs + r * a_rs + c];
+                                    const bool said = mi::operands_overlap(buffer + 2 * (origin - 128 + at), a_rs, a_bs, buffer + 2 * origin, b_rs, b_bs, batch, rows, len);
+                                    CHECK(said || !shared);                                 // never missed
+                                    const bool whole_items = batch == 1 || odd == 0;
+                                    // column slices of one buffer, one beside the other
+                                    const long column = ((at - 128) % a_rs + a_rs) % a_rs;
+                                    if (a_rs == b_rs && whole_items && column >= len && column <= a_rs - len) CHECK(!said);
+                                }
+}
+
 int main() {
     int cases = 0;
+    check_operands_overlap();
     for (int n_blocks : {256, 257, 300, 312, 384, 432, 511, 520, 1000, 4097})
         for (int T : {16, 17, 52, 64, 72, 1000})
             for (int cu_g : {8, 32, 38}) {

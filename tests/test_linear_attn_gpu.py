@@ -239,3 +239,25 @@ def test_linear_attention_sums_partial_states_on_apply(oracle, B, H, d, N):
         assert np.max(np.abs(wsn[b, :, d * d:] - z)) <= 1e-4 * max(1.0, np.max(np.abs(z)))
     ws2 = torch.empty_like(ws)
     assert torch.equal(bd.linear_attention_relu_forward(dq, dk, dv, H, workspace=ws2, form=1), out) and torch.equal(ws2, ws)
+
+
+@pytest.mark.parametrize("B,H,d,N", [(1, 20, 112, 300), (1, 20, 112, 1024), (2, 5, 72, 700), (1, 2, 64, 257), (1, 4, 128, 900), (3, 3, 32, 1100), (1, 40, 112, 256)])
+@pytest.mark.parametrize("target", ["q", "k", "v", "slice"])
+def test_linear_attention_output_in_the_place_of_an_operand(oracle, B, H, d, N, target):
+    """O written over Q, K or V: every form reads a row before it, or any other work group, writes it. And O next to the others as a
+    column slice of one buffer, which shares no element with them."""
+    dtype, D = "bf16", H * d
+    q, k, v = (randn(5200 + i + N, (B, N, D), dtype) for i in range(3))
+    for form in (0, 1, 2):
+        for scratch in (None, False):
+            wide = torch.full((B, N, 4 * D + 8), 7.0, dtype=torch.bfloat16, device="cuda")
+            ops = [wide[:, :, i * D:(i + 1) * D] if target == "slice" else torch.empty(B, N, D, dtype=torch.bfloat16, device="cuda") for i in range(3)]
+            for t, x in zip(ops, (q, k, v)):
+                t.copy_(to_dev(x, dtype))
+            out = wide[:, :, 3 * D:4 * D] if target == "slice" else ops["qkv".index(target)]
+            bd.linear_attention_relu_forward(*ops, H, out=out, scratch=scratch, form=form)
+            for b in range(B):
+                assert_close(oracle.linear_attn_relu(q[b], k[b], v[b], H), to_np(out[b]), dtype, f"form {form}, batch {b}")
+            if target == "slice":
+                dense = bd.linear_attention_relu_forward(*(to_dev(x, dtype) for x in (q, k, v)), H, scratch=scratch, form=form)
+                assert torch.equal(out, dense) and (wide[:, :, 4 * D:] == 7).all()
