@@ -261,3 +261,21 @@ def test_linear_attention_output_in_the_place_of_an_operand(oracle, B, H, d, N, 
             if target == "slice":
                 dense = bd.linear_attention_relu_forward(*(to_dev(x, dtype) for x in (q, k, v)), H, scratch=scratch, form=form)
                 assert torch.equal(out, dense) and (wide[:, :, 4 * D:] == 7).all()
+
+
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("H,d,N", [(20, 112, 1024), (3, 32, 1500), (2, 64, 1024)])
+def test_partial_states_are_added_in_pairs(H, d, N, accumulate):
+    """A state entry whose first token contributes 2^24 and the first token of every other 128-token chunk 1: added one after the other
+    onto the 2^24 the ones vanish; in pairs the sum is off by at most its spacing, 2."""
+    D = H * d
+    q, k, v = (torch.zeros(1, N, D, dtype=torch.bfloat16, device="cuda") for _ in range(3))
+    q[:] = 1
+    k[0, 0::128], v[0, 0::128] = 1, 1
+    k[0, 0], v[0, 0] = 2.0 ** 12, 2.0 ** 12
+    ws = torch.zeros(H * (d * d + d), dtype=torch.float32, device="cuda")
+    bd.linear_attention_relu_forward(q, k, v, H, workspace=ws, accumulate_state=accumulate, form=1)
+    S = ws.view(H, d * d + d)[:, :d * d].double()
+    chunks = (N + 127) // 128
+    assert chunks == 8 or N > 1024
+    assert (S - (2.0 ** 24 + chunks - 1)).abs().max().item() <= (2 if chunks == 8 else chunks)
