@@ -111,7 +111,7 @@ int launch_sdpa_wide(const SdpaDev& p, int dtype, int head_dim, hipStream_t stre
 bool sdpa_small_takes(const SdpaDev& p, int head_dim);
 bool sdpa_flow_runs(const SdpaDev& p);
 bool sdpa_flow_takes(const SdpaDev& p, int head_dim, int n_cu);
-int launch_sdpa_flow(const SdpaDev& p, int dtype, int head_dim, hipStream_t stream);
+int launch_sdpa_flow(const SdpaDev& p, int dtype, int head_dim, int n_cu, bool short_keys, hipStream_t stream);   // short_keys: the keys fit LDS
 int launch_sdpa_small(const SdpaDev& p, int dtype, int head_dim, hipStream_t stream);
 
 // Device-side view of the head-averaged attention map launch (batch 1).

@@ -37,9 +37,17 @@ template <int D> struct FlowGeo {
     static constexpr bool ZERO_PAD = D == 40 || D == 72;
 };
 
+// How far the probabilities' rounding to 16 bits reaches a result is set by the row's reference (the probability of the key that it was
+// taken from is 1, exactly) and by what the denominator sums.
+struct FlowRounding {
+    float sum_max;      // the reference moves to a later tile's maximum when a lane's sum reaches this
+    int two_tiles;      // it is the maximum of the first two tiles, not of the first
+    bool pair_sum;      // the denominators sum the rounded probabilities, in FP32 (see softmax_tile_rel), not the FP32 exponentials
+};
+
 // (40: the cap at 128 registers lets four groups share a CU; 64 spills there)
-template <typename T, int D>
-__global__ void __launch_bounds__(kThreads, (D == 40 ? 4 : D <= 96 ? 3 : 2)) sdpa_flow_kernel(const SdpaDev p) {
+template <typename T, int D, bool PAIR_SUM>
+__global__ void __launch_bounds__(kThreads, (D == 40 ? 4 : D <= 96 ? 3 : 2)) sdpa_flow_kernel(const SdpaDev p, const float sum_max, const int two_tiles) {
     using G = HeadGeo<D>;
     using FG = FlowGeo<D>;
     using V8 = typename Mma<T>::v8;
@@ -198,8 +206,11 @@ __global__ void __launch_bounds__(kThreads, (D == 40 ? 4 : D <= 96 ? 3 : 2)) sdp
                     const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[kb][e + 1], mul, add));
                     pf[c4][i] = static_cast<T>(p0);
                     pf[c4][i + 1] = static_cast<T>(p1);
-                    sum[i & 2] += p0;
-                    sum[(i & 2) + 1] += p1;
+                    if constexpr (PAIR_SUM) sum[i >> 1] = pair_sum<T>(pf[c4], i >> 1, sum[i >> 1]);
+                    else {
+                        sum[i & 2] += p0;
+                        sum[(i & 2) + 1] += p1;
+                    }
                 }
             // (packed here: left to itself the compiler keeps the 32 FP32 values through the branch that follows)
 #pragma unroll
@@ -207,8 +218,9 @@ __global__ void __launch_bounds__(kThreads, (D == 40 ? 4 : D <= 96 ? 3 : 2)) sdp
             return (sum[0] + sum[1]) + (sum[2] + sum[3]);
         };
         float ls = exponentiate(cl2, st.neg_ref);
-        if (__any(!(st.started && ls < kRelSumMax))) {
-            // first tile, or terms that grew: the reference moves to the row's maximum (see softmax_tile_rel)
+        const bool second = D >= 80 && D <= 112 && !PAIR_SUM && decltype(parity)::value && two_tiles && t == 1;
+        if (__any(!(st.started && ls < sum_max && !second))) {
+            // first tiles, or terms that grew: the reference moves to the row's maximum (see softmax_tile_rel)
             float mloc = fmaxf(sacc[0][0], sacc[1][0]);
 #pragma unroll
             for (int e = 1; e < 16; ++e) mloc = fmaxf(mloc, fmaxf(sacc[0][e], sacc[1][e]));
@@ -257,26 +269,50 @@ __global__ void __launch_bounds__(kThreads, (D == 40 ? 4 : D <= 96 ? 3 : 2)) sdp
 }
 
 template <typename T, int D>
-int launch_flow(SdpaDev p, hipStream_t stream) {
+int launch_flow(SdpaDev p, const FlowRounding& r, hipStream_t stream) {
     p.n_q_tiles = (p.Lq + kRows - 1) / kRows;
     p.n_blocks = p.B * p.H * p.n_q_tiles;
-    hipLaunchKernelGGL((sdpa_flow_kernel<T, D>), dim3((p.n_blocks + 7) / 8 * 8), dim3(kThreads), FlowGeo<D>::LDS, stream, p);
+    const dim3 grid((p.n_blocks + 7) / 8 * 8), block(kThreads);
+    if (D <= 96 && r.pair_sum) hipLaunchKernelGGL((sdpa_flow_kernel<T, D, D <= 96>), grid, block, FlowGeo<D>::LDS, stream, p, r.sum_max, r.two_tiles);
+    else hipLaunchKernelGGL((sdpa_flow_kernel<T, D, false>), grid, block, FlowGeo<D>::LDS, stream, p, r.sum_max, r.two_tiles);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail("sdpa_fwd launch: %s", hipGetErrorString(e));
     return 0;
 }
 
+// As exact as the kernels that these calls would otherwise take:
+//   a 256-row tile or more per CU, more keys than the short-key kernel holds: the 256-row kernels, which sum rounded probabilities up to
+//     head_dim 96 and move the reference at 2^10;
+//   below, at 40 and 64 always, at 72 from 5 and at 128 from 8 key tiles: their instances that sum exponentials;
+//   otherwise the 128-row kernel or (few keys) the short-key one: exponentials, reference moved at 2^8. At 80 to 112 and four key tiles
+//     or more two halves of a work group took every other tile, each with a reference of its own: hence the first two tiles here, and 2^6.
+// Relative error against 64 bits, with the first tile's maximum, 2^10 and exponentials for all / so (bf16, scores N(0, 1); N(0, 3)):
+//   80, 8 x 4096 rows, 231 keys 2.27e-3 / 2.22e-3; 2.18e-3 / 1.97e-3 (before there was this kernel 2.21e-3; 1.99e-3), 1000 keys 2.33e-3 /
+//   2.31e-3; 2.28e-3 / 2.12e-3; 96, 16 x 4096, 300 keys 2.30e-3 / 2.28e-3; 2.22e-3 / 1.90e-3; 160, 8 x 4096, 4096 keys 2.27e-3 / 2.19e-3 (N(0, 3)).
+// Time, so against that: N(0, 1) equal but for 80 to 112 with few keys (80, 231 keys 8.7 -> 9.1 us, 1000 keys 19.4 -> 19.9) and with rounded sums (40, 1.25
+// rounds 99 -> 96 us; 80, 2 x 8 x 4096 bf16 90.5 -> 94); N(0, 3) up to 12 % more at 80 to 112 below a round, where the reference moves more often.
+FlowRounding flow_rounding(const SdpaDev& p, int head_dim, int n_cu, bool short_keys) {
+    const long heads = static_cast<long>(p.B) * p.H;
+    const bool full = heads * ((p.Lq + 255) / 256) >= n_cu && !short_keys, middle = head_dim >= 80 && head_dim <= 112;
+    const int tiles = (p.Lk + kBN - 1) / kBN, many = head_dim <= 64 ? 1 : head_dim == 72 ? 5 : head_dim == 128 ? 8 : 1 << 30;
+    FlowRounding r;
+    r.pair_sum = full && head_dim <= 96;
+    r.sum_max = (full && head_dim <= 128) || (tiles >= many && p.Lp == 0 && !short_keys) ? kRelSumMax : middle ? 64.f : 256.f;
+    r.two_tiles = middle && !full && tiles >= 4;
+    return r;
+}
+
 template <typename T>
-int launch_flow_t(const SdpaDev& p, int head_dim, hipStream_t stream) {
+int launch_flow_t(const SdpaDev& p, int head_dim, const FlowRounding& r, hipStream_t stream) {
     switch (head_dim) {
-        case 40: return launch_flow<T, 40>(p, stream);
-        case 64: return launch_flow<T, 64>(p, stream);
-        case 72: return launch_flow<T, 72>(p, stream);
-        case 80: return launch_flow<T, 80>(p, stream);
-        case 96: return launch_flow<T, 96>(p, stream);
-        case 112: return launch_flow<T, 112>(p, stream);
-        case 128: return launch_flow<T, 128>(p, stream);
-        default: return launch_flow<T, 160>(p, stream);
+        case 40: return launch_flow<T, 40>(p, r, stream);
+        case 64: return launch_flow<T, 64>(p, r, stream);
+        case 72: return launch_flow<T, 72>(p, r, stream);
+        case 80: return launch_flow<T, 80>(p, r, stream);
+        case 96: return launch_flow<T, 96>(p, r, stream);
+        case 112: return launch_flow<T, 112>(p, r, stream);
+        case 128: return launch_flow<T, 128>(p, r, stream);
+        default: return launch_flow<T, 160>(p, r, stream);
     }
 }
 
@@ -317,9 +353,10 @@ bool sdpa_flow_takes(const SdpaDev& p, int head_dim, int n_cu) {
     }
 }
 
-int launch_sdpa_flow(const SdpaDev& p, int dtype, int head_dim, hipStream_t stream) {
-    if (dtype == MI_DTYPE_BF16) return launch_flow_t<__bf16>(p, head_dim, stream);
-    return launch_flow_t<_Float16>(p, head_dim, stream);
+int launch_sdpa_flow(const SdpaDev& p, int dtype, int head_dim, int n_cu, bool short_keys, hipStream_t stream) {
+    const FlowRounding r = flow_rounding(p, head_dim, n_cu, short_keys);
+    if (dtype == MI_DTYPE_BF16) return launch_flow_t<__bf16>(p, head_dim, r, stream);
+    return launch_flow_t<_Float16>(p, head_dim, r, stream);
 }
 
 }  // namespace mi

@@ -1345,7 +1345,7 @@ int launch_d(SdpaDev p, int n_cu, hipStream_t stream) {
                             shortkv_lds_bytes<D>(n_kt, p.key_mask != nullptr) <= 160 * 1024;
     const ShortPlan short_plan = short_keys ? plan_short(static_cast<long>(p.B) * p.H, (p.Lq + 255) / 256, n_cu) : ShortPlan{};
     const bool flow = short_keys ? sdpa_flow_runs(p) && !shortkv_pays<D>(short_plan, tiles256, n_cu) : choice == 0 && sdpa_flow_takes(p, D, n_cu);
-    if (flow) return launch_sdpa_flow(p, std::is_same_v<T, __bf16> ? MI_DTYPE_BF16 : MI_DTYPE_F16, D, stream);
+    if (flow) return launch_sdpa_flow(p, std::is_same_v<T, __bf16> ? MI_DTYPE_BF16 : MI_DTYPE_F16, D, n_cu, short_keys, stream);
     if constexpr (dma_kernel_available<D>()) {
         if (p.split_scratch != nullptr && plan_split<D>(p, n_cu) &&
             p.split_scratch_bytes >= static_cast<size_t>(8) * p.split.max_tail * p.split.max_parts * SplitGeo::slot_bytes(D)) {
