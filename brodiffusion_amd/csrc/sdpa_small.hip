@@ -315,10 +315,18 @@ __global__ void __launch_bounds__(64 * kMaxWaves, PROJ ? 2 : D <= 64 ? 4 : D <= 
     for (int vb = 0; vb < G::VB; ++vb)
 #pragma unroll
         for (int e = 0; e < 16; ++e) oacc[vb][e] = 0.f;
-    float m = kNegInf, mc = 0.f, l = 0.f;
+    float m = kNegInf, mc = 0.f, l = 0.f, m_keep = kNegInf;      // (m_keep: the maximum up to which the reference stays)
     bool started = false;      // a block has been accumulated
     const float cl2 = p.scale_log2;
     const float lazy_raw = kLazyLog2 / cl2;
+    // A wavefront's reference is the maximum of its first blocks, as many as hold the keys from which the kernels before took theirs (the
+    // first 64; at head_dim 80 to 112 two halves of a work group, 64 each): the probability of the key that it comes from is 1, exactly,
+    // in 16 bits too. (Error against 64 bits, bf16, scores of N(0, 3), from one block / so / before there was this kernel: causal, 256 tokens, 80
+    // 2.01e-3 / 1.81e-3 / 1.81e-3, 128 2.01e-3 / 1.93e-3 / 1.93e-3; N(0, 1), 2000 tokens, 160 2.11e-3 / 2.08e-3 / 2.09e-3. Time: causal 1 % more, windows of
+    // 64 in 256 tokens 6 %, others the same.)
+    constexpr bool MIDDLE = D >= 80 && D <= 112;
+    int exact_blocks = S == 1 ? (MIDDLE ? 4 : 2) : S == 2 && (MIDDLE || D == 160) ? 2 : 1;
+    if constexpr (MASKED) { if (ext.window > 0 && S <= (MIDDLE ? 2 : 1)) exact_blocks += 2; }      // (rows whose first key lies in a later block)
     const PanelReads at(lane);
 
     const int n_steps = (n_blocks + S - 1) / S;
@@ -380,7 +388,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves, PROJ ? 2 : D <= 64 ? 4 : D <= 
 #pragma unroll
             for (int e = 1; e < 16; ++e) mloc = fmaxf(mloc, sacc[e]);
             mloc = exchange_max(mloc);
-            if (__any(mloc > m + lazy_raw)) {
+            if (__any(mloc > m_keep)) {
                 const float m_new = fmaxf(m, mloc);
                 const float mc_new = (m_new == kNegInf) ? 0.f : m_new * cl2;
                 if (started) {
@@ -393,8 +401,10 @@ __global__ void __launch_bounds__(64 * kMaxWaves, PROJ ? 2 : D <= 64 ? 4 : D <= 
                 }
                 m = m_new;
                 mc = mc_new;
+                m_keep = m_new + (exact_blocks > 1 ? 0.f : lazy_raw);
             }
             started = true;
+            --exact_blocks;
             V8 pf[2];
             float l0 = 0.f, l1 = 0.f;
 #pragma unroll

@@ -53,3 +53,17 @@ def test_reference_moves_to_terms_above_two_to_the_eighth(dtype, d, H, Lq, Lk):
 @pytest.mark.parametrize("H,Lq,Lk", [(8, 4096, 231), (8, 2500, 1030), (16, 2000, 300)])
 def test_reference_is_the_maximum_of_the_first_two_tiles(dtype, d, H, Lq, Lk):
     one_heavy_key(dtype, d, H, Lq, Lk, 100, 5)
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("d", [40, 64, 72, 80, 96, 112, 128, 160])
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("H,Lq,Lk,at", [(16, 1285, 190, 40), (16, 1285, 300, 40), (9, 993, 190, 40), (2, 100, 190, 40), (2, 100, 1500, 63)])
+def test_few_rows_reference_is_the_maximum_of_the_first_64_keys(dtype, d, masked, H, Lq, Lk, at):
+    one_heavy_key(dtype, d, H, Lq, Lk, at, 5, **({"mask": bd.SdpaMask.causal(Lk)} if masked else {}))
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("d", [80, 96, 112])
+def test_few_rows_reference_is_the_maximum_of_the_first_128_keys_of_two_wavefronts(dtype, d):
+    one_heavy_key(dtype, d, 16, 1285, 300, 70, 5, mask=bd.SdpaMask.causal(300))
