@@ -510,8 +510,9 @@ int key_blocks(const SdpaDev& p) { return (p.Lp + kKB - 1) / kKB + (p.Lk - p.Lp 
 // Calls without extras (key mask, logit bias, denominators), tile-wise K rotation, the prefix dial or packed sequences. The lines
 // are from 8 head dimensions x 64 to 8192 units (32 query rows of a head) x 1 to 256 key blocks of 8 fp16 heads, every R and two S
 // against the kernel that took the call before (us, before / here; n = compute units). Masked calls (causal, windowed, block-causal;
-// 8 dimensions x 64 to 1008 units) take 0.35 to 0.98 of the time up to 4 n units, except windowed ones of 80 to 112 above 3 n (1008
-// units, window 256: 96 15.9 / 17.3); beyond 4 n they are left where their longest tiles start first.
+// 8 dimensions x 64 to 1008 units) take 0.35 to 0.98 of the time up to 4 n units (windowed ones of 96, 1008 units, 128-row kernel / here: window
+// 64 11.5 / 9.3, 256 15.9 / 12.8, 1024 32.3 / 24.4, 4000 92 / 65; 1024 units of 250 tokens, window 64 11.0 / 10.0, 128 12.5 / 11.6); beyond 4 n
+// they are left where their longest tiles start first.
 //   units <= n       R = 1: 256 units, 5, 32 and 128 blocks: 40 8.4 / 4.8, 18.2 / 8.9, 56 / 25; 72 10.5 / 5.4, 23 / 10.2, 73 / 27; 128
 //                    10.5 / 6.7, 25.7 / 12, 79 / 30; 160 13.4 / 7.9, 37 / 16.5, 134 / 43
 //   units <= 2 n     R = 2: 512 units, 5, 32 and 128 blocks: 40 8.5 / 5.5, 18 / 11, 56 / 32; 80 10.5 / 6.5, 23 / 15, 73 / 40; 128 10.8 /
@@ -529,7 +530,6 @@ SmallPlan plan_small(const SdpaDev& p, int D, int n_cu) {
     if (units <= 2L * n_cu) return {2, kMaxWaves};
     if (units > 4L * n_cu) return {};
     if (!masked) return D == 64 && nb >= 48 ? SmallPlan{2, kMaxWaves} : SmallPlan{};
-    if (p.window > 0 && units > 3L * n_cu && D >= 80 && D <= 112) return {};
     return {4, nb <= (D <= 64 ? 6 : 8) ? 4 : kMaxWaves};
 }
 

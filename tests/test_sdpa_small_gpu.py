@@ -72,6 +72,19 @@ def test_masks(oracle, dtype, d, H, n):
         assert_close(ref[rows], to_np(out)[rows], dtype, f"{name}, {H} x {n}")
 
 
+# 776 to 1024 units of 32 rows, the most that come here: one and two wavefronts to a row, windows below, of and above a block
+@pytest.mark.parametrize("dtype,d", [("fp16", 80), ("bf16", 96), ("fp16", 112), ("bf16", 128)])
+@pytest.mark.parametrize("H,n,windows", [(8, 4032, (1, 31, 256, 1024, 4000)), (110, 250, (5, 32, 100)), (24, 1100, (33, 700))])
+def test_windows_at_the_most_rows(oracle, dtype, d, H, n, windows):
+    q, k, v = (randn(9661 + i, (n, H * d), dtype) for i in range(3))
+    dq, dk, dv = (to_dev(x, dtype) for x in (q, k, v))
+    rows, pos = sampled(n), np.arange(n)
+    for w in windows:
+        out = bd.sdpa_forward(dq, dk, dv, H, mask=bd.SdpaMask.causal(0, w))
+        ref = oracle.sdpa(q, k, v, H, row_lo=np.maximum(0, pos + 1 - w).astype(np.int32), row_hi=(pos + 1).astype(np.int32), rows=rows)
+        assert_close(ref[rows], to_np(out)[rows], dtype, f"window {w}, {H} x {n}")
+
+
 @pytest.mark.parametrize("split_half", [False, True])
 @pytest.mark.parametrize("dtype,d", DIMS)
 def test_grouped_heads_batches_and_rope(oracle, dtype, d, split_half):
