@@ -61,6 +61,7 @@ HOST_DIR = os.path.join(HERE, "host")
 HOST_LIB = os.path.join(LIB_DIR, "libbrodiffusion_amd_host.so")
 HOST_TEST = os.path.join(LIB_DIR, "test_host_ops")
 SPLIT_TEST = os.path.join(LIB_DIR, "test_split_geo")
+FORMS_LIB = os.path.join(LIB_DIR, "liblinear_forms_test.so")
 WAITING_LIB = os.path.join(LIB_DIR, "libwaiting_test.so")
 CXX = os.environ.get("CXX", "g++")
 
@@ -92,6 +93,12 @@ def build_host(with_test: bool = True, verbose: bool = False) -> str:
         if r.returncode != 0:
             sys.stderr.write(r.stdout + r.stderr)
             raise RuntimeError("split-geometry test build failed")
+        cmd = [HIPCC, "-std=c++20", "-O1", "-Wall", "-fPIC", "-shared", "--offload-host-only", "-x", "hip", "-I" + os.path.join(ROOT, "include"), "-I" + CSRC,
+               os.path.join(ROOT, "tests", "cpp", "linear_forms.cpp"), "-o", FORMS_LIB]
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        if r.returncode != 0:
+            sys.stderr.write(r.stdout + r.stderr)
+            raise RuntimeError("test library build failed")
         cmd = [*common, "-shared", os.path.join(ROOT, "tests", "cpp", "waiting_library.cpp"), "-o", WAITING_LIB]
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
