@@ -1,5 +1,6 @@
-"""Calls with few query rows or few keys: work groups of R x S wavefronts, R groups of 32 rows (by the number of query
-rows: up to one such unit per compute unit, two, four, more), S blocks of 32 keys at a time. Key counts around a block and around
+"""Calls with few query rows: work groups of R x S wavefronts, R groups of 32 rows (1 up to one such unit per compute unit, 2 up to
+two; masked calls 4 up to four), S blocks of 32 keys at a time. Unmasked calls of more units, 16 x 1285 rows here, belong to the kernel of
+tests/test_sdpa_flow_gpu.py but for those of many keys at head_dim 64 (test_two_groups_to_a_compute_unit). Key counts around a block and around
 one round of S blocks, the last rows, cached prefixes that end inside a block, valid lengths, grouped heads and RoPE on the query,
 against the CPU checker; infinities and NaN next to rows that do not exist."""
 import numpy as np
@@ -17,7 +18,7 @@ def sampled(Lq):
     return np.unique(np.concatenate([np.arange(0, Lq, max(1, Lq // 40)), [min(31, Lq - 1), min(32, Lq - 1), Lq - 1]])).astype(np.int32)
 
 
-# (heads, rows): R = 1, 2, 4 at 256 compute units; keys around one block, one round of S blocks, two rounds
+# (heads, rows): R = 1 (twice), R = 2, more units than come here, at 256 compute units; keys around one block, one round of S blocks, two rounds
 @pytest.mark.parametrize("dtype,d", DIMS)
 @pytest.mark.parametrize("H,Lq", [(2, 1), (3, 65), (9, 993), (16, 1285)])
 @pytest.mark.parametrize("Lk", [1, 32, 33, 129, 257, 515])
@@ -33,6 +34,10 @@ def test_rows_and_keys(oracle, dtype, d, H, Lq, Lk):
 @pytest.mark.parametrize("H,Lq", [(3, 40), (9, 993), (16, 1285)])
 @pytest.mark.parametrize("Lp,Lk", [(1, 64), (31, 1), (33, 130), (64, 33), (300, 95)])
 def test_prefix_and_valid_length(oracle, dtype, d, H, Lq, Lp, Lk):
+    check_prefix_and_valid_length(oracle, dtype, d, H, Lq, Lp, Lk, (None, 0, 1, Lp, Lp + 1, Lp + Lk - 1))
+
+
+def check_prefix_and_valid_length(oracle, dtype, d, H, Lq, Lp, Lk, lengths):
     """Prefix rows of a stride of their own; rows behind both segments poisoned."""
     q, k, v = randn(9621, (Lq, H * d), dtype), randn(9622, (Lp + Lk, H * d), dtype), randn(9623, (Lp + Lk, H * d), dtype)
     def placed(x, width):
@@ -42,14 +47,23 @@ def test_prefix_and_valid_length(oracle, dtype, d, H, Lq, Lp, Lk):
     kp, vp, kf, vf = placed(k[:Lp], 2 * H * d), placed(v[:Lp], H * d + 8), placed(k[Lp:], H * d), placed(v[Lp:], H * d + 8)
     rows = sampled(Lq)
     dq = to_dev(q, dtype)
-    for valid in (None, 0, 1, Lp, Lp + 1, Lp + Lk - 1):
+    for valid in lengths:
         vl = None if valid is None else torch.tensor([valid], dtype=torch.int32, device="cuda")
-        out = bd.sdpa_forward(dq, kf, vf, H, k_prefix=kp, v_prefix=vp, kv_valid_len=vl)
+        out = bd.sdpa_forward(dq, kf, vf, H, kv_valid_len=vl, **({"k_prefix": kp, "v_prefix": vp} if Lp else {}))
         n = Lp + Lk if valid is None else valid
         if n == 0:
             assert (out == 0).all()
         else:
             assert_close(oracle.sdpa(q, k[:n], v[:n], H, rows=rows)[rows], to_np(out)[rows], dtype, f"prefix {Lp} + {Lk}, valid {valid}")
+
+
+# head_dim 64, 528 to 1024 units and 48 or more blocks of keys: R = 2 with two groups to a compute unit
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("H,Lq,Lp,Lk", [(16, 1050, 0, 1505), (8, 4090, 45, 1500), (11, 2000, 1601, 33)])
+def test_two_groups_to_a_compute_unit(oracle, dtype, H, Lq, Lp, Lk):
+    assert 2 < H * ((Lq + 31) // 32) / bd.device_info()["compute_units"] <= 4 and (Lp + 31) // 32 + (Lk + 31) // 32 >= 48
+    v_of = (None, 0, Lp + 1, Lp + Lk - 1) if Lp else (None, 0, 1, 1000, Lk - 1)
+    check_prefix_and_valid_length(oracle, dtype, 64, H, Lq, Lp, Lk, v_of)
 
 
 @pytest.mark.parametrize("dtype,d", DIMS)
@@ -102,7 +116,7 @@ def test_grouped_heads_batches_and_rope(oracle, dtype, d, split_half):
 
 
 @pytest.mark.parametrize("dtype,d", DIMS)
-@pytest.mark.parametrize("H,Lq", [(2, 40), (16, 1285)])
+@pytest.mark.parametrize("H,Lq", [(2, 40), (9, 993), (16, 1285)])
 def test_values_of_the_last_row_do_not_leak(dtype, d, H, Lq):
     """Rows past the last key repeat it in LDS: an infinite value there stays an infinity (0 x Inf would make it NaN), and a NaN key in
     one block makes exactly its head NaN whichever wavefront has it."""
