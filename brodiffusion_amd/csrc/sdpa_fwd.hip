@@ -1268,8 +1268,12 @@ bool same_keys_for_all_rows(const SdpaDev& p) {
 // 128-row tiles. With a 256-row tile or more per CU the former always. Below that the 128-row kernel keeps more CUs busy, but
 // each of them runs one wavefront per SIMD whose softmax nothing hides, and from the 257th work group on two share a CU
 // anyway ("crowded"); a CU with eight wavefronts needs 2/3 of the time per row and key, and costs about 1.5 us more to start
-// (rings, two-part Q staging). The lines are where the two sides meet (us, 128-row / 256-row, 8 heads of 40 and 80, 16 of 64, 72
-// and 96, 24 of 128; over a sweep of 156 such calls the side taken is at most 7 % slower than the other, 0.6 % on average):
+// (rings, two-part Q staging).
+// What asks below a tile per CU: calls with extras or K rotated by tile, masked ones of more rows than sdpa_small.hip takes, and plain ones
+// of 40, 64 and 128 above the lines of sdpa_flow_takes (all of them on 256 rows: those of 128 are crowded and have more than three key
+// tiles). The other plain lines are met only by K or V of 2 GiB and more, whose offsets sdpa_small.hip and sdpa_flow.hip do not hold. The lines are where the two sides meet (us, 128-row /
+// 256-row, 8 heads of 40 and 80, 16 of 64, 72 and 96, 24 of 128; over a sweep of 156 such calls the side taken is at most 7 % slower than the
+// other, 0.6 % on average):
 //   128, no mask:      T = 4 11.5 / 12.5, 5 13.3 / 13.9, 8 18.0 / 17.3, 16 30.8 / 26.9, 32 (192 tiles) 74.7 / 52.7; cross, 3 key
 //                      tiles, 216 query tiles 15.0 / 14.6, 96 query tiles 11.1 / 12.7
 //   72, no mask:       T = 4 11.4 / 10.8, 5 12.9 / 12.0, cross with 2 9.2 / 10.1, with 5 13.4 / 13.5, 16 29.3 / 23.6, 36 (144
@@ -1437,7 +1441,7 @@ int launch_d(SdpaDev p, int n_cu, hipStream_t stream) {
                             return;
                         }
                     }
-                    // (below one tile per CU only 80 and 96 come here: rows256_pay)
+                    // (below one tile per CU only 80 and 96 come here, with K or V of 2 GiB and more: rows256_pay)
                     if constexpr (!F || D > 72) hipLaunchKernelGGL((sdpa_fwd_pp_kernel<T, D, false, kGeneral, false, F>), grid, block, lds_bytes_8<D>(), stream, p);
                 };
                 // the form of the denominators (from head_dim 112 on there is one)
