@@ -8,8 +8,8 @@
 //   turns the scores into probabilities relative to the row's reference, as the 256-row kernels do (softmax_tile_rel), with FP32
 //   row sums in four chains;
 //   multiplies the values, fragments read four ahead.
-// No LDS read waits for a DMA load: measured, a read issued right behind four of them returns in the usual 56 clocks. Two or three
-// such groups share a CU (154 to 208 registers) and drift apart, so that the softmax of one runs under the products of the other
+// No LDS read waits for a DMA load: measured, a read issued right behind four of them returns in the usual 56 clocks. Two to four
+// such groups share a CU (121 to 126 registers at head_dim 40, 126 to 166 at 64 to 96, 202 to 244 above) and drift apart, so that the softmax of one runs under the products of the other
 // without a schedule between them, and 128-row tiles leave half as much of a last round idle as 256-row ones.
 // At head_dim 40 and 72 the places past the end of a row are not loaded but zeroed once: the products that they feed are of zeros,
 // which costs the power-limited matrix unit less (72, 8192 tokens 378 -> 365 us); at 80 to 112 that masking costs more than it saves.
