@@ -9,12 +9,14 @@
 //   row sums in four chains;
 //   multiplies the values, fragments read four ahead.
 // No LDS read waits for a DMA load: measured, a read issued right behind four of them returns in the usual 56 clocks. Two to four
-// such groups share a CU (121 to 126 registers at head_dim 40, 126 to 166 at 64 to 96, 202 to 244 above) and drift apart, so that the softmax of one runs under the products of the other
-// without a schedule between them, and 128-row tiles leave half as much of a last round idle as 256-row ones.
+// such groups share a CU (121 to 126 registers at head_dim 40, 126 to 166 at 64 to 96, 202 to 244 above) and drift apart, so that the
+// softmax of one runs under the products of the other without a schedule between them, and 128-row tiles leave half as much of a last
+// round idle as 256-row ones.
 // At head_dim 40 and 72 the places past the end of a row are not loaded but zeroed once: the products that they feed are of zeros,
 // which costs the power-limited matrix unit less (72, 8192 tokens 378 -> 365 us); at 80 to 112 that masking costs more than it saves.
-// What bounds it: with all of the GPU at work the clock that the power limit leaves (random data 27 % slower than zeros at head_dim
-// 40, 40 % at 72); with fewer groups than CUs the chain above (about 2000 clocks per tile at head_dim 72, of which 700 are products).
+// What bounds it: with all of the GPU at work the clock that the power limit leaves (72, 16 x 4096 tokens: as many cycles on zeros as on
+// N(0, 1), but 2.12 against 1.65 GHz, 71 against 91 us: profiles/model_blocks_counters.txt); with fewer groups than CUs the chain above
+// (about 2000 clocks per tile at head_dim 72, of which 700 are products).
 // Measured (us, before -> now; 256-row kernels, 128-row kernel for 160): 16 heads of 72, 2304 tokens 45.0 -> 41.1, 4096 100 -> 97; 8
 // heads of 80, batch 2, 2048 55 -> 32, 3072 93 -> 63, 4096 128 -> 98; 8 of 160, 4096 140 -> 92; 24 of 128, 1100 29.6 -> 24.2; 8 of 40, 1.25
 // rounds of 256-row tiles 309 -> 234.
