@@ -123,3 +123,23 @@ def test_elementwise_and_rope_beyond_2_31_elements(oracle):
     ref = oracle.linear(xs, to_np(w))
     got = to_np(out[idx])
     assert np.all(np.abs(got - ref) <= unit * np.maximum(np.abs(ref), 2.0 ** -6) * 1.05 + 2e-6)
+
+
+@pytest.mark.parametrize("d", [40, 64, 72, 80, 96, 112, 128, 160])
+def test_rows_of_keys_that_span_2_gib(oracle, d):
+    """K and V are rows of a few hundred bytes per head in a buffer of more than 2 GiB: the kernels for few rows and for mid
+    sizes hold 32-bit offsets and leave these calls, plain and causal, to the 128- and 256-row ones (whose offsets inside a tile of
+    64 rows stay within 32 bits: 64 x 2^25 bytes)."""
+    for H, Lq, Lk, stride in [(8, 70, 70, 1 << 24), (16, 1100, 1100, 1 << 20)]:
+        assert Lk * stride * 2 > 2 ** 31
+        g = torch.Generator(device="cuda").manual_seed(d + Lk)
+        q, k0, v0 = (torch.randn(L, H * d, device="cuda", generator=g).to(torch.bfloat16) for L in (Lq, Lk, Lk))
+        k, v = (torch.empty((Lk - 1) * stride + H * d, dtype=torch.bfloat16, device="cuda").as_strided((Lk, H * d), (stride, 1)) for _ in range(2))
+        k.copy_(k0)
+        v.copy_(v0)
+        for causal in (False, True):
+            what = f"d {d}, {H} x {Lq} rows, {Lk} keys {stride} elements apart, {'causal' if causal else 'plain'}"
+            print(what, flush=True)
+            out = bd.sdpa_forward(q, k, v, H, mask=bd.SdpaMask.causal(0) if causal else None)
+            lo, hi = np.zeros(Lq, np.int32), np.arange(1, Lq + 1, dtype=np.int32) if causal else np.full(Lq, Lk, np.int32)
+            assert_close(oracle.sdpa(to_np(q), to_np(k0), to_np(v0), H, row_lo=lo, row_hi=hi), to_np(out), "bf16", what)
