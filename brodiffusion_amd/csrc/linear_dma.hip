@@ -2,7 +2,7 @@
 // by DMA into rings.
 //
 // The work group's 512 threads are 8 wavefronts in a 2 (feature halves) x 4 (token quarters) arrangement; a wavefront owns
-// 128 features x 64 tokens = 4 x 2 accumulator blocks of v_mfma_f32_32x32x16 (128 registers). As in linear.hip the product
+// 128 features x 64 tokens = 8 x 4 accumulator blocks of v_mfma_f32_16x16x32 (128 registers; linear_pipe.hip says why that one). As in linear.hip the product
 // is computed transposed (MFMA rows = features), so both operands are read along their contiguous contraction index.
 //
 // Operands arrive in blocks of 64 contraction elements: per operand a 256-row x 128-byte tile (32 KB) = 32 LDS-DMA
@@ -13,20 +13,18 @@
 // are avoided by an XOR swizzle applied for free on the global side: the piece that lands in position c of row r is piece
 // c ^ ((r >> 1) & 7). X blocks live in a ring of two stages, W blocks in a ring of three (160 KB in all).
 //
-// A block is multiplied in two half-steps of 32 contraction elements (16 MFMAs per wavefront each). Half-step t of block b:
-//   1. read the 12 fragments of half-step t + 1 into the other register set
-//   2. issue this wavefront's 4 DMA instructions: first half of a block: W of block b + 2 (into the stage of W block b - 1);
-//      second half: X of block b + 2 (into the stage of X block b, whose fragments are all in registers by now)
-//   3. 16 MFMAs
-//   4. first half: wait until all but this wavefront's 4 youngest DMA instructions have landed (X and W of block b + 1);
+// A block is multiplied in two half-steps of 32 contraction elements (32 MFMAs per wavefront each). Half-step t of block b:
+//   1. the MFMAs, and between the first 24 of them the reads of the 12 fragments of half-step t + 1 into the other register set,
+//      between the last 8 this wavefront's 4 DMA instructions: first half of a block: W of block b + 2 (into the stage of W block
+//      b - 1); second half: X of block b + 2 (into the stage of X block b, whose fragments are all in registers by now)
+//   2. first half: wait until all but this wavefront's 4 youngest DMA instructions have landed (X and W of block b + 1);
 //      barrier
-// The order of 1 and 2 matters: an LDS read issued behind an LDS-DMA load of the same wavefront does not return before
-// that load has landed; issuing the DMA in two small bursts, a whole half-step before the next reads, keeps that wait short
-// (one burst of 8 per block measured 25 % slower).
+// With the reads and the DMA in front of the MFMAs a block took 3078 clocks of which 2048 are products, 2700 to 2890 so. The DMA comes
+// in two small bursts, each a whole half-step before what it loads is waited for (one burst of 8 per block measured 25 % slower).
 // The accumulators leave through LDS (bias added in FP32, one rounding) so that global stores are full 16-byte pieces of
 // consecutive threads along a row. A launch of one tile per CU spends about 14 us outside the loop (1.35 us per block inside it):
 // hence the start after one block instead of two, the bias requested ahead of the operands and the write-out in batches of 8
-// (us, before -> now: 4096 x 1152 x 4608 52.6 -> 50.4, x 3456 36.1 -> 35.1, 4608 x 3072 x 3072 78.5 -> 77.6).
+// (us, before -> now: 4096 x 1152 x 4608 52.6 -> 50.4, x 3456 36.1 -> 35.1, 4608 x 3072 x 3072 78.5 -> 77.6; with the half-steps as they are now 4096 x 3456 x 1152 36.2 -> 32.8).
 #include <type_traits>
 #include <utility>
 
@@ -39,19 +37,19 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 template <typename T> struct Mma;
 template <> struct Mma<__bf16> {
     using v8 = bf16x8;
     using v4 = bf16x4;
-    static __device__ __forceinline__ f32x16 run(v8 a, v8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
+    static __device__ __forceinline__ f32x4 run(v8 a, v8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 };
 template <> struct Mma<_Float16> {
     using v8 = f16x8;
     using v4 = f16x4;
-    static __device__ __forceinline__ f32x16 run(v8 a, v8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0); }
+    static __device__ __forceinline__ f32x4 run(v8 a, v8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
 };
 
 constexpr int kTile = 256;                       // tokens and features per work group
@@ -87,7 +85,7 @@ __global__ void __launch_bounds__(kThreads, 2) linear_dma_kernel(const LinearBat
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
+    const int lane = tid & 63, lr = lane & 15, lg = lane >> 4;      // (row of a 16-row block, group of 8 contraction elements)
     const int wn = wave & 1, wm = wave >> 1;
 
     // ── DMA duty: instructions 4 wave .. 4 wave + 3 of either operand; instruction j fills rows 8 j .. 8 j + 7 ──
@@ -111,89 +109,82 @@ __global__ void __launch_bounds__(kThreads, 2) linear_dma_kernel(const LinearBat
         // (the LDS destination travels in m0; the s_nop is the wait state an LDS-DMA instruction needs behind a write of m0)
         asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(base), "{m0}"(dst) : "memory");
     };
-    auto dma_x = [&](int stage) {
-        const unsigned dst = lds_base + stage * kOpBytes + 4 * wave * 1024;
+    // instruction u of this wavefront's four of a block; xg / wg stand on that block
+    auto dma_x = [&](int stage, int u) { dma(xoff[u], xg, lds_base + stage * kOpBytes + (4 * wave + u) * 1024); };
+    auto dma_w = [&](int stage, int u) { dma(woff[u], wg, lds_base + kWRing + stage * kOpBytes + (4 * wave + u) * 1024); };
+    auto dma_block = [&](int stage) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) dma(xoff[u], xg, dst + u * 1024);
+        for (int u = 0; u < 4; ++u) dma_x(stage, u);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) dma_w(stage, u);
         xg += kBK * 2;
-    };
-    auto dma_w = [&](int stage) {
-        const unsigned dst = lds_base + kWRing + stage * kOpBytes + 4 * wave * 1024;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) dma(woff[u], wg, dst + u * 1024);
         wg += kBK * 2;
     };
 
-    // ── fragment reads: row lq of a 32-row block, 16-byte piece 4 h + 2 kc + lh of the row (swizzled position) ──
-    const int f = (lq >> 1) & 7;
-    unsigned frag[2][2];   // [half][kc]
+    // ── fragment reads: row lr of a 16-row block, 16-byte piece 4 h + lg of the row (swizzled position) ──
+    unsigned frag[2];   // [half]
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int kc = 0; kc < 2; ++kc) frag[h][kc] = lq * 128 + (((4 * h + 2 * kc + lh) ^ f) << 4);
+    for (int h = 0; h < 2; ++h) frag[h] = lr * 128 + (((4 * h + lg) ^ ((lr >> 1) & 7)) << 4);
     const unsigned x_blk = wm * 64 * 128;                         // this wavefront's first token row, in bytes
     const unsigned w_blk = kWRing + wn * 128 * 128;
-    V8 wf[2][4][2], xf[2][2][2];   // [register set][block][kc]
-    // fragments of half-step t (block t / 2, half t % 2) into register set t % 2
-    auto read_frags = [&](auto set_tag, int t) {
-        constexpr int S = decltype(set_tag)::value;
+    V8 wf[2][8], xf[2][4];   // [register set][block]
+    // reads [R0, R1) of the 12 fragments of half-step t (block t / 2, half t % 2) into register set t % 2, in the order in which its
+    // products use them: two token blocks, the feature blocks, the other token blocks
+    auto read_frags = [&](auto set_tag, auto r0_tag, auto r1_tag, int t) {
+        constexpr int S = decltype(set_tag)::value, R0 = decltype(r0_tag)::value, R1 = decltype(r1_tag)::value;
         const int b = t >> 1;
         const unsigned char* xs = lds + (b & 1) * kOpBytes + x_blk;
         const unsigned char* ws = lds + (b % 3) * kOpBytes + w_blk;
-#pragma unroll
-        for (int kc = 0; kc < 2; ++kc) {
-            const unsigned fr = frag[S][kc];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) wf[S][i][kc] = *reinterpret_cast<const V8*>(ws + i * 4096 + fr);
-#pragma unroll
-            for (int j = 0; j < 2; ++j) xf[S][j][kc] = *reinterpret_cast<const V8*>(xs + j * 4096 + fr);
-        }
+        [&]<int... R>(std::integer_sequence<int, R...>) {
+            ([&] {
+                constexpr int k = R0 + R;
+                if constexpr (k >= 2 && k < 10) wf[S][k - 2] = *reinterpret_cast<const V8*>(ws + (k - 2) * 2048 + frag[S]);
+                else xf[S][k < 2 ? k : k - 8] = *reinterpret_cast<const V8*>(xs + (k < 2 ? k : k - 8) * 2048 + frag[S]);
+            }(), ...);
+        }(std::make_integer_sequence<int, R1 - R0>{});
     };
 
-    f32x16 acc[4][2];
+    f32x4 acc[8][4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 8; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     const int nb = p.K / kBK;      // blocks
     const int nt = 2 * nb;         // half-steps
     // prologue: blocks 0 and 1 requested, block 0 in LDS (block 1 has landed by the first close_half; waiting for it here too
     // made every work group of the launch wait for twice the bytes before its first product)
-    dma_x(0);
-    dma_w(0);
+    dma_block(0);
     if (nb > 1) {
-        dma_x(1);
-        dma_w(1);
+        dma_block(1);
         asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
     } else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     using Set0 = std::integral_constant<int, 0>;
     using Set1 = std::integral_constant<int, 1>;
-    using Kc0 = std::integral_constant<int, 0>;
-    using Kc1 = std::integral_constant<int, 1>;
-    read_frags(Set0{}, 0);
+    read_frags(Set0{}, std::integral_constant<int, 0>{}, std::integral_constant<int, 12>{}, 0);
 
-    auto mfma_half = [&](auto set_tag, auto kc_tag) {
-        constexpr int S = decltype(set_tag)::value, kc = decltype(kc_tag)::value;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) acc[i][j] = M::run(wf[S][i][kc], xf[S][j][kc], acc[i][j]);
-    };
-    // half-step t (set S = t % 2): fragment reads of half-step t + 1, then the DMA of half of the block after next
-    auto feed = [&](auto set_tag, int t) -> bool {
+    // half-step t (set S = t % 2): its 32 products, between them the fragment reads of half-step t + 1 and the DMA of half of the block
+    // after next
+    auto half_step = [&](auto set_tag, int t) -> bool {
         constexpr int S = decltype(set_tag)::value;
-        read_frags(std::integral_constant<int, 1 - S>{}, t + 1);   // (behind the last half-step: a stage of no block, never used)
         const int nxt = (t >> 1) + 2;
         const bool more = nxt < nb;
-        if (more) {
-            if constexpr (S == 0) dma_w(nxt % 3);
-            else dma_x(nxt & 1);
-        }
-        __builtin_amdgcn_sched_barrier(0);
+        [&]<int... Q>(std::integer_sequence<int, Q...>) {
+            ([&] {
+                // (two token blocks at a time, each feature block meets both in a row)
+                constexpr int i = (Q >> 1) & 7, j = 2 * (Q >> 4) + (Q & 1);
+                acc[i][j] = M::run(wf[S][i], xf[S][j], acc[i][j]);
+                if constexpr (Q < 24 && Q % 2 == 1)    // (behind the last half-step: a stage of no block, never used)
+                    read_frags(std::integral_constant<int, 1 - S>{}, std::integral_constant<int, Q / 2>{}, std::integral_constant<int, Q / 2 + 1>{}, t + 1);
+                else if (Q >= 24 && Q % 2 == 1 && more) {
+                    if constexpr (S == 0) dma_w(nxt % 3, Q / 2 - 12);
+                    else dma_x(nxt & 1, Q / 2 - 12);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }(), ...);
+        }(std::make_integer_sequence<int, 32>{});
+        if (more) { if constexpr (S == 0) wg += kBK * 2; else xg += kBK * 2; }
         return more;
     };
     auto close_half = [&](auto set_tag, bool more) {
@@ -208,35 +199,29 @@ __global__ void __launch_bounds__(kThreads, 2) linear_dma_kernel(const LinearBat
         __builtin_amdgcn_s_barrier();
     };
     for (int t = 0; t < nt; t += 2) {
-        const bool m0_ = feed(Set0{}, t);
-        mfma_half(Set0{}, Kc0{});
-        mfma_half(Set0{}, Kc1{});
+        const bool m0_ = half_step(Set0{}, t);
         close_half(Set0{}, m0_);
-        const bool m1_ = feed(Set1{}, t + 1);
-        mfma_half(Set1{}, Kc0{});
-        mfma_half(Set1{}, Kc1{});
+        const bool m1_ = half_step(Set1{}, t + 1);
         close_half(Set1{}, m1_);
     }
 
-    // ── epilogue: acc[i][j][4 g + e] is feature wn*128 + 32 i + 8 g + 4 lh + e of token wm*64 + 32 j + lq ──
+    // ── epilogue: acc[i][j][e] is feature wn*128 + 16 i + 4 lg + e of token wm*64 + 16 j + lr ──
     typedef T t2 __attribute__((ext_vector_type(2)));
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 8; ++i) {
+        const int feat = wn * 128 + 16 * i + 4 * lg;
+        const int src = 4 * (8 * i + 2 * lg);      // byte index of the lane that holds the bias of this and the next feature
+        const t2 b01 = __builtin_bit_cast(t2, __builtin_amdgcn_ds_bpermute(src, static_cast<int>(bias2)));
+        const t2 b23 = __builtin_bit_cast(t2, __builtin_amdgcn_ds_bpermute(src + 4, static_cast<int>(bias2)));
+        const float bv[4] = {static_cast<float>(b01[0]), static_cast<float>(b01[1]), static_cast<float>(b23[0]), static_cast<float>(b23[1])};
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const int feat = wn * 128 + 32 * i + 8 * g + 4 * lh;
-            const int src = 4 * (16 * i + 4 * g + 2 * lh);      // byte index of the lane that holds the bias of this and the next feature
-            const t2 b01 = __builtin_bit_cast(t2, __builtin_amdgcn_ds_bpermute(src, static_cast<int>(bias2)));
-            const t2 b23 = __builtin_bit_cast(t2, __builtin_amdgcn_ds_bpermute(src + 4, static_cast<int>(bias2)));
-            const float bv[4] = {static_cast<float>(b01[0]), static_cast<float>(b01[1]), static_cast<float>(b23[0]), static_cast<float>(b23[1])};
+        for (int j = 0; j < 4; ++j) {
+            typename M::v4 o;
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                typename M::v4 o;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) o[e] = static_cast<T>(acc[i][j][4 * g + e] + bv[e]);
-                *reinterpret_cast<typename M::v4*>(lds + (wm * 64 + 32 * j + lq) * kOutStride + feat * 2) = o;
-            }
+            for (int e = 0; e < 4; ++e) o[e] = static_cast<T>(acc[i][j][e] + bv[e]);
+            *reinterpret_cast<typename M::v4*>(lds + (wm * 64 + 16 * j + lr) * kOutStride + feat * 2) = o;
         }
+    }
     __syncthreads();
     // (8 pieces read before the first is stored; read and stored one by one, each waited for the one before)
     const int cc = tid & 31;   // 16-byte piece of a row

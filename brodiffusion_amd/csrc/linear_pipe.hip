@@ -9,14 +9,22 @@
 // the global side: the 16-byte piece in position c of row r is piece c ^ ((r >> 1) & 7) (INT8 rows: c ^ ((r >> 2) & 3)).
 //
 // A work group is WM x WN wavefronts over tokens x features; a wavefront owns TM x TN blocks of 32 x 32 (as in linear.hip the
-// product is computed transposed: MFMA rows are features). A stage is read in two halves into two register sets. Step t:
-//   read half 1 of stage t; multiply half 0
+// product is computed transposed: MFMA rows are features). A stage is multiplied in two halves of 32 contraction elements, each
+// read into a register set of its own while the other is multiplied. Step t:
+//   multiply half 0 of stage t, between the products read half 1
 //   wait until stage t + 1 has landed and this wavefront's reads of stage t have returned; barrier (for everybody)
-//   read half 0 of stage t + 1; multiply half 1 of stage t
+//   multiply half 1 of stage t, between the products read half 0 of stage t + 1
 // and the DMA of stage t + S, which goes into the ring slot of stage t, is dealt out between the MFMAs of the second half of
 // step t and the first half of step t + 1: issued in one burst behind the barrier it made a step of 128 x 128 take 0.57 us
 // on an otherwise empty compute unit, 0.4 dealt out. The accumulation order is the same in every form (and in linear_dma.hip):
 // a problem gives the same bits whichever one takes it, alone or in a launch with others.
+//
+// Products are v_mfma_f32_16x16x32, two token blocks with one feature block in a row. What bounds the large forms on values of a
+// real spread is the power limit, and a loop of these keeps up 2.07 PFLOP/s (bf16, N(0, 1); 1.84 fp16) at it, one of
+// v_mfma_f32_32x32x16, which moves twice the accumulator registers per FLOP, 1.78 (1.65): the same bits. Reads in one burst in
+// front of the products of a half kept the matrix pipe waiting for the LDS queue of all wavefronts behind each barrier: a step of
+// 256 x 128 took 1427 clocks of which 1024 are products, 1260 so (halves of up to 8 products of 16-bit weights keep the burst). Both
+// together (us): 4096 x 1152 x 1152 16.1 -> 14.8, 1024 x 6720 x 2240 37.6 -> 34, three of 16384 x 512 x 512 34.1 -> 32.8.
 //
 // With NL > 0 the work group has NL further wavefronts that do nothing but load (a whole stage behind the barrier that frees its slot)
 // and the others nothing but read and multiply: an LDS-DMA instruction keeps its wavefront from issuing for 33 clocks, the products of
@@ -91,6 +99,7 @@ __global__ void __launch_bounds__(64 * (WM * WN + NL), 2) linear_pipe_kernel(con
     using V8 = typename M::v8;
     using V4 = typename M::v4;
     constexpr int BM = G::BM, BN = G::BN, BN_OUT = G::BN_OUT, MI = G::MI;
+    constexpr int FB = 2 * TN, TB = 2 * TM;      // blocks of 16 features and of 16 tokens of a wavefront
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
 
     // Tiles of all problems in one row; consecutive work-group ids go to the 8 XCDs in turn, and every XCD (one L2) takes a
@@ -111,7 +120,7 @@ __global__ void __launch_bounds__(64 * (WM * WN + NL), 2) linear_pipe_kernel(con
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lane = tid & 63, lq = lane & 31, lh = lane >> 5;
+    const int lane = tid & 63, lr = lane & 15, lg = lane >> 4;      // (row of a 16-row block, group of 8 contraction elements)
     const int wm = wave % WM, wn = wave / WM;
 
     const int lw = NL ? wave - G::NW : wave;     // (NL: the loading wavefronts come last)
@@ -167,72 +176,84 @@ __global__ void __launch_bounds__(64 * (WM * WN + NL), 2) linear_pipe_kernel(con
     // (N is a multiple of 8, so 4 features are in or out together; those past the end are not stored.)
     typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
     const T* const bias = static_cast<const T*>(p.bias);
-    V4 braw[TN][4];
-    f32x4_a4 sraw[W8 ? TN : 1][4];
-    auto feature = [&](int a, int g) { return min(n0 + (GEGLU ? wn : wn * TN + a) * 32 + 8 * g + 4 * lh, p.N - 4) + (GEGLU ? a * p.N : 0); };
+    V4 braw[FB];
+    f32x4_a4 sraw[W8 ? FB : 1];
+    // (GEGLU: blocks 0 and 1 are values, 2 and 3 the gates of the same features)
+    auto feature = [&](int a) { return min(n0 + (GEGLU ? wn * 32 + 16 * (a & 1) : wn * TN * 32 + 16 * a) + 4 * lg, p.N - 4) + (GEGLU ? (a >> 1) * p.N : 0); };
 #pragma unroll
-    for (int a = 0; a < TN; ++a)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            if constexpr (W8) sraw[a][g] = *reinterpret_cast<const f32x4_a4*>(p.w_scale + feature(a, g));
-            braw[a][g] = V4{};
-        }
+    for (int a = 0; a < FB; ++a) {
+        if constexpr (W8) sraw[a] = *reinterpret_cast<const f32x4_a4*>(p.w_scale + feature(a));
+        braw[a] = V4{};
+    }
     if (bias != nullptr) {
 #pragma unroll
-        for (int a = 0; a < TN; ++a)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) braw[a][g] = *reinterpret_cast<const V4*>(bias + feature(a, g));
+        for (int a = 0; a < FB; ++a) braw[a] = *reinterpret_cast<const V4*>(bias + feature(a));
     }
 
-    // ── fragment reads: a stage is four chunks of 16 contraction elements, read two at a time ──
-    unsigned xaddr[4], waddr[4];
+    // ── fragment reads: a stage is two halves of 32 contraction elements, one MFMA operand each ──
+    unsigned xaddr[2], waddr[2];
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-        xaddr[kk] = wm * TM * 4096 + lq * 128 + (((2 * kk + lh) ^ ((lq >> 1) & 7)) << 4);
-        waddr[kk] = G::X_BYTES + wn * TN * 32 * G::WROW + (W8 ? lq * 64 + ((kk ^ ((lq >> 2) & 3)) << 4) + 8 * lh : lq * 128 + (((2 * kk + lh) ^ ((lq >> 1) & 7)) << 4));
+    for (int h = 0; h < 2; ++h) {
+        xaddr[h] = wm * TM * 4096 + lr * 128 + (((4 * h + lg) ^ ((lr >> 1) & 7)) << 4);
+        waddr[h] = G::X_BYTES + wn * TN * 32 * G::WROW +
+                   (W8 ? lr * 64 + (((2 * h + (lg >> 1)) ^ ((lr >> 2) & 3)) << 4) + 8 * (lg & 1) : lr * 128 + (((4 * h + lg) ^ ((lr >> 1) & 7)) << 4));
     }
     using WRaw = std::conditional_t<W8, u32x2, V8>;
-    V8 xf[2][2][TM];
-    WRaw wf[2][2][TN];
-    auto read_half = [&](auto half_tag, unsigned slot) {
-        constexpr int H = decltype(half_tag)::value;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-#pragma unroll
-            for (int b = 0; b < TM; ++b) xf[H][i][b] = *reinterpret_cast<const V8*>(lds + slot + xaddr[2 * H + i] + b * 4096);
-#pragma unroll
-            for (int a = 0; a < TN; ++a) wf[H][i][a] = *reinterpret_cast<const WRaw*>(lds + slot + waddr[2 * H + i] + a * 32 * G::WROW);
-        }
+    V8 xf[2][TB];
+    WRaw wf[2][FB];
+    // reads [R0, R1) of the NR of a half, in the order in which its products use them: two token blocks, the feature blocks, the other
+    // token blocks
+    constexpr int NR = TB + FB;
+    auto read_pieces = [&](auto half_tag, auto r0_tag, auto r1_tag, unsigned slot) {
+        constexpr int H = decltype(half_tag)::value, R0 = decltype(r0_tag)::value, R1 = decltype(r1_tag)::value;
+        [&]<int... R>(std::integer_sequence<int, R...>) {
+            ([&] {
+                constexpr int k = R0 + R;
+                if constexpr (k >= 2 && k < 2 + FB) wf[H][k - 2] = *reinterpret_cast<const WRaw*>(lds + slot + waddr[H] + (k - 2) * 16 * G::WROW);
+                else {
+                    constexpr int b = k < 2 ? k : k - FB;
+                    xf[H][b] = *reinterpret_cast<const V8*>(lds + slot + xaddr[H] + b * 2048);
+                }
+            }(), ...);
+        }(std::make_integer_sequence<int, R1 - R0>{});
     };
-    f32x16 acc[TN][TM];
+    auto read_half = [&](auto half_tag, unsigned slot) { read_pieces(half_tag, std::integral_constant<int, 0>{}, std::integral_constant<int, NR>{}, slot); };
+    f32x4 acc[FB][TB];
 #pragma unroll
-    for (int a = 0; a < TN; ++a)
+    for (int a = 0; a < FB; ++a)
 #pragma unroll
-        for (int b = 0; b < TM; ++b)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[a][b][e] = 0.f;
-    // the MFMAs of a half stage, with DMA pieces [J0, J1) of the stage that goes to `slot` between them: issued in one burst they
-    // would keep the wavefront from its MFMAs for as long as the burst takes (16 clocks per instruction and compute unit)
-    auto multiply_half = [&](auto half_tag, auto j0_tag, auto j1_tag, unsigned slot) {
-        constexpr int H = decltype(half_tag)::value, J0 = decltype(j0_tag)::value, J1 = decltype(j1_tag)::value, NM = 2 * TM * TN;
-        V8 w[2][TN];
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int a = 0; a < TN; ++a) {
-                if constexpr (W8) w[i][a] = widen<T>(wf[H][i][a]);
-                else w[i][a] = wf[H][i][a];
-            }
+        for (int b = 0; b < TB; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // the MFMAs of a half stage, and between them the reads of the next one (READ: half 1 - H from `from`) and DMA pieces [J0, J1) of
+    // the stage that goes to `slot`
+    auto multiply_half = [&](auto half_tag, auto read_tag, unsigned from, auto j0_tag, auto j1_tag, unsigned slot) {
+        constexpr int H = decltype(half_tag)::value, J0 = decltype(j0_tag)::value, J1 = decltype(j1_tag)::value, NM = TB * FB;
+        constexpr bool READ = decltype(read_tag)::value;
+        V8 w[W8 ? FB : 1];
+        // (a half of few MFMAs: all reads ahead of them, as dealt out the last one returns too late; INT8: behind the first two, under the
+        //  widening of the others: 2048 x 640 x 640 5.5 us, 5.9 with the burst)
+        constexpr bool BURST = NM <= 8 && !W8;
+        constexpr int SPAN = NM <= 8 ? 2 : NM * 3 / 4;      // MFMAs that have reads behind them
+        if constexpr (READ && BURST) {
+            read_pieces(std::integral_constant<int, 1 - H>{}, std::integral_constant<int, 0>{}, std::integral_constant<int, NR>{}, from);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         [&]<int... Q>(std::integer_sequence<int, Q...>) {
             ([&] {
-                constexpr int i = Q / (TM * TN), a = Q / TM % TN, b = Q % TM;
-                acc[a][b] = M::run(w[i][a], xf[H][i][b], acc[a][b]);
+                // (two token blocks at a time, each feature block meets both in a row)
+                constexpr int a = Q / 2 % FB, b = Q / (2 * FB) * 2 + Q % 2;
+                if constexpr (!W8) acc[a][b] = M::run16(wf[H][a], xf[H][b], acc[a][b]);
+                else {
+                    if constexpr (b == 0) w[a] = widen<T>(wf[H][a]);
+                    acc[a][b] = M::run16(w[a], xf[H][b], acc[a][b]);
+                }
+                if constexpr (READ && !BURST && Q < SPAN)
+                    read_pieces(std::integral_constant<int, 1 - H>{}, std::integral_constant<int, NR * Q / SPAN>{}, std::integral_constant<int, NR * (Q + 1) / SPAN>{}, from);
                 constexpr int j0 = J0 + (J1 - J0) * Q / NM, j1 = J0 + (J1 - J0) * (Q + 1) / NM;
                 if constexpr (j1 > j0) {
 #pragma unroll
                     for (int j = j0; j < j1; ++j) dma_piece(j, slot);
-                    __builtin_amdgcn_sched_barrier(0);
                 }
+                if constexpr (j1 > j0 || (READ && !BURST && Q < SPAN)) __builtin_amdgcn_sched_barrier(0);
             }(), ...);
         }(std::make_integer_sequence<int, NM>{});
     };
@@ -248,22 +269,21 @@ __global__ void __launch_bounds__(64 * (WM * WN + NL), 2) linear_pipe_kernel(con
     auto step = [&](auto d0_tag, auto d1_tag, int t) {
         constexpr bool D0 = decltype(d0_tag)::value, D1 = decltype(d1_tag)::value;
         const unsigned nxt = cur + G::STAGE == S * G::STAGE ? 0u : cur + G::STAGE;
-        read_half(Half1{}, cur);
-        __builtin_amdgcn_sched_barrier(0);
         if constexpr (D0) {
-            multiply_half(Half0{}, Mid{}, All{}, prev);
+            multiply_half(Half0{}, std::true_type{}, cur, Mid{}, All{}, prev);
             next_stage();
         } else {
-            multiply_half(Half0{}, Half0{}, Half0{}, 0u);
+            multiply_half(Half0{}, std::true_type{}, cur, Half0{}, Half0{}, 0u);
         }
         __builtin_amdgcn_sched_barrier(0);
         if (D1 || t + 1 < n) {
             wait_barrier(D1 ? S - 2 : (t + S - 1 < n - 1 ? t + S - 1 : n - 1) - (t + 1));
-            read_half(Half0{}, nxt);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (D1) multiply_half(Half1{}, std::true_type{}, nxt, Half0{}, Mid{}, cur);
+            else multiply_half(Half1{}, std::true_type{}, nxt, Half0{}, Half0{}, 0u);
+        } else {
+            multiply_half(Half1{}, std::false_type{}, 0u, Half0{}, Half0{}, 0u);
         }
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr (D1) multiply_half(Half1{}, Half0{}, Mid{}, cur);
-        else multiply_half(Half1{}, Half0{}, Half0{}, 0u);
         __builtin_amdgcn_sched_barrier(0);
         prev = cur;
         cur = nxt;
@@ -295,20 +315,16 @@ __global__ void __launch_bounds__(64 * (WM * WN + NL), 2) linear_pipe_kernel(con
         read_half(Half0{}, 0);
         for (int t = 0; t < n - 1; ++t) {
             const unsigned nxt = cur + G::STAGE == S * G::STAGE ? 0u : cur + G::STAGE;
-            read_half(Half1{}, cur);
-            __builtin_amdgcn_sched_barrier(0);
-            multiply_half(Half0{}, Half0{}, Half0{}, 0u);
+            multiply_half(Half0{}, std::true_type{}, cur, Half0{}, Half0{}, 0u);
             __builtin_amdgcn_sched_barrier(0);
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // stage t is in registers
-            read_half(Half0{}, nxt);
             __builtin_amdgcn_sched_barrier(0);
-            multiply_half(Half1{}, Half0{}, Half0{}, 0u);
+            multiply_half(Half1{}, std::true_type{}, nxt, Half0{}, Half0{}, 0u);
             __builtin_amdgcn_sched_barrier(0);
             cur = nxt;
         }
-        read_half(Half1{}, cur);
-        multiply_half(Half0{}, Half0{}, Half0{}, 0u);
-        multiply_half(Half1{}, Half0{}, Half0{}, 0u);
+        multiply_half(Half0{}, std::true_type{}, cur, Half0{}, Half0{}, 0u);
+        multiply_half(Half1{}, std::false_type{}, 0u, Half0{}, Half0{}, 0u);
     } else if (n < S) {   // everything fits the ring
         for (int s = 0; s < n; ++s) {
 #pragma unroll
@@ -336,48 +352,42 @@ __global__ void __launch_bounds__(64 * (WM * WN + NL), 2) linear_pipe_kernel(con
     }
 
     __syncthreads();   // the ring is used up
-    // ── epilogue: acc[a][b][4g + i] is feature n0 + (wn TN + a) 32 + 8g + 4 lh + i of token m0 + (wm TM + b) 32 + lq; the tile
+    // ── epilogue: acc[a][b][i] is feature n0 + wn TN 32 + 16 a + 4 lg + i of token m0 + wm TM 32 + 16 b + lr; the tile
     //    leaves through LDS as 16-byte pieces of rows of Y ──
     if constexpr (GEGLU) {
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const int feat = wn * 32 + 8 * g + 4 * lh;
+        for (int a = 0; a < 2; ++a)
 #pragma unroll
-            for (int b = 0; b < TM; ++b) {
-                    V4 o;
+            for (int b = 0; b < TB; ++b) {
+                V4 o;
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const float bv = static_cast<float>(braw[0][g][i]), bg = static_cast<float>(braw[1][g][i]);
-                        float val, gate;
-                        if constexpr (W8) {   // the two halves are rounded where the reference's 16-bit intermediate would
-                            val = static_cast<float>(static_cast<T>(scaled_acc(acc[0][b][4 * g + i], sraw[0][g][i], bv)));
-                            gate = static_cast<float>(static_cast<T>(scaled_acc(acc[1][b][4 * g + i], sraw[1][g][i], bg)));
-                        } else {
-                            val = acc[0][b][4 * g + i] + bv;
-                            gate = acc[1][b][4 * g + i] + bg;
-                        }
-                        o[i] = static_cast<T>(val * gelu_erf(gate));
+                for (int i = 0; i < 4; ++i) {
+                    const float bv = static_cast<float>(braw[a][i]), bg = static_cast<float>(braw[2 + a][i]);
+                    float val, gate;
+                    if constexpr (W8) {   // the two halves are rounded where the reference's 16-bit intermediate would
+                        val = static_cast<float>(static_cast<T>(scaled_acc(acc[a][b][i], sraw[a][i], bv)));
+                        gate = static_cast<float>(static_cast<T>(scaled_acc(acc[2 + a][b][i], sraw[2 + a][i], bg)));
+                    } else {
+                        val = acc[a][b][i] + bv;
+                        gate = acc[2 + a][b][i] + bg;
                     }
-                    *reinterpret_cast<V4*>(lds + ((wm * TM + b) * 32 + lq) * G::OUT_ROW + feat * 2) = o;
+                    o[i] = static_cast<T>(val * gelu_erf(gate));
                 }
-        }
+                *reinterpret_cast<V4*>(lds + (wm * TM * 32 + 16 * b + lr) * G::OUT_ROW + (wn * 32 + 16 * a + 4 * lg) * 2) = o;
+            }
     } else {
 #pragma unroll
-        for (int a = 0; a < TN; ++a)
+        for (int a = 0; a < FB; ++a)
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int feat = (wn * TN + a) * 32 + 8 * g + 4 * lh;
+            for (int b = 0; b < TB; ++b) {
+                V4 o;
 #pragma unroll
-                for (int b = 0; b < TM; ++b) {
-                        V4 o;
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const float bv = static_cast<float>(braw[a][g][i]);
-                            if constexpr (W8) o[i] = static_cast<T>(scaled_acc(acc[a][b][4 * g + i], sraw[a][g][i], bv));
-                            else o[i] = static_cast<T>(acc[a][b][4 * g + i] + bv);
-                        }
-                        *reinterpret_cast<V4*>(lds + ((wm * TM + b) * 32 + lq) * G::OUT_ROW + feat * 2) = o;
-                    }
+                for (int i = 0; i < 4; ++i) {
+                    const float bv = static_cast<float>(braw[a][i]);
+                    if constexpr (W8) o[i] = static_cast<T>(scaled_acc(acc[a][b][i], sraw[a][i], bv));
+                    else o[i] = static_cast<T>(acc[a][b][i] + bv);
+                }
+                *reinterpret_cast<V4*>(lds + (wm * TM * 32 + 16 * b + lr) * G::OUT_ROW + (wn * TN * 32 + 16 * a + 4 * lg) * 2) = o;
             }
     }
     __syncthreads();
