@@ -105,6 +105,8 @@ bool sdpa_supported(int dtype, int head_dim);
 bool sdpa_wide_head(int head_dim);
 size_t sdpa_wide_split_scratch_bytes(const SdpaDev& p, int head_dim);
 int launch_sdpa_wide(const SdpaDev& p, int dtype, int head_dim, hipStream_t stream);
+// head_dim 512, long calls: the launch alone, planned and merged by launch_sdpa_wide
+int launch_sdpa_wide_long(const SdpaDev& p, bool bf16, int n_q_tiles, int n_split, int n_blocks, hipStream_t stream);
 
 // Calls with few query rows (sdpa_small.hip) and unmasked ones of some sizes (sdpa_flow.hip): whether the kernel takes a call at kernel
 // choice 0, and the launch.

@@ -18,6 +18,8 @@
 //   chunks, f(r) = 4 (r % 4) + (r / 4) % 4: the K fragment reads (16 rows, one chunk column) and the V transpose reads
 //   (4 rows, one 64-byte window) are both free of bank conflicts.
 //
+// Long calls of head_dim 512 take the form of sdpa_wide_long.hip; planning, scratch and merge are the same.
+//
 // A query tile is 128 rows, so a VAE mid-block has 32 (64 x 64 latent) to 128 tiles for 256 compute units: the key axis is
 // cut into as many pieces as shorten the launch (wide_split), each leaving its output accumulators and softmax statistics in
 // the caller's scratch, all FP32, merged in a fixed order by wide_combine_kernel: the result is rounded once.
@@ -25,33 +27,12 @@
 // Masks work as everywhere (per-row visible key interval, kv_valid_len, key mask); cached prefixes, logit bias, lse output,
 // packed sequences and K rotated tile by tile are not offered at these widths (K rotated into a scratch and Q rotated on
 // load are).
-#include "sdpa_tiles.h"
+#include "sdpa_wide.h"
 
 namespace mi {
 namespace {
 
 using namespace sdpa;
-
-constexpr int kWideThreads = 256;
-constexpr int kWideRows = 128;    // query rows per work group, 32 per wavefront
-constexpr int kWideKeys = 32;     // key rows per step
-
-template <int D> struct WideGeo {
-    using G = HeadGeo<D>;
-    static constexpr int ROWB = D * 2;                  // bytes per row in LDS
-    static constexpr int TILE = kWideKeys * ROWB;       // one operand stage
-    static constexpr int VOFF = 2 * TILE;               // the V stages follow the K stages
-    static constexpr int NDMA = TILE / 1024 / 4;        // DMA instructions per wavefront and operand tile
-    static constexpr int KC = D / 16;                   // 16-element contraction chunks of K Q^T
-    static constexpr int VB = D / 32;                   // 32-row blocks of O^T
-    static constexpr int STAGED = kWideRows * G::O_STRIDE;   // the staged Q tile, later the staged output, over the rings
-    static constexpr int LDS_BYTES = 4 * TILE > STAGED ? 4 * TILE : STAGED;
-    static_assert(D % 128 == 0 && TILE % 4096 == 0, "whole swizzle groups per row, whole DMA instructions per wavefront");
-    static_assert(LDS_BYTES <= 160 * 1024, "one work group must fit the LDS of a compute unit");
-    // A partial result, FP32: the accumulators of the four wavefronts as their lanes hold them (16-byte piece ((w D / 8 + c) 64 +
-    // lane): head-dim elements 8 c + 4 lh .. + 3 of row 32 w + lq), then 128 references and 128 denominators
-    static constexpr long SLOT = static_cast<long>(kWideRows) * (D * 4 + 8);
-};
 
 // The MFMAs of this kernel are inline assembly. At head_dim 512 the output accumulator of a wavefront is exactly the 256
 // accumulation registers; left to the compiler, which also puts every other MFMA result there, the scores spill (640 to
@@ -61,12 +42,6 @@ template <int D> struct WideGeo {
 // MFMA of 8 passes (11 wait states); it is kept by construction: the last MFMA of a score tile and the two that follow it
 // are one statement (wide_tail), so the scores are complete before anything can read them, and wide_settle stands in front
 // of the code that works on O.
-#define MI_A10(t) "a" #t "0", "a" #t "1", "a" #t "2", "a" #t "3", "a" #t "4", "a" #t "5", "a" #t "6", "a" #t "7", "a" #t "8", "a" #t "9"
-#define MI_AGPRS                                                                                                              \
-    "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", MI_A10(1), MI_A10(2), MI_A10(3), MI_A10(4), MI_A10(5),       \
-        MI_A10(6), MI_A10(7), MI_A10(8), MI_A10(9), MI_A10(10), MI_A10(11), MI_A10(12), MI_A10(13), MI_A10(14), MI_A10(15),  \
-        MI_A10(16), MI_A10(17), MI_A10(18), MI_A10(19), MI_A10(20), MI_A10(21), MI_A10(22), MI_A10(23), MI_A10(24), "a250",  \
-        "a251", "a252", "a253", "a254", "a255"
 template <typename T> struct WideMma;
 #define MI_WIDE_MMA(TYPE, NAME)                                                                                               \
     template <> struct WideMma<TYPE> {                                                                                        \
@@ -92,16 +67,7 @@ MI_WIDE_MMA(_Float16, "v_mfma_f32_32x32x16_f16")
 #undef MI_WIDE_MMA
 // every MFMA in flight has written its result when this returns
 __device__ __forceinline__ void wide_settle(f32x16& s) { asm volatile("s_nop 15\n\ts_nop 15" : "+v"(s) : : MI_AGPRS); }
-template <int R> __device__ __forceinline__ float o_get() {
-    float f;
-    asm volatile("v_accvgpr_read_b32 %0, a[%1]" : "=v"(f) : "n"(R) : MI_AGPRS);
-    return f;
-}
-template <int R> __device__ __forceinline__ void o_set(float f) { asm volatile("v_accvgpr_write_b32 a[%1], %0" : : "v"(f), "n"(R) : MI_AGPRS); }
-// O = 0; O *= f (the reads of a block go out before its writes: a value just read is not touched in the next instruction)
-template <int N> __device__ __forceinline__ void o_clear() {
-    [&]<int... I>(std::integer_sequence<int, I...>) { (o_set<I>(0.f), ...); }(std::make_integer_sequence<int, N>{});
-}
+// O *= f (the reads of a block go out before its writes: a value just read is not touched in the next instruction)
 template <int B> __device__ __forceinline__ void o_scale_block(float f) {
     [&]<int... I>(std::integer_sequence<int, I...>) {
         const float v[16] = {o_get<16 * B + I>()...};
@@ -121,7 +87,7 @@ __global__ void __launch_bounds__(kWideThreads, 1) sdpa_wide_kernel(const SdpaDe
     using G = HeadGeo<D>;
     using W = WideGeo<D>;
     using V8 = typename Mma<T>::v8;
-    constexpr int KC = W::KC, VB = W::VB;
+    constexpr int KC = D / 16, VB = D / 32;     // 16-element chunks of K Q^T, 32-row blocks of O^T
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
     // pieces of the key axis outermost: the work groups of one XCD walk the same keys
@@ -470,6 +436,13 @@ int wide_split(const SdpaDev& p, int head_dim, int n_cu) {
     return best;
 }
 
+// Whether a call of head_dim 512 goes to sdpa_wide_long.hip, by the key steps of the launch. Below one power-limited round the higher
+// clock does not come and its fixed part (2000 clocks more: twice the instructions to fetch once) shows. One head, fp16, us (this file's
+// kernel / that one): 1024 tokens 33.5 / 34.4, 4096 (16 steps per compute unit) 62.7 / 62.3, 9216 184 / 173, 16384 498 / 454. At 256
+// and 384 there are fewer products per exponential, and that form is the slower one at nearly every length (256: 4096 tokens
+// 41.3 / 42.4, 9216 105 / 110; 384 bf16: 9216 141 / 146).
+bool wide_long_pays(long tiles, int keys, int n_cu) { return tiles * ((keys + kWideKeys - 1) / kWideKeys) >= 16L * n_cu; }
+
 template <typename T, int D>
 int launch_wide_d(const SdpaDev& p, hipStream_t stream) {
     using W = WideGeo<D>;
@@ -485,8 +458,11 @@ int launch_wide_d(const SdpaDev& p, hipStream_t stream) {
                                          W::LDS_BYTES));
         raised = true;
     }
-    hipLaunchKernelGGL((sdpa_wide_kernel<T, D>), dim3(static_cast<unsigned>((blocks + 7) / 8 * 8)), dim3(kWideThreads), W::LDS_BYTES, stream, p,
-                       n_q_tiles, n_split, static_cast<int>(blocks));
+    if (D == 512 && wide_long_pays(tiles, p.Lk, device_cu_count())) {
+        if (launch_sdpa_wide_long(p, std::is_same_v<T, __bf16>, n_q_tiles, n_split, static_cast<int>(blocks), stream) != 0) return -1;
+    } else
+        hipLaunchKernelGGL((sdpa_wide_kernel<T, D>), dim3(static_cast<unsigned>((blocks + 7) / 8 * 8)), dim3(kWideThreads), W::LDS_BYTES, stream, p,
+                           n_q_tiles, n_split, static_cast<int>(blocks));
     if (n_split > 1)
         hipLaunchKernelGGL((wide_combine_kernel<T, D>), dim3(static_cast<unsigned>(tiles), kWideRows * (D / 8) / 256), dim3(256), 0, stream, p,
                            n_q_tiles, n_split);

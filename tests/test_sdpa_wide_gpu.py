@@ -6,7 +6,7 @@ import pytest
 import torch
 
 import brodiffusion_amd as bd
-from helpers import assert_close, randn, to_dev, to_np
+from helpers import TOL, TORCH_DT, assert_close, randn, to_dev, to_np
 
 pytestmark = pytest.mark.gpu
 
@@ -165,3 +165,45 @@ def test_pieces_are_as_close_to_the_exact_result_as_the_whole(dtype, d):
     assert not torch.equal(whole, pieces), "this shape is expected to be cut"
     error = [((x.double() - exact).norm() / exact.norm()).item() for x in (whole, pieces)]
     assert error[1] <= 1.05 * error[0], error
+
+
+@pytest.mark.parametrize("dtype,B,Lq,Lk,kind", [
+    ("fp16", 4096, 1, 1, "plain"),         # one step, one row
+    ("bf16", 2100, 1, 33, "plain"),        # two steps, one key in the second
+    ("fp16", 140, 300, 300, "plain"),      # ragged rows and keys
+    ("bf16", 140, 257, 320, "peaked"),     # the softmax reference is raised along the keys
+    ("bf16", 140, 300, 300, "valid"),      # valid lengths from none to all
+    ("fp16", 140, 300, 300, "key_mask"),
+    ("bf16", 1, 4100, 4113, "causal"),
+    ("fp16", 1, 4096, 4096, "plain"),      # the shortest single head of the long form, its key axis in pieces
+    ("fp16", 1, 3968, 4096, "plain"),      # below it
+])
+def test_wide_head_long_calls(dtype, B, Lq, Lk, kind):
+    """Calls of head_dim 512 with enough key steps for the form of sdpa_wide_long.hip (16 per compute unit), against FP32."""
+    d, dt = 512, TORCH_DT[dtype]
+    g = torch.Generator(device="cuda").manual_seed(8600 + Lq + Lk)
+    q, k, v = (torch.randn(B, n, d, generator=g, device="cuda") for n in (Lq, Lk, Lk))
+    q, k, v = (q * 4 if kind == "peaked" else q).to(dt), k.to(dt), v.to(dt)
+    see = torch.ones(B, Lq, Lk, dtype=torch.bool, device="cuda")
+    if kind == "valid":
+        n = torch.linspace(0, Lk, B, device="cuda").round().int()
+        see &= torch.arange(Lk, device="cuda")[None, None, :] < n[:, None, None]
+        out = bd.sdpa_forward(q, k, v, 1, kv_valid_len=n)
+    elif kind == "key_mask":
+        m = (torch.rand(B, Lk, generator=g, device="cuda") > 0.5).float()
+        m[:, 64:128] = 0
+        see &= m[:, None, :] != 0
+        out = bd.sdpa_forward(q, k, v, 1, key_mask=m)
+    elif kind == "causal":
+        see &= torch.arange(Lk, device="cuda")[None, None, :] <= torch.arange(Lq, device="cuda")[None, :, None] + Lk - Lq
+        out = bd.flash_attention_windowed_forward(q[0], k[0], v[0], None, 1, 0)[None]
+    else:
+        out = bd.sdpa_forward(q, k, v, 1)
+    s = torch.bmm(q.float(), k.float().transpose(1, 2).contiguous()) * d ** -0.5
+    p = torch.softmax(s.masked_fill(~see, float("-inf")), 2).nan_to_num(0.0)     # rows without a visible key are zero
+    ref = torch.bmm(p, v.float())
+    # An output is a mean of values with weights rounded to the type, and is rounded once itself: the largest error of the millions
+    # here is below 2 u max |v| (u the unit roundoff, 2^-8 and 2^-11) and what FP32 sums add, so a fixed bound does not fit
+    err, u = (out.float() - ref).abs().max().item(), 2.0 ** (-8 if dtype == "bf16" else -11)
+    assert torch.isfinite(out).all() and err <= 2 * u * v.float().abs().max().item() + 1e-4, err
+    assert ((out.float() - ref).norm() / ref.norm()).item() <= TOL[dtype][0]
