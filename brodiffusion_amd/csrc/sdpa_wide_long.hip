@@ -9,7 +9,7 @@
 // scale and reference of the scores go under the PV product. 16384 tokens, fp16, us: 498 with v_mfma_f32_32x32x16, 455 so; without the
 // turns 459; mid-block around it (540 before): DMA ahead of the second product 521, exponentials there 537, fragments 5 or 7 ahead
 // instead of 6 523 and 526 (518 in that build).
-// Mid-block of 16384 tokens on four GPUs: 545 -> 508, 540 -> 518 (without the turns), 560 -> 553, 559 -> 549.
+// Mid-block of 16384 tokens on four GPUs: 545 -> 508 and 540 -> 518 (without the turns), 560 -> 553 and 559 -> 549 (as built).
 //   Register layouts (lq = lane % 16, g = lane / 16): A row lq, B column lq, 8 contraction elements from 8 g on; C column lq, element
 //   i is row 4 g + i. A lane holds scores of two query rows (16 r + lq of the wavefront's 32), each shared with the lanes 16, 32 and
 //   48 away; P goes into the PV product as it lies (slot 8 g + t of the contraction is key 4 g + t, for t >= 4 key 16 + 4 g + t - 4).
