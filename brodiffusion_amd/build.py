@@ -27,11 +27,13 @@ FLAGS = [
     "-fno-honor-nans",
     "-Wall", "-Wno-unused-value", "-Wno-unknown-pragmas",
 ]
+# flags of one source alone; the reason stands at its top
+SOURCE_FLAGS = {"linear_pipe.hip": ["-falign-loops=64"]}
 
 
 def _compile(src: str, obj_dir: str, save_temps: bool) -> str:
     obj = os.path.join(obj_dir, src.replace(".hip", ".o"))
-    cmd = [HIPCC, *FLAGS, "-c", os.path.join(CSRC, src), "-o", obj]
+    cmd = [HIPCC, *FLAGS, *SOURCE_FLAGS.get(src, []), "-c", os.path.join(CSRC, src), "-o", obj]
     if save_temps:
         cmd.append("-save-temps=obj")
     r = subprocess.run(cmd, capture_output=True, text=True)

@@ -5,8 +5,10 @@
 // store instructions, and as many steps in flight as the LDS holds (a problem of this size is a chain of memory latencies
 // before it is anything else: with one step in flight, 2048 x 640 x 640 took 10 to 12 us of which 1 us is arithmetic). A
 // stage holds BM rows of X and BN rows of W, 128 bytes each (INT8: 64), back to back as the DMA deposits them; bank
-// conflicts of the fragment reads (one row per lane, 16 consecutive rows per phase) are avoided by an XOR swizzle applied on
-// the global side: the 16-byte piece in position c of row r is piece c ^ ((r >> 1) & 7) (INT8 rows: c ^ ((r >> 2) & 3)).
+// conflicts of the fragment reads (16 rows, one 16-byte piece of each, per phase) are avoided by an XOR swizzle applied on
+// the global side: the 16-byte piece in position c of row r is piece c ^ ((r >> 1) & 7). INT8 rows: c ^ ((r >> 2) & 3), which keeps
+// reads of 8 bytes from 16 rows and two pieces apart (the operands of v_mfma_f32_16x16x32); those of 32 rows and one half of a
+// piece (v_mfma_f32_32x32x16) meet in half of the banks and take two phases.
 //
 // A work group is WM x WN wavefronts over tokens x features; a wavefront owns TM x TN blocks of 32 x 32 (as in linear.hip the
 // product is computed transposed: MFMA rows are features). A stage is multiplied in two halves of 32 contraction elements, each
@@ -25,6 +27,11 @@
 // front of the products of a half kept the matrix pipe waiting for the LDS queue of all wavefronts behind each barrier: a step of
 // 256 x 128 took 1427 clocks of which 1024 are products, 1260 so (halves of up to 8 products of 16-bit weights keep the burst). Both
 // together (us): 4096 x 1152 x 1152 16.1 -> 14.8, 1024 x 6720 x 2240 37.6 -> 34, three of 16384 x 512 x 512 34.1 -> 32.8.
+// A wavefront with one block of INT8 weights multiplies with v_mfma_f32_32x32x16 instead: its step is a chain of latencies and of
+// widening, far from the power limit, and with the other product it is longer in every order of reads and widening tried (us, 32x32x16 /
+// 16x16x32: fp16 32 x 1280 x 5120 15.5 / 16.7, 512 x 1280 x 5120 19.7 / 21.0; bf16 512 x 1280 x 5120 19.1 / 22.0, 1024 x 1280 x 5120
+// 26.3 / 29.4, 77 x 6720 x 2240 10.5 / 11.6). Such loops of 80 to 100 instructions also take up to 3 % more or less by where they start in a cache line
+// of instructions, so that this file is compiled with its loops aligned to 64 bytes (fp16, 64 x 64 tiles: 3 % faster than before).
 //
 // With NL > 0 the work group has NL further wavefronts that do nothing but load (a whole stage behind the barrier that frees its slot)
 // and the others nothing but read and multiply: an LDS-DMA instruction keeps its wavefront from issuing for 33 clocks, the products of
@@ -99,7 +106,11 @@ __global__ void __launch_bounds__(64 * (WM * WN + NL), 2) linear_pipe_kernel(con
     using V8 = typename M::v8;
     using V4 = typename M::v4;
     constexpr int BM = G::BM, BN = G::BN, BN_OUT = G::BN_OUT, MI = G::MI;
-    constexpr int FB = 2 * TN, TB = 2 * TM;      // blocks of 16 features and of 16 tokens of a wavefront
+    // one block of INT8 weights per wavefront: v_mfma_f32_32x32x16 (see the top)
+    constexpr bool ONE = W8 && TM == 1 && TN == 1;
+    constexpr int BS = ONE ? 32 : 16, FB = TN * 32 / BS, TB = TM * 32 / BS;      // rows of a block; feature and token blocks of a wavefront
+    constexpr int KS = BS / 16;                  // products of a half per pair of blocks
+    constexpr int NG = ONE ? 4 : 1;              // groups of 4 features that a lane holds of a block, 8 apart
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
 
     // Tiles of all problems in one row; consecutive work-group ids go to the 8 XCDs in turn, and every XCD (one L2) takes a
@@ -120,7 +131,7 @@ __global__ void __launch_bounds__(64 * (WM * WN + NL), 2) linear_pipe_kernel(con
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lane = tid & 63, lr = lane & 15, lg = lane >> 4;      // (row of a 16-row block, group of 8 contraction elements)
+    const int lane = tid & 63, lr = lane % BS, lg = lane / BS;      // (row of a block, group of 8 contraction elements)
     const int wm = wave % WM, wn = wave / WM;
 
     const int lw = NL ? wave - G::NW : wave;     // (NL: the loading wavefronts come last)
@@ -176,40 +187,45 @@ __global__ void __launch_bounds__(64 * (WM * WN + NL), 2) linear_pipe_kernel(con
     // (N is a multiple of 8, so 4 features are in or out together; those past the end are not stored.)
     typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
     const T* const bias = static_cast<const T*>(p.bias);
-    V4 braw[FB];
-    f32x4_a4 sraw[W8 ? FB : 1];
+    V4 braw[FB * NG];
+    f32x4_a4 sraw[W8 ? FB * NG : 1];
+    // the 4 features from feature(a) on are the lane's group a % NG of block a / NG
     // (GEGLU: blocks 0 and 1 are values, 2 and 3 the gates of the same features)
-    auto feature = [&](int a) { return min(n0 + (GEGLU ? wn * 32 + 16 * (a & 1) : wn * TN * 32 + 16 * a) + 4 * lg, p.N - 4) + (GEGLU ? (a >> 1) * p.N : 0); };
+    auto feature = [&](int a) { return min(n0 + (GEGLU ? wn * 32 + 16 * (a & 1) : wn * TN * 32 + BS / NG * a) + 4 * lg, p.N - 4) + (GEGLU ? (a >> 1) * p.N : 0); };
 #pragma unroll
-    for (int a = 0; a < FB; ++a) {
+    for (int a = 0; a < FB * NG; ++a) {
         if constexpr (W8) sraw[a] = *reinterpret_cast<const f32x4_a4*>(p.w_scale + feature(a));
         braw[a] = V4{};
     }
     if (bias != nullptr) {
 #pragma unroll
-        for (int a = 0; a < FB; ++a) braw[a] = *reinterpret_cast<const V4*>(bias + feature(a));
+        for (int a = 0; a < FB * NG; ++a) braw[a] = *reinterpret_cast<const V4*>(bias + feature(a));
     }
 
-    // ── fragment reads: a stage is two halves of 32 contraction elements, one MFMA operand each ──
-    unsigned xaddr[2], waddr[2];
+    // ── fragment reads: a stage is two halves of 32 contraction elements, KS MFMA operands each ──
+    unsigned xaddr[2 * KS], waddr[2 * KS];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        xaddr[h] = wm * TM * 4096 + lr * 128 + (((4 * h + lg) ^ ((lr >> 1) & 7)) << 4);
-        waddr[h] = G::X_BYTES + wn * TN * 32 * G::WROW +
-                   (W8 ? lr * 64 + (((2 * h + (lg >> 1)) ^ ((lr >> 2) & 3)) << 4) + 8 * (lg & 1) : lr * 128 + (((4 * h + lg) ^ ((lr >> 1) & 7)) << 4));
+    for (int c = 0; c < 2 * KS; ++c) {
+        const int piece = c * (64 / BS) + lg;       // of 8 contraction elements
+        xaddr[c] = wm * TM * 4096 + lr * 128 + ((piece ^ ((lr >> 1) & 7)) << 4);
+        waddr[c] = G::X_BYTES + wn * TN * 32 * G::WROW +
+                   (W8 ? lr * 64 + (((piece >> 1) ^ ((lr >> 2) & 3)) << 4) + 8 * (piece & 1) : lr * 128 + ((piece ^ ((lr >> 1) & 7)) << 4));
     }
     using WRaw = std::conditional_t<W8, u32x2, V8>;
-    V8 xf[2][TB];
-    WRaw wf[2][FB];
+    V8 xf[2][KS * TB];
+    WRaw wf[2][KS * FB];
     // reads [R0, R1) of the NR of a half, in the order in which its products use them: two token blocks, the feature blocks, the other
     // token blocks
-    constexpr int NR = TB + FB;
+    constexpr int NR = KS * (TB + FB);
     auto read_pieces = [&](auto half_tag, auto r0_tag, auto r1_tag, unsigned slot) {
         constexpr int H = decltype(half_tag)::value, R0 = decltype(r0_tag)::value, R1 = decltype(r1_tag)::value;
         [&]<int... R>(std::integer_sequence<int, R...>) {
             ([&] {
                 constexpr int k = R0 + R;
-                if constexpr (k >= 2 && k < 2 + FB) wf[H][k - 2] = *reinterpret_cast<const WRaw*>(lds + slot + waddr[H] + (k - 2) * 16 * G::WROW);
+                if constexpr (ONE) {
+                    if constexpr (k % 2 == 0) xf[H][k / 2] = *reinterpret_cast<const V8*>(lds + slot + xaddr[2 * H + k / 2]);
+                    else wf[H][k / 2] = *reinterpret_cast<const WRaw*>(lds + slot + waddr[2 * H + k / 2]);
+                } else if constexpr (k >= 2 && k < 2 + FB) wf[H][k - 2] = *reinterpret_cast<const WRaw*>(lds + slot + waddr[H] + (k - 2) * 16 * G::WROW);
                 else {
                     constexpr int b = k < 2 ? k : k - FB;
                     xf[H][b] = *reinterpret_cast<const V8*>(lds + slot + xaddr[H] + b * 2048);
@@ -218,34 +234,39 @@ __global__ void __launch_bounds__(64 * (WM * WN + NL), 2) linear_pipe_kernel(con
         }(std::make_integer_sequence<int, R1 - R0>{});
     };
     auto read_half = [&](auto half_tag, unsigned slot) { read_pieces(half_tag, std::integral_constant<int, 0>{}, std::integral_constant<int, NR>{}, slot); };
-    f32x4 acc[FB][TB];
+    std::conditional_t<ONE, f32x16, f32x4> acc[FB][TB];
 #pragma unroll
     for (int a = 0; a < FB; ++a)
 #pragma unroll
-        for (int b = 0; b < TB; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int b = 0; b < TB; ++b)
+#pragma unroll
+            for (int e = 0; e < 4 * NG; ++e) acc[a][b][e] = 0.f;
     // the MFMAs of a half stage, and between them the reads of the next one (READ: half 1 - H from `from`) and DMA pieces [J0, J1) of
     // the stage that goes to `slot`
     auto multiply_half = [&](auto half_tag, auto read_tag, unsigned from, auto j0_tag, auto j1_tag, unsigned slot) {
-        constexpr int H = decltype(half_tag)::value, J0 = decltype(j0_tag)::value, J1 = decltype(j1_tag)::value, NM = TB * FB;
+        constexpr int H = decltype(half_tag)::value, J0 = decltype(j0_tag)::value, J1 = decltype(j1_tag)::value, NM = KS * TB * FB;
         constexpr bool READ = decltype(read_tag)::value;
-        V8 w[W8 ? FB : 1];
-        // (a half of few MFMAs: all reads ahead of them, as dealt out the last one returns too late; INT8: behind the first two, under the
-        //  widening of the others: 2048 x 640 x 640 5.5 us, 5.9 with the burst)
-        constexpr bool BURST = NM <= 8 && !W8;
+        // (a half of few MFMAs: all reads ahead of them, as dealt out the last one returns too late; INT8 of two blocks: behind the first
+        //  two, under the widening)
+        constexpr bool BURST = ONE || (NM <= 8 && !W8);
         constexpr int SPAN = NM <= 8 ? 2 : NM * 3 / 4;      // MFMAs that have reads behind them
         if constexpr (READ && BURST) {
             read_pieces(std::integral_constant<int, 1 - H>{}, std::integral_constant<int, 0>{}, std::integral_constant<int, NR>{}, from);
             __builtin_amdgcn_sched_barrier(0);
         }
+        // (INT8: all blocks widened ahead of the products; between them steps of two and more blocks take 1 to 4 % longer)
+        V8 w[W8 ? KS * FB : 1];
+        if constexpr (W8) {
+#pragma unroll
+            for (int a = 0; a < KS * FB; ++a) w[a] = widen<T>(wf[H][a]);
+        }
         [&]<int... Q>(std::integer_sequence<int, Q...>) {
             ([&] {
                 // (two token blocks at a time, each feature block meets both in a row)
-                constexpr int a = Q / 2 % FB, b = Q / (2 * FB) * 2 + Q % 2;
-                if constexpr (!W8) acc[a][b] = M::run16(wf[H][a], xf[H][b], acc[a][b]);
-                else {
-                    if constexpr (b == 0) w[a] = widen<T>(wf[H][a]);
-                    acc[a][b] = M::run16(w[a], xf[H][b], acc[a][b]);
-                }
+                constexpr int a = ONE ? 0 : Q / 2 % FB, b = ONE ? 0 : Q / (2 * FB) * 2 + Q % 2;
+                if constexpr (ONE) acc[0][0] = M::run(w[Q], xf[H][Q], acc[0][0]);
+                else if constexpr (W8) acc[a][b] = M::run16(w[a], xf[H][b], acc[a][b]);
+                else acc[a][b] = M::run16(wf[H][a], xf[H][b], acc[a][b]);
                 if constexpr (READ && !BURST && Q < SPAN)
                     read_pieces(std::integral_constant<int, 1 - H>{}, std::integral_constant<int, NR * Q / SPAN>{}, std::integral_constant<int, NR * (Q + 1) / SPAN>{}, from);
                 constexpr int j0 = J0 + (J1 - J0) * Q / NM, j1 = J0 + (J1 - J0) * (Q + 1) / NM;
@@ -379,17 +400,17 @@ __global__ void __launch_bounds__(64 * (WM * WN + NL), 2) linear_pipe_kernel(con
             }
     } else {
 #pragma unroll
-        for (int a = 0; a < FB; ++a)
+        for (int a = 0; a < FB * NG; ++a)
 #pragma unroll
             for (int b = 0; b < TB; ++b) {
                 V4 o;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const float bv = static_cast<float>(braw[a][i]);
-                    if constexpr (W8) o[i] = static_cast<T>(scaled_acc(acc[a][b][i], sraw[a][i], bv));
-                    else o[i] = static_cast<T>(acc[a][b][i] + bv);
+                    const float bv = static_cast<float>(braw[a][i]), sum = acc[a / NG][b][4 * (a % NG) + i];
+                    if constexpr (W8) o[i] = static_cast<T>(scaled_acc(sum, sraw[a][i], bv));
+                    else o[i] = static_cast<T>(sum + bv);
                 }
-                *reinterpret_cast<V4*>(lds + (wm * TM * 32 + 16 * b + lr) * G::OUT_ROW + (wn * TN * 32 + 16 * a + 4 * lg) * 2) = o;
+                *reinterpret_cast<V4*>(lds + (wm * TM * 32 + BS * b + lr) * G::OUT_ROW + (wn * TN * 32 + BS / NG * a + 4 * lg) * 2) = o;
             }
     }
     __syncthreads();
