@@ -96,7 +96,7 @@ def build_host(with_test: bool = True, verbose: bool = False) -> str:
             sys.stderr.write(r.stdout + r.stderr)
             raise RuntimeError("split-geometry test build failed")
         cmd = [HIPCC, "-std=c++20", "-O1", "-Wall", "-fPIC", "-shared", "--offload-host-only", "-x", "hip", "-I" + os.path.join(ROOT, "include"), "-I" + CSRC,
-               os.path.join(ROOT, "tests", "cpp", "linear_forms.cpp"), "-o", FORMS_LIB]
+               os.path.join(ROOT, "tests", "cpp", "linear_forms.cpp"), os.path.join(ROOT, "tests", "cpp", "wide_plan.cpp"), "-o", FORMS_LIB]
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             sys.stderr.write(r.stdout + r.stderr)

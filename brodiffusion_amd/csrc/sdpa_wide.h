@@ -2,13 +2,12 @@
 // output accumulators, which live in accumulation registers by name.
 #pragma once
 #include "sdpa_tiles.h"
+#include "sdpa_wide_plan.h"
 
 namespace mi {
 namespace sdpa {
 
 constexpr int kWideThreads = 256;
-constexpr int kWideRows = 128;    // query rows per work group, 32 per wavefront
-constexpr int kWideKeys = 32;     // key rows per step
 
 template <int D> struct WideGeo {
     using G = HeadGeo<D>;

@@ -18,7 +18,8 @@
 //   chunks, f(r) = 4 (r % 4) + (r / 4) % 4: the K fragment reads (16 rows, one chunk column) and the V transpose reads
 //   (4 rows, one 64-byte window) are both free of bank conflicts.
 //
-// Long calls of head_dim 512 take the form of sdpa_wide_long.hip; planning, scratch and merge are the same.
+// Long calls of head_dim 512 that fill the GPU take the form of sdpa_wide_long.hip; planning (sdpa_wide_plan.h), scratch and merge are
+// the same.
 //
 // A query tile is 128 rows, so a VAE mid-block has 32 (64 x 64 latent) to 128 tiles for 256 compute units: the key axis is
 // cut into as many pieces as shorten the launch (wide_split), each leaving its output accumulators and softmax statistics in
@@ -406,63 +407,27 @@ __global__ void __launch_bounds__(256) wide_combine_kernel(const SdpaDev p, int 
     *reinterpret_cast<t8*>(static_cast<T*>(p.o) + b * p.o_bs + static_cast<long>(q0 + row) * p.o_rs + h * D + cc * 8) = out;
 }
 
-// Pieces of the key axis: as many as minimise the launch, counted in steps: rounds x (steps of a piece + kOverhead: Q staging,
-// first tiles, write-out), and for the merge kMerge plus kParts per part on every compute unit (128 x D FP32 values written and
-// read again), the same once more for what the parts of the launch exceed kNear by (the L2s no longer hold them). Fitted on
-// MI355X to up to 16 pieces of 45 problems (1 to 24 batch items, 300 to 16384 rows, 320 to 16384 keys) at each head dimension:
-// the number taken is 1.2 % slower than the best one on average, 10 % at worst (counting no parts: 3.1 and 21 %). At 512, us:
-//   1024 tokens (8 tiles)      1 piece 54.6   3 34.6   5 32.4           6 33.2 (taken)   8 35.4
-//   4096 (32)                  1 168          4 67.0   6 63.6 (taken)   8 67.1   9 (a second round) 91.8
-//   9216 (72)                  1 358          2 208    3 185 (taken)    7 210
-//   16384 (128)                1 638          2 493 (taken)             4 515
-//   8 x 600 (40)               1 45.7         3 38.0   4 37.2           5 40.1       3 taken
-// Only unmasked calls (a valid length or key mask may be on): with causal masks the tiles are unequal and fill the GPU in their
-// own way.
-int wide_split(const SdpaDev& p, int head_dim, int n_cu) {
-    if (p.mask_mode != MI_MASK_NONE) return 1;
-    const long tiles = static_cast<long>(p.B) * p.H * ((p.Lq + kWideRows - 1) / kWideRows);
-    const int steps = (p.Lk + kWideKeys - 1) / kWideKeys;
-    constexpr int kMaxSplit = 16, kMinSteps = 5;
-    constexpr double kOverhead = 6, kMerge = 1, kParts = 16, kNear = 47e6;
-    int best = 1;
-    double best_cost = 0;
-    for (int s = 1; s <= kMaxSplit && (s == 1 || steps / s >= kMinSteps); ++s) {
-        const double parts = static_cast<double>(tiles) * s, far = parts * kWideRows * head_dim * 4 - kNear;
-        const double rounds = static_cast<double>((tiles * s + n_cu - 1) / n_cu);
-        double cost = rounds * ((steps + s - 1) / s + kOverhead);
-        if (s > 1) cost += kMerge + kParts * (parts / n_cu + (far > 0 ? far / (n_cu * kWideRows * 512.0 * 4) : 0));
-        if (s == 1 || cost < best_cost) { best = s; best_cost = cost; }
-    }
-    return best;
-}
-
-// Whether a call of head_dim 512 goes to sdpa_wide_long.hip, by the key steps of the launch. Below one power-limited round the higher
-// clock does not come and its fixed part (2000 clocks more: twice the instructions to fetch once) shows. One head, fp16, us (this file's
-// kernel / that one): 1024 tokens 33.5 / 34.4, 4096 (16 steps per compute unit) 62.7 / 62.3, 9216 184 / 173, 16384 498 / 454. At 256
-// and 384 there are fewer products per exponential, and that form is the slower one at nearly every length (256: 4096 tokens
-// 41.3 / 42.4, 9216 105 / 110; 384 bf16: 9216 141 / 146).
-bool wide_long_pays(long tiles, int keys, int n_cu) { return tiles * ((keys + kWideKeys - 1) / kWideKeys) >= 16L * n_cu; }
-
 template <typename T, int D>
 int launch_wide_d(const SdpaDev& p, hipStream_t stream) {
     using W = WideGeo<D>;
     const int n_q_tiles = (p.Lq + kWideRows - 1) / kWideRows;
-    const long tiles = static_cast<long>(p.B) * p.H * n_q_tiles;
+    const long tiles = wide_tiles(p);
     int n_split = wide_split(p, D, device_cu_count());
     if (p.split_scratch == nullptr || p.split_scratch_bytes < static_cast<size_t>(tiles) * n_split * W::SLOT) n_split = 1;
     const long blocks = tiles * n_split;
     if (blocks > 0x7fffff00L) return fail("mi_sdpa_forward: problem too large for one launch");
-    static thread_local bool raised = false;
-    if (!raised) {
-        MI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&sdpa_wide_kernel<T, D>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         W::LDS_BYTES));
-        raised = true;
-    }
-    if (D == 512 && wide_long_pays(tiles, p.Lk, device_cu_count())) {
+    if (D == 512 && wide_long_pays(p, n_split, device_cu_count())) {
         if (launch_sdpa_wide_long(p, std::is_same_v<T, __bf16>, n_q_tiles, n_split, static_cast<int>(blocks), stream) != 0) return -1;
-    } else
+    } else {
+        static thread_local bool raised = false;
+        if (!raised) {
+            MI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&sdpa_wide_kernel<T, D>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             W::LDS_BYTES));
+            raised = true;
+        }
         hipLaunchKernelGGL((sdpa_wide_kernel<T, D>), dim3(static_cast<unsigned>((blocks + 7) / 8 * 8)), dim3(kWideThreads), W::LDS_BYTES, stream, p,
                            n_q_tiles, n_split, static_cast<int>(blocks));
+    }
     if (n_split > 1)
         hipLaunchKernelGGL((wide_combine_kernel<T, D>), dim3(static_cast<unsigned>(tiles), kWideRows * (D / 8) / 256), dim3(256), 0, stream, p,
                            n_q_tiles, n_split);
@@ -479,7 +444,7 @@ size_t sdpa_wide_split_scratch_bytes(const SdpaDev& p, int head_dim) {
     const int n_split = wide_split(p, head_dim, device_cu_count());
     if (n_split == 1) return 0;
     const size_t slot = static_cast<size_t>(kWideRows) * (static_cast<size_t>(head_dim) * 4 + 8);
-    return static_cast<size_t>(p.B) * p.H * ((p.Lq + kWideRows - 1) / kWideRows) * n_split * slot;
+    return static_cast<size_t>(wide_tiles(p)) * n_split * slot;
 }
 
 int launch_sdpa_wide(const SdpaDev& p, int dtype, int head_dim, hipStream_t stream) {

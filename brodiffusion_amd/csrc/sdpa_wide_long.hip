@@ -1,5 +1,5 @@
-// Softmax attention of head_dim 512 on gfx950, the form for long calls (sdpa_wide.hip says which those are, plans them and merges their
-// parts): the same work group, LDS rings and softmax, other matrix instructions.
+// Softmax attention of head_dim 512 on gfx950, the form for long calls that fill the GPU (sdpa_wide_plan.h says which those are; sdpa_wide.hip merges
+// their parts): the same work group, LDS rings and softmax, other matrix instructions.
 //
 // Products are v_mfma_f32_16x16x32, each LDS fragment with both blocks of 16 query rows in turn: at the power limit they run at a
 // 14 % higher clock than v_mfma_f32_32x32x16 (1.86 against 1.63 GHz, head_dim 512, N(0, 1)). But a product covers 16 clocks instead

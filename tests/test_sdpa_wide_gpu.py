@@ -175,11 +175,12 @@ def test_pieces_are_as_close_to_the_exact_result_as_the_whole(dtype, d):
     ("bf16", 140, 300, 300, "valid"),      # valid lengths from none to all
     ("fp16", 140, 300, 300, "key_mask"),
     ("bf16", 1, 4100, 4113, "causal"),
-    ("fp16", 1, 4096, 4096, "plain"),      # the shortest single head of the long form, its key axis in pieces
-    ("fp16", 1, 3968, 4096, "plain"),      # below it
+    ("fp16", 1, 4096, 4096, "plain"),      # key axis in pieces
+    ("fp16", 1, 3968, 4096, "plain"),
 ])
 def test_wide_head_long_calls(dtype, B, Lq, Lk, kind):
-    """Calls of head_dim 512 with enough key steps for the form of sdpa_wide_long.hip (16 per compute unit), against FP32."""
+    """Calls of head_dim 512 with many key steps (16 per compute unit and more), against FP32. The kernel for long calls takes the last
+    but one and leaves the others, which do not fill the GPU to their end or have few steps a work group."""
     d, dt = 512, TORCH_DT[dtype]
     g = torch.Generator(device="cuda").manual_seed(8600 + Lq + Lk)
     q, k, v = (torch.randn(B, n, d, generator=g, device="cuda") for n in (Lq, Lk, Lk))
