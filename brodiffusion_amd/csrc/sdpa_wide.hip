@@ -40,7 +40,7 @@ using namespace sdpa;
 // 1840 bytes of scratch per lane). Here O lives in a[0 : 16 VB) by name (block vb in a[16 vb : 16 vb + 16)), every statement
 // that touches it declares all of a0..a255 clobbered, so that the compiler keeps nothing of its own there, and the scores are
 // in ordinary registers. The compiler does not see the wait that VALU code needs before it touches the result of an
-// MFMA of 8 passes (11 wait states); it is kept by construction: the last MFMA of a score tile and the two that follow it
+// MFMA of 8 passes (12 wait states); it is kept by construction: the last MFMA of a score tile and the two that follow it
 // are one statement (wide_tail), so the scores are complete before anything can read them, and wide_settle stands in front
 // of the code that works on O.
 template <typename T> struct WideMma;

@@ -4,12 +4,12 @@
 // Products are v_mfma_f32_16x16x32, each LDS fragment with both blocks of 16 query rows in turn: at the power limit they run at a
 // 14 % higher clock than v_mfma_f32_32x32x16 (1.86 against 1.63 GHz, head_dim 512, N(0, 1)). But a product covers 16 clocks instead
 // of 32, and what stands between two of them in one piece (two V reads; a DMA instruction behind a read) no longer fits: cycles
-// per CU 794 k before, 963 k so, 16384 tokens of one head 485 -> 518 us. Hence the order of a slot: first product, one LDS
+// per CU 794 k before, 963 k so, 16384 tokens of one head 485 -> 518 us on one GPU. Hence the order of a slot: first product, one LDS
 // read, second product, then one other thing (the second half of a V fragment; a DMA instruction or an exponential in turn), and the
-// scale and reference of the scores go under the PV product. 16384 tokens, fp16, us: 498 with v_mfma_f32_32x32x16, 455 so; without the
-// turns 459; mid-block around it (540 before): DMA ahead of the second product 521, exponentials there 537, fragments 5 or 7 ahead
-// instead of 6 523 and 526 (518 in that build).
-// Mid-block of 16384 tokens on four GPUs: 545 -> 508 and 540 -> 518 (without the turns), 560 -> 553 and 559 -> 549 (as built).
+// scale and reference of the scores go under the PV product. The times differ from GPU to GPU: 16384 tokens, fp16, us, the kernel of
+// sdpa_wide.hip / this one, three of them: 498 / 455 (without the turns 459), 490 / 454, 508 / 468. Mid-block around it on another (540 before): DMA
+// ahead of the second product 521, exponentials there 537, fragments 5 or 7 ahead instead of 6 523 and 526 (518 in that build).
+// Mid-block of 16384 tokens: 560 -> 553 and 559 -> 549 on two GPUs.
 //   Register layouts (lq = lane % 16, g = lane / 16): A row lq, B column lq, 8 contraction elements from 8 g on; C column lq, element
 //   i is row 4 g + i. A lane holds scores of two query rows (16 r + lq of the wavefront's 32), each shared with the lanes 16, 32 and
 //   48 away; P goes into the PV product as it lies (slot 8 g + t of the contraction is key 4 g + t, for t >= 4 key 16 + 4 g + t - 4).
@@ -24,7 +24,7 @@ namespace {
 using namespace sdpa;
 
 // (inline assembly with O in a[0 : 8 VB) by name, block vb of query rows r in a[8 vb + 4 r : + 4), for the reasons given in
-// sdpa_wide.hip. The wait that VALU code needs before it touches the result of an MFMA of 4 passes, 7 wait states, is kept by
+// sdpa_wide.hip. The wait that VALU code needs before it touches the result of an MFMA of 4 passes, 8 wait states, is kept by
 // construction: the last MFMAs of a score tile and the four that follow them are one statement, four slots pass before the
 // scores are scaled, and wide_settle stands in front of the code that works on O.)
 template <typename T> struct WideMma;
@@ -86,7 +86,9 @@ __device__ __forceinline__ float quad_sum(float v) {
 // position of 16-byte chunk `c` of row `row` (XOR within groups of 16 chunks)
 __device__ __forceinline__ int wide_swz(int row) { return 2 * ((row ^ ((row >> 1) & 4)) & 7) + ((row >> 3) & 1); }
 
-template <typename T, int D>
+constexpr int D = 512;     // a row of K or V is one DMA instruction
+
+template <typename T>
 __global__ void __launch_bounds__(kWideThreads, 1) sdpa_wide_long_kernel(const SdpaDev p, int n_q_tiles, int n_split, int n_blocks) {
     using G = HeadGeo<D>;
     using W = WideGeo<D>;
@@ -158,19 +160,17 @@ __global__ void __launch_bounds__(kWideThreads, 1) sdpa_wide_long_kernel(const S
     const unsigned char* kptr = reinterpret_cast<const unsigned char*>(static_cast<const T*>(p.k) + b * p.k_bs + hk * D) + static_cast<unsigned long>(k_first) * k_rsb;
     const unsigned char* vptr = reinterpret_cast<const unsigned char*>(static_cast<const T*>(p.v) + b * p.v_bs + hk * D) + static_cast<unsigned long>(k_first) * v_rsb;
     int k_left = g_hi - k_first, v_left = k_left;     // rows from the tile under the cursor on
-    // this lane's tile row in its m-th instruction, and the byte offset of its chunk in that row (at 512 a row is one instruction,
-    // and the chunk depends on m % 4 only: a scalar row and four registers)
-    auto drow = [&](int m) -> int { return D == 512 ? wave + 4 * m : (64 * (wave + 4 * m) + lane) / G::CPR; };
-    constexpr int NCOL = D == 512 ? 4 : W::NDMA;
-    unsigned dcol[NCOL];
+    // the tile row of the wavefront's m-th instruction, and the byte offset of this lane's chunk in that row, which depends on m % 4 only
+    auto drow = [&](int m) -> int { return wave + 4 * m; };
+    unsigned dcol[4];
 #pragma unroll
-    for (int m = 0; m < NCOL; ++m) dcol[m] = static_cast<unsigned>((64 * (wave + 4 * m) + lane - drow(m) * G::CPR) ^ wide_swz(drow(m))) * 16u;
+    for (int m = 0; m < 4; ++m) dcol[m] = static_cast<unsigned>(lane ^ wide_swz(drow(m))) * 16u;
     const unsigned lds_base = static_cast<unsigned>(reinterpret_cast<size_t>((__attribute__((address_space(3))) unsigned char*)smem));
     // (inline assembly: for the compiler's builtin every later LDS read may alias the DMA's LDS write, so it would wait for the
     //  load to land before the next LDS read. The s_nop is the wait state an LDS-DMA instruction needs behind a write of m0.
     //  Rows past the last visible key repeat it: their scores are blanked.)
     auto dma = [&](const unsigned char* base, unsigned rsb, int left, int m, unsigned dst) {
-        const unsigned voff = dcol[m % NCOL] + static_cast<unsigned>(min(drow(m), left - 1)) * rsb;
+        const unsigned voff = dcol[m % 4] + static_cast<unsigned>(min(drow(m), left - 1)) * rsb;
         asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(base), "{m0}"(lds_base + dst + (wave + 4 * m) * 1024) : "memory");
     };
     auto dma_tile = [&](bool is_k, unsigned dst) {
@@ -416,14 +416,14 @@ __global__ void __launch_bounds__(kWideThreads, 1) sdpa_wide_long_kernel(const S
 
 template <typename T>
 int launch(const SdpaDev& p, int n_q_tiles, int n_split, int n_blocks, hipStream_t stream) {
-    using W = WideGeo<512>;
+    using W = WideGeo<D>;
     static thread_local bool raised = false;
     if (!raised) {
-        MI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&sdpa_wide_long_kernel<T, 512>), hipFuncAttributeMaxDynamicSharedMemorySize,
+        MI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&sdpa_wide_long_kernel<T>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                          W::LDS_BYTES));
         raised = true;
     }
-    hipLaunchKernelGGL((sdpa_wide_long_kernel<T, 512>), dim3(static_cast<unsigned>((n_blocks + 7) / 8 * 8)), dim3(kWideThreads), W::LDS_BYTES,
+    hipLaunchKernelGGL((sdpa_wide_long_kernel<T>), dim3(static_cast<unsigned>((n_blocks + 7) / 8 * 8)), dim3(kWideThreads), W::LDS_BYTES,
                        stream, p, n_q_tiles, n_split, n_blocks);
     return 0;
 }
