@@ -22,9 +22,11 @@
 // With the reads and the DMA in front of the MFMAs a block took 3078 clocks of which 2048 are products, 2700 to 2890 so. The DMA comes
 // in two small bursts, each a whole half-step before what it loads is waited for (one burst of 8 per block measured 25 % slower).
 // The accumulators leave through LDS (bias added in FP32, one rounding) so that global stores are full 16-byte pieces of
-// consecutive threads along a row. A launch of one tile per CU spends about 14 us outside the loop (1.35 us per block inside it):
-// hence the start after one block instead of two, the bias requested ahead of the operands and the write-out in batches of 8
-// (us, before -> now: 4096 x 1152 x 4608 52.6 -> 50.4, x 3456 36.1 -> 35.1, 4608 x 3072 x 3072 78.5 -> 77.6; with the half-steps as they are now 4096 x 3456 x 1152 36.2 -> 32.8).
+// consecutive threads along a row. A launch of one tile per CU spends about 11 us outside the loop (bf16, 4096 x 3456 with contractions
+// of 576 to 3456: 23.8 to 81.6 us, 1.3 us per block; 25.4 to 90.9 with the half-steps as they were): hence the start after one block
+// instead of two, the bias requested ahead of the operands and the write-out in batches of 8 (all three together 1 to 4 %). Rows x
+// features x contraction, us, half-steps as they were / as they are, on one GPU: bf16 4096 x 3456 x 1152 37.1 / 34.3, 4608 x 3072 x 3072
+// 80.4 / 72.7; fp16 38.2 / 34.5, 83.4 / 74.6.
 #include <type_traits>
 #include <utility>
 

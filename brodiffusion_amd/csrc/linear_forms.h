@@ -14,20 +14,22 @@ namespace gemm {
 // with steps = K / 64: phi what a launch of one tile per compute unit costs beyond its steps (start, first loads, write-out), lam
 // a step when the compute unit has one tile, tau and eps a step and the rest of every further tile. The constants (us) are fitted
 // on MI355X to 350 problems (32 to 16384 rows, eleven layers of the supported models, one or three of a launch; 16-bit: jointly with a
-// term for the bytes of the operands, the same for every form). Every form timed as built on 452 such problems
-// (profiles/linear_form_times.txt): the form taken is 0.3 (INT8 1.1, GEGLU 1.4, GEGLU of INT8 0.3) % slower than the fastest one on average;
-// at worst 35 %, where the same form in a graph of its own differs by as much (three of INT8 6144 x 320 x 320 15.6 and 10.6). Large tiles
+// term for the bytes of the operands, the same for every form), with all products v_mfma_f32_32x32x16. As built now steps of the large
+// tiles are 6 to 12 % shorter and the others much as they were, and the constants still rank the forms: every form timed on 452 such
+// problems (profiles/linear_form_times.txt), the form taken is 0.7 (INT8 0.5 to 0.8, GEGLU 1.2 to 1.7, GEGLU of INT8 0.6 to 0.7) % slower
+// than the fastest one on average, where the same form timed twice differs by 0.8 %; at worst 16 % (GEGLU 6144 x 640 -> 2 x 2560 56.5 us on
+// 192 x 128 tiles, 48.5 on 128 x 64). Large tiles
 // need fewer bytes per FLOP: a compute unit takes 1 KB from its L2 in 16 to 24 clocks, so a step of 128 x 128 (32 KB) takes 600 to 700 where its products take 512, one of 128 x 64 (24 KB) 450 to 650 where they take
 // 256. Small ones fill the GPU: 128 x 1280 x 1280 takes 4.9 us with 160 tiles of 32 x 32, 5.2 with 80 of 64 x 32, 7.5 with 20 of
-// 128 x 64; 1024 x 2240 x 2240 takes 16 us with 192 tiles of 128 x 96, 23 with 280 of 128 x 64, 50 with 36 of 256 x 256.
+// 128 x 64; 1024 x 2240 x 2240 takes 15.6 us with 192 tiles of 128 x 96, 23 with 280 of 128 x 64, 46 with 36 of 256 x 256.
 // The tiles 96 features wide and the GEGLU tile of 192 x 128 (constants set by hand from 17 problems of their own) are for
-// the counts between (us on one GPU, without / with them): 1024 x 2240 x 2240 16.7 -> 14.8 on
-// 192 tiles of 128 x 96, 2048 x 1152 x 1152 10.3 -> 9.0, 2048 x 640 x 2560 15.0 -> 12.6 on 224 of 64 x 96; GEGLU 2048 x 640 ->
-// 2 x 2560 21.9 -> 19.1 and 1024 x 1280 -> 2 x 5120 37.3 -> 31.6 (INT8 24.1 -> 22.2, 40.9 -> 35.1) on 220 and 240 of 192 x 128; INT8
-// 2048 x 640 x 640 6.4 -> 5.8, 1024 x 1280 x 1280 9.4 -> 8.2, 4096 x 640 x 640 8.7 -> 7.7. Wavefronts that own 128 x 64
-// or 96 x 64 instead of 64 x 64 (a quarter fewer LDS reads) gave nothing: 1024 x 6720 x 2240 32.8 -> 32.9.
+// the counts between (us, best other form / theirs, profiles/linear_form_times.txt): 1024 x 2240 x 2240 16.8 / 15.6 on
+// 192 tiles of 128 x 96, 2048 x 1152 x 1152 10.5 / 9.9, 2048 x 640 x 2560 15.0 / 13.2 on 224 of 64 x 96; GEGLU 2048 x 640 ->
+// 2 x 2560 21.6 / 21.1 and 1024 x 1280 -> 2 x 5120 35.5 / 33.8 (INT8 22.9 / 21.3, 38.2 / 33.1) on 220 and 240 of 192 x 128; INT8
+// 1024 x 1280 x 1280 8.7 (128 x 64) / 8.8, 4096 x 640 x 640 8.4 / 7.8. Wavefronts that own 128 x 64
+// or 96 x 64 instead of 64 x 64 (a quarter fewer LDS reads) gave nothing with products of 32 x 32 x 16: 1024 x 6720 x 2240 32.8 -> 32.9.
 // Loading wavefronts (see the top) pay where the products of a step are short. They are no help where a compute unit holds two work
-// groups of large register use: GEGLU 3072 x 640 -> 2 x 2560 29 -> 37 us, three of 16384 x 512 x 512 37 -> 42.
+// groups of large register use (products of 32 x 32 x 16): GEGLU 3072 x 640 -> 2 x 2560 29 -> 37 us, three of 16384 x 512 x 512 37 -> 42.
 struct Form {
     int bm, bn_out;
     float phi, lam, tau, eps;

@@ -22,8 +22,8 @@
 // a problem gives the same bits whichever one takes it, alone or in a launch with others.
 //
 // Products are v_mfma_f32_16x16x32, two token blocks with one feature block in a row. What bounds the large forms on values of a
-// real spread is the power limit, and a loop of these keeps up 2.07 PFLOP/s (bf16, N(0, 1); 1.84 fp16) at it, one of
-// v_mfma_f32_32x32x16, which moves twice the accumulator registers per FLOP, 1.78 (1.65): the same bits. Reads in one burst in
+// real spread is the power limit, and a loop of these keeps up 2.03 PFLOP/s (bf16, N(0, 1); 1.90 fp16) at it, one of
+// v_mfma_f32_32x32x16, which moves twice the accumulator registers per FLOP, 1.78 (1.64): the same bits. Reads in one burst in
 // front of the products of a half kept the matrix pipe waiting for the LDS queue of all wavefronts behind each barrier: a step of
 // 256 x 128 took 1427 clocks of which 1024 are products, 1260 so (halves of up to 8 products of 16-bit weights keep the burst). Both
 // together (us): 4096 x 1152 x 1152 16.1 -> 14.8, 1024 x 6720 x 2240 37.6 -> 34, three of 16384 x 512 x 512 34.1 -> 32.8.
@@ -42,11 +42,12 @@
 // instruction 1900 -> 1250 (PipeArgs), first stage landed 2900, bias and last barrier 950 -> 390 (the bias is requested ahead of the
 // loop), tile staged 1000, stored 1300 -> 570 (all pieces read before the first is stored).
 //
-// Measured (fp16 / bf16, one launch, us; first: 64 x 64 tiles through registers, one step ahead; then: this pipeline with the fixed part
-// as it was; now, with the tiles that the rule below takes): 4096 x 1152 x 1152 30 / 16.9 / 14.5 to 17.3 (192 x 128 tiles; it differs
-// from GPU to GPU); 1024 x 2240 x 2240 30 / 16.3 / 14.8; 2048 x 640 x 640 8.4 / 6.9 / 6.0 (INT8 weights 11.5 / 7.8 / 5.8);
-// 128 x 1280 x 1280 8.2 / 6.4 / 4.6 (INT8 - / 8.2 / 5.7), three of them - / 6.9 / 5.7 (INT8 - / 8.7 / 6.7); 256 x 1152 x 1152 - / 6.2 / 5.0;
-// 3072 x 640 x 2560 - / 17.4 / 15.8; GEGLU 3072 x 640 -> 2 x 2560 39 / 32.0 / 29; three of 16384 x 512 x 512 - / 42.3 / 36.
+// Measured (fp16, one launch, us, each column on a GPU of its own; first: 64 x 64 tiles through registers, one step ahead; then: this
+// pipeline with the fixed part as it was; then: products of 32 x 32 x 16; now, on that GPU): 4096 x 1152 x 1152 30 / 16.9 / 15.7 / 14.3;
+// 1024 x 2240 x 2240 30 / 16.3 / 15.5 / 15.2; 2048 x 640 x 640 8.4 / 6.9 / 5.3 / 5.4 (INT8 weights 11.5 / 7.8 / 6.05 / 6.04);
+// 128 x 1280 x 1280 8.2 / 6.4 / 4.7 / 4.65 (INT8 - / 8.2 / 5.85 / 5.85), three of them - / 6.9 / 5.3 / 5.2 (INT8 - / 8.7 / 6.7 / 6.7);
+// 256 x 1152 x 1152 - / 6.2 / 5.0 / 4.8; 3072 x 640 x 2560 - / 17.4 / 17.3 / 17.0; GEGLU 3072 x 640 -> 2 x 2560 39 / 32.0 / 29.2 / 27.2;
+// three of 16384 x 512 x 512 - / 42.3 / 36.3 / 34.0.
 #include <cmath>
 #include <type_traits>
 #include <utility>

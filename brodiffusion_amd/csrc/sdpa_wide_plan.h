@@ -16,7 +16,7 @@ inline long wide_tiles(const SdpaDev& p) { return static_cast<long>(p.B) * p.H *
 // read again), the same once more for what the parts of the launch exceed kNear by (the L2s no longer hold them). Fitted on
 // MI355X to up to 16 pieces of 45 problems (1 to 24 batch items, 300 to 16384 rows, 320 to 16384 keys) at each head dimension:
 // the number taken is 1.2 % slower than the best one on average, 10 % at worst (counting no parts: 3.1 and 21 %). The kernel of
-// sdpa_wide_long.hip, 21 problems of 3 to 192 tiles: 0.5 % on average, 5 % at worst. At 512 with the kernel of sdpa_wide.hip, us:
+// sdpa_wide_long.hip, 22 problems of 3 to 192 tiles: 0.6 % on average, 6 % at worst. At 512 with the kernel of sdpa_wide.hip, us:
 //   1024 tokens (8 tiles)      1 piece 54.6   3 34.6   5 32.4           6 33.2 (taken)   8 35.4
 //   4096 (32)                  1 168          4 67.0   6 63.6 (taken)   8 67.1   9 (a second round) 91.8
 //   9216 (72)                  1 358          2 208    3 185 (taken)    7 210
