@@ -7,8 +7,9 @@
 // stage holds BM rows of X and BN rows of W, 128 bytes each (INT8: 64), back to back as the DMA deposits them; bank
 // conflicts of the fragment reads (16 rows, one 16-byte piece of each, per phase) are avoided by an XOR swizzle applied on
 // the global side: the 16-byte piece in position c of row r is piece c ^ ((r >> 1) & 7). INT8 rows: c ^ ((r >> 2) & 3), which keeps
-// reads of 8 bytes from 16 rows and two pieces apart (the operands of v_mfma_f32_16x16x32); those of 32 rows and one half of a
-// piece (v_mfma_f32_32x32x16) meet in half of the banks and take two phases.
+// reads of 8 bytes from 16 rows and two pieces apart (an operand of v_mfma_f32_16x16x32); those of 32 rows and one half of a piece
+// (v_mfma_f32_32x32x16) meet in half of the banks and take two phases, and so do the operands of two blocks where the compiler
+// fetches them with one ds_read2 (64 x 96 tiles: conflicts in 21 % of the busy cycles with the one, 35 % with the other).
 //
 // A work group is WM x WN wavefronts over tokens x features; a wavefront owns TM x TN blocks of 32 x 32 (as in linear.hip the
 // product is computed transposed: MFMA rows are features). A stage is multiplied in two halves of 32 contraction elements, each
@@ -367,7 +368,7 @@ __global__ void __launch_bounds__(64 * (WM * WN + NL), 2) linear_pipe_kernel(con
         for (++t; t < n - 1; ++t) step(std::false_type{}, std::false_type{}, t);
     }
     // The last step: nothing behind it to wait for or to read. It stands here once and not as a branch inside `step`: where that branch
-    // met the others again, the compiler moved all accumulators, 130 to 219 registers became 166 to 256 and the GEGLU tile of 192 x 128
+    // met the others again, the compiler moved all accumulators, 115 to 238 registers became 131 to 256 and the GEGLU tile of 192 x 128
     // put 215 to 356 of them in scratch, each reload behind a wait for the DMA as well (GEGLU, fp16, us with the branch / without:
     // 2048 x 640 -> 2 x 2560 28.7 / 20.0, INT8 36.0 / 20.9; 4096 x 320 -> 2 x 1280 23.0 / 14.1, INT8 29.5 / 15.2; 1024 x 1280 ->
     // 2 x 5120 41.2 / 32.5, INT8 48.8 / 32.9).
