@@ -19,8 +19,8 @@ namespace gemm {
 // problems (profiles/linear_form_times.txt), the form taken is 0.7 (INT8 0.5 to 0.8, GEGLU 1.2 to 1.7, GEGLU of INT8 0.6 to 0.7) % slower
 // than the fastest one on average, where the same form timed twice differs by 0.8 %; at worst 16 % (GEGLU 6144 x 640 -> 2 x 2560 56.5 us on
 // 192 x 128 tiles, 48.5 on 128 x 64). Large tiles
-// need fewer bytes per FLOP: a compute unit takes 1 KB from its L2 in 16 to 24 clocks, so a step of 128 x 128 (32 KB) takes 600 to 700 where its products take 512, one of 128 x 64 (24 KB) 450 to 650 where they take
-// 256. Small ones fill the GPU: 128 x 1280 x 1280 takes 4.9 us with 160 tiles of 32 x 32, 5.2 with 80 of 64 x 32, 7.5 with 20 of
+// need fewer bytes per FLOP: a compute unit takes 1 KB from its L2 in 16 to 24 clocks, so a step of 128 x 128 (32 KB) took 600 to 700 where its products take 512, one of 128 x 64 (24 KB) 450 to 650 where they take
+// 256 (with products of 32 x 32 x 16). Small ones fill the GPU: 128 x 1280 x 1280 takes 4.8 us with 160 tiles of 32 x 32, 5.1 with 80 of 64 x 32, 7.0 with 20 of
 // 128 x 64; 1024 x 2240 x 2240 takes 15.6 us with 192 tiles of 128 x 96, 23 with 280 of 128 x 64, 46 with 36 of 256 x 256.
 // The tiles 96 features wide and the GEGLU tile of 192 x 128 (constants set by hand from 17 problems of their own) are for
 // the counts between (us, best other form / theirs, profiles/linear_form_times.txt): 1024 x 2240 x 2240 16.8 / 15.6 on
