@@ -624,7 +624,9 @@ __device__ __forceinline__ int swz(int row) { return 4 * (row & 3) + ((row >> 2)
 
 // SPLIT: the launch follows p.split — a work group either processes one whole query tile or one piece of the last
 // round, i.e. one or more (tile, key range) parts in sequence, each leaving a partial result in its scratch slot
-// (merged by sdpa_combine_kernel). Only for unmasked calls without prefix.
+// (merged by sdpa_combine_kernel). Only for unmasked calls without prefix, whose parts are of the ragged form (in the general form, with
+// its interval per row, the Flux calls below took, head norms and rotation included: bf16, 24 heads of 128, 2816 tokens 139.7 -> 136.6 us, 3328
+// 180.9 -> 176.4, 4096 226.3 -> 222.2; 16 heads, 9216 tokens 633.8 -> 624.1; PixArt block of 16 heads of 72, 4608 tokens 224.6 -> 220.6).
 // FORM kDense: no mask of any kind and key counts (cached prefix, if any, and fresh) that are multiples of 64: every tile is
 // whole and visible to every row, so the masked form of the softmax and the per-step bookkeeping (which tile, its limit,
 // whether this wavefront sees it whole) drop out of the kernel, and with them their registers: measured 6 % faster at
@@ -643,8 +645,8 @@ __device__ __forceinline__ int swz(int row) { return 4 * (row & 3) + ((row >> 2)
 template <typename T, int D, bool SPLIT, int FORM = kGeneral, bool PSCALE = false, bool XTRA = false, bool F32SUM = false>
 __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const SdpaDev p) {
     constexpr bool DENSE = FORM != kGeneral, RAGGED = FORM == kRagged, LISTED = XTRA && RAGGED;
-    static_assert(!(SPLIT && DENSE), "the split launch clips key ranges per part");
-    static_assert(!PSCALE || (!SPLIT && !DENSE), "the dial belongs to the general form");
+    static_assert(!SPLIT || RAGGED, "the parts of a split launch end anywhere");
+    static_assert(!PSCALE || !DENSE, "the dial belongs to the general form");
     static_assert(!XTRA || (!SPLIT && FORM != kDense && !PSCALE), "key mask, bias and denominators are not in these forms");
     using G = HeadGeo<D>;
     using DG = DmaGeo<D>;
@@ -723,11 +725,6 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
     // (rows past the end count as the last row where they share a wavefront with it: as rows without keys they put every tile
     //  of that wavefront on the masked path; 24 heads of 128, 2500 tokens, block-causal: 83.8 -> 74.5 us)
     if constexpr (!DENSE) row_interval(p, b, min(qrow, p.Lq - 1), q0 + wave * 32 < p.Lq, lo, hi);
-    if constexpr (SPLIT) {
-        lo = max(lo, kv_begin);
-        hi = min(hi, kv_end);
-        if (hi <= lo) { lo = 0; hi = 0; }
-    }
     WaveExtent we{0, 0, n_keys, n_keys};
     if constexpr (!DENSE) {
         we = wave_extent(lo, hi);
@@ -754,7 +751,8 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
         g_lo = __builtin_amdgcn_readfirstlane(g_lo);
         kv_stop = __builtin_amdgcn_readfirstlane(kv_stop);
     }
-    const TilePlan plan(g_lo == 0x7fffffff ? 0 : g_lo, kv_stop, p.Lp);
+    // (a part begins at a multiple of 64 keys; its tiles are numbered from there)
+    const TilePlan plan(SPLIT ? kv_begin : g_lo == 0x7fffffff ? 0 : g_lo, SPLIT ? min(kv_stop, kv_end) : kv_stop, p.Lp);
     int n_tiles = plan.n_tiles;
     // XTRA: visibility words of the plan's tiles (made visible to all wavefronts by the barrier that ends the prologue)
     const unsigned long long* const kbits = (XTRA && p.key_mask) ? reinterpret_cast<const unsigned long long*>(smem + p.kbits_off) : nullptr;
@@ -1358,7 +1356,7 @@ int launch_d(SdpaDev p, int n_cu, hipStream_t stream) {
             int per_group = 0;
             for (int xg = 0; xg < 8; ++xg)
                 per_group = max(per_group, p.split.full_of(xg) + p.split.pieces_for(p.split.tail_of(xg) * p.split.T));
-            hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, true>), dim3(8 * per_group), dim3(kThreads8), DmaGeo<D>::lds_bytes(), stream, p);
+            hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, true, kRagged>), dim3(8 * per_group), dim3(kThreads8), DmaGeo<D>::lds_bytes(), stream, p);
             hipLaunchKernelGGL((sdpa_combine_kernel<T, D>), dim3(8 * p.split.max_tail, (256 * (D / 8) + 255) / 256), dim3(256), 0, stream, p);
             const hipError_t e = hipGetLastError();
             if (e != hipSuccess) return fail("sdpa_fwd launch: %s", hipGetErrorString(e));

@@ -147,3 +147,18 @@ def test_own_split_scratch_is_per_stream():
     for (_, _, _, ref), o in zip(probs, outs):
         for got in o:
             assert torch.equal(got, ref)
+
+
+@pytest.mark.parametrize("dtype,d,Lk", [("bf16", 128, 2497), ("fp16", 72, 2559), ("fp16", 128, 2560)])
+def test_parts_around_the_last_key(oracle, dtype, d, Lk):
+    """The last part ends inside a key tile (or on its edge); the rows behind the last key and between the rows are poisoned."""
+    H, Lq = 17, 4096      # 272 tiles, two of the last round per XCD
+    q, k, v = randn(8151, (Lq, H * d), dtype), randn(8152, (Lk, H * d), dtype), randn(8153, (Lk, H * d), dtype)
+    k[Lk // 2:] *= 2      # parts with references of their own
+    dq = to_dev(q, dtype)
+    kb, vb = (torch.full((Lk + 70, H * d + 8), float("nan"), device="cuda", dtype=dq.dtype) for _ in range(2))
+    kb[:Lk, :H * d], vb[:Lk, :H * d] = to_dev(k, dtype), to_dev(v, dtype)
+    assert split_bytes(dq, kb[:Lk], vb[:Lk], H, head_dim=d, num_heads=H) > 0
+    out = bd.sdpa_forward(dq, kb[:Lk, :H * d], vb[:Lk, :H * d], H)
+    rows = np.unique(np.concatenate([np.arange(0, Lq, 89), np.arange(Lq - 300, Lq, 13)])).astype(np.int32)
+    assert_close(oracle.sdpa(q, k, v, H, rows=rows)[rows], to_np(out)[rows], dtype, f"{Lk} keys")
