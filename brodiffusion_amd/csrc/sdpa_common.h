@@ -163,6 +163,12 @@ struct QTileLoad {
     static constexpr int NI = (NCH + NT - 1) / NT;
     u32x4 raw[NI];
     f32x4 cs[NI], sn[NI];
+    // Gives the table registers a value, any value, without an instruction. In a loop a call without tables would otherwise keep those of
+    // the pass before: the compiler carries all of them (64 registers at head_dim 128) through the key loop and spills others.
+    __device__ __forceinline__ void define_tables() {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) asm volatile("" : "=v"(cs[i]), "=v"(sn[i]));
+    }
     __device__ __forceinline__ void issue(const SdpaDev& p, const T* q_base, int q0, int tid, int last_row) {
         const bool rope = p.cos_q != nullptr && !p.rope_split;
 #pragma unroll

@@ -627,6 +627,10 @@ __device__ __forceinline__ int swz(int row) { return 4 * (row & 3) + ((row >> 2)
 // (merged by sdpa_combine_kernel). Only for unmasked calls without prefix, whose parts are of the ragged form (in the general form, with
 // its interval per row, the Flux calls below took, head norms and rotation included: bf16, 24 heads of 128, 2816 tokens 139.7 -> 136.6 us, 3328
 // 180.9 -> 176.4, 4096 226.3 -> 222.2; 16 heads, 9216 tokens 633.8 -> 624.1; PixArt block of 16 heads of 72, 4608 tokens 224.6 -> 220.6).
+// The loop over parts keeps nothing of a pass for the next: with the RoPE tables' registers left undefined where there are no tables
+// (QTileLoad::define_tables) it carried them through the key loop, and each table piece was waited for and spilled as it arrived (24 heads of 128
+// with RoPE, K rotation included: 2816 tokens 129.0 -> 119.4 us, 3328 169.4 -> 154.6, 4096 213.5 -> 203.1, 6144 432.9 -> 417.1; 48 heads, 4608
+// 512.9 -> 491.5; without RoPE 3328 147.2 -> 143.1).
 // FORM kDense: no mask of any kind and key counts (cached prefix, if any, and fresh) that are multiples of 64: every tile is
 // whole and visible to every row, so the masked form of the softmax and the per-step bookkeeping (which tile, its limit,
 // whether this wavefront sees it whole) drop out of the kernel, and with them their registers: measured 6 % faster at
@@ -736,6 +740,7 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
     using QL = QTileLoad<T, D, kThreads8, BM>;
     static_assert(!DG::Q_HALVES || (QL::NI % 2 == 0 && kThreads8 * (QL::NI / 2) == 128 * QL::CPRK), "half of the load rounds must be half of the rows");
     QL ql;
+    if constexpr (SPLIT) ql.define_tables();
     ql.issue(p, q_base, q0, tid, p.Lq - 1);
     // the first pass through the MFMA stream multiplies a zero P with the last V buffer; the slack behind both rings is zero
     for (int i = tid; i < (DG::TILE + DG::SLACK) / 16; i += kThreads8)
@@ -1220,8 +1225,9 @@ __global__ void __launch_bounds__(256) sdpa_combine_kernel(const SdpaDev p) {
 // shortens the last round by more than that — and only when the last round would fill at most half of the GPU:
 // under sustained MFMA load the GPU runs at its power limit, a partly idle last round runs at a higher clock, and
 // measured time follows the total work rather than the number of rounds (432 tiles on 256 compute units take 1.70
-// times one full round, not 2). Measured on head_dim 128, 24 heads: last round 7/32 full: 12 % faster with the
-// split, 10/32: 10 %, 16/32: 6 %, 22/32: 5 % slower.
+// times one full round, not 2). Measured at head_dim 128 (us, unsplit / split, with RoPE and K rotation; last round of a part in 32): 24 heads, 1.03
+// rounds (1/32) 144.6 / 119.4, 1.22 (7) 166.9 / 154.6, 1.31 (10) 178.9 / 171.5, 1.5 (16) 204.2 / 203.1, 2.25 (8) 459.0 / 417.1, 2.44 (14) 498.8 /
+// 495.4; 32 heads, 2.25 (8) 354.4 / 326.7; 48 heads, 3.19 (6) 463.0 / 444.1, 3.375 (12) 489.5 / 491.5.
 template <int D>
 bool plan_split(SdpaDev& p, int n_cu) {
     p.split = SplitGeo{};
