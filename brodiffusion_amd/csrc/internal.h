@@ -22,7 +22,7 @@ int device_cu_count();
         if (_e != hipSuccess) return ::mi::fail("%s: %s", #expr, hipGetErrorString(_e)); \
     } while (0)
 
-// Split of the last, partly filled round of an unmasked attention launch.
+// Split of the last, partly filled round of an attention launch without a mask other than a key mask.
 //
 // A launch of n_blocks equal query tiles on a GPU that runs n_cu work groups at a time takes ceil(n_blocks / n_cu)
 // rounds even when the last round fills only part of the GPU (432 tiles on 256 compute units: 2 rounds for 1.69

@@ -624,7 +624,7 @@ __device__ __forceinline__ int swz(int row) { return 4 * (row & 3) + ((row >> 2)
 
 // SPLIT: the launch follows p.split — a work group either processes one whole query tile or one piece of the last
 // round, i.e. one or more (tile, key range) parts in sequence, each leaving a partial result in its scratch slot
-// (merged by sdpa_combine_kernel). Only for unmasked calls without prefix, whose parts are of the ragged form (in the general form, with
+// (merged by sdpa_combine_kernel). Only for calls without prefix and without a mask other than a key mask, whose parts are of the ragged form (in the general form, with
 // its interval per row, the Flux calls below took, head norms and rotation included: bf16, 24 heads of 128, 2816 tokens 139.7 -> 136.6 us, 3328
 // 180.9 -> 176.4, 4096 226.3 -> 222.2; 16 heads, 9216 tokens 633.8 -> 624.1; PixArt block of 16 heads of 72, 4608 tokens 224.6 -> 220.6).
 // The loop over parts keeps nothing of a pass for the next: with the RoPE tables' registers left undefined where there are no tables
@@ -644,14 +644,17 @@ __device__ __forceinline__ int swz(int row) { return 4 * (row & 3) + ((row >> 2)
 // XTRA with kRagged: a key mask but no bias. The mask hides the same keys from every row (the padding of a prompt in
 // the middle of a joint sequence), so the tiles without a visible key are taken out of the walk: `vis` lists the others, and a
 // step looks up the tile that it loads. 48 query / 12 K/V heads of 128, 4608 tokens of which 435 are padding (6 of 72 tiles):
-// 520 -> 472 us; the words used to blank the scores of a hidden tile, whose MFMAs and loads ran all the same.
+// 520 -> 472 us; the words used to blank the scores of a hidden tile, whose MFMAs and loads ran all the same. With SPLIT every pass lists
+// the tiles anew and a part [s0, s1) of T tiles takes entries [s0 n / T, s1 n / T) of the n listed ones, so that hidden tiles shorten all parts
+// alike (with RoPE and K rotation, unsplit -> split: the call above 472 -> 447; 24 heads, 435 keys hidden, 2816 tokens 137 -> 109, 3328 162 -> 145,
+// 4096 201 -> 187; 16 heads, 200 hidden, 4608 231 -> 174; 16 heads of 72, 4608 199 -> 140).
 // F32SUM: see softmax_tile_rel.
 template <typename T, int D, bool SPLIT, int FORM = kGeneral, bool PSCALE = false, bool XTRA = false, bool F32SUM = false>
 __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const SdpaDev p) {
     constexpr bool DENSE = FORM != kGeneral, RAGGED = FORM == kRagged, LISTED = XTRA && RAGGED;
     static_assert(!SPLIT || RAGGED, "the parts of a split launch end anywhere");
     static_assert(!PSCALE || !DENSE, "the dial belongs to the general form");
-    static_assert(!XTRA || (!SPLIT && FORM != kDense && !PSCALE), "key mask, bias and denominators are not in these forms");
+    static_assert(!XTRA || (FORM != kDense && !PSCALE), "key mask, bias and denominators are not in these forms");
     using G = HeadGeo<D>;
     using DG = DmaGeo<D>;
     using V8 = typename Mma<T>::v8;
@@ -715,6 +718,7 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
             seg_s = tt * p.split.T + s1;
         }
     }
+    const int Lp = SPLIT ? 0 : p.Lp;      // (LISTED: a third of the key loop's scalar instructions are the choice between prefix and fresh rows)
     const int h = bh % p.H;
     const int b = bh / p.H;
     const int q0 = qt * BM;
@@ -757,14 +761,15 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
         kv_stop = __builtin_amdgcn_readfirstlane(kv_stop);
     }
     // (a part begins at a multiple of 64 keys; its tiles are numbered from there)
-    const TilePlan plan(SPLIT ? kv_begin : g_lo == 0x7fffffff ? 0 : g_lo, SPLIT ? min(kv_stop, kv_end) : kv_stop, p.Lp);
+    constexpr bool RANGE = SPLIT && !LISTED;
+    const TilePlan plan(RANGE ? kv_begin : g_lo == 0x7fffffff ? 0 : g_lo, RANGE ? min(kv_stop, kv_end) : kv_stop, Lp);
     int n_tiles = plan.n_tiles;
     // XTRA: visibility words of the plan's tiles (made visible to all wavefronts by the barrier that ends the prologue)
     const unsigned long long* const kbits = (XTRA && p.key_mask) ? reinterpret_cast<const unsigned long long*>(smem + p.kbits_off) : nullptr;
     if constexpr (XTRA) build_key_bits(p, plan, b, smem + p.kbits_off, wave, lane);
     // LISTED: tile numbers of the tiles with a visible key, in order, behind the words; every wavefront writes the whole list
     // (the same values) and reads only what it wrote. vis_t .. vis_t3: the list's entries t .. t + 3 in step t.
-    unsigned short* const vis = LISTED ? reinterpret_cast<unsigned short*>(smem + p.kbits_off + 8 * ((p.Lk + kBN - 1) / kBN + 2)) : nullptr;
+    unsigned short* vis = LISTED ? reinterpret_cast<unsigned short*>(smem + p.kbits_off + 8 * ((p.Lk + kBN - 1) / kBN + 2)) : nullptr;
     int vis_t = 0, vis_t1 = 0, vis_t2 = 0, vis_t3 = 0;
     if constexpr (LISTED) {
         __syncthreads();
@@ -779,6 +784,14 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if constexpr (SPLIT) {
+            // a part is its share of the list (keys counted in tiles: at most 3070 of them, what the LDS holds words for)
+            if (!whole) {
+                const int first = kv_begin / kBN * n_tiles / p.split.T, stop = kv_end / kBN * n_tiles / p.split.T;
+                vis += first;
+                n_tiles = stop - first;
+            }
+        }
     }
     auto listed = [&](int i) { return __builtin_amdgcn_readfirstlane(static_cast<int>(vis[min(i, n_tiles - 1)])); };   // n_tiles > 0
     const float* const bias_row = (XTRA && p.bias && qvalid && qrow >= p.bias_q0) ? p.bias + static_cast<long>(qrow - p.bias_q0) * p.bias_rs : nullptr;
@@ -796,14 +809,14 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
     //    instruction j of an operand fills LDS bytes [1024 j, 1024 j + 1024) of the tile = chunks 64 j + lane ──
     TileCursor kc, vc;
     kc.init(plan, reinterpret_cast<const unsigned char*>(static_cast<const T*>(p.kp) + b * p.kp_bs + hk * D), static_cast<unsigned>(p.kp_rs) * 2u,
-            reinterpret_cast<const unsigned char*>(static_cast<const T*>(p.k) + b * p.k_bs + hk * D), static_cast<unsigned>(p.k_rs) * 2u, p.Lp);
+            reinterpret_cast<const unsigned char*>(static_cast<const T*>(p.k) + b * p.k_bs + hk * D), static_cast<unsigned>(p.k_rs) * 2u, Lp);
     vc.init(plan, reinterpret_cast<const unsigned char*>(static_cast<const T*>(p.vp) + b * p.vp_bs + hk * D), static_cast<unsigned>(p.vp_rs) * 2u,
-            reinterpret_cast<const unsigned char*>(static_cast<const T*>(p.v) + b * p.v_bs + hk * D), static_cast<unsigned>(p.v_rs) * 2u, p.Lp);
+            reinterpret_cast<const unsigned char*>(static_cast<const T*>(p.v) + b * p.v_bs + hk * D), static_cast<unsigned>(p.v_rs) * 2u, Lp);
     auto seek = [&](TileCursor& c, int t, const void* pre, long pre_bs, const void* fresh, long fresh_bs) {   // (LISTED: one row stride for both)
         const int j0 = plan.j0(t);
         c.ptr = plan.in_prefix(t)
                     ? reinterpret_cast<const unsigned char*>(static_cast<const T*>(pre) + b * pre_bs + hk * D) + static_cast<unsigned long>(j0) * c.rsb
-                    : reinterpret_cast<const unsigned char*>(static_cast<const T*>(fresh) + b * fresh_bs + hk * D) + static_cast<unsigned long>(j0 - p.Lp) * c.rsb;
+                    : reinterpret_cast<const unsigned char*>(static_cast<const T*>(fresh) + b * fresh_bs + hk * D) + static_cast<unsigned long>(j0 - Lp) * c.rsb;
         c.rows_left = plan.limit(t) - j0;
     };
     int drow[DG::MAXI];        // tile row this lane fetches in its m-th instruction
@@ -970,7 +983,7 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
                 return;
             }
             issued = dma_tiles(load_k, KD, load_v, VD);
-            if (DENSE && !RAGGED && p.Lp == 0) {
+            if (DENSE && !RAGGED && Lp == 0) {
                 if (load_k) kc.ptr += kBN * kc.rsb;
                 if (load_v) vc.ptr += kBN * vc.rsb;
             } else {
@@ -1220,6 +1233,15 @@ __global__ void __launch_bounds__(256) sdpa_combine_kernel(const SdpaDev p) {
     }
 }
 
+// LDS behind the tile buffers for the visibility words of a key mask, and with the list of the tiles that have a visible key (kRagged with XTRA)
+long kbits_bytes_of(const SdpaDev& p) { return p.key_mask ? 8L * ((p.Lk + kBN - 1) / kBN + 2) : 0; }
+long listed_bytes_of(const SdpaDev& p) { return kbits_bytes_of(p) + kbits_bytes_of(p) / 4; }
+constexpr long kMaxKbits = 24 * 1024;     // (the words share the LDS with rings and Q staging)
+template <int D>
+bool listed_fits(const SdpaDev& p) {
+    return kbits_bytes_of(p) <= kMaxKbits && DmaGeo<D>::lds_bytes() + listed_bytes_of(p) + 256 <= 160 * 1024;
+}
+
 // Decides whether the launch splits its last round (see SplitGeo) and fills p.split. The split costs every tail work
 // group a second prologue and the launch a merge pass (together about ten key steps), so it is taken only when it
 // shortens the last round by more than that — and only when the last round would fill at most half of the GPU:
@@ -1233,9 +1255,12 @@ bool plan_split(SdpaDev& p, int n_cu) {
     p.split = SplitGeo{};
     if constexpr (!dma_kernel_available<D>()) return false;
     if (sdpa_kernel_choice() == 0 && sdpa_flow_takes(p, D, n_cu)) return false;
-    if (p.mask_mode != MI_MASK_NONE || p.kv_valid_len || p.key_mask || p.Lp > 0 || p.cos_k || p.cu_q) return false;
+    if (p.mask_mode != MI_MASK_NONE || p.kv_valid_len || p.Lp > 0 || p.cos_k || p.cu_q) return false;
     // (the split form neither adds a logit bias nor writes the softmax denominators)
     if (p.bias != nullptr || p.lse != nullptr) return false;
+    if constexpr (dma_kernel_available<D>()) {
+        if (p.key_mask && !listed_fits<D>(p)) return false;
+    }
     if (n_cu < 8 || n_cu % 8 != 0 || sdpa_kernel_choice() == 1 || sdpa_kernel_choice() == 3) return false;
     const long tiles = static_cast<long>(p.B) * p.H * ((p.Lq + 255) / 256);
     const int T = (p.Lk + kBN - 1) / kBN;
@@ -1246,7 +1271,8 @@ bool plan_split(SdpaDev& p, int n_cu) {
     if (tail0 == 0 || 2 * tail0 > g.cu_g) return false;
     const int np0 = g.pieces_for(tail0 * T);
     const int piece_len = (tail0 * T + np0 - 1) / np0;
-    if (T - piece_len < 12) return false;
+    // (a key mask may hide tiles, which is known on the GPU only: it pays from half of them visible on)
+    if (T - piece_len < (p.key_mask ? 24 : 12)) return false;
     for (int xg = 0; xg < 8; ++xg) {
         const int tail = g.tail_of(xg), S = tail * T, np = g.pieces_for(S);
         g.max_tail = max(g.max_tail, tail);
@@ -1362,7 +1388,10 @@ int launch_d(SdpaDev p, int n_cu, hipStream_t stream) {
             int per_group = 0;
             for (int xg = 0; xg < 8; ++xg)
                 per_group = max(per_group, p.split.full_of(xg) + p.split.pieces_for(p.split.tail_of(xg) * p.split.T));
-            hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, true, kRagged>), dim3(8 * per_group), dim3(kThreads8), DmaGeo<D>::lds_bytes(), stream, p);
+            const dim3 grid(8 * per_group), block(kThreads8);
+            p.kbits_off = DmaGeo<D>::lds_bytes();
+            if (p.key_mask) hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, true, kRagged, false, true>), grid, block, DmaGeo<D>::lds_bytes() + listed_bytes_of(p), stream, p);
+            else hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, true, kRagged>), grid, block, DmaGeo<D>::lds_bytes(), stream, p);
             hipLaunchKernelGGL((sdpa_combine_kernel<T, D>), dim3(8 * p.split.max_tail, (256 * (D / 8) + 255) / 256), dim3(256), 0, stream, p);
             const hipError_t e = hipGetLastError();
             if (e != hipSuccess) return fail("sdpa_fwd launch: %s", hipGetErrorString(e));
@@ -1375,8 +1404,8 @@ int launch_d(SdpaDev p, int n_cu, hipStream_t stream) {
     // kernels (visibility words of all key tiles in LDS behind the tile buffers), unless K is rotated tile by tile, the
     // prefix-KV dial is on as well, or the key sequence is too long for the words to fit: then the 128-row kernel
     const bool xtra = p.key_mask != nullptr || p.bias != nullptr || p.lse != nullptr;
-    const long kbits_bytes = p.key_mask ? 8L * ((p.Lk + kBN - 1) / kBN + 2) : 0;
-    const bool xtra_ok = !xtra || (!rope_k && !p.prefix_scaled && kbits_bytes <= 24 * 1024);   // (the words share the LDS with rings and Q staging)
+    const long kbits_bytes = kbits_bytes_of(p);
+    const bool xtra_ok = !xtra || (!rope_k && !p.prefix_scaled && kbits_bytes <= kMaxKbits);
     // calls with the prefix-KV dial stay on the 128-row kernel unless the DMA kernel (which has an instance for it) takes them
     const bool dial_ok = !p.prefix_scaled || (dma_kernel_available<D>() && !rope_k && choice != 3);
     const bool pingpong = D <= 128 && xtra_ok && dial_ok && (choice >= 2 || (choice == 0 && rows256_pay<D>(p, n_cu, xtra)));
@@ -1401,11 +1430,10 @@ int launch_d(SdpaDev p, int n_cu, hipStream_t stream) {
             if (xtra) {
                 const bool dma = dma_kernel_available<D>() && sdpa_kernel_choice() != 3;
                 if constexpr (dma_kernel_available<D>()) {
-                    const long listed_bytes = kbits_bytes + kbits_bytes / 4;
-                    if (dma && p.key_mask && !p.bias && same_keys_for_all_rows(p) && DmaGeo<D>::lds_bytes() + listed_bytes + 256 <= 160 * 1024) {
+                    if (dma && p.key_mask && !p.bias && same_keys_for_all_rows(p) && listed_fits<D>(p)) {
                         p.kbits_off = DmaGeo<D>::lds_bytes();
                         hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, false, kRagged, false, true>), grid, block,
-                                           DmaGeo<D>::lds_bytes() + listed_bytes, stream, p);
+                                           DmaGeo<D>::lds_bytes() + listed_bytes_of(p), stream, p);
                     }
                     else if (dma) {
                         p.kbits_off = DmaGeo<D>::lds_bytes();

@@ -213,8 +213,8 @@ typedef struct mi_sdpa_args {
 
 MI_API int mi_sdpa_forward(const mi_sdpa_args* args);
 /* Bytes of split_scratch with which this call (same args, split_scratch fields ignored) would split its last round;
- * 0 when it would not (masked calls, short key sequences, a last round that is nearly full, kernels without the
- * split). No reference counterpart. */
+ * 0 when it would not (calls with a prefix or a mask other than key_mask, short key sequences, a last round that is more
+ * than half full, kernels without the split). No reference counterpart. */
 MI_API size_t mi_sdpa_split_scratch_bytes(const mi_sdpa_args* args);
 /* Tuning / testing knob for the calling thread: 0 = choose the kernel by problem size (default),
  * 1 = always the 4-wavefront kernel (128 query rows per work group), 2 = always the 8-wavefront

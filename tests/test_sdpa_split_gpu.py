@@ -162,3 +162,38 @@ def test_parts_around_the_last_key(oracle, dtype, d, Lk):
     out = bd.sdpa_forward(dq, kb[:Lk, :H * d], vb[:Lk, :H * d], H)
     rows = np.unique(np.concatenate([np.arange(0, Lq, 89), np.arange(Lq - 300, Lq, 13)])).astype(np.int32)
     assert_close(oracle.sdpa(q, k, v, H, rows=rows)[rows], to_np(out)[rows], dtype, f"{Lk} keys")
+
+
+@pytest.mark.parametrize("dtype,B,H,Hkv,d,Lq,Lk", [
+    ("bf16", 1, 20, 5, 128, 4500, 2925),     # 360 tiles, the last key tile of 45 keys
+    ("fp16", 2, 17, 17, 72, 2048, 3008),     # batch 2, a mask for each item, whole key tiles
+])
+@pytest.mark.parametrize("seen", ["padding", "few", "one key", "nothing"])
+def test_parts_of_the_tiles_that_a_key_mask_leaves(oracle, dtype, B, H, Hkv, d, Lq, Lk, seen):
+    """Parts are shares of the list of tiles with a visible key, which may be shorter than the parts are many. Tiles without one are not
+    read: NaN there must not matter."""
+    q = randn(8161, (B, Lq, H * d), dtype)
+    k, v = randn(8162, (B, Lk, Hkv * d), dtype), randn(8163, (B, Lk, Hkv * d), dtype)
+    m = np.zeros((B, Lk), np.float32)
+    if seen == "padding":
+        m[:, :70] = m[:, 300:] = 1
+    elif seen == "few":
+        m[:, 130::640] = m[:, Lk - 1] = 1
+    elif seen == "one key":
+        m[:, Lk // 2] = 1
+    if B > 1:
+        m[1] = np.random.default_rng(8164).integers(0, 2, Lk)
+    rep = lambda x: x.reshape(Lk, Hkv, d).repeat(H // Hkv, axis=1).reshape(Lk, H * d)
+    dq, dk, dv, dm = to_dev(q, dtype), to_dev(k, dtype), to_dev(v, dtype), torch.from_numpy(m).cuda()
+    for b in range(B):
+        for j in range(0, Lk, 64):
+            if not m[b, j:j + 64].any():
+                dk[b, j:j + 64] = dv[b, j:j + 64] = float("nan")
+    need = split_bytes(dq, dk, dv, H, num_kv_heads=Hkv, key_mask=dm.data_ptr(), key_mask_batch_stride=Lk)
+    assert need > 0
+    split = bd.sdpa_forward(dq, dk, dv, H, num_kv_heads=Hkv, key_mask=dm, split_scratch=torch.full((need,), 0xFF, dtype=torch.uint8, device="cuda"))
+    plain = bd.sdpa_forward(dq, dk, dv, H, num_kv_heads=Hkv, key_mask=dm, split_scratch=False)
+    assert max_ulp_diff(split, plain) <= 2.0
+    rows = np.unique(np.concatenate([np.arange(0, Lq, 197), np.arange(255, Lq, 256)])).astype(np.int32)
+    for b in range(B):
+        assert_close(oracle.sdpa(q[b], rep(k[b]), rep(v[b]), H, key_mask=m[b], rows=rows)[rows], to_np(split[b])[rows], dtype, f"{seen}, batch {b}")
