@@ -624,7 +624,9 @@ __device__ __forceinline__ int swz(int row) { return 4 * (row & 3) + ((row >> 2)
 
 // SPLIT: the launch follows p.split — a work group either processes one whole query tile or one piece of the last
 // round, i.e. one or more (tile, key range) parts in sequence, each leaving a partial result in its scratch slot
-// (merged by sdpa_combine_kernel). Only for calls without prefix and without a mask other than a key mask, whose parts are of the ragged form (in the general form, with
+// (merged by sdpa_combine_kernel). Only for calls without prefix and without a mask other than a key mask, in the dense form where the key tiles are
+// whole (ragged -> dense, with RoPE and K rotation: 24 heads of 128, 3328 tokens 154.8 -> 148.9 us, 4096 202.1 -> 194.5, 6656 489.6 -> 471.0, 9472
+// 943.5 -> 895.6; 16 of 72, 4608 tokens 138.0 -> 136.1) and else in the ragged form (in the general form, with
 // its interval per row, the Flux calls below took, head norms and rotation included: bf16, 24 heads of 128, 2816 tokens 139.7 -> 136.6 us, 3328
 // 180.9 -> 176.4, 4096 226.3 -> 222.2; 16 heads, 9216 tokens 633.8 -> 624.1; PixArt block of 16 heads of 72, 4608 tokens 224.6 -> 220.6).
 // The loop over parts keeps nothing of a pass for the next: with the RoPE tables' registers left undefined where there are no tables
@@ -652,7 +654,7 @@ __device__ __forceinline__ int swz(int row) { return 4 * (row & 3) + ((row >> 2)
 template <typename T, int D, bool SPLIT, int FORM = kGeneral, bool PSCALE = false, bool XTRA = false, bool F32SUM = false>
 __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const SdpaDev p) {
     constexpr bool DENSE = FORM != kGeneral, RAGGED = FORM == kRagged, LISTED = XTRA && RAGGED;
-    static_assert(!SPLIT || RAGGED, "the parts of a split launch end anywhere");
+    static_assert(!SPLIT || DENSE, "every row of a split launch sees the same keys");
     static_assert(!PSCALE || !DENSE, "the dial belongs to the general form");
     static_assert(!XTRA || (FORM != kDense && !PSCALE), "key mask, bias and denominators are not in these forms");
     using G = HeadGeo<D>;
@@ -1391,6 +1393,7 @@ int launch_d(SdpaDev p, int n_cu, hipStream_t stream) {
             const dim3 grid(8 * per_group), block(kThreads8);
             p.kbits_off = DmaGeo<D>::lds_bytes();
             if (p.key_mask) hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, true, kRagged, false, true>), grid, block, DmaGeo<D>::lds_bytes() + listed_bytes_of(p), stream, p);
+            else if (p.Lk % kBN == 0) hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, true, kDense>), grid, block, DmaGeo<D>::lds_bytes(), stream, p);
             else hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, true, kRagged>), grid, block, DmaGeo<D>::lds_bytes(), stream, p);
             hipLaunchKernelGGL((sdpa_combine_kernel<T, D>), dim3(8 * p.split.max_tail, (256 * (D / 8) + 255) / 256), dim3(256), 0, stream, p);
             const hipError_t e = hipGetLastError();
