@@ -1435,8 +1435,18 @@ int launch_d(SdpaDev p, int n_cu, hipStream_t stream) {
                 if constexpr (dma_kernel_available<D>()) {
                     if (dma && p.key_mask && !p.bias && same_keys_for_all_rows(p) && listed_fits<D>(p)) {
                         p.kbits_off = DmaGeo<D>::lds_bytes();
-                        hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, false, kRagged, false, true>), grid, block,
-                                           DmaGeo<D>::lds_bytes() + listed_bytes_of(p), stream, p);
+                        const long lds = DmaGeo<D>::lds_bytes() + listed_bytes_of(p);
+                        if (p.Lp == 0) {
+                            // the instance of split launches, which looks for no prefix, as one without a tail (with RoPE and K rotation, us:
+                            // 48 / 12 heads of 128, 435 keys hidden, 4928 tokens 508 -> 500, 24 / 6 heads 4608 231 -> 228; 16 of 72, 4096 96.7 -> 95.1,
+                            // 5376 without a scratch 229 -> 221)
+                            p.split.T = (p.Lk + kBN - 1) / kBN;
+                            p.split.n_blocks = p.n_blocks;
+                            p.split.chunk = (p.n_blocks + 7) / 8;
+                            p.split.cu_g = 1;
+                            hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, true, kRagged, false, true>), dim3(8 * p.split.chunk), block, lds, stream, p);
+                        }
+                        else hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, false, kRagged, false, true>), grid, block, lds, stream, p);
                     }
                     else if (dma) {
                         p.kbits_off = DmaGeo<D>::lds_bytes();

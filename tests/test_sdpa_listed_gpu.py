@@ -74,3 +74,29 @@ def test_block_causal_tiles(oracle, rows256, ends, causal, prefix, d):
     mask = bd.SdpaMask.block_causal(prefix, ends, [prefix + e for e in ends], causal)
     out = bd.sdpa_forward(dev(q), dev(k[prefix:]), dev(v[prefix:]), H, mask=mask, **kw)
     assert_close(ref, to_np(out), dtype, f"{ends} {causal} prefix {prefix}")
+
+
+@pytest.mark.parametrize("d,H,L", [(128, 3, 1300), (72, 5, 1024)])
+def test_key_mask_with_a_valid_length_and_denominators(oracle, rows256, d, H, L):
+    """Batch items of different valid lengths (one of them 0), tiles hidden on both sides of it; denominators as an output."""
+    dtype, B = "bf16", 3
+    q, k, v = (randn(9431 + i, (B, L, H * d), dtype) for i in range(3))
+    m = np.ones((B, L), np.float32)
+    m[:, 64:200] = 0
+    m[2, 640:] = 0
+    n = [L, 0, 777]
+    lse = torch.full((B, H, L), float("nan"), device="cuda")
+    out = bd.sdpa_forward(*(to_dev(x, dtype) for x in (q, k, v)), H, key_mask=torch.from_numpy(m).cuda(),
+                          kv_valid_len=torch.tensor(n, dtype=torch.int32, device="cuda"), lse_out=lse)
+    for b in range(B):
+        m[b, n[b]:] = 0
+        assert_close(oracle.sdpa(q[b], k[b], v[b], H, key_mask=m[b]), to_np(out[b]), dtype, f"batch {b}")
+        if n[b] == 0:
+            assert (out[b] == 0).all() and (lse[b] == float("inf")).all()
+            continue
+        qh, kh = (torch.from_numpy(x[b]).double().view(L, H, d).transpose(0, 1).contiguous() for x in (q, k))
+        s = (qh @ kh.transpose(1, 2).contiguous()) * d ** -0.5
+        s[:, :, torch.from_numpy(m[b]) == 0] = float("-inf")
+        exact = torch.logsumexp(s, -1) / np.log(2.0)       # base 2
+        # raw scores below 2^6 summed from 128 products in 32 bits (2^-17), times 0.18, and a sum of at most L rounded exponentials
+        assert (lse[b].double().cpu() - exact).abs().max().item() < 2e-5
