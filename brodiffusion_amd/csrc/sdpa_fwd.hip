@@ -920,11 +920,16 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
     // One step t of the loop with S = (t + 1) % 3 known at compile time:
     //   reads K_{t+1} from K stage S and V_t from V stage (S + 2) % 3,
     //   loads K_{t+3} into K stage (S + 2) % 3 and V_{t+2} into V stage (S + 1) % 3.
+    // What a step asks is asked once, by scalar selections where that is possible: a load flag for each operand, branches around each cursor and
+    // three questions for the wait made 22 scalar branches a step of which 9 are left (with RoPE and K rotation, us: 24 heads, 4608 tokens 242.5 -> 237.6,
+    // 4600 248.2 -> 244.5, 4096 198.3 -> 197.5, 1997 62.3 -> 61.5; 48 heads, 4928 540 -> 530; 16 of 72, 8192 342 -> 340, 4608 136.2 -> 134.9, without a
+    // scratch 190.7 -> 193.4).
     auto step = [&](auto stage_tag, int t) {
         constexpr int S = decltype(stage_tag)::value;
         constexpr int KS = S * DG::TILE, VS = ((S + 2) % 3) * DG::TILE;
         constexpr int KD = ((S + 2) % 3) * DG::TILE, VD = DG::VOFF + ((S + 1) % 3) * DG::TILE;
-        const bool load_k = t + 3 < n_tiles, load_v = t + 2 < n_tiles;
+        // (behind K's last tile that one is loaded once more, into the free stage: one question for both operands)
+        const bool load = t + 2 < n_tiles;
         int issued = 0;
         // XTRA: the visibility word of the tile whose softmax this wavefront runs in this step, fetched here, ahead of this
         // step's DMA instructions (an LDS read behind them would wait for them to land)
@@ -978,19 +983,15 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
         // read takes the full memory latency), so the DMA instructions of a step go where the wavefront has no
         // LDS access ahead of it for a long time: right before its softmax.
         auto issue_dma = [&]() {
+            if (!load) return;
             if constexpr (LISTED) {
                 seek(kc, vis_t3, p.kp, p.kp_bs, p.k, p.k_bs);
                 seek(vc, vis_t2, p.vp, p.vp_bs, p.v, p.v_bs);
-                issued = dma_tiles(load_k, KD, load_v, VD);
-                return;
             }
-            issued = dma_tiles(load_k, KD, load_v, VD);
-            if (DENSE && !RAGGED && Lp == 0) {
-                if (load_k) kc.ptr += kBN * kc.rsb;
-                if (load_v) vc.ptr += kBN * vc.rsb;
-            } else {
-                if (load_k) kc.next();
-                if (load_v) vc.next();
+            issued = dma_tiles(true, KD, true, VD);
+            if constexpr (!LISTED) {
+                kc.next(t + 4 < n_tiles);
+                vc.next(t + 3 < n_tiles);
             }
         };
         // group 1 turns the scores of its previous step into P first, so that its MFMA stream meets group 0's softmax
@@ -1060,10 +1061,8 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
         // The tiles loaded in the PREVIOUS step are read in the next one: wait for those only (this step's
         // loads stay in flight), then meet the other wavefronts.
         if constexpr (DG::NDMA % 8 == 0) {
-            // every wavefront issues NDMA / 8 loads per operand tile: the count follows from the flags alone
-            if (load_k) wait_all_but(DG::NDMA / 4);
-            else if (load_v) wait_all_but(DG::NDMA / 8);
-            else wait_all_but(0);
+            // every wavefront issues NDMA / 8 loads per operand tile
+            wait_all_but(load ? DG::NDMA / 4 : 0);
         } else {
             wait_all_but(issued);
         }

@@ -106,6 +106,16 @@ struct TileCursor {
         if (t == n_pre) { ptr = fresh_ptr; rsb = fresh_rsb; rows_left = fresh_rows; }
         else { ptr += kBN * rsb; rows_left -= kBN; }
     }
+    // the same by selections instead of branches, in a key loop that asks in every step; stays where it is unless `more`
+    __device__ __forceinline__ void next(bool more) {
+        t += more ? 1 : 0;
+        const bool enters = more && t == n_pre;
+        const unsigned char* const on = ptr + (more ? kBN * rsb : 0u);
+        const int left = rows_left - (more ? kBN : 0);
+        ptr = enters ? fresh_ptr : on;
+        rsb = enters ? fresh_rsb : rsb;
+        rows_left = enters ? fresh_rows : left;
+    }
 };
 
 // Forms of the 256-row kernels by what the launch can look like:
