@@ -1445,10 +1445,11 @@ int launch_d(SdpaDev p, int n_cu, hipStream_t stream) {
                     if (dma && p.key_mask && !p.bias && same_keys_for_all_rows(p) && listed_fits<D>(p)) {
                         p.kbits_off = DmaGeo<D>::lds_bytes();
                         const long lds = DmaGeo<D>::lds_bytes() + listed_bytes_of(p);
-                        if (p.Lp == 0) {
-                            // the instance of split launches, which looks for no prefix, as one without a tail (with RoPE and K rotation, us:
-                            // 48 / 12 heads of 128, 435 keys hidden, 4928 tokens 508 -> 500, 24 / 6 heads 4608 231 -> 228; 16 of 72, 4096 96.7 -> 95.1,
-                            // 5376 without a scratch 229 -> 221)
+                        if (p.Lp == 0 && n_kt >= 20) {
+                            // the instance of split launches, which looks for no prefix, as one without a tail: about 1.5 % less per key step, 0.7 us
+                            // more to start (with RoPE and K rotation, us: 48 / 12 heads of 128, 435 keys hidden, 768 tokens 22.1 -> 23.0, 1000 28.9 ->
+                            // 29.4, 1300 67.8 -> 67.9, 1700 87.5 -> 86.7, 4928 508 -> 500; 112 hidden, 1100 43.1 -> 43.3, 1300 82.7 -> 82.1; 24 / 6 heads,
+                            // 4608 231 -> 228; 16 of 72, 4096 96.7 -> 95.1, 5376 without a scratch 229 -> 221)
                             p.split.T = (p.Lk + kBN - 1) / kBN;
                             p.split.n_blocks = p.n_blocks;
                             p.split.chunk = (p.n_blocks + 7) / 8;
