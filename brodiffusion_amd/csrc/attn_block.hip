@@ -52,7 +52,8 @@ LinearProblem problem(const void* x, const void* w, const void* bias, void* y, l
 
 // What the attention launch of a block uses to cut the key axis into pieces.
 size_t split_bytes(int batch, int q_len, int kv_len, int num_heads, int head_dim, bool causal = false, const float* key_mask = nullptr) {
-    if (q_len == 0 || kv_len == 0 || !sdpa_supported(MI_DTYPE_F16, head_dim)) return 0;
+    // (under a key mask a block's scratch stays what callers lay out for it, its buffers; a larger one is used all the same)
+    if (q_len == 0 || kv_len == 0 || (key_mask != nullptr && !sdpa_wide_head(head_dim)) || !sdpa_supported(MI_DTYPE_F16, head_dim)) return 0;
     SdpaDev p;
     std::memset(&p, 0, sizeof(p));
     p.B = batch; p.H = num_heads; p.Lq = q_len; p.Lk = kv_len;
