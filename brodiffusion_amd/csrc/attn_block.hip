@@ -50,10 +50,13 @@ LinearProblem problem(const void* x, const void* w, const void* bias, void* y, l
     return p;
 }
 
+// Whether a block lends its attention launch a scratch to cut the key axis with. Under a key mask only one of wide heads: the scratch of other
+// masked blocks is their buffers, and a larger one (left by another call, say) must not change the launch and with it the rounding.
+bool lends_split_scratch(int head_dim, const float* key_mask) { return key_mask == nullptr || sdpa_wide_head(head_dim); }
+
 // What the attention launch of a block uses to cut the key axis into pieces.
 size_t split_bytes(int batch, int q_len, int kv_len, int num_heads, int head_dim, bool causal = false, const float* key_mask = nullptr) {
-    // (under a key mask a block's scratch stays what callers lay out for it, its buffers; a larger one is used all the same)
-    if (q_len == 0 || kv_len == 0 || (key_mask != nullptr && !sdpa_wide_head(head_dim)) || !sdpa_supported(MI_DTYPE_F16, head_dim)) return 0;
+    if (q_len == 0 || kv_len == 0 || !lends_split_scratch(head_dim, key_mask) || !sdpa_supported(MI_DTYPE_F16, head_dim)) return 0;
     SdpaDev p;
     std::memset(&p, 0, sizeof(p));
     p.B = batch; p.H = num_heads; p.Lq = q_len; p.Lk = kv_len;
@@ -82,7 +85,7 @@ SdpaDev cached_view(const mi_attn_block_args* a, const BlockDims& d, void* o) {
     return p;
 }
 
-// [scratch_used, scratch_bytes) of the caller's scratch is lent to the attention launch.
+// [scratch_used, scratch_bytes) of the caller's scratch is lent to the attention launch where it is counted in the scratch's size.
 int attend(const mi_attn_block_args* a, const BlockDims& d, const void* q, const void* k, const void* v, void* o, int kv_len, size_t scratch_used) {
     mi_sdpa_args s;
     std::memset(&s, 0, sizeof(s));
@@ -93,8 +96,10 @@ int attend(const mi_attn_block_args* a, const BlockDims& d, const void* q, const
     s.q_len = a->q_len; s.kv_len = kv_len;
     s.key_mask = a->key_mask; s.key_mask_batch_stride = a->key_mask_batch_stride;
     if (a->causal) { s.mask_mode = MI_MASK_CAUSAL; s.q_offset = kv_len - a->q_len; }
-    s.split_scratch = static_cast<char*>(a->scratch) + scratch_used;
-    s.split_scratch_bytes = a->scratch_bytes - scratch_used;
+    if (lends_split_scratch(d.head_dim, a->key_mask)) {
+        s.split_scratch = static_cast<char*>(a->scratch) + scratch_used;
+        s.split_scratch_bytes = a->scratch_bytes - scratch_used;
+    }
     s.stream = a->stream;
     return mi_sdpa_forward(&s);
 }

@@ -619,7 +619,7 @@ def flash_attention_qkvo_forward(X, Ctx, Wq, bq, Wk, bk, Wv, bv, Wo, bo, d_mask,
                                  out: Optional[torch.Tensor] = None, scratch: Optional[torch.Tensor] = None):
     """out = attention(X Wq^T + bq, S Wk^T + bk, S Wv^T + bv) Wo^T + bo with S = Ctx, or X when Ctx is None.
     `scratch` (flash_attention_scratch_bytes(..., with_kv=True) bytes) holds the projections; None allocates it, together with
-    what the attention launch can use to cut its key axis."""
+    what an attention launch without d_mask can use to cut its key axis (with d_mask only one of head_dim 256, 384 or 512)."""
     return _attn_block("flash_attention_qkvo_forward", "mi_flash_attention_qkvo_forward", X, Ctx, None, None,
                        Wq, bq, Wk, bk, Wv, bv, Wo, bo, d_mask, num_heads, causal, out, scratch)
 

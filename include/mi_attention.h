@@ -490,7 +490,8 @@ typedef struct mi_attn_block_args {
     void* stream;
 } mi_attn_block_args;
 /* Scratch bytes of this call (qkvo form if k is NULL, else the kv_cached form; the scratch fields are ignored), with all that its
- * attention launch can use. project_kv needs none. */
+ * attention launch uses (under a key mask only one of head_dim 256, 384 or 512 cuts its key axis: other masked blocks use their buffers, however
+ * large the scratch is). project_kv needs none. */
 MI_API size_t mi_attn_block_scratch_bytes(const mi_attn_block_args* args);
 /* The same for callers that size the scratch before they know the call: the required bytes of the qkvo form (with_kv != 0) or the
  * kv_cached form (with_kv == 0), and what cutting the key axis takes where `inner` is the head dimension of one wide head

@@ -214,6 +214,30 @@ def test_qkvo_key_mask_and_causal(oracle, causal):
         assert np.array_equal(rows, np.broadcast_to(to_np(d["bo"]), rows.shape))
 
 
+@pytest.mark.parametrize("cached", [False, True])
+def test_a_larger_scratch_changes_no_bit_under_a_key_mask(cached):
+    """264 query tiles, 8 of them in the last round: a launch that would be cut if its scratch held the parts. What the host layers lend
+    depends on the calls before."""
+    L, C, H, inner = 2816, 64, 24, 3072
+    x = to_dev(randn(7541, (L, C), "bf16"), "bf16")
+    wq, wk, wv = (to_dev(randn(7542 + i, (inner, C), "bf16") / 8, "bf16") for i in range(3))
+    wo = to_dev(randn(7545, (C, inner), "bf16") / 55, "bf16")
+    mask = torch.ones(L, device="cuda")
+    mask[77:512] = 0
+    need = bd.flash_attention_scratch_bytes(1, L, L, inner, not cached)
+    more = bd.flash_attention_scratch_bytes(1, L, L, inner, not cached, num_heads=H)
+    assert more > need
+    outs = []
+    for size in (need, more, 2 * more):
+        scratch = torch.empty(size, dtype=torch.uint8, device="cuda")
+        if cached:
+            k, v = bd.flash_attention_project_kv(x, wk, None, wv, None)
+            outs.append(bd.flash_attention_q_with_kv_cached_forward(x, k, v, wq, None, wo, None, mask, H, False, scratch=scratch))
+        else:
+            outs.append(bd.flash_attention_qkvo_forward(x, None, wq, None, wk, None, wv, None, wo, None, mask, H, False, scratch=scratch))
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
 def test_attn_block_argument_errors():
     dt = torch.bfloat16
     z = lambda *s: torch.zeros(*s, device="cuda", dtype=dt)

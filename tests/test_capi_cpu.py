@@ -145,7 +145,7 @@ def test_block_scratch_is_what_the_call_can_use(capi):
     # one wide head
     mine, buffers, any_heads = block(1, 4096, 512, 1)
     assert mine == any_heads == buffers + cut(1, 4096, 1, 512) > buffers
-    # heads of 128 whose last round is cut, and not when a mask makes the tiles unequal
+    # heads of 128 whose last round is cut; a causal launch is not, and a block lends its launch nothing under a key mask
     mine, buffers, any_heads = block(1, 3328, 3072, 24)
     assert mine == buffers + cut(1, 3328, 24, 128) > any_heads == buffers
     assert block(1, 3328, 3072, 24, causal=1)[0] == block(1, 3328, 3072, 24, key_mask=0x1000)[0] == buffers
