@@ -847,9 +847,7 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
         unsigned voff = dcol[m];
         if constexpr (!DENSE) voff += static_cast<unsigned>(min(drow[m], min(c.rows_left, kBN) - 1)) * c.rsb;
         // the last tile of a segment: rows past its end repeat the last one. A scalar branch that no other tile takes: the empty
-        // statement keeps the compiler from computing it for every tile and selecting (a branch for all loads of a step, not
-        // for each: 24 heads with RoPE, 4600 tokens 241.8 -> 239.6 us, 1997 61.3 -> 60.7; 48 heads, 4920 541.8 -> 536.3; under a key mask 48 / 12 heads, 4928
-        // tokens 503.8 -> 500.9)
+        // statement keeps the compiler from computing it for every tile and selecting
         if (RAGGED && last) {
             asm volatile("" : "+v"(voff));
             voff -= static_cast<unsigned>(max(drow[m] - (c.rows_left - 1), 0)) * c.rsb;
@@ -859,7 +857,11 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
         //  the s_nop is the wait state an LDS-DMA instruction needs behind a write of m0)
         asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(c.ptr), "{m0}"(dst) : "memory");
     };
-    // this wavefront's share of the loads of one K tile (if do_k) and one V tile (if do_v); returns how many it issued
+    // this wavefront's share of the loads of one K tile (if do_k) and one V tile (if do_v); returns how many it issued.
+    // head_dim 128 asks once for all loads of a step whether one of the tiles is the last (24 heads with RoPE, 4600 tokens 241.8 -> 239.6 us; under a key
+    // mask 48 / 12 heads, 3000 tokens 249 -> 246), but under a key mask with a prefix for each (48 / 12 heads, 200 prefix rows: 1300 tokens 74.9 -> 73.8,
+    // 2304 127.0 -> 125.6)
+    constexpr bool EACH = LISTED && !SPLIT;
     auto dma_tiles = [&](bool do_k, int k_off, bool do_v, int v_off) -> int {
         int n = 0;
         if constexpr (DG::NDMA % 8 == 0) {
@@ -868,11 +870,11 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
 #pragma unroll
                 for (int m = 0; m < DG::MAXI; ++m) {
                     const int i = wave + 8 * m;
-                    if (m < DG::MAXI / 2) { if (do_k) { dma(kc, m, i, k_off, last); ++n; } }
-                    else { if (do_v) { dma(vc, m, i - DG::NDMA, v_off, last); ++n; } }
+                    if (m < DG::MAXI / 2) { if (do_k) { dma(kc, m, i, k_off, EACH ? kc.rows_left < kBN : last); ++n; } }
+                    else { if (do_v) { dma(vc, m, i - DG::NDMA, v_off, EACH ? vc.rows_left < kBN : last); ++n; } }
                 }
             };
-            if (RAGGED && ((do_k && kc.rows_left < kBN) || (do_v && vc.rows_left < kBN))) all(true);
+            if (RAGGED && !EACH && ((do_k && kc.rows_left < kBN) || (do_v && vc.rows_left < kBN))) all(true);
             else all(false);
         } else {
 #pragma unroll
@@ -930,16 +932,18 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
     // One step t of the loop with S = (t + 1) % 3 known at compile time:
     //   reads K_{t+1} from K stage S and V_t from V stage (S + 2) % 3,
     //   loads K_{t+3} into K stage (S + 2) % 3 and V_{t+2} into V stage (S + 1) % 3.
-    // What a step asks is asked once, by scalar selections where that is possible: a load flag for each operand, branches around each cursor and
-    // three questions for the wait made 22 scalar branches a step of which 9 are left (with RoPE and K rotation, us: 24 heads, 4608 tokens 242.5 -> 237.6,
-    // 4600 248.2 -> 244.5, 4096 198.3 -> 197.5, 1997 62.3 -> 61.5; 48 heads, 4928 540 -> 530; 16 of 72, 8192 342 -> 340, 4608 136.2 -> 134.9, without a
-    // scratch 190.7 -> 193.4).
+    // head_dim 128: what a step asks is asked once, by scalar selections where that is possible. A load flag for each operand, branches around each
+    // cursor and three questions for the wait are 22 scalar branches a step in the dense form, of which 9 are left (24 heads, us, with RoPE and K
+    // rotation: 4608 tokens 242 -> 238, 4096 205 -> 200, 1997 62.2 -> 61.2; causal 2048 49.9 -> 49.2; with 669 prefix rows 4096 229 -> 223).
+    // head_dim 72, with 9 loads per operand tile dealt to 8 wavefronts, must count its loads for the wait and is slower that way (16 heads,
+    // flags for each operand / one: 4608 tokens unsplit 200.4 / 203.8, causal 4096 86.1 / 88.2, biased under a key mask 244 / 251).
+    constexpr bool ONE_FLAG = DG::NDMA % 8 == 0;
     auto step = [&](auto stage_tag, int t) {
         constexpr int S = decltype(stage_tag)::value;
         constexpr int KS = S * DG::TILE, VS = ((S + 2) % 3) * DG::TILE;
         constexpr int KD = ((S + 2) % 3) * DG::TILE, VD = DG::VOFF + ((S + 1) % 3) * DG::TILE;
-        // (behind K's last tile that one is loaded once more, into the free stage: one question for both operands)
-        const bool load = t + 2 < n_tiles;
+        // (ONE_FLAG: behind K's last tile that one is loaded once more, into the free stage)
+        const bool load_v = t + 2 < n_tiles, load_k = ONE_FLAG ? load_v : t + 3 < n_tiles;
         int issued = 0;
         // XTRA: the visibility word of the tile whose softmax this wavefront runs in this step, fetched here, ahead of this
         // step's DMA instructions (an LDS read behind them would wait for them to land)
@@ -993,15 +997,22 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
         // read takes the full memory latency), so the DMA instructions of a step go where the wavefront has no
         // LDS access ahead of it for a long time: right before its softmax.
         auto issue_dma = [&]() {
-            if (!load) return;
+            if (ONE_FLAG && !load_v) return;
             if constexpr (LISTED) {
                 seek(kc, vis_t3, p.kp, p.kp_bs, p.k, p.k_bs);
                 seek(vc, vis_t2, p.vp, p.vp_bs, p.v, p.v_bs);
             }
-            issued = dma_tiles(true, KD, true, VD);
-            if constexpr (!LISTED) {
+            issued = dma_tiles(ONE_FLAG || load_k, KD, ONE_FLAG || load_v, VD);
+            if constexpr (LISTED) return;
+            if constexpr (ONE_FLAG) {
                 kc.next(t + 4 < n_tiles);
                 vc.next(t + 3 < n_tiles);
+            } else if (DENSE && !RAGGED && Lp == 0) {
+                if (load_k) kc.ptr += kBN * kc.rsb;
+                if (load_v) vc.ptr += kBN * vc.rsb;
+            } else {
+                if (load_k) kc.next();
+                if (load_v) vc.next();
             }
         };
         // group 1 turns the scores of its previous step into P first, so that its MFMA stream meets group 0's softmax
@@ -1072,7 +1083,7 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
         // loads stay in flight), then meet the other wavefronts.
         if constexpr (DG::NDMA % 8 == 0) {
             // every wavefront issues NDMA / 8 loads per operand tile
-            wait_all_but(load ? DG::NDMA / 4 : 0);
+            wait_all_but(load_v ? DG::NDMA / 4 : 0);
         } else {
             wait_all_but(issued);
         }
