@@ -653,10 +653,12 @@ __device__ __forceinline__ int swz(int row) { return 4 * (row & 3) + ((row >> 2)
 // F32SUM: see softmax_tile_rel.
 template <typename T, int D, bool SPLIT, int FORM = kGeneral, bool PSCALE = false, bool XTRA = false, bool F32SUM = false>
 __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const SdpaDev p) {
-    constexpr bool DENSE = FORM != kGeneral, RAGGED = FORM == kRagged, LISTED = XTRA && RAGGED;
+    constexpr bool DENSE = FORM != kGeneral, RAGGED = FORM == kRagged || FORM == kFresh, LISTED = XTRA && RAGGED;
+    constexpr bool FRESH = SPLIT || FORM == kFresh;     // no prefix
     static_assert(!SPLIT || DENSE, "every row of a split launch sees the same keys");
     static_assert(!PSCALE || !DENSE, "the dial belongs to the general form");
     static_assert(!XTRA || (FORM != kDense && !PSCALE), "key mask, bias and denominators are not in these forms");
+    static_assert(FORM != kFresh || (XTRA && !SPLIT), "only calls under a key mask gain by it");
     using G = HeadGeo<D>;
     using DG = DmaGeo<D>;
     using V8 = typename Mma<T>::v8;
@@ -720,7 +722,7 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
             seg_s = tt * p.split.T + s1;
         }
     }
-    const int Lp = SPLIT ? 0 : p.Lp;      // (LISTED: a third of the key loop's scalar instructions are the choice between prefix and fresh rows)
+    const int Lp = FRESH ? 0 : p.Lp;      // (LISTED: a third of the key loop's scalar instructions are the choice between prefix and fresh rows)
     const int h = bh % p.H;
     const int b = bh / p.H;
     const int q0 = qt * BM;
@@ -730,7 +732,7 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
     const T* const q_base = static_cast<const T*>(p.q) + b * p.q_bs + h * D;
     T* const o_base = static_cast<T*>(p.o) + b * p.o_bs + h * D;
 
-    const int n_keys = RAGGED ? visible_keys(p, b) : p.Lk;   // counts the cached prefix rows, which come first
+    const int n_keys = RAGGED && !SPLIT ? visible_keys(p, b) : p.Lk;   // counts the cached prefix rows, which come first
     int lo = 0, hi = n_keys;   // DENSE: rows past the end of Q repeat its last row and are never stored
     // (rows past the end count as the last row where they share a wavefront with it: as rows without keys they put every tile
     //  of that wavefront on the masked path; 24 heads of 128, 2500 tokens, block-causal: 83.8 -> 74.5 us)
@@ -861,7 +863,7 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
     // head_dim 128 asks once for all loads of a step whether one of the tiles is the last (24 heads with RoPE, 4600 tokens 241.8 -> 239.6 us; under a key
     // mask 48 / 12 heads, 3000 tokens 249 -> 246), but under a key mask with a prefix for each (48 / 12 heads, 200 prefix rows: 1300 tokens 74.9 -> 73.8,
     // 2304 127.0 -> 125.6)
-    constexpr bool EACH = LISTED && !SPLIT;
+    constexpr bool EACH = LISTED && !FRESH;
     auto dma_tiles = [&](bool do_k, int k_off, bool do_v, int v_off) -> int {
         int n = 0;
         if constexpr (DG::NDMA % 8 == 0) {
@@ -1153,7 +1155,7 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
 
     const float l_tot = exchange_sum(st.l);
     const float inv = row_inverse(l_tot);
-    if constexpr (XTRA) {
+    if constexpr (XTRA && !SPLIT) {
         // base-2 log of the row's denominator in exponent units: p(key) = exp2(score * scale_log2 [+ bias * log2 e] - lse);
         // +inf for a row without visible keys, so that every p is 0
         if (p.lse && qvalid && lh == 0)
@@ -1456,17 +1458,9 @@ int launch_d(SdpaDev p, int n_cu, hipStream_t stream) {
                     if (dma && p.key_mask && !p.bias && same_keys_for_all_rows(p) && listed_fits<D>(p)) {
                         p.kbits_off = DmaGeo<D>::lds_bytes();
                         const long lds = DmaGeo<D>::lds_bytes() + listed_bytes_of(p);
-                        if (p.Lp == 0 && n_kt >= 20) {
-                            // the instance of split launches, which looks for no prefix, as one without a tail: about 1.5 % less per key step, 0.7 us
-                            // more to start (with RoPE and K rotation, us: 48 / 12 heads of 128, 435 keys hidden, 768 tokens 22.1 -> 23.0, 1000 28.9 ->
-                            // 29.4, 1300 67.8 -> 67.9, 1700 87.5 -> 86.7, 4928 508 -> 500; 112 hidden, 1100 43.1 -> 43.3, 1300 82.7 -> 82.1; 24 / 6 heads,
-                            // 4608 231 -> 228; 16 of 72, 4096 96.7 -> 95.1, 5376 without a scratch 229 -> 221)
-                            p.split.T = (p.Lk + kBN - 1) / kBN;
-                            p.split.n_blocks = p.n_blocks;
-                            p.split.chunk = (p.n_blocks + 7) / 8;
-                            p.split.cu_g = 1;
-                            hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, true, kRagged, false, true>), dim3(8 * p.split.chunk), block, lds, stream, p);
-                        }
+                        // (without a prefix, with RoPE and K rotation, us, looking for one / not: 48 / 12 heads of 128, 1100 tokens 43.2 / 42.4, 3000 255 / 245,
+                        // 4928 548 / 532, one key visible of 3000 48.0 / 46.9; 16 of 72, 1100 34.5 / 32.9, 3000 76.6 / 72.5)
+                        if (p.Lp == 0) hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, false, kFresh, false, true>), grid, block, lds, stream, p);
                         else hipLaunchKernelGGL((sdpa_fwd_pp_dma_kernel<T, D, false, kRagged, false, true>), grid, block, lds, stream, p);
                     }
                     else if (dma) {

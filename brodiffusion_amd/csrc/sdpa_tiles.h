@@ -122,7 +122,8 @@ struct TileCursor {
 //   kGeneral  any mask: a visible-key interval per query row, K and V of prefix and fresh rows with their own strides
 //   kDense    no mask of any kind and whole key tiles only
 //   kRagged   every query row sees the same keys [0, n) of its batch item, n any number (kv_valid_len included), prefix of any length
-enum { kGeneral = 0, kDense = 1, kRagged = 2 };
+//   kFresh    as kRagged, no prefix (256-row DMA kernel under a key mask)
+enum { kGeneral = 0, kDense = 1, kRagged = 2, kFresh = 3 };
 
 // keys that every query row of batch item b sees, where no mask but kv_valid_len (and a key mask) applies (uniform)
 __device__ __forceinline__ int visible_keys(const SdpaDev& p, int b) {
