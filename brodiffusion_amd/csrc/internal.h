@@ -37,6 +37,7 @@ struct SplitGeo {
     int T, chunk, n_blocks, cu_g;
     int max_tail;   // most tail tiles of any group
     int max_parts;  // partial slots per tail tile
+    int min_visible;  // under a key mask: a query tile with fewer visible key tiles than this is not cut, its first part takes it whole
     static constexpr int kMinPiece = 8;   // shortest piece worth a work group of its own, in steps
     __host__ __device__ int tiles_of(int g) const { const int n = n_blocks - g * chunk; return n < 0 ? 0 : (n > chunk ? chunk : n); }
     __host__ __device__ int full_of(int g) const { return tiles_of(g) / cu_g * cu_g; }

@@ -620,6 +620,14 @@ template <int D> struct DmaGeo {
 // (head_dim 40 works the same way but measured no faster than the register-staged kernel: not instantiated)
 template <int D> constexpr bool dma_kernel_available() { return D == 72 || D == 128; }
 
+// The statistics of a part's scratch slot: 256 references, then 256 denominators; in their place kWholeTile where the first part took the tile
+// whole (LISTED) and wrote the result itself.
+template <int D>
+__device__ __forceinline__ float* part_stats(unsigned char* slot) { return reinterpret_cast<float*>(slot + 256L * D * 4); }
+template <int D>
+__device__ __forceinline__ const float* part_stats(const unsigned char* slot) { return reinterpret_cast<const float*>(slot + 256L * D * 4); }
+constexpr float kWholeTile = -1.f;
+
 __device__ __forceinline__ int swz(int row) { return 4 * (row & 3) + ((row >> 2) & 3); }
 
 // SPLIT: the launch follows p.split — a work group either processes one whole query tile or one piece of the last
@@ -646,10 +654,10 @@ __device__ __forceinline__ int swz(int row) { return 4 * (row & 3) + ((row >> 2)
 // XTRA with kRagged: a key mask but no bias. The mask hides the same keys from every row (the padding of a prompt in
 // the middle of a joint sequence), so the tiles without a visible key are taken out of the walk: `vis` lists the others, and a
 // step looks up the tile that it loads. 48 query / 12 K/V heads of 128, 4608 tokens of which 435 are padding (6 of 72 tiles):
-// 520 -> 472 us; the words used to blank the scores of a hidden tile, whose MFMAs and loads ran all the same. With SPLIT every pass lists
-// the tiles anew and a part [s0, s1) of T tiles takes entries [s0 n / T, s1 n / T) of the n listed ones, so that hidden tiles shorten all parts
-// alike (with RoPE and K rotation, unsplit -> split: the call above 472 -> 447; 24 heads, 435 keys hidden, 2816 tokens 137 -> 109, 3328 162 -> 145,
-// 4096 201 -> 187; 16 heads, 200 hidden, 4608 231 -> 174; 16 heads of 72, 4608 199 -> 140).
+// 520 -> 472 us; the words used to blank the scores of a hidden tile, whose MFMAs and loads ran all the same. With SPLIT a part [s0, s1) of T
+// tiles takes entries [s0 n / T, s1 n / T) of the n listed ones, so that hidden tiles shorten all parts alike; a query tile with fewer than
+// split.min_visible listed ones is not cut: its first part takes it whole and writes the result, the others and the merge have nothing to do
+// (cut all the same, an empty part staged Q and wrote a slot of FP32 like any other: 24 heads of 128, one key visible of 3328, unsplit 37 us, cut 59).
 // F32SUM: see softmax_tile_rel.
 template <typename T, int D, bool SPLIT, int FORM = kGeneral, bool PSCALE = false, bool XTRA = false, bool F32SUM = false>
 __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const SdpaDev p) {
@@ -694,6 +702,38 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
             qt = bh = 0;
         }
     }
+    // XTRA: the visibility words of the key tiles (published by the barrier that ends the prologue). LISTED: behind them the numbers of the tiles
+    // with a visible key, in order; every wavefront writes the whole list (the same values) and reads only what it wrote.
+    const unsigned long long* const kbits = (XTRA && p.key_mask) ? reinterpret_cast<const unsigned long long*>(smem + p.kbits_off) : nullptr;
+    unsigned short* const vis_list = LISTED ? reinterpret_cast<unsigned short*>(smem + p.kbits_off + 8 * ((p.Lk + kBN - 1) / kBN + 2)) : nullptr;
+    int listed_b = -1, n_visible = 0;     // the batch item whose list it is, and its length
+    auto list_tiles = [&](const TilePlan& plan, int b, int wave, int lane) -> int {
+        build_key_bits(p, plan, b, smem + p.kbits_off, wave, lane);
+        __syncthreads();
+        int n = 0;
+        for (int t0 = 0; t0 < plan.n_tiles; t0 += 64) {
+            const bool on = t0 + lane < plan.n_tiles && kbits[t0 + lane] != 0ull;
+            const unsigned long long m = __ballot(on);
+            if (on) vis_list[n + __popcll(m & ((1ull << lane) - 1ull))] = static_cast<unsigned short>(t0 + lane);
+            n += __popcll(m);
+        }
+        n = __builtin_amdgcn_readfirstlane(n);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        return n;
+    };
+    if constexpr (SPLIT && LISTED) {
+        // a piece that begins inside a tile has nothing to do there if the tile is not cut; it reaches into one other tile at most, whose first part it is
+        if (!whole && seg_s % p.split.T != 0) {
+            listed_b = (xg * p.split.chunk + n_full + seg_s / p.split.T) / p.n_q_tiles / p.H;
+            n_visible = list_tiles(TilePlan(0, p.Lk, 0), listed_b, __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6), threadIdx.x & 63);
+            if (n_visible < p.split.min_visible) {
+                seg_s = (seg_s / p.split.T + 1) * p.split.T;
+                if (seg_s >= seg_end) return;
+            }
+        }
+    }
   for (;;) {   // one pass per part (a single pass unless SPLIT)
     // The thread id is made opaque per pass: otherwise every address computation of the prologue and the epilogue,
     // being the same for all parts, is hoisted out of this loop and stays in registers through the key loop.
@@ -722,6 +762,7 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
             seg_s = tt * p.split.T + s1;
         }
     }
+    bool alone = false;                   // LISTED: the first part of a tile that is not cut
     const int Lp = FRESH ? 0 : p.Lp;      // (LISTED: a third of the key loop's scalar instructions are the choice between prefix and fresh rows)
     const int h = bh % p.H;
     const int b = bh / p.H;
@@ -768,32 +809,23 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
     constexpr bool RANGE = SPLIT && !LISTED;
     const TilePlan plan(RANGE ? kv_begin : g_lo == 0x7fffffff ? 0 : g_lo, RANGE ? min(kv_stop, kv_end) : kv_stop, Lp);
     int n_tiles = plan.n_tiles;
-    // XTRA: visibility words of the plan's tiles (made visible to all wavefronts by the barrier that ends the prologue)
-    const unsigned long long* const kbits = (XTRA && p.key_mask) ? reinterpret_cast<const unsigned long long*>(smem + p.kbits_off) : nullptr;
-    if constexpr (XTRA) build_key_bits(p, plan, b, smem + p.kbits_off, wave, lane);
-    // LISTED: tile numbers of the tiles with a visible key, in order, behind the words; every wavefront writes the whole list
-    // (the same values) and reads only what it wrote. vis_t .. vis_t3: the list's entries t .. t + 3 in step t.
-    unsigned short* vis = LISTED ? reinterpret_cast<unsigned short*>(smem + p.kbits_off + 8 * ((p.Lk + kBN - 1) / kBN + 2)) : nullptr;
+    if constexpr (XTRA && !LISTED) build_key_bits(p, plan, b, smem + p.kbits_off, wave, lane);
+    // LISTED: vis_t .. vis_t3 are the list's entries t .. t + 3 in step t
+    const unsigned short* vis = vis_list;
     int vis_t = 0, vis_t1 = 0, vis_t2 = 0, vis_t3 = 0;
     if constexpr (LISTED) {
-        __syncthreads();
-        int n = 0;
-        for (int t0 = 0; t0 < plan.n_tiles; t0 += 64) {
-            const bool on = t0 + lane < plan.n_tiles && kbits[t0 + lane] != 0ull;
-            const unsigned long long m = __ballot(on);
-            if (on) vis[n + __popcll(m & ((1ull << lane) - 1ull))] = static_cast<unsigned short>(t0 + lane);
-            n += __popcll(m);
-        }
-        n_tiles = __builtin_amdgcn_readfirstlane(n);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (!SPLIT || b != listed_b) n_visible = list_tiles(plan, b, wave, lane);
+        listed_b = b;
+        n_tiles = n_visible;
         if constexpr (SPLIT) {
-            // a part is its share of the list (keys counted in tiles: at most 3070 of them, what the LDS holds words for)
             if (!whole) {
-                const int first = kv_begin / kBN * n_tiles / p.split.T, stop = kv_end / kBN * n_tiles / p.split.T;
-                vis += first;
-                n_tiles = stop - first;
+                if (n_visible < p.split.min_visible) alone = true;
+                else {
+                    // a part is its share of the list (keys counted in tiles: at most 3070 of them, what the LDS holds words for)
+                    const int first = kv_begin / kBN * n_visible / p.split.T, stop = kv_end / kBN * n_visible / p.split.T;
+                    vis += first;
+                    n_tiles = stop - first;
+                }
             }
         }
     }
@@ -1161,10 +1193,13 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
         if (p.lse && qvalid && lh == 0)
             p.lse[(static_cast<long>(b) * p.H + h) * p.Lq + qrow] = l_tot > 0.f ? __builtin_amdgcn_logf(l_tot) - st.neg_ref : __builtin_huge_valf();
     }
-    if (!SPLIT || part == nullptr) {
+    if (SPLIT && LISTED && part != nullptr && !alone && n_tiles == 0) {
+        if (tid < BM) part_stats<D>(part)[BM + tid] = 0.f;      // a part without a tile: the merge looks no further
+    } else if (!SPLIT || part == nullptr || alone) {
         stage_output<T, D>(smem, wave * 32 + lq, lh, oacc, inv);
         __syncthreads();
         write_output<T, D, kThreads8>(smem, o_base, p.o_rs, q0, p.Lq, BM, tid);
+        if (SPLIT && LISTED && alone && part != nullptr && tid < BM) part_stats<D>(part)[BM + tid] = kWholeTile;
     } else {
         // the accumulators of the part as the lanes hold them: 16-byte piece (wave D / 8 + c) 64 + lane is head-dim elements
         // 8 c + 4 lh .. + 3 of row 32 wave + lq; then per row the softmax reference (log2 domain) and the denominator relative
@@ -1177,7 +1212,7 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
             slot[c * 64] = f32x4{block[e], block[e + 1], block[e + 2], block[e + 3]};
         }
         if (lh == 0) {
-            float* const stat = reinterpret_cast<float*>(part + static_cast<long>(BM) * D * 4);
+            float* const stat = part_stats<D>(part);
             stat[wave * 32 + lq] = -st.neg_ref;
             stat[BM + wave * 32 + lq] = l_tot;
         }
@@ -1228,19 +1263,20 @@ __global__ void __launch_bounds__(256) sdpa_combine_kernel(const SdpaDev p) {
             asm volatile("" : "+v"(bits));
             return (bits & 0x7fffffffu) == 0u;
         };
+        if (__builtin_bit_cast(unsigned, part_stats<D>(slots)[BM + row]) == __builtin_bit_cast(unsigned, kWholeTile)) return;
         float ref = kNegInf;
         for (int k = 0; k < n_parts; ++k) {
-            const float* stat = reinterpret_cast<const float*>(slots + k * SplitGeo::slot_bytes(D) + static_cast<long>(BM) * D * 4);
+            const float* stat = part_stats<D>(slots + k * SplitGeo::slot_bytes(D));
             if (!empty(stat[BM + row])) ref = fmaxf(ref, stat[row]);
         }
         float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         float lsum = 0.f;
         for (int k = 0; k < n_parts; ++k) {
             const unsigned char* slot = slots + k * SplitGeo::slot_bytes(D);
-            const float* stat = reinterpret_cast<const float*>(slot + static_cast<long>(BM) * D * 4);
-            const f32x4 lo = reinterpret_cast<const f32x4*>(slot)[piece0], hi = reinterpret_cast<const f32x4*>(slot)[piece0 + 32];
+            const float* stat = part_stats<D>(slot);
             const float l = stat[BM + row];
-            if (empty(l)) continue;
+            if (empty(l)) continue;           // (its values may not be written)
+            const f32x4 lo = reinterpret_cast<const f32x4*>(slot)[piece0], hi = reinterpret_cast<const f32x4*>(slot)[piece0 + 32];
             const float w = __builtin_amdgcn_exp2f(stat[row] - ref);
             lsum = __builtin_fmaf(w, l, lsum);
 #pragma unroll
@@ -1271,9 +1307,22 @@ bool listed_fits(const SdpaDev& p) {
 // shortens the last round by more than that — and only when the last round would fill at most half of the GPU:
 // under sustained MFMA load the GPU runs at its power limit, a partly idle last round runs at a higher clock, and
 // measured time follows the total work rather than the number of rounds (432 tiles on 256 compute units take 1.70
-// times one full round, not 2). Measured at head_dim 128 (us, unsplit / split, with RoPE and K rotation; last round of a part in 32): 24 heads, 1.03
-// rounds (1/32) 144.6 / 119.4, 1.22 (7) 166.9 / 154.6, 1.31 (10) 178.9 / 171.5, 1.5 (16) 204.2 / 203.1, 2.25 (8) 459.0 / 417.1, 2.44 (14) 498.8 /
-// 495.4; 32 heads, 2.25 (8) 354.4 / 326.7; 48 heads, 3.19 (6) 463.0 / 444.1, 3.375 (12) 489.5 / 491.5.
+// times one full round, not 2). Both sides (us, unsplit / split, with RoPE and K rotation; rounds, and the last one's share in 32):
+//   dense, 128:  24 heads, 2816 tokens (1.03, 1) 142.6 / 116.6, 3328 (1.22, 7) 164.1 / 151.8, 3584 (1.31, 10) 175.7 / 167.5, 4096 (1.5, 16) 199.3 / 197.6,
+//                6144 (2.25, 8) 449 / 403, 6656 (2.44, 14) 486 / 475; 32 heads, 4608 (2.25, 8) 348 / 316; 48 heads, 4352 (3.19, 6) 454 / 429, 4608
+//                (3.38, 12) 479 / 471
+//   ragged, 128: 24 heads, 2800 (1.03, 1) 147.3 / 120.1, 3300 (1.22, 7) 169.7 / 154.9, 4080 (1.5, 16) 207.5 / 203.0, 6600 (2.44, 14) 499 / 485; 48 heads,
+//                4600 (3.38, 12) 493 / 482
+//   72:          16 heads, 4608 (1.13, 4) 201.3 / 143.7, 4600 203.6 / 145.1; 40 heads, 1792 (1.09, 3) 90.9 / 82.4
+// A key mask may hide tiles, which is known on the GPU only: planned as if all were visible, where that gains twice what an unmasked call has to, and
+// decided there for each batch item. Visible keys: all, half, a quarter, an eighth, one:
+//   48 / 12 heads of 128, 4608 (3.38, 12)  485 / 471, 271 / 277, 164 / 171, 110 / 118, 67 / 75
+//   24 heads of 128, 2816 (1.03, 1)        149.5 / 122.2, 88.4 / 81.0, 58.4 / 63.5, 45.6 / 50.7, 32.9 / 39.3
+//                    3328 (1.22, 7)        172.4 / 157.5, 101.0 / 104.9, 65.1 / 70.8, 49.2 / 55.0, 34.1 / 40.6
+//                    4096 (1.5, 16)        209.2 / 203.6, 121.5 / 125.2, 77.8 / 83.9, 55.7 / 61.9, 38.5 / 44.8
+//   16 heads of 128, 4608 (1.13, 4)        229.3 / 181.1, 130.1 / 114.6, 80.4 / 81.6, 55.7 / 61.1, 35.6 / 41.1
+//   16 heads of 72, 4608 (1.13, 4)         203.6 / 149.4, 113.7 / 95.0, 68.7 / 68.4, 46.6 / 51.4, 28.2 / 33.1
+// Where nothing is cut the launch still takes the merge pass (2.3 us, which then finds nothing to do) and a longer start of every tile (about 1 us at 128).
 template <int D>
 bool plan_split(SdpaDev& p, int n_cu) {
     p.split = SplitGeo{};
@@ -1295,8 +1344,12 @@ bool plan_split(SdpaDev& p, int n_cu) {
     if (tail0 == 0 || 2 * tail0 > g.cu_g) return false;
     const int np0 = g.pieces_for(tail0 * T);
     const int piece_len = (tail0 * T + np0 - 1) / np0;
-    // (a key mask may hide tiles, which is known on the GPU only: it pays from half of them visible on)
     if (T - piece_len < (p.key_mask ? 24 : 12)) return false;
+    // Under a key mask a tile is cut if that shortens it by 12 visible tiles, by 18 where a piece may hold two parts and so starts twice (pieces
+    // that do not divide the tiles evenly). The sides meet at (visible tiles saved): 24 heads, 4096 tokens 12; 16 of 72, 4608 10, of 128 12; 24 heads, 2816 7;
+    // pieces of two parts: 48 / 12 heads, 4608 19; 24 heads, 3328 18.
+    const int pays = np0 % tail0 == 0 ? 12 : 18;
+    g.min_visible = (pays * T + T - piece_len - 1) / (T - piece_len);
     for (int xg = 0; xg < 8; ++xg) {
         const int tail = g.tail_of(xg), S = tail * T, np = g.pieces_for(S);
         g.max_tail = max(g.max_tail, tail);

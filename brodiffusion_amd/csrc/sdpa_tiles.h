@@ -71,12 +71,21 @@ __device__ __forceinline__ void build_key_bits(const SdpaDev& p, const TilePlan&
     if (!p.key_mask) return;
     const float* const km = p.key_mask + b * p.key_mask_bs;
     unsigned long long* const out = reinterpret_cast<unsigned long long*>(dst);
-    for (int t = wave; t < plan.n_tiles; t += n_waves) {
-        const int j = plan.j0(t) + lane;
-        unsigned bits = 0;
-        if (j < plan.limit(t)) bits = __builtin_bit_cast(unsigned, km[j]) & 0x7fffffffu;
-        const unsigned long long w = __ballot(bits != 0u);
-        if (lane == 0) out[t] = w;
+    // the loads of eight tiles are under way together: one by one each waits out the latency, which every query tile pays before its first key tile
+    // (with RoPE and K rotation, 48 / 12 heads of 128, 4608 tokens, one by one / now: one key visible 80.8 / 75.7 us, half of them 286 / 281)
+    constexpr int kBatch = 8;
+    for (int t0 = wave; t0 < plan.n_tiles; t0 += kBatch * n_waves) {
+        unsigned bits[kBatch];
+#pragma unroll
+        for (int i = 0; i < kBatch; ++i) {
+            const int t = min(t0 + i * n_waves, plan.n_tiles - 1), last = plan.limit(t) - 1, j = plan.j0(t) + lane;
+            bits[i] = __builtin_bit_cast(unsigned, km[min(j, last)]) & (j <= last ? 0x7fffffffu : 0u);
+        }
+#pragma unroll
+        for (int i = 0; i < kBatch; ++i) {
+            const unsigned long long w = __ballot(bits[i] != 0u);
+            if (lane == 0 && t0 + i * n_waves < plan.n_tiles) out[t0 + i * n_waves] = w;
+        }
     }
 }
 

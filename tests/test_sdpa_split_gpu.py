@@ -197,3 +197,29 @@ def test_parts_of_the_tiles_that_a_key_mask_leaves(oracle, dtype, B, H, Hkv, d, 
     rows = np.unique(np.concatenate([np.arange(0, Lq, 197), np.arange(255, Lq, 256)])).astype(np.int32)
     for b in range(B):
         assert_close(oracle.sdpa(q[b], rep(k[b]), rep(v[b]), H, key_mask=m[b], rows=rows)[rows], to_np(split[b])[rows], dtype, f"{seen}, batch {b}")
+
+
+@pytest.mark.parametrize("dtype,d", [("bf16", 128), ("fp16", 72)])
+def test_tiles_that_a_key_mask_leaves_uncut(oracle, dtype, d):
+    """Whether a query tile is cut depends on the visible key tiles of its batch item (from 24 of these 40 on); pieces of the last round reach from one
+    item into the next, cut or not. A tile that is not cut has the bits of an unsplit launch."""
+    B, H, Lq, Lk = 4, 11, 1772, 2500         # 308 query tiles: 7 of a group's last round, 3 of the last group's
+    q, k, v = (randn(8171 + i, (B, n, H * d), dtype) for i, n in enumerate((Lq, Lk, Lk)))
+    m = np.zeros((B, Lk), np.float32)
+    m[0, 5:24 * 64:3] = 1                    # 24 tiles
+    m[1, 64:24 * 64] = 1                     # 23
+    m[2] = 1
+    m[3, Lk - 1] = 1
+    dq, dk, dv, dm = to_dev(q, dtype), to_dev(k, dtype), to_dev(v, dtype), torch.from_numpy(m).cuda()
+    for b in range(B):
+        for j in range(0, Lk, 64):
+            if not m[b, j:j + 64].any():
+                dk[b, j:j + 64] = dv[b, j:j + 64] = float("nan")
+    need = split_bytes(dq, dk, dv, H, key_mask=dm.data_ptr(), key_mask_batch_stride=Lk)
+    assert need > 0
+    split = bd.sdpa_forward(dq, dk, dv, H, key_mask=dm, split_scratch=torch.full((need,), 0xFF, dtype=torch.uint8, device="cuda"))
+    plain = bd.sdpa_forward(dq, dk, dv, H, key_mask=dm, split_scratch=False)
+    rows = np.unique(np.concatenate([np.arange(0, Lq, 101), np.arange(255, Lq, 256)])).astype(np.int32)
+    for b, cut in enumerate((True, False, True, False)):
+        assert max_ulp_diff(split[b], plain[b]) <= 2.0 and torch.equal(split[b], plain[b]) != cut, b
+        assert_close(oracle.sdpa(q[b], k[b], v[b], H, key_mask=m[b], rows=rows)[rows], to_np(split[b])[rows], dtype, f"batch {b}")
