@@ -160,6 +160,32 @@ def test_block_scratch_is_what_the_call_can_use(capi):
     assert bd.flash_attention_scratch_bytes(2, 64, 77, 1280, True, 8) == bd.flash_attention_scratch_bytes(2, 64, 77, 1280, True)
 
 
+def test_which_attention_calls_cut_their_last_round(capi):
+    """(No GPU: the planner assumes 256 compute units.) 24 heads of 128, 4096 queries: 384 query tiles, half a round left. Under a key mask from
+    24 key tiles saved on, without one from 12; never with a prefix, a valid length, a bias, the denominators or another mask."""
+    lib = capi.lib()
+
+    def cut(key_tiles, **kw):
+        a = capi.MiSdpaArgs()
+        a.struct_size = C.sizeof(a)
+        a.dtype, a.batch, a.num_heads, a.head_dim, a.q_len, a.kv_len = capi.MI_DTYPE_BF16, 1, 24, 128, 4096, 64 * key_tiles - 5
+        a.q = a.k = a.v = a.o = 0x1000              # never dereferenced
+        for k, v in kw.items():
+            setattr(a, k, v)
+        n = lib.mi_sdpa_split_scratch_bytes(C.byref(a))
+        assert capi.last_error() == ""              # 0 because it does not cut, not because it is refused
+        return n
+    masked = {"key_mask": 0x1000}
+    assert cut(24) > 0 and cut(22) == 0
+    assert cut(48, **masked) > 0 and cut(47, **masked) == 0 < cut(47)
+    assert cut(48, **masked) == cut(48)
+    for no in ({"kv_valid_len": 0x1000}, {"k_prefix": 0x1000, "v_prefix": 0x1000, "prefix_len": 64}, {"lse_out": 0x1000}, {"mask_mode": capi.MI_MASK_CAUSAL},
+               {"logit_bias": 0x1000, "bias_cols": 64, "bias_row_stride": 64}):
+        assert cut(64, **masked, **no) == cut(64, **no) == 0, no
+    # the list of visible tiles has to fit the LDS behind the rings: 2993 tiles at head_dim 128
+    assert cut(2993, **masked) > 0 and cut(2994, **masked) == 0 < cut(2994)
+
+
 def test_python_mirror_refuses_cpu_tensors():
     import torch
     import brodiffusion_amd as bd

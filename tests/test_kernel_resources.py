@@ -56,7 +56,8 @@ def kernels():
     ("linear_pipe_kernel", 54),        # 11 plain forms, 5 GEGLU, 7 of INT8 and 4 of both, by two types
     ("linear_dma_kernel", 2),
     ("sdpa_wide_long_kernel", 2),
-    ("sdpa_fwd_pp_dma_kernelIDF16bLi128ELb1E", 1), ("sdpa_fwd_pp_dma_kernelIDF16_Li72ELb1E", 1),       # split launches
+    *((f"sdpa_fwd_pp_dma_kernelI{t}Li{d}ELb1E", 3) for t in ("DF16_", "DF16b") for d in (72, 128)),      # split launches: dense, ragged, key mask
+    *((f"sdpa_fwd_pp_dma_kernelI{t}Li{d}ELb0ELi3E", 1) for t in ("DF16_", "DF16b") for d in (72, 128)),  # a key mask without prefix
 ])
 def test_kernels_with_loads_in_flight_use_no_scratch(kernels, kernel, at_least):
     found = {name: (k[".private_segment_fixed_size"], k[".vgpr_spill_count"]) for name, k in kernels.items() if kernel in name}

@@ -223,3 +223,28 @@ def test_tiles_that_a_key_mask_leaves_uncut(oracle, dtype, d):
     for b, cut in enumerate((True, False, True, False)):
         assert max_ulp_diff(split[b], plain[b]) <= 2.0 and torch.equal(split[b], plain[b]) != cut, b
         assert_close(oracle.sdpa(q[b], k[b], v[b], H, key_mask=m[b], rows=rows)[rows], to_np(split[b])[rows], dtype, f"batch {b}")
+
+
+@pytest.mark.parametrize("dtype,H,Hkv,d,L,split_half", [("bf16", 24, 6, 128, 2700, False), ("fp16", 24, 6, 128, 2816, True), ("bf16", 16, 16, 72, 4400, False)])
+def test_key_mask_with_rotated_queries_and_keys(oracle, dtype, H, Hkv, d, L, split_half):
+    """A masked block's attention as a program calls it: RoPE on Q as it is loaded (a tile of each part anew), K rotated into a scratch, the padding of
+    the prompt hidden, the last round cut."""
+    q, k, v = randn(8181, (L, H * d), dtype), randn(8182, (L, Hkv * d), dtype), randn(8183, (L, Hkv * d), dtype)
+    angle = np.random.default_rng(8184).uniform(-3, 3, (L, d // 2)).astype(np.float32)
+    cos, sin = np.cos(angle), np.sin(angle)
+    m = np.ones(L, np.float32)
+    m[77:512] = 0
+    dq, dk, dv, dm = to_dev(q, dtype), to_dev(k, dtype), to_dev(v, dtype), torch.from_numpy(m).cuda()
+    tables, kr = (torch.from_numpy(cos).cuda(), torch.from_numpy(sin).cuda()), torch.empty_like(dk)
+    assert split_bytes(dq, dk, dv, H, num_kv_heads=Hkv, key_mask=dm.data_ptr(), key_mask_batch_stride=L) > 0
+
+    def call(**kw):
+        return bd.sdpa_forward(dq, dk, dv, H, num_kv_heads=Hkv, key_mask=dm, rope_q=tables, rope_k=tables, rope_k_scratch=kr, rope_split_half=split_half, **kw)
+    out = call() if split_half else bd.gqa_attention_masked(dq, dk, dv, *tables, d, H, Hkv, dm, Kr=kr)
+    plain = call(split_scratch=False)
+    assert max_ulp_diff(out, plain) <= 2.0 and not torch.equal(out, plain)
+    qr = oracle.rope_apply(q, cos, sin, H, d, split_half=split_half, round_to_dtype=dtype)
+    rep = lambda x: x.reshape(L, Hkv, d).repeat(H // Hkv, axis=1).reshape(L, H * d)
+    kx = rep(oracle.rope_apply(k, cos, sin, Hkv, d, split_half=split_half, round_to_dtype=dtype))
+    rows = np.unique(np.concatenate([np.arange(0, L, 149), np.arange(255, L, 256)])).astype(np.int32)
+    assert_close(oracle.sdpa(qr, kx, rep(v), H, key_mask=m, rows=rows)[rows], to_np(out)[rows], dtype, "rotated, masked, cut")
