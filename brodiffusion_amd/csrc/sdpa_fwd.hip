@@ -632,15 +632,10 @@ __device__ __forceinline__ int swz(int row) { return 4 * (row & 3) + ((row >> 2)
 
 // SPLIT: the launch follows p.split — a work group either processes one whole query tile or one piece of the last
 // round, i.e. one or more (tile, key range) parts in sequence, each leaving a partial result in its scratch slot
-// (merged by sdpa_combine_kernel). Only for calls without prefix and without a mask other than a key mask, in the dense form where the key tiles are
-// whole (ragged -> dense, with RoPE and K rotation: 24 heads of 128, 3328 tokens 154.8 -> 148.9 us, 4096 202.1 -> 194.5, 6656 489.6 -> 471.0, 9472
-// 943.5 -> 895.6; 16 of 72, 4608 tokens 138.0 -> 136.1) and else in the ragged form (in the general form, with
-// its interval per row, the Flux calls below took, head norms and rotation included: bf16, 24 heads of 128, 2816 tokens 139.7 -> 136.6 us, 3328
-// 180.9 -> 176.4, 4096 226.3 -> 222.2; 16 heads, 9216 tokens 633.8 -> 624.1; PixArt block of 16 heads of 72, 4608 tokens 224.6 -> 220.6).
-// The loop over parts keeps nothing of a pass for the next: with the RoPE tables' registers left undefined where there are no tables
-// (QTileLoad::define_tables) it carried them through the key loop, and each table piece was waited for and spilled as it arrived (24 heads of 128
-// with RoPE, K rotation included: 2816 tokens 129.0 -> 119.4 us, 3328 169.4 -> 154.6, 4096 213.5 -> 203.1, 6144 432.9 -> 417.1; 48 heads, 4608
-// 512.9 -> 491.5; without RoPE 3328 147.2 -> 143.1).
+// (merged by sdpa_combine_kernel; plan_split has the times). Only for calls without prefix and without a mask other than a key mask: in the dense form
+// where the key tiles are whole, else in the ragged form (24 heads of 128 with RoPE and K rotation, 4096 tokens: ragged 202.1, dense 194.5 us).
+// The loop over parts keeps nothing of a pass for the next, the RoPE tables' registers included (QTileLoad::define_tables; carried through the key
+// loop they made it spill 21 others, and each table piece was waited for as it arrived: the same call 213.5, without 203.1).
 // FORM kDense: no mask of any kind and key counts (cached prefix, if any, and fresh) that are multiples of 64: every tile is
 // whole and visible to every row, so the masked form of the softmax and the per-step bookkeeping (which tile, its limit,
 // whether this wavefront sees it whole) drop out of the kernel, and with them their registers: measured 6 % faster at
@@ -648,10 +643,11 @@ __device__ __forceinline__ int swz(int row) { return 4 * (row & 3) + ((row >> 2)
 // FORM kRagged: every row sees the same keys, their number is free. All tiles but the last of a segment are as in kDense; that
 // one is met by scalar branches (DMA rows clamped to the last that exists, scores past it blanked). The general form clamps and
 // compares in every step: 24 heads of 128, 2500 tokens 77.5 -> 75.3 us, 16 heads of 72, 3600 tokens 84.0 -> 82.0.
+// FORM kFresh: kRagged without a prefix, for calls under a key mask (the choice between prefix and fresh rows in every step is gone; launch_d has the times).
 // PSCALE: the general form with the prefix-KV dial (factors on the rows of the cached prefix) in its softmax.
 // XTRA: the general form with a key mask (one visibility bit per key, 64-bit words per key tile built once per work group
 // in LDS behind the rings), an additive logit bias and the softmax denominators as an output (traced attention).
-// XTRA with kRagged: a key mask but no bias. The mask hides the same keys from every row (the padding of a prompt in
+// XTRA with kRagged or kFresh: a key mask but no bias. The mask hides the same keys from every row (the padding of a prompt in
 // the middle of a joint sequence), so the tiles without a visible key are taken out of the walk: `vis` lists the others, and a
 // step looks up the tile that it loads. 48 query / 12 K/V heads of 128, 4608 tokens of which 435 are padding (6 of 72 tiles):
 // 520 -> 472 us; the words used to blank the scores of a hidden tile, whose MFMAs and loads ran all the same. With SPLIT a part [s0, s1) of T

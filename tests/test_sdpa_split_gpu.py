@@ -170,8 +170,8 @@ def test_parts_around_the_last_key(oracle, dtype, d, Lk):
 ])
 @pytest.mark.parametrize("seen", ["padding", "few", "one key", "nothing"])
 def test_parts_of_the_tiles_that_a_key_mask_leaves(oracle, dtype, B, H, Hkv, d, Lq, Lk, seen):
-    """Parts are shares of the list of tiles with a visible key, which may be shorter than the parts are many. Tiles without one are not
-    read: NaN there must not matter."""
+    """Parts are shares of the list of tiles with a visible key; where it is short ("few", "one key", "nothing") the first part takes its tile whole.
+    Tiles without a visible key are not read: NaN there must not matter."""
     q = randn(8161, (B, Lq, H * d), dtype)
     k, v = randn(8162, (B, Lk, Hkv * d), dtype), randn(8163, (B, Lk, Hkv * d), dtype)
     m = np.zeros((B, Lk), np.float32)
