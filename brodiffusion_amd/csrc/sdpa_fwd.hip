@@ -731,10 +731,7 @@ __global__ void __launch_bounds__(kThreads8, 2) sdpa_fwd_pp_dma_kernel(const Sdp
         }
     }
   for (;;) {   // one pass per part (a single pass unless SPLIT)
-    // The thread id is made opaque per pass: otherwise every address computation of the prologue and the epilogue,
-    // being the same for all parts, is hoisted out of this loop and stays in registers through the key loop.
-    int tid = threadIdx.x;
-    if constexpr (SPLIT) asm volatile("" : "+v"(tid));
+    const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int grp = wave >> 2;
     const int lane = tid & 63;
@@ -1304,21 +1301,21 @@ bool listed_fits(const SdpaDev& p) {
 // under sustained MFMA load the GPU runs at its power limit, a partly idle last round runs at a higher clock, and
 // measured time follows the total work rather than the number of rounds (432 tiles on 256 compute units take 1.70
 // times one full round, not 2). Both sides (us, unsplit / split, with RoPE and K rotation; rounds, and the last one's share in 32):
-//   dense, 128:  24 heads, 2816 tokens (1.03, 1) 142.6 / 116.6, 3328 (1.22, 7) 164.1 / 151.8, 3584 (1.31, 10) 175.7 / 167.5, 4096 (1.5, 16) 199.3 / 197.6,
-//                6144 (2.25, 8) 449 / 403, 6656 (2.44, 14) 486 / 475; 32 heads, 4608 (2.25, 8) 348 / 316; 48 heads, 4352 (3.19, 6) 454 / 429, 4608
-//                (3.38, 12) 479 / 471
-//   ragged, 128: 24 heads, 2800 (1.03, 1) 147.3 / 120.1, 3300 (1.22, 7) 169.7 / 154.9, 4080 (1.5, 16) 207.5 / 203.0, 6600 (2.44, 14) 499 / 485; 48 heads,
-//                4600 (3.38, 12) 493 / 482
-//   72:          16 heads, 4608 (1.13, 4) 201.3 / 143.7, 4600 203.6 / 145.1; 40 heads, 1792 (1.09, 3) 90.9 / 82.4
+//   dense, 128:  24 heads, 2816 tokens (1.03, 1) 140.1 / 113.9, 3328 (1.22, 7) 162.9 / 149.7, 3584 (1.31, 10) 175.1 / 166.0, 4096 (1.5, 16) 200.0 / 197.7,
+//                6144 (2.25, 8) 448 / 400, 6656 (2.44, 14) 484 / 472; 32 heads, 4608 (2.25, 8) 346 / 314; 48 heads, 4352 (3.19, 6) 455 / 428, 4608
+//                (3.38, 12) 480 / 470
+//   ragged, 128: 24 heads, 2800 (1.03, 1) 145.7 / 117.3, 3300 (1.22, 7) 169.2 / 152.1, 4080 (1.5, 16) 205.5 / 199.3, 6600 (2.44, 14) 498 / 480; 48 heads,
+//                4600 (3.38, 12) 493 / 479
+//   72:          16 heads, 4608 (1.13, 4) 198.9 / 139.6, 4600 201.0 / 141.8; 40 heads, 1792 (1.09, 3) 89.5 / 79.6
 // A key mask may hide tiles, which is known on the GPU only: planned as if all were visible, where that gains twice what an unmasked call has to, and
 // decided there for each batch item. Visible keys: all, half, a quarter, an eighth, one:
-//   48 / 12 heads of 128, 4608 (3.38, 12)  485 / 471, 271 / 277, 164 / 171, 110 / 118, 67 / 75
-//   24 heads of 128, 2816 (1.03, 1)        149.5 / 122.2, 88.4 / 81.0, 58.4 / 63.5, 45.6 / 50.7, 32.9 / 39.3
-//                    3328 (1.22, 7)        172.4 / 157.5, 101.0 / 104.9, 65.1 / 70.8, 49.2 / 55.0, 34.1 / 40.6
-//                    4096 (1.5, 16)        209.2 / 203.6, 121.5 / 125.2, 77.8 / 83.9, 55.7 / 61.9, 38.5 / 44.8
-//   16 heads of 128, 4608 (1.13, 4)        229.3 / 181.1, 130.1 / 114.6, 80.4 / 81.6, 55.7 / 61.1, 35.6 / 41.1
-//   16 heads of 72, 4608 (1.13, 4)         203.6 / 149.4, 113.7 / 95.0, 68.7 / 68.4, 46.6 / 51.4, 28.2 / 33.1
-// Where nothing is cut the launch still takes the merge pass (2.3 us, which then finds nothing to do) and a longer start of every tile (about 1 us at 128).
+//   48 / 12 heads of 128, 4608 (3.38, 12)  484 / 469, 268 / 272, 162 / 168, 110 / 115, 68 / 73
+//   24 heads of 128, 2816 (1.03, 1)        146.7 / 119.1, 87.5 / 79.2, 58.0 / 62.0, 45.2 / 49.2, 33.1 / 37.0
+//                    3328 (1.22, 7)        169.8 / 154.2, 99.6 / 102.2, 64.7 / 69.2, 49.3 / 53.7, 34.5 / 39.0
+//                    4096 (1.5, 16)        206.2 / 200.0, 120.1 / 122.4, 77.2 / 81.9, 55.4 / 60.4, 38.8 / 43.6
+//   16 heads of 128, 4608 (1.13, 4)        224.7 / 178.1, 127.9 / 112.3, 79.2 / 79.9, 55.0 / 59.1, 35.8 / 39.9
+//   16 heads of 72, 4608 (1.13, 4)         200.5 / 145.4, 112.2 / 92.5, 67.7 / 66.6, 46.0 / 49.9, 28.1 / 32.5
+// Where nothing is cut the launch still takes the merge pass (2.3 us, which then finds nothing to do) and a longer start of every tile.
 template <int D>
 bool plan_split(SdpaDev& p, int n_cu) {
     p.split = SplitGeo{};
